@@ -96,6 +96,7 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     ncurves = (int)offsets.size() - 1;
     coff_h = offsets;
     n = offsets.back();
+    longest = 0;
     G = G_;
     ntaps = ntaps_;
     olo = -((ntaps - 1) / 2);
@@ -124,6 +125,7 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     for (int c = 0; c < ncurves; ++c) {
         int nc = offsets[c + 1] - offsets[c];
         require(nc >= 0, "curve offsets must be non-decreasing");
+        longest = std::max(longest, nc);
         int k = (int)ceil_div(nc, CH);
         nch[c] = k;
         base[c] = total_chunks;
@@ -401,11 +403,19 @@ bool Plan<T>::bootstrap_fused_ok(bool window) const {
            (!window || has_pts2);
 }
 
+// partial maxima of |y| per curve: the longest curve's values in at most two
+// rounds of kAbsmaxLoads loads per thread, up to 64 parts
+template <typename T>
+int Plan<T>::ymax_parts() const {
+    const long two_rounds = 2L * kAbsmaxLoads * kAbsmaxThreads;
+    return (int)std::min(64L, std::max(1L, ceil_div(pts.longest, two_rounds)));
+}
+
 template <typename T>
 void Plan<T>::prepare_bootstrap(int nbs, bool window) {
     if (bootstrap_fused_ok(window)) {
         counter.ensure(sizeof(int));
-        ymax.ensure(sizeof(T) * (size_t)ncurves());
+        ymax.ensure(sizeof(T) * (size_t)ncurves() * ymax_parts());
         cover.ensure(sizeof(int) * 2 * (size_t)ncurves());
         return;
     }
@@ -427,12 +437,14 @@ BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t 
         }
         cover_ready = true;
     }
-    if (y) launch_curve_absmax<T>(y, pts.coff.template as<int>(), nc, ymax.as<T>(), s);
+    launch_boot_prepare<T>(y, pts.coff.template as<int>(), nc, ymax_parts(), ymax.as<T>(),
+                           counter.as<int>(), s);
     BootArgs<T> B{};
     B.rec_x = pts.rec_orig.template as<PointRec<T>>();
     B.rec_2x = has_pts2 ? pts2.rec_orig.template as<PointRec<T>>() : nullptr;
     B.y = y;
     B.ymax = ymax.as<T>();
+    B.ymax_parts = ymax_parts();
     B.cover_x = cov;
     B.cover_2x = cov + nc;
     B.coff = pts.coff.template as<int>();

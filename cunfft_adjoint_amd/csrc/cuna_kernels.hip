@@ -578,8 +578,6 @@ static void boot_fused_one(BootArgs<T> A, hipStream_t s) {
         require(A.ls_w != nullptr && A.ls_w_slots >= 1, "Lomb-Scargle workspace missing");
         nblk = std::min(nblk, A.ls_w_slots);
     }
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, s, A.counter);
-    CUNA_LAUNCH_CHECK();
     hipLaunchKernelGGL(k, dim3(nblk), dim3(NT), lds, s, A);
     CUNA_LAUNCH_CHECK();
 }
@@ -597,9 +595,11 @@ void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, in
 }
 
 template <typename T>
-void launch_curve_absmax(const T *y, const int *coff, int ncurves, T *out, hipStream_t s) {
-    if (ncurves <= 0) return;
-    hipLaunchKernelGGL(k_curve_absmax<T>, dim3(ncurves), dim3(256), 0, s, y, coff, out);
+void launch_boot_prepare(const T *y, const int *coff, int ncurves, int parts, T *ymax,
+                         int *counter, hipStream_t s) {
+    const int nblk = y ? ncurves * parts : 1;
+    hipLaunchKernelGGL(k_boot_prepare<T>, dim3(std::max(nblk, 1)), dim3(kAbsmaxThreads), 0, s,
+                       ncurves > 0 ? y : nullptr, coff, parts, ymax, counter);
     CUNA_LAUNCH_CHECK();
 }
 
@@ -649,6 +649,7 @@ template bool boot_fused_supported<dTyp>(int, int);
 template void launch_boot_fused<dTyp>(BootArgs<dTyp>, int, int, int, hipStream_t);
 template void launch_curve_cover<dTyp>(const PointRec<dTyp> *, const int *, int, int, int, int *,
                                        hipStream_t);
-template void launch_curve_absmax<dTyp>(const dTyp *, const int *, int, dTyp *, hipStream_t);
+template void launch_boot_prepare<dTyp>(const dTyp *, const int *, int, int, dTyp *, int *,
+                                        hipStream_t);
 
 }  // namespace cuna

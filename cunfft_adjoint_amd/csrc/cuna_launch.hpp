@@ -89,12 +89,15 @@ void launch_tile_order(const int *bucket, int Kc, int ntiles, int ncurves, bool 
 // fused kernel
 template <typename T>
 bool boot_fused_supported(int lgN, int ntaps);
-// per-curve densest tap window (G <= 2^15) and max |y|
+// per-curve densest tap window (G <= 2^15)
 template <typename T>
 void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, int G, int ntaps,
                         int *cover, hipStream_t s);
 template <typename T>
-void launch_curve_absmax(const T *y, const int *coff, int ncurves, T *out, hipStream_t s);
+// zeroes the work-queue head and, with y, fills `parts` partial maxima of |y|
+// per curve (launched before every fused bootstrap)
+void launch_boot_prepare(const T *y, const int *coff, int ncurves, int parts, T *ymax,
+                         int *counter, hipStream_t s);
 template <typename T>
 // mode 0: spectra of y at x and of the window at 2x; 1: Lomb-Scargle power
 void launch_boot_fused(BootArgs<T> A, int lgN, int ntaps, int mode, hipStream_t s);

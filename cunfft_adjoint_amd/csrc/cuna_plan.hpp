@@ -57,6 +57,7 @@ struct TiledPoints {
     int ncurves = 0;
     long n = 0;
     std::vector<int> coff_h;
+    int longest = 0;  // points of the longest curve
     int G = 0, tlog = 0, ntiles = 0, Kc = 0, olo = 0, ntaps = 0;
     bool periodic = true;
     DevMem arena;  // one allocation; the buffers below are views into it
@@ -165,6 +166,7 @@ struct Plan {
     // the call can be captured into a graph without allocating)
     void prepare_bootstrap(int nbs, bool window);
     bool bootstrap_fused_ok(bool window) const;
+    int ymax_parts() const;
 
     SpreadArgs<T> spread_args(const TiledPoints<T> &P) const;
     BootArgs<T> fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s);
