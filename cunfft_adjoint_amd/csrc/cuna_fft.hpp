@@ -469,42 +469,54 @@ struct LoadGrid {
     __device__ __forceinline__ cplx<T> at(long n) const { return z[n]; }
 };
 
-// Backward (C2R of a Hermitian spectrum): builds Z[q] = E_q + i O_q with
-// E_q = H_q + H_{q+N}, O_q = w_G^{-q} (H_q - H_{q+N}),
-// H_f = (c_f + conj c_{G-f})/2, c_f = D(k) g[M/2 + k] for f = k mod G in band.
+// Backward (C2R of a Hermitian spectrum): Z[q] = E_q + i O_q, 0 <= q < N, with
+//   E_q = H_q + H_{q+N},  O_q = w_G^{-q} (H_q - H_{q+N}),
+//   H_f = (c_f + conj c_{G-f})/2,  c_f = D(k) g[M/2 + k] for f = k mod G, |k| in band.
+// The band reaches |k| <= M/2 <= N/2, and H_{q+N} = conj H_{N-q}.  So at most one
+// of the two terms is non-zero, H_q for q <= N/2 and H_{q+N} above, except at q =
+// N/2 = M/2, where w_G^{-q} = -i makes H_q's term the whole of Z[q] = 2 H_q.
+// With k = min(q, N - q), sigma = +1 for q <= N/2 and -1 above:
+//   Z[q] = (1 + sigma i w_G^{-q}) h,  h = H_k, conjugated above N/2,
+// which takes two values of g, one D(k) and one twiddle.
 template <typename T>
 struct LoadHermitian {
-    static constexpr bool kStage = false;  // heavy loader: twiddles stay in global memory
+    static constexpr bool kStage = true;
     const cplx<T> *g;  // M values, natural order k = -M/2..M/2-1
-    int rot;           // 1: use -i g (the grid then gives the imaginary part)
-    long gstride;      // per batch
-    long M, G, N;
+    int parts;         // 2: batch row 2c + part holds the transform of (part ? -i : 1) g_c,
+                       // whose grid gives the real and the imaginary part
+    int rot;           // 1: this row (with parts = 1, every row) uses -i g
+    long gstride;      // per spectrum
+    int M, N;
     T invG, coef, pref;
     Tw2<T> twG;
-    __device__ __forceinline__ void advance(long b) { g += b * gstride; }
-    __device__ __forceinline__ cplx<T> c(long f) const {
-        long k;
-        if (f < M / 2)
-            k = f;
-        else if (f >= G - M / 2 && f < G)
-            k = f - G;
-        else
-            return cmk(T(0), T(0));
-        T kk = (T)k * invG;
-        T D = pref * dexp(coef * kk * kk);
-        const cplx<T> v = g[M / 2 + k] * D;
-        return rot ? cmk(v.y, -v.x) : v;  // -i v: imaginary part of the forward transform
+    __device__ __forceinline__ void advance(long b) {
+        if (parts == 2) {
+            rot = (int)(b & 1);
+            b >>= 1;
+        }
+        g += b * gstride;
     }
-    __device__ __forceinline__ cplx<T> H(long f) const {
-        long mf = f == 0 ? 0 : G - f;
-        return (c(f) + conjg(c(mf))) * T(0.5);
-    }
-    __device__ __forceinline__ cplx<T> at(long q) const {
-        cplx<T> h0 = H(q), h1 = H(q + N);
-        cplx<T> E = h0 + h1;
-        cplx<T> w = conjg(twG(q));
-        cplx<T> O = w * (h0 - h1);
-        return E + mul_i(O);
+    __device__ __forceinline__ cplx<T> at(long q_) const {
+        const int q = (int)q_, half = M / 2;
+        const bool hi = N - q < q;
+        const int k = hi ? N - q : q;
+        // clamped loads, so that they need no branch; values out of the band
+        // are dropped below
+        const int kc = k < half ? k : half;
+        cplx<T> u = g[half - kc];                            // c_{-k}
+        cplx<T> v = g[half + (kc < half ? kc : half - 1)];   // c_k (none at k = M/2)
+        const cplx<T> w = conjg(twG[q]);
+        if (k >= half) v = cmk(T(0), T(0));
+        if (rot) {
+            u = cmk(u.y, -u.x);
+            v = cmk(v.y, -v.x);
+        }
+        const T kk = (T)k * invG;
+        const T D = pref * dexp(coef * kk * kk) * T(0.5);
+        cplx<T> h = k <= half ? (v + conjg(u)) * D : cmk(T(0), T(0));
+        if (hi) h.y = -h.y;
+        const cplx<T> O = mul_i(w * h);
+        return hi ? h - O : h + O;
     }
 };
 
@@ -734,7 +746,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
 
 // Pass 2, plain: H consecutive rows per workgroup, length-L1 FFT, result
 // X[r2 + L2 r1] stored in natural order.
-template <typename T, int S, int LG1, int H, int NT>
+template <typename T, int S, int LG1, int H, int NT, int MR = 4>
 __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long src_stride,
                                                       int L2, cplx<T> *dst, long dst_stride,
                                                       const cplx<T> *tw, long b0) {
@@ -752,9 +764,9 @@ __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long s
     auto fetch = [&](int e, int h) __attribute__((always_inline)) { return z[(long)(i * H + h) * L1 + e]; };
     if constexpr (TAB) {
         auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
-        lds_fft<T, S, LG1, H, NT>(lds, twl, fetch, hook);
+        lds_fft<T, S, LG1, H, NT, MR>(lds, twl, fetch, hook);
     } else {
-        lds_fft<T, S, LG1, H, NT>(lds, tw, fetch);
+        lds_fft<T, S, LG1, H, NT, MR>(lds, tw, fetch);
     }
     cplx<T> *o = dst + b * dst_stride;
     for (int idx = tid; idx < H * L1; idx += NT) {

@@ -111,11 +111,11 @@ static void run_row_real(const FftShape &sh, const cplx<T> *src, int L2, const S
 template <typename T, int S, int LG1, int H>
 static void run_row_plain(const FftShape &sh, const cplx<T> *src, int L2, cplx<T> *dst,
                           hipStream_t s) {
-    constexpr int NT = fft_threads(LG1, H);
+    constexpr int NT = fft_threads(LG1, H, kRowMr);
     auto &tc = TwiddleCache<T>::get();
     const long N = 1L << sh.lgN;
     size_t lds = (sizeof(cplx<T>) << LG1) * (H + (lds_table(LG1) ? 1 : 0));
-    auto k = k_fft_row_plain<T, S, LG1, H, NT>;
+    auto k = k_fft_row_plain<T, S, LG1, H, NT, kRowMr>;
     set_lds(k, lds);
     require(L2 % H == 0, "fft row split");
     for (long b0 = 0; b0 < sh.batch; b0 += kMaxGridY) {
@@ -276,8 +276,8 @@ void fft_c2r_inverse(const FftShape &sh, const LoadHermitian<T> &ld, cplx<T> *wo
         return;
     }
     const int lg1 = split_lg1(sh.lgN), lg2 = sh.lgN - lg1;
-    const int W = pick_seq<T>(lg2, 1L << lg1, sh.batch, 1, "CUNA_FFT_W", sh.w);
-    const int H = pick_seq<T>(lg1, 1L << lg2, sh.batch, 1, "CUNA_FFT_H", sh.h);
+    const int W = pick_seq<T>(lg2, 1L << lg1, sh.batch, 1, "CUNA_FFT_W", sh.w, num_cus());
+    const int H = pick_seq<T>(lg1, 1L << lg2, sh.batch, 1, "CUNA_FFT_H", sh.h, num_cus());
     dispatch_lg<7, 12>(lg2, [&](auto c) {
         constexpr int LG2 = decltype(c)::value;
         dispatch_w<T, LG2>(W, [&](auto w) {
@@ -313,8 +313,8 @@ void fft_complex(const FftShape &sh, cplx<T> *data, cplx<T> *work, int sign, hip
         return;
     }
     const int lg1 = split_lg1(sh.lgN), lg2 = sh.lgN - lg1;
-    const int W = pick_seq<T>(lg2, 1L << lg1, sh.batch, 1, "CUNA_FFT_W", sh.w);
-    const int H = pick_seq<T>(lg1, 1L << lg2, sh.batch, 1, "CUNA_FFT_H", sh.h);
+    const int W = pick_seq<T>(lg2, 1L << lg1, sh.batch, 1, "CUNA_FFT_W", sh.w, num_cus());
+    const int H = pick_seq<T>(lg1, 1L << lg2, sh.batch, 1, "CUNA_FFT_H", sh.h, num_cus());
     dispatch_lg<7, 12>(lg2, [&](auto c) {
         constexpr int LG2 = decltype(c)::value;
         dispatch_w<T, LG2>(W, [&](auto w) {
@@ -529,21 +529,40 @@ void launch_tile_order(const int *bucket, int Kc, int ntiles, int ncurves, bool 
     CUNA_LAUNCH_CHECK();
 }
 
+template <typename T, int NTP, int NG>
+static void gather_one(GatherArgs<T> A, int nslabs, long npts, hipStream_t s) {
+    // tiles per workgroup: on average at most one point per thread, LDS for
+    // 4096 cells, and still a few workgroups per CU
+    const long slots = (long)nslabs * A.ntiles;
+    const long per_tile = std::max(1L, npts / std::max(1L, slots));
+    int gl = 0;
+    while (gl < 4 && (per_tile << (gl + 1)) <= 256 && A.tlog + gl + 1 <= 12 &&
+           (1 << (gl + 1)) <= A.ntiles && (slots >> (gl + 1)) >= 4L * num_cus())
+        ++gl;
+    A.glog = gl;
+    const size_t lds = NG * sizeof(T) * (((size_t)1 << (A.tlog + gl)) + NTP);
+    require(lds <= kMaxLds, "gather tile too large", CUNA_ERROR_UNSUPPORTED);
+    auto k = k_gather<T, NTP, NG>;
+    set_lds(k, lds);
+    const int nblk = (int)ceil_div(A.ntiles, 1L << gl);
+    for (int s0 = 0; s0 < nslabs; s0 += kMaxGridY) {
+        GatherArgs<T> B = A;
+        B.slab0 = s0;
+        hipLaunchKernelGGL(k, dim3(nblk, std::min(kMaxGridY, nslabs - s0)), dim3(256), lds, s, B);
+        CUNA_LAUNCH_CHECK();
+    }
+}
+
 template <typename T>
-void launch_gather(const GatherArgs<T> &A, int ntaps, int nslabs, hipStream_t s) {
+void launch_gather(const GatherArgs<T> &A, int ntaps, int nslabs, int ngrids, long npts,
+                   hipStream_t s) {
     require(ntaps % 2 == 0, "unsupported filter width", CUNA_ERROR_UNSUPPORTED);
     dispatch_m<2, kMaxTaps / 2>(ntaps / 2, [&](auto c) {
         constexpr int NTP = decltype(c)::value;
-        size_t lds = sizeof(T) * (((size_t)1 << A.tlog) + NTP);
-        auto k = k_gather<T, NTP>;
-        set_lds(k, lds);
-        for (int s0 = 0; s0 < nslabs; s0 += kMaxGridY) {
-            GatherArgs<T> B = A;
-            B.slab0 = s0;
-            hipLaunchKernelGGL(k, dim3(A.ntiles, std::min(kMaxGridY, nslabs - s0)), dim3(256),
-                               lds, s, B);
-            CUNA_LAUNCH_CHECK();
-        }
+        if (ngrids == 2)
+            gather_one<T, NTP, 2>(A, nslabs, npts, s);
+        else
+            gather_one<T, NTP, 1>(A, nslabs, npts, s);
     });
 }
 
@@ -643,7 +662,7 @@ template void launch_buckets<dTyp>(const int *, int, int, const PointRec<dTyp> *
                                    int *, hipStream_t);
 template void launch_spread<dTyp>(const SpreadArgs<dTyp> &, int, int, int, hipStream_t, hipEvent_t,
                                   hipEvent_t);
-template void launch_gather<dTyp>(const GatherArgs<dTyp> &, int, int, hipStream_t);
+template void launch_gather<dTyp>(const GatherArgs<dTyp> &, int, int, int, long, hipStream_t);
 template void launch_tile_cover<dTyp>(const SpreadArgs<dTyp> &, int, int *, hipStream_t);
 template bool boot_fused_supported<dTyp>(int, int);
 template void launch_boot_fused<dTyp>(BootArgs<dTyp>, int, int, int, hipStream_t);

@@ -77,7 +77,10 @@ template <typename T>
 void launch_spread(const SpreadArgs<T> &A, int ntaps, int vm, int nslabs, hipStream_t s,
                    hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 template <typename T>
-void launch_gather(const GatherArgs<T> &A, int ntaps, int nslabs, hipStream_t s);
+// ngrids real grids per slab (2: their sums are the parts of one complex
+// output); npts: points of all slabs (for the launch shape)
+void launch_gather(const GatherArgs<T> &A, int ntaps, int nslabs, int ngrids, long npts,
+                   hipStream_t s);
 // per (curve, tile) point cover of the spread's scale (A: rec, bucket, tiles)
 template <typename T>
 void launch_tile_cover(const SpreadArgs<T> &A, int ncurves, int *cover, hipStream_t s);

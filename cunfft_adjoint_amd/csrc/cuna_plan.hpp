@@ -169,6 +169,8 @@ struct Plan {
     int ymax_parts() const;
 
     SpreadArgs<T> spread_args(const TiledPoints<T> &P) const;
+    GatherArgs<T> gather_args() const;
+    void spectrum_to_grid(const cplx<T> *g, int parts, int rot, hipStream_t s);
     BootArgs<T> fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s);
     void run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s,
                  hipEvent_t mid = nullptr) const;

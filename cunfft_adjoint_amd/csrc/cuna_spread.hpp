@@ -1635,66 +1635,90 @@ __global__ void k_curve_cover(const PointRec<T> *rec, const int *coff, int G, in
 }
 
 // ----------------------------------------------------------- gather --
-// Transpose of the accurate spread, for the backward pass: for each point of
-// a tile, sum_o w(o) h[a+o] and sum_o (o - e) w(o) h[a+o] over the real grid h.
+// Transpose of the accurate spread, for the backward and the forward transform:
+// for each point, sum_o w(o) h[a+o] and sum_o (o - e) w(o) h[a+o] over the real
+// grid h; with NG = 2 grids per curve (forward) the first sum over both, as the
+// real and imaginary part of one complex value.
 template <typename T>
 struct GatherArgs {
     const PointRec<T> *rec;
     const int *perm;
     const int *bucket;
-    const T *h;         // real grid per slab (slab = curve * nrep + rep)
+    const T *h;         // NG real grids of G cells per slab (slab = curve * nrep + rep)
     long h_stride;
     const T *y;         // values (for d/dx), nullable -> 1
     long y_stride;      // per rep
-    T *dy;              // nullable
+    T *dy;              // nullable (NG = 2: interleaved complex values)
     T *dx;              // nullable
     long out_stride;    // per rep
     int dy_elem;        // element stride of dy (2: one part of an interleaved complex array)
     int G, tlog, ntiles, Kc, olo, nrep;
+    int glog;  // a workgroup takes 2^glog consecutive tiles
     int slab0;  // slab of blockIdx.y = 0
     T bi, wscale, dxscale;  // dxscale = 2 G / beta
     T e3[kMaxTaps];
 };
 
-template <typename T, int NTAPS>
+// A workgroup stages the cells of its tiles (and the taps' halo) in LDS, then
+// takes their points, which are adjacent in the sorted order.  2^glog tiles
+// share a workgroup so that its threads have a point each: one 256-cell tile
+// per workgroup left 85 % of the threads idle at 20,000 points on 2^17 cells.
+template <typename T, int NTAPS, int NG>
 __global__ __launch_bounds__(256) void k_gather(GatherArgs<T> A) {
     constexpr int NT = 256;
     constexpr int Q0 = (NTAPS - 1) / 2;
-    const int TT = 1 << A.tlog;
-    T *hs = reinterpret_cast<T *>(cuna_smem);  // cells tstart-Q0 .. tstart+TT-Q0+NTAPS-1
-    const int tile = xcd_remap(blockIdx.x, A.ntiles);
+    struct alignas(NG * sizeof(T)) Cell {
+        T v[NG];
+    };
+    Cell *hs = reinterpret_cast<Cell *>(cuna_smem);  // cells tstart-Q0 .. tstart+span-Q0-1
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
     const int slab = A.slab0 + blockIdx.y;
     const int c = slab / A.nrep, rep = slab % A.nrep;
     const int *bk = A.bucket + (long)c * (A.Kc + 1);
-    const int tstart = tile << A.tlog;
-    const T *h = A.h + (long)slab * A.h_stride;
-    const int span = TT + NTAPS;
+    const int tile0 = blk << A.glog, tile1 = min(tile0 + (1 << A.glog), A.ntiles);
+    const int tstart = tile0 << A.tlog;
+    const T *h = A.h + (long)slab * NG * A.h_stride;
+    const int span = ((tile1 - tile0) << A.tlog) + NTAPS;
     for (int i = threadIdx.x; i < span; i += NT) {
-        int cell = (tstart - Q0 + i) % A.G;
-        if (cell < 0) cell += A.G;
-        hs[i] = h[cell];
+        int cell = tstart - Q0 + i;
+        if (cell < 0 || cell >= A.G) {
+            cell %= A.G;
+            if (cell < 0) cell += A.G;
+        }
+        Cell v;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) v.v[k] = h[k * A.h_stride + cell];
+        hs[i] = v;
     }
+    const long s0 = bk[3 * tile0], send = bk[3 * tile1];
     __syncthreads();
-    const long send = bk[3 * tile + 3];
-    for (long s = bk[3 * tile] + threadIdx.x; s < send; s += NT) {
-        const PointRec<T> pr = A.rec[s];
+    for (long s = s0 + threadIdx.x; s < send; s += NT) {
         const int p = A.perm[s];
+        const PointRec<T> pr = A.rec[s];
         const T e = pr.e;
         const int rel = pr.a - tstart;  // hs index of tap q is rel + q
         T w[NTAPS];
         tap_weights<T, NTAPS>(A.wscale, e, A.bi, A.e3, w);
-        T sw = T(0), sd = T(0);
+        T sw[NG] = {}, sd = T(0);
 #pragma unroll
         for (int q = 0; q < NTAPS; ++q) {
-            const T hv = hs[rel + q] * w[q];
-            sw += hv;
-            sd += ((T)(q - Q0) - e) * hv;
+            const Cell hv = hs[rel + q];
+#pragma unroll
+            for (int k = 0; k < NG; ++k) {
+                const T t = hv.v[k] * w[q];
+                sw[k] += t;
+                if constexpr (NG == 1) sd += ((T)(q - Q0) - e) * t;
+            }
         }
         const long oo = (long)rep * A.out_stride;
-        if (A.dy) A.dy[oo + (long)p * A.dy_elem] = sw;
-        if (A.dx) {
-            const T v = A.y ? A.y[(long)rep * A.y_stride + p] : T(1);
-            A.dx[oo + p] = A.dxscale * v * sd;
+        if constexpr (NG == 2) {
+            reinterpret_cast<cplx<T> *>(A.dy)[oo + p] = cmk(sw[0], sw[1]);
+        } else {
+            if (A.dy) A.dy[oo + (long)p * A.dy_elem] = sw[0];
+            if (A.dx) {
+                const T v = A.y ? A.y[(long)rep * A.y_stride + p] : T(1);
+                A.dx[oo + p] = A.dxscale * v * sd;
+            }
         }
     }
 }
