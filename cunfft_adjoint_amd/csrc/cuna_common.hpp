@@ -130,6 +130,18 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
     return (bid % kNumXcd) * per + bid / kNumXcd;
 }
 
+// (block, slab) of workgroup (bx, by) of an nx x ny grid whose slabs (curves of
+// a batch) are independent.  Slabs in groups of eight go one to an XCD, so that
+// all blocks of a slab share one L2; the blocks of the slabs left over are
+// spread over the XCDs as by xcd_remap.
+__device__ __forceinline__ int2 xcd_block(int bx, int by, int nx, int ny) {
+    const int grouped = ny & ~(kNumXcd - 1);
+    if (by >= grouped) return make_int2(xcd_remap(bx, nx), by);
+    // eight slabs hold 8 nx workgroups with ids l in dispatch order, XCD l % 8
+    const int l = (by & (kNumXcd - 1)) * nx + bx;
+    return make_int2(l / kNumXcd, (by & ~(kNumXcd - 1)) + (l & (kNumXcd - 1)));
+}
+
 inline int ilog2(long v) {
     int r = 0;
     while ((1L << r) < v) r++;

@@ -605,8 +605,9 @@ __global__ __launch_bounds__(NT) void k_fft_col(Loader ld, cplx<T> *dst, long ds
     cplx<T> *twl = lds + W * L2;
     const int tid = threadIdx.x;
     const int nblk = L1 / W;
-    const int blk = xcd_remap(blockIdx.x, nblk);
-    const long b = b0 + blockIdx.y;  // launches span at most kMaxGridY batches
+    const int2 bs = xcd_block(blockIdx.x, blockIdx.y, nblk, gridDim.y);
+    const int blk = bs.x;
+    const long b = b0 + bs.y;  // launches span at most kMaxGridY batches
     const int n10 = blk * W;
     Loader lb = ld;
     lb.advance(b);
@@ -671,8 +672,9 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
     cplx<T> *twl = lds + W * L1;
     const int tid = threadIdx.x;
     const int nblk = L2 / (2 * H);
-    const int i = xcd_remap(blockIdx.x, nblk);
-    const long b = b0 + blockIdx.y;  // launches span at most kMaxGridY batches
+    const int2 bs = xcd_block(blockIdx.x, blockIdx.y, nblk, gridDim.y);
+    const int i = bs.x;
+    const long b = b0 + bs.y;  // launches span at most kMaxGridY batches
     const long N = (long)L1 * L2;
     const cplx<T> *z = src + b * src_stride;
     TableStage<T, (TAB ? L1 : 1), NT> tab;
@@ -756,8 +758,9 @@ __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long s
     cplx<T> *twl = lds + H * L1;
     const int tid = threadIdx.x;
     const int nblk = L2 / H;
-    const int i = xcd_remap(blockIdx.x, nblk);
-    const long b = b0 + blockIdx.y;  // launches span at most kMaxGridY batches
+    const int2 bs = xcd_block(blockIdx.x, blockIdx.y, nblk, gridDim.y);
+    const int i = bs.x;
+    const long b = b0 + bs.y;  // launches span at most kMaxGridY batches
     const cplx<T> *z = src + b * src_stride;
     TableStage<T, (TAB ? L1 : 1), NT> tab;
     if constexpr (TAB) tab.load(tw, tid);

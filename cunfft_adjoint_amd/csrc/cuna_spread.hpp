@@ -997,17 +997,20 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
     Acc *acc = acc_all + wave * NC;
     T *facc = facc_all + wave * TT;
 
-    const int slab = A.slab0 + blockIdx.y;
+    // (entry of the work order, slab); a few slabs keep the order as it is
+    const int2 bs = gridDim.y < kNumXcd ? make_int2(blockIdx.x, blockIdx.y)
+                                        : xcd_block(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
+    const int slab = A.slab0 + bs.y;
     const int c = slab / A.nrep, rep = slab % A.nrep;
     TileRanges R;
     int cover = CAP;
     if (A.tile_desc) {
-        const TileDesc d = ldc_desc(A.tile_desc + (long)c * A.ntiles + blockIdx.x);
+        const TileDesc d = ldc_desc(A.tile_desc + (long)c * A.ntiles + bs.x);
         R.from_desc(A, d, NTAPS);
         cover = d.cover;
     } else {
-        R.init(A, blockIdx.x, c, NTAPS);
-        if (A.tile_cover) cover = A.tile_cover[(long)c * A.ntiles + blockIdx.x];
+        R.init(A, bs.x, c, NTAPS);
+        if (A.tile_cover) cover = A.tile_cover[(long)c * A.ntiles + bs.x];
     }
     const int total = R.total;
     const bool multi = total > CAP;
@@ -1671,8 +1674,8 @@ __global__ __launch_bounds__(256) void k_gather(GatherArgs<T> A) {
         T v[NG];
     };
     Cell *hs = reinterpret_cast<Cell *>(cuna_smem);  // cells tstart-Q0 .. tstart+span-Q0-1
-    const int blk = xcd_remap(blockIdx.x, gridDim.x);
-    const int slab = A.slab0 + blockIdx.y;
+    const int2 bs = xcd_block(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
+    const int blk = bs.x, slab = A.slab0 + bs.y;
     const int c = slab / A.nrep, rep = slab % A.nrep;
     const int *bk = A.bucket + (long)c * (A.Kc + 1);
     const int tile0 = blk << A.glog, tile1 = min(tile0 + (1 << A.glog), A.ntiles);
