@@ -90,6 +90,18 @@ __global__ void k_compose(int *perm, const int *idx, long n) {
 }
 
 // ------------------------------------------------------------ TiledPoints --
+namespace {
+// offsets of 256-byte aligned pieces of one allocation
+struct Carve {
+    size_t total = 0;
+    size_t add(size_t b) {
+        const size_t o = total;
+        total += (b + 255) & ~size_t(255);
+        return o;
+    }
+};
+}  // namespace
+
 template <typename T>
 void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int G_, int tlog_,
                            int ntaps_, bool periodic_, bool keep_eps, hipStream_t s) {
@@ -113,46 +125,19 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
         ntiles = 1;
     }
     Kc = 3 * ntiles;
-    const int K1 = 1 << tlog;
-
-    // chunk table: chunks of at most CH points, never crossing a curve.  One
-    // wave ranks a chunk against per-chunk counts of every key: 512 points
-    // for the 256-key passes, up to 2048 for larger tiles (first digit)
-    const int CH = std::max(512, std::min(2048, 2 * K1));
-    std::vector<int4> chunks;
-    std::vector<int> base(ncurves), nch(ncurves);
-    int total_chunks = 0;
     for (int c = 0; c < ncurves; ++c) {
-        int nc = offsets[c + 1] - offsets[c];
+        const int nc = offsets[c + 1] - offsets[c];
         require(nc >= 0, "curve offsets must be non-decreasing");
         longest = std::max(longest, nc);
-        int k = (int)ceil_div(nc, CH);
-        nch[c] = k;
-        base[c] = total_chunks;
-        for (int q = 0; q < k; ++q) {
-            int st = offsets[c] + q * CH;
-            chunks.push_back(make_int4(c, st, std::min(CH, offsets[c + 1] - st), q));
-        }
-        total_chunks += k;
     }
-    const long hist_len = (long)std::max(K1, 256) * std::max(total_chunks, 1);
     // work-queue order of the curves for the fused batched kernels
     std::vector<int> ord(ncurves);
     for (int c = 0; c < ncurves; ++c) ord[c] = c;
     std::stable_sort(ord.begin(), ord.end(), [&](int u, int v) {
         return offsets[u + 1] - offsets[u] > offsets[v + 1] - offsets[v];
     });
-    // device memory in two allocations, the plan's buffers and the sort's
-    // stream-ordered temporaries, each filled by one upload: allocation and
-    // copy calls are most of a plan build's host time
-    struct Carve {
-        size_t total = 0;
-        size_t add(size_t b) {
-            const size_t o = total;
-            total += (b + 255) & ~size_t(255);
-            return o;
-        }
-    };
+    // the plan's device memory in one allocation, filled by one upload:
+    // allocation and copy calls are most of a plan build's host time
     const long n1 = std::max<long>(n, 1);
     const size_t ncov = (size_t)std::max(ncurves, 1) * std::max(ntiles, 1);
     Carve pc;
@@ -162,7 +147,6 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     const size_t o_orig = pc.add(sizeof(PointRec<T>) * n1);
     const size_t o_bk = pc.add(sizeof(int) * (size_t)ncurves * (Kc + 1));
     const size_t o_eps = keep_eps ? pc.add(sizeof(T) * n1) : 0;
-    const size_t o_cov = pc.add(sizeof(int) * ncov);
     const size_t o_desc = pc.add(sizeof(TileDesc) * ncov);
     arena.alloc(pc.total);
     char *pb = arena.as<char>();
@@ -178,12 +162,63 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     } else {
         eps_orig.release();
     }
-    tile_cover.view(pb + o_cov, sizeof(int) * ncov);
     tile_desc.view(pb + o_desc, sizeof(TileDesc) * ncov);
     plan_h.assign(offsets.begin(), offsets.end());
     plan_h.insert(plan_h.end(), ord.begin(), ord.end());
     CUNA_HIP(hipMemcpyAsync(pb + o_up, plan_h.data(), sizeof(int) * plan_h.size(),
                             hipMemcpyHostToDevice, s));
+    A.n = n;
+    A.G = G;
+    A.rec = rec_orig.as<PointRec<T>>();
+    // phase reduction / compat decisions, then the sort by anchor
+    launch_point_setup<T>(A, s);
+    if (!launch_plan_curves<T>(rec_orig.as<PointRec<T>>(), coff.as<int>(), ncurves, longest, tlog,
+                               G, Kc, olo, olo + ntaps - 1, rec.as<PointRec<T>>(), perm.as<int>(),
+                               bucket.as<int>(), s))
+        sort_points(s);
+    // the spread's work order, with each tile's cover (bounds the sums any
+    // cell receives)
+    SpreadArgs<T> C{};
+    C.rec = rec.as<PointRec<T>>();
+    C.bucket = bucket.as<int>();
+    C.coff = coff.as<int>();
+    C.G = G;
+    C.tlog = tlog;
+    C.ntiles = ntiles;
+    C.Kc = Kc;
+    C.olo = olo;
+    C.ntaps = ntaps;
+    C.periodic = periodic ? 1 : 0;
+    C.wrap1 = (periodic && ntiles == 1) ? 1 : 0;
+    launch_tile_order<T>(C, ncurves, tile_desc.as<TileDesc>(), s);
+}
+
+// Sort and buckets of curves of any length, in several launches.
+template <typename T>
+void TiledPoints<T>::sort_points(hipStream_t s) {
+    const std::vector<int> &offsets = coff_h;
+    const int K1 = 1 << tlog;
+    // chunk table: chunks of at most CH points, never crossing a curve.  One
+    // wave ranks a chunk against per-chunk counts of every key: 512 points
+    // for the 256-key passes, up to 2048 for larger tiles (first digit)
+    const int CH = std::max(512, std::min(2048, 2 * K1));
+    std::vector<int4> chunks;
+    std::vector<int> base(ncurves), nch(ncurves);
+    int total_chunks = 0;
+    for (int c = 0; c < ncurves; ++c) {
+        int nc = offsets[c + 1] - offsets[c];
+        int k = (int)ceil_div(nc, CH);
+        nch[c] = k;
+        base[c] = total_chunks;
+        for (int q = 0; q < k; ++q) {
+            int st = offsets[c] + q * CH;
+            chunks.push_back(make_int4(c, st, std::min(CH, offsets[c + 1] - st), q));
+        }
+        total_chunks += k;
+    }
+    const long hist_len = (long)std::max(K1, 256) * std::max(total_chunks, 1);
+    const long n1 = std::max<long>(n, 1);
+    // the sort's stream-ordered temporaries, in one allocation
     Carve tc;
     const size_t o_chunks = tc.add(sizeof(int4) * std::max<size_t>(chunks.size(), 1));
     const size_t o_base = tc.add(sizeof(int) * ncurves);
@@ -216,15 +251,10 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     W.total_chunks = total_chunks;
     W.hist = reinterpret_cast<int *>(tb + o_hist);
     W.bsum = reinterpret_cast<int *>(tb + o_bsum);
-    // phase reduction / compat decisions, then an LSD sort by anchor: the cell
-    // within the tile, then the tile index in digits of at most 8 bits; the
-    // passes alternate between rec/perm and recA/permA, ending in rec/perm
-    A.n = n;
-    A.G = G;
-    A.tlog = tlog;
-    A.rec = rec_orig.as<PointRec<T>>();
-    A.key = keys;
-    launch_point_setup<T>(A, s);
+    // an LSD sort by anchor: the cell within the tile, then the tile index in
+    // digits of at most 8 bits; the passes alternate between rec/perm and
+    // recA/permA, ending in rec/perm
+    launch_digit_keys<T>(rec_orig.as<PointRec<T>>(), n, 0, K1 - 1, keys, s);
     const int tbits = ilog2(ntiles);
     const int npass = 1 + (tbits + 7) / 8;
     PointRec<T> *const rbuf[2] = {rec.as<PointRec<T>>(), recA};
@@ -240,24 +270,6 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     }
     launch_buckets<T>(coff.as<int>(), ncurves, Kc, rec.as<PointRec<T>>(), tlog, olo,
                       olo + ntaps - 1, G, bucket.as<int>(), s);
-    // the spread's per-tile cover (bounds the sums any cell receives)
-    {
-        SpreadArgs<T> C{};
-        C.rec = rec.as<PointRec<T>>();
-        C.bucket = bucket.as<int>();
-        C.coff = coff.as<int>();
-        C.G = G;
-        C.tlog = tlog;
-        C.ntiles = ntiles;
-        C.Kc = Kc;
-        C.olo = olo;
-        C.ntaps = ntaps;
-        C.periodic = periodic ? 1 : 0;
-        C.wrap1 = (periodic && ntiles == 1) ? 1 : 0;
-        launch_tile_cover<T>(C, ncurves, tile_cover.as<int>(), s);
-        launch_tile_order(bucket.as<int>(), Kc, ntiles, ncurves, periodic, tile_cover.as<int>(),
-                          tile_desc.as<TileDesc>(), s);
-    }
 }
 
 // --------------------------------------------------------------- Plan --
@@ -283,7 +295,6 @@ SpreadArgs<T> Plan<T>::spread_args(const TiledPoints<T> &P) const {
     A.bi = T(1) / beta;
     A.wscale = wscale;
     A.cpar = cpar_c;
-    A.tile_cover = P.tile_cover.template as<int>();
     A.tile_desc = P.tile_desc.template as<TileDesc>();
     for (int q = 0; q < kMaxTaps; ++q) A.e3[q] = e3[q];
     return A;

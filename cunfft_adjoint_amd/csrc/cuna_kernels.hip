@@ -502,31 +502,51 @@ void launch_spread(const SpreadArgs<T> &A, int ntaps, int vm, int nslabs, hipStr
 }
 
 template <typename T>
-void launch_tile_cover(const SpreadArgs<T> &A, int ncurves, int *cover, hipStream_t s) {
+void launch_tile_order(const SpreadArgs<T> &A, int ncurves, TileDesc *desc, hipStream_t s) {
     if (ncurves <= 0 || A.ntiles <= 0) return;
-    const size_t lds = sizeof(int) * (((size_t)1 << A.tlog) + 2 * (size_t)A.ntaps);
+    require(A.ntiles <= kOrderMaxTiles, "too many spread tiles for the work order",
+            CUNA_ERROR_UNSUPPORTED);
+    hipLaunchKernelGGL(k_tile_order, dim3(ncurves), dim3(kOrderThreads), 0, s, A.bucket, A.Kc,
+                       A.ntiles, desc);
+    CUNA_LAUNCH_CHECK();
+    const size_t lds = sizeof(int) * kDescWaves * (((size_t)1 << A.tlog) + 2 * (size_t)A.ntaps + 1);
     require(lds <= kMaxLds, "spread tile too large", CUNA_ERROR_UNSUPPORTED);
-    set_lds(k_tile_cover<T>, lds);
-    for (int c0 = 0; c0 < ncurves; c0 += kMaxGridY) {  // blockIdx.y = curve - slab0
-        SpreadArgs<T> B = A;
-        B.slab0 = c0;
-        hipLaunchKernelGGL(k_tile_cover<T>, dim3(A.ntiles, std::min(kMaxGridY, ncurves - c0)),
-                           dim3(256), lds, s, B, cover);
-        CUNA_LAUNCH_CHECK();
-    }
+    set_lds(k_tile_desc<T>, lds);
+    const long npos = (long)ncurves * A.ntiles;
+    hipLaunchKernelGGL(k_tile_desc<T>, dim3(ceil_div(npos, kDescWaves)), dim3(64 * kDescWaves), lds,
+                       s, A, npos, desc);
+    CUNA_LAUNCH_CHECK();
 }
 
-void launch_tile_order(const int *bucket, int Kc, int ntiles, int ncurves, bool periodic,
-                       const int *cover, TileDesc *desc, hipStream_t s) {
-    if (ncurves <= 0 || ntiles <= 0) return;
-    require(ntiles <= kOrderMaxTiles, "too many spread tiles for the work order",
-            CUNA_ERROR_UNSUPPORTED);
-    hipLaunchKernelGGL(k_tile_order, dim3(ncurves), dim3(kOrderThreads), 0, s, bucket, Kc, ntiles,
-                       desc);
-    CUNA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_tile_desc, dim3(ceil_div(ntiles, 256) * ncurves), dim3(256), 0, s, bucket,
-                       Kc, ntiles, periodic ? 1 : 0, cover, desc);
-    CUNA_LAUNCH_CHECK();
+// sort and buckets of short curves in one launch; false when a curve is too
+// long or its (anchor, index) pairs too wide for it
+template <typename T>
+bool launch_plan_curves(const PointRec<T> *rec_orig, const int *coff, int ncurves, int longest,
+                        int tlog, int G, int Kc, int olo, int ohi, PointRec<T> *rec, int *perm,
+                        int *bucket, hipStream_t s) {
+    const int abits = std::max(1, ilog2(G)), ibits = std::max(1, ilog2(std::max(longest, 1)));
+    if (longest > kPlanCurveMax || abits + ibits > 32) return false;
+    if (ncurves <= 0) return true;
+    // 256 threads where they hold a curve in 8 points each, so that several
+    // curves share a CU
+    const int NT = longest <= 2048 ? 256 : 1024;
+    const int cap = (std::max(longest, 1) + 7) & ~7;
+    const int npass = (int)ceil_div(abits, kPlanDigitBits), bits = (int)ceil_div(abits, npass);
+    const size_t lds = (sizeof(unsigned) + sizeof(short)) * (size_t)cap +
+                       sizeof(short) * ((size_t)(NT / 64) << bits);
+    auto go = [&](auto k) {
+        set_lds(k, lds);
+        hipLaunchKernelGGL(k, dim3(ncurves), dim3(NT), lds, s, rec_orig, coff, cap, abits, ibits,
+                           tlog, G, Kc, olo, ohi, rec, perm, bucket);
+        CUNA_LAUNCH_CHECK();
+    };
+    if (NT == 256)
+        go(k_plan_curve<T, 256, 8>);
+    else if (longest <= 8 * 1024)
+        go(k_plan_curve<T, 1024, 8>);
+    else
+        go(k_plan_curve<T, 1024, 23>);
+    return true;
 }
 
 template <typename T, int NTP, int NG>
@@ -663,7 +683,9 @@ template void launch_buckets<dTyp>(const int *, int, int, const PointRec<dTyp> *
 template void launch_spread<dTyp>(const SpreadArgs<dTyp> &, int, int, int, hipStream_t, hipEvent_t,
                                   hipEvent_t);
 template void launch_gather<dTyp>(const GatherArgs<dTyp> &, int, int, int, long, hipStream_t);
-template void launch_tile_cover<dTyp>(const SpreadArgs<dTyp> &, int, int *, hipStream_t);
+template void launch_tile_order<dTyp>(const SpreadArgs<dTyp> &, int, TileDesc *, hipStream_t);
+template bool launch_plan_curves<dTyp>(const PointRec<dTyp> *, const int *, int, int, int, int, int,
+                                       int, int, PointRec<dTyp> *, int *, int *, hipStream_t);
 template bool boot_fused_supported<dTyp>(int, int);
 template void launch_boot_fused<dTyp>(BootArgs<dTyp>, int, int, int, hipStream_t);
 template void launch_curve_cover<dTyp>(const PointRec<dTyp> *, const int *, int, int, int, int *,

@@ -81,12 +81,16 @@ template <typename T>
 // output); npts: points of all slabs (for the launch shape)
 void launch_gather(const GatherArgs<T> &A, int ntaps, int nslabs, int ngrids, long npts,
                    hipStream_t s);
-// per (curve, tile) point cover of the spread's scale (A: rec, bucket, tiles)
+// per curve, the scatter's work order (tiles by decreasing point count) with
+// each tile's ranges and cover (A: rec, bucket, tiles)
 template <typename T>
-void launch_tile_cover(const SpreadArgs<T> &A, int ncurves, int *cover, hipStream_t s);
-// per curve, the scatter's work order (tiles by decreasing point count)
-void launch_tile_order(const int *bucket, int Kc, int ntiles, int ncurves, bool periodic,
-                       const int *cover, TileDesc *desc, hipStream_t s);
+void launch_tile_order(const SpreadArgs<T> &A, int ncurves, TileDesc *desc, hipStream_t s);
+// sort by anchor and buckets of short curves in one launch; false, and nothing
+// launched, when the longest curve or the grid is too large for it
+template <typename T>
+bool launch_plan_curves(const PointRec<T> *rec_orig, const int *coff, int ncurves, int longest,
+                        int tlog, int G, int Kc, int olo, int ohi, PointRec<T> *rec, int *perm,
+                        int *bucket, hipStream_t s);
 
 // fused batched bootstrap (grid in LDS): false when this size/filter has no
 // fused kernel

@@ -64,12 +64,14 @@ struct TiledPoints {
     DevMem coff, rec, perm, bucket, eps_orig;
     DevMem rec_orig;  // (anchor, e) by original index
     DevMem order;     // curves by decreasing length (work-queue order)
-    DevMem tile_cover;  // per (curve, tile): most points in one window of ntaps anchors
     DevMem tile_desc;   // per curve: the scatter's work order (TileDesc per tile)
 
     // src: setup arguments with x/t/mode/compat fields filled
     void build(SetupArgs<T> A, const std::vector<int> &offsets, int G_, int tlog_, int ntaps_,
                bool periodic_, bool keep_eps, hipStream_t s);
+
+  private:
+    void sort_points(hipStream_t s);
 };
 
 struct ModeSpec {

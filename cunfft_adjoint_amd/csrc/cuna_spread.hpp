@@ -88,9 +88,7 @@ struct SetupArgs {
     T *E1, *E2, *E3;   // compat filter_properties arrays (nullable)
     T *eps_orig;       // compat: eps by original index (nullable)
     long n;
-    int tlog;          // tile = 2^tlog cells
     PointRec<T> *rec;  // out: (anchor, e) by original index
-    int *key;          // out: anchor & (tile - 1), the first sort digit
 };
 
 // compat decisions in the build's precision, one rounding per operation
@@ -156,7 +154,6 @@ __global__ void k_point_setup(SetupArgs<T> A) {
     pr.a = a;
     pr.e = e;
     A.rec[i] = pr;
-    A.key[i] = a & ((1 << A.tlog) - 1);
 }
 
 __device__ __forceinline__ int tile_key(int a, int tlog, int olo, int ohi, int G) {
@@ -270,6 +267,167 @@ __global__ void k_buckets(const int *coff, int ncurves, int Kc, const PointRec<T
             hi = mid;
     }
     bucket[idx] = lo;
+}
+
+// ---------------------------------------- sort of short curves: one launch --
+// The sort by anchor and the buckets of one curve in one workgroup, for curves
+// of at most kPlanCurveMax points whose (anchor, index) pairs fit 32 bits.  A
+// point is the word anchor << ibits | index, held in LDS; an LSD radix sort over
+// the anchor's bits (digits of at most 9) permutes the words: stable, so the
+// order is that of the multi-launch sort.  Wave w ranks the consecutive words
+// [w seg, (w + 1) seg), 64 per step: a word's rank is the count of equal digits
+// in the wave's earlier steps (16-bit counters per wave) plus the lower lanes
+// with the same digit (nine ballots); the scan of the
+// counters turns it into a place, and every thread moves its IPT words through
+// registers.  Bound by instruction issue in the ranking steps (one workgroup
+// per CU, four waves per SIMD).  It stands in for the sort's launches (digits,
+// histogram, three scan steps and scatter per digit, and the buckets): at 64
+// curves of 20,000 points and 2^17 cells 18 launches and 172 us -> 1 launch and
+// 52 us; at one curve of 20,011 points and 2^16 cells (FP64) 77 -> 55 us.
+constexpr int kPlanCurveMax = 23 * 1024, kPlanDigitBits = 9;
+
+template <typename T, int NT, int IPT>
+__global__ __launch_bounds__(NT) void k_plan_curve(const PointRec<T> *rec_orig, const int *coff,
+                                                   int cap, int abits, int ibits, int tlog, int G,
+                                                   int Kc, int olo, int ohi, PointRec<T> *rec,
+                                                   int *perm, int *bucket) {
+    constexpr int NW = NT / 64, UN = 4;
+    unsigned *sv = reinterpret_cast<unsigned *>(cuna_smem);              // cap words
+    unsigned short *rk = reinterpret_cast<unsigned short *>(sv + cap);   // cap ranks
+    unsigned short *cnt = rk + cap;                                      // [wave][digit]
+    __shared__ int wsum[NW];
+    const int c = blockIdx.x, c0 = coff[c], n = coff[c + 1] - c0;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int seg = (n + NT - 1) / NT * 64;  // words per wave
+    const int w0 = min(wave * seg, n), w1 = min(w0 + seg, n);
+    for (int p0 = tid; p0 < n; p0 += UN * NT) {
+        int a[UN];  // (clamped loads: all issue together)
+#pragma unroll
+        for (int k = 0; k < UN; ++k) a[k] = rec_orig[c0 + min(p0 + k * NT, n - 1)].a;
+#pragma unroll
+        for (int k = 0; k < UN; ++k) {
+            const int p = p0 + k * NT;
+            if (p < n) sv[p] = (unsigned)a[k] << ibits | (unsigned)p;
+        }
+    }
+    int shift = ibits, left = abits;
+    for (int pass = (abits + kPlanDigitBits - 1) / kPlanDigitBits; pass > 0; --pass) {
+        const int bits = (left + pass - 1) / pass, K = 1 << bits;
+        const unsigned mask = K - 1;
+        unsigned short *cw = cnt + wave * K;
+        for (int i = tid; i < NW * K / 2; i += NT) reinterpret_cast<unsigned *>(cnt)[i] = 0;
+        __syncthreads();
+        for (int q0 = w0; q0 < w1; q0 += 64) {  // uniform
+            const int na = min(64, w1 - q0);
+            const unsigned long long act = na == 64 ? ~0ull : (1ull << na) - 1ull;
+            const int q = min(q0 + lane, w1 - 1);
+            const unsigned d = (sv[q] >> shift) & mask;
+            unsigned plo = (unsigned)act, phi = (unsigned)(act >> 32);
+#pragma unroll
+            for (int b = 0; b < kPlanDigitBits; ++b) {  // (bits past the digit's are 0)
+                const int t = __builtin_amdgcn_sbfe((int)d, b, 1);  // 0 or ~0
+                const unsigned long long m = __ballot(t < 0);
+                plo &= ~((unsigned)m ^ (unsigned)t);
+                phi &= ~((unsigned)(m >> 32) ^ (unsigned)t);
+            }
+            // (a lane past the end counts all its peers as lower: it never writes)
+            const int r = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0));
+            const int cur = cw[d];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (r == __popc(plo) + __popc(phi) - 1) cw[d] = (unsigned short)(cur + r + 1);
+            if (lane < na) rk[q] = (unsigned short)(cur + r);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        // exclusive scan of the counters, by digit and then wave; a thread
+        // takes every NT-th digit
+        int carry = 0;
+        for (int d0 = 0; d0 < K; d0 += NT) {
+            const int d = d0 + tid;
+            int own[NW], tot = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                own[w] = d < K ? cnt[w * K + d] : 0;
+                tot += own[w];
+            }
+            int incl = tot;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(incl, o);
+                if (lane >= o) incl += u;
+            }
+            if (lane == 63) wsum[wave] = incl;
+            __syncthreads();
+            int at = carry + incl - tot, all = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                if (w < wave) at += wsum[w];
+                all += wsum[w];
+            }
+            carry += all;
+            if (d < K) {
+#pragma unroll
+                for (int w = 0; w < NW; ++w) {
+                    cnt[w * K + d] = (unsigned short)at;
+                    at += own[w];
+                }
+            }
+            __syncthreads();
+        }
+        // every word to its place, through registers
+        unsigned v[IPT];
+        unsigned short to[IPT];
+#pragma unroll
+        for (int s = 0; s < IPT; ++s) {
+            const int q = max(min(w0 + s * 64 + lane, w1 - 1), 0);
+            v[s] = sv[q];
+            to[s] = (unsigned short)(rk[q] + cw[(v[s] >> shift) & mask]);
+            if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // fewer registers
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < IPT; ++s)
+            if (w0 + s * 64 + lane < w1) sv[to[s]] = v[s];
+        __syncthreads();
+        shift += bits;
+        left -= bits;
+    }
+    // sorted records and original indices
+    const unsigned imask = (1u << ibits) - 1u;
+    for (int j0 = tid; j0 < n; j0 += UN * NT) {
+        unsigned w[UN];
+        T e[UN];
+#pragma unroll
+        for (int k = 0; k < UN; ++k) w[k] = sv[min(j0 + k * NT, n - 1)];
+#pragma unroll
+        for (int k = 0; k < UN; ++k) e[k] = rec_orig[c0 + (w[k] & imask)].e;
+#pragma unroll
+        for (int k = 0; k < UN; ++k) {
+            const int j = j0 + k * NT;
+            if (j < n) {
+                PointRec<T> pr;
+                pr.a = (int)(w[k] >> ibits);
+                pr.e = e[k];
+                rec[c0 + j] = pr;
+                perm[c0 + j] = c0 + (int)(w[k] & imask);
+            }
+        }
+    }
+    // bucket[k]: first sorted point with tile_key >= k, as in k_buckets
+    for (int k = tid; k <= Kc; k += NT) {
+        int lo = k < Kc ? 0 : n, hi = n;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (tile_key((int)(sv[mid] >> ibits), tlog, olo, ohi, G) < k)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        bucket[(long)c * (Kc + 1) + k] = c0 + lo;
+    }
 }
 
 // ------------------------------------------------ exclusive int scan --
@@ -386,11 +544,8 @@ struct SpreadArgs {
     // nullable: per curve (bi, wscale, exp(-bi)) in place of the three above,
     // for batches of compat curves whose filter widths differ
     const T *cpar;
-    // nullable: per (curve, tile), the most points whose anchors fall in one
-    // window of ntaps consecutive anchors (no cell receives more weights)
-    const int *tile_cover;
-    // nullable: per curve, ntiles work-order entries (the scatter kernels
-    // take entry blockIdx.x of their curve instead of tile blockIdx.x)
+    // per curve, ntiles work-order entries (the scatter kernel takes the next
+    // entry of its curve per workgroup)
     const TileDesc *tile_desc;
     // VAL_COMPAT_BOOT (src/gridding.cu:86-117): value y[d] and weight
     // parameter eps_orig[d] of the drawn point d, position of point p
@@ -685,46 +840,6 @@ __device__ __forceinline__ unsigned long long to_fixed64(double x) {
     return ((unsigned long long)(unsigned)(int)h << 32) | (unsigned)l;
 }
 
-// Plan time, one workgroup per (tile, curve): cover[c * ntiles + tile] = the
-// most points (the tile's own and its neighbours' edge classes) whose anchors
-// fall in one window of ntaps consecutive anchors that reaches a cell of the
-// tile, from a histogram of the anchors in LDS.
-template <typename T>
-__global__ __launch_bounds__(256) void k_tile_cover(SpreadArgs<T> A, int *cover) {
-    constexpr int NT = 256;
-    int *hist = reinterpret_cast<int *>(cuna_smem);
-    __shared__ int red[NT / 64];
-    const int tile = blockIdx.x, c = A.slab0 + blockIdx.y;
-    const int TT = 1 << A.tlog, nt = A.ntaps, Q0 = (nt - 1) / 2, NH = TT + 2 * nt;
-    TileRanges R;
-    R.init(A, tile, c, nt);
-    for (int i = threadIdx.x; i < NH; i += NT) hist[i] = 0;
-    __syncthreads();
-    for (int j = threadIdx.x; j < R.total; j += NT) {
-        int s, ro;
-        R.get(j, s, ro);
-        const int a = A.rec[s].a - ro + nt;
-        if (a >= 0 && a < NH) atomicAdd(&hist[a], 1);
-    }
-    __syncthreads();
-    // cell g takes the points with anchors g - (nt - 1 - Q0) .. g + Q0
-    int best = 0;
-    for (int g = threadIdx.x; g < TT; g += NT) {
-        int sum = 0;
-        for (int q = 0; q < nt; ++q) sum += hist[g - (nt - 1 - Q0) + nt + q];
-        best = max(best, sum);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) best = max(best, __shfl_xor(best, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int m = red[0];
-        for (int w = 1; w < NT / 64; ++w) m = max(m, red[w]);
-        cover[(long)c * A.ntiles + tile] = m;
-    }
-}
-
 // Work order of the scatter kernels, one workgroup per curve: the curve's
 // tiles by decreasing own point count, as a stable counting sort over
 // kOrderBins bins of the count (exact below 128 points, in steps of 8 up to
@@ -814,30 +929,77 @@ static __global__ __launch_bounds__(kOrderThreads) void k_tile_order(const int *
     for (int i = tid; i < ntiles; i += kOrderThreads) desc[(long)c * ntiles + i].tile = order[i];
 }
 
-// The rest of each TileDesc: tile t's own range and its neighbours' edge
-// classes (prev = t - 1 and next = t + 1, wrapping when periodic).  Many
-// workgroups share the random reads of the bucket table.
-static __global__ __launch_bounds__(256) void k_tile_desc(const int *bucket, int Kc, int ntiles,
-                                                          int periodic, const int *cover,
-                                                          TileDesc *desc) {
-    const int nblk = (ntiles + 255) / 256;  // workgroups per curve
-    const int c = blockIdx.x / nblk, i = (blockIdx.x % nblk) * 256 + threadIdx.x;
-    if (i >= ntiles) return;
-    const int *bk = bucket + (long)c * (Kc + 1);
-    TileDesc *dp = desc + (long)c * ntiles + i;
-    const int t = dp->tile;
-    const int prev = t > 0 ? t - 1 : ntiles - 1, next = t + 1 < ntiles ? t + 1 : 0;
-    const bool hp = t > 0 || periodic != 0, hn = t + 1 < ntiles || periodic != 0;
-    TileDesc d;
-    d.tile = t;
-    d.b1 = bk[3 * t];
-    d.e1 = bk[3 * t + 3];
-    d.b0 = hp ? bk[3 * prev + 2] : 0;
-    d.e0 = hp ? bk[3 * prev + 3] : 0;
-    d.b2 = hn ? bk[3 * next] : 0;
-    d.e2 = hn ? bk[3 * next + 1] : 0;
-    d.cover = cover ? cover[(long)c * ntiles + t] : 0x7fffffff;
-    *dp = d;
+// The rest of each TileDesc, one wave per work-order position: the tile's own
+// range, its neighbours' edge classes (prev = t - 1 and next = t + 1, wrapping
+// when periodic) and its cover, the most of these points whose anchors fall in
+// one window of ntaps consecutive anchors that reaches a cell of the tile.  The
+// wave counts the anchors in LDS, turns the counts into prefix sums (lane l
+// scans a contiguous piece) and takes each cell's window as a difference of
+// two.  One 256-thread workgroup per tile adding ntaps counts per cell took
+// 33 us at 32,768 tiles of 39 points; this takes 17.5 us.
+constexpr int kDescWaves = 4;
+
+template <typename T>
+__global__ __launch_bounds__(64 * kDescWaves) void k_tile_desc(SpreadArgs<T> A, long npos,
+                                                               TileDesc *desc) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int TT = 1 << A.tlog, nt = A.ntaps, Q0 = (nt - 1) / 2, NH = TT + 2 * nt;
+    int *h = reinterpret_cast<int *>(cuna_smem) + wave * (NH + 1);  // cells -nt .. TT+nt-1
+    const long pos = (long)blockIdx.x * kDescWaves + wave;
+    if (pos >= npos) return;  // no workgroup barriers below
+    const int c = (int)(pos / A.ntiles);
+    const int tile = desc[pos].tile;
+    TileRanges R;
+    R.init(A, tile, c, nt);
+    for (int i = lane; i <= NH; i += 64) h[i] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int j = lane; j < R.total; j += 64) {
+        int s, ro;
+        R.get(j, s, ro);
+        const int a = A.rec[s].a - ro + nt;
+        if (a >= 0 && a < NH) atomicAdd(&h[a], 1);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // h[i] := points with anchors before cell i, i = 0 .. NH
+    const int per = (NH + 64) / 64, i0 = min(lane * per, NH + 1), i1 = min(i0 + per, NH + 1);
+    int sum = 0;
+    for (int i = i0; i < i1; ++i) sum += h[i];
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o);
+        if (lane >= o) incl += u;
+    }
+    int run = incl - sum;
+    for (int i = i0; i < i1; ++i) {
+        const int v = h[i];
+        h[i] = run;
+        run += v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // cell g takes the points with anchors g - (nt - 1 - Q0) .. g + Q0
+    int best = 0;
+    for (int g = lane; g < TT; g += 64) {
+        const int lo = g + Q0 + 1;  // = g - (nt - 1 - Q0) + nt
+        best = max(best, h[lo + nt] - h[lo]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) best = max(best, __shfl_xor(best, o));
+    if (lane == 0) {
+        TileDesc d;
+        d.tile = tile;
+        d.b0 = R.b0;
+        d.e0 = R.b0 + R.n0;
+        d.b1 = R.b1;
+        d.e1 = R.b1 + R.n1;
+        d.b2 = R.b2;
+        d.e2 = R.b2 + R.n2;
+        d.cover = best;
+        desc[pos] = d;
+    }
 }
 
 // Accumulators of the scatter: 32-bit cells (ds_add_u32) hold sums within
@@ -1003,15 +1165,9 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
     const int slab = A.slab0 + bs.y;
     const int c = slab / A.nrep, rep = slab % A.nrep;
     TileRanges R;
-    int cover = CAP;
-    if (A.tile_desc) {
-        const TileDesc d = ldc_desc(A.tile_desc + (long)c * A.ntiles + bs.x);
-        R.from_desc(A, d, NTAPS);
-        cover = d.cover;
-    } else {
-        R.init(A, bs.x, c, NTAPS);
-        if (A.tile_cover) cover = A.tile_cover[(long)c * A.ntiles + bs.x];
-    }
+    const TileDesc desc = ldc_desc(A.tile_desc + (long)c * A.ntiles + bs.x);
+    R.from_desc(A, desc, NTAPS);
+    const int cover = desc.cover;
     const int total = R.total;
     const bool multi = total > CAP;
     const T c1 = A.cpar ? A.cpar[3 * c + 2] : A.e3[Q0 + 1];  // exp(-bi)
