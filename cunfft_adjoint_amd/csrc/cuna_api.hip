@@ -89,6 +89,99 @@ __global__ void k_compose(int *perm, const int *idx, long n) {
     if (i < n) perm[i] = idx[perm[i]];
 }
 
+// ------------------------------------------------------------- BlockPool --
+namespace {
+struct Block {
+    void *p;
+    size_t bytes;
+    int dev;
+};
+// (never destroyed: at process exit the runtime may be gone already)
+struct Kept {
+    std::mutex mu;
+    std::list<Block> blocks;  // oldest first
+    size_t bytes = 0;
+};
+Kept &kept() {
+    static Kept *k = new Kept;
+    return *k;
+}
+
+// eighths of a power of two: at most 12.5 % over
+size_t size_class(size_t n) {
+    size_t p = size_t(1) << 12;
+    while (p < n) p <<= 1;
+    const size_t step = std::max<size_t>(p >> 4, 256);
+    return (n + step - 1) / step * step;
+}
+}  // namespace
+
+void *BlockPool::take(size_t nbytes, size_t *got, int *dev, hipStream_t s) {
+    CUNA_HIP(hipGetDevice(dev));
+    const size_t n = nbytes >= kMinBlock ? size_class(nbytes) : nbytes;
+    if (nbytes >= kMinBlock) {
+        Kept &K = kept();
+        std::lock_guard<std::mutex> lk(K.mu);
+        for (auto it = K.blocks.begin(); it != K.blocks.end(); ++it) {
+            if (it->bytes != n || it->dev != *dev) continue;
+            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+            CUNA_HIP(hipStreamIsCapturing(s, &st));
+            require(st == hipStreamCaptureStatusNone,
+                    "device memory cannot be allocated while the stream is captured "
+                    "(run the call once before capturing it)",
+                    CUNA_ERROR_HIP);
+            void *p = it->p;
+            K.bytes -= n;
+            K.blocks.erase(it);
+            *got = n;
+            return p;
+        }
+    }
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, n);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        clear();
+        e = hipMalloc(&p, n);
+    }
+    hip_check(e, "hipMalloc", __FILE__, __LINE__);
+    *got = n;
+    return p;
+}
+
+void BlockPool::give(void *p, size_t bytes, int dev) {
+    if (bytes < kMinBlock || bytes > kMaxBlock) {
+        (void)hipFree(p);
+        return;
+    }
+    int cur = dev;
+    (void)hipGetDevice(&cur);
+    if (cur != dev) (void)hipSetDevice(dev);
+    const hipError_t e = hipDeviceSynchronize();
+    if (cur != dev) (void)hipSetDevice(cur);
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return;
+    }
+    Kept &K = kept();
+    std::lock_guard<std::mutex> lk(K.mu);
+    K.blocks.push_back(Block{p, bytes, dev});
+    K.bytes += bytes;
+    while (K.bytes > kMaxKept) {
+        (void)hipFree(K.blocks.front().p);
+        K.bytes -= K.blocks.front().bytes;
+        K.blocks.pop_front();
+    }
+}
+
+void BlockPool::clear() {
+    Kept &K = kept();
+    std::lock_guard<std::mutex> lk(K.mu);
+    for (const Block &b : K.blocks) (void)hipFree(b.p);
+    K.blocks.clear();
+    K.bytes = 0;
+}
+
 // ------------------------------------------------------------ TiledPoints --
 namespace {
 // offsets of 256-byte aligned pieces of one allocation
@@ -148,7 +241,7 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     const size_t o_bk = pc.add(sizeof(int) * (size_t)ncurves * (Kc + 1));
     const size_t o_eps = keep_eps ? pc.add(sizeof(T) * n1) : 0;
     const size_t o_desc = pc.add(sizeof(TileDesc) * ncov);
-    arena.alloc(pc.total);
+    arena.alloc(pc.total, s);
     char *pb = arena.as<char>();
     coff.view(pb + o_up, sizeof(int) * (ncurves + 1));
     order.view(pb + o_up + sizeof(int) * (ncurves + 1), sizeof(int) * ncurves);
@@ -309,7 +402,7 @@ void Plan<T>::prepare_fft(hipStream_t s) {
     require(spec.mode == CUNA_MODE_COMPAT, "accurate-mode grids are powers of two");
     blu = std::make_unique<Bluestein<T>>();
     blu->init(G, s);
-    blu->ensure(std::max(ncurves(), 1));
+    blu->ensure(std::max(ncurves(), 1), s);
 }
 
 template <typename T>
@@ -349,7 +442,7 @@ void Plan<T>::run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s, hipEv
 template <typename T>
 void Plan<T>::adjoint(const T *y, cplx<T> *out, hipStream_t s) {
     require(out != nullptr, "output pointer is NULL");
-    grid.ensure(sizeof(T) * (size_t)G * ncurves());
+    grid.ensure(sizeof(T) * (size_t)G * ncurves(), s);
     adjoint_into(y, out, grid.as<T>(), s);
 }
 
@@ -378,7 +471,7 @@ void Plan<T>::adjoint_many(const T *y, int nrhs, cplx<T> *out, hipStream_t s) {
     require(nrhs >= 1, "nrhs must be positive");
     const int nc = ncurves();
     require((long)nc * nrhs <= INT_MAX, "ncurves * nrhs too large", CUNA_ERROR_UNSUPPORTED);
-    grid.ensure(sizeof(T) * (size_t)G * nc * nrhs);
+    grid.ensure(sizeof(T) * (size_t)G * nc * nrhs, s);
     SpreadArgs<T> A = spread_args(pts);
     A.y = y;
     A.y_slab_stride = n();
@@ -395,8 +488,8 @@ void Plan<T>::bootstrap_compat(const T *y, cplx<T> *out, int nbs, uint32_t seed,
     require(spec.mode == CUNA_MODE_COMPAT && ncurves() == 1, "compat bootstrap needs a compat plan");
     require(nbs > 0, "nbs must be positive");
     require(out != nullptr, "output pointer is NULL");
-    grid.ensure(sizeof(T) * (size_t)G * nbs);
-    if (blu) blu->ensure(nbs);
+    grid.ensure(sizeof(T) * (size_t)G * nbs, s);
+    if (blu) blu->ensure(nbs, s);
     SpreadArgs<T> A = spread_args(pts);
     A.y = y;
     A.grid = grid.as<T>();
@@ -423,15 +516,15 @@ int Plan<T>::ymax_parts() const {
 }
 
 template <typename T>
-void Plan<T>::prepare_bootstrap(int nbs, bool window) {
+void Plan<T>::prepare_bootstrap(int nbs, bool window, hipStream_t s) {
     if (bootstrap_fused_ok(window)) {
-        counter.ensure(sizeof(int));
-        ymax.ensure(sizeof(T) * (size_t)ncurves() * ymax_parts());
-        cover.ensure(sizeof(int) * 2 * (size_t)ncurves());
+        counter.ensure(sizeof(int), s);
+        ymax.ensure(sizeof(T) * (size_t)ncurves() * ymax_parts(), s);
+        cover.ensure(sizeof(int) * 2 * (size_t)ncurves(), s);
         return;
     }
-    counts.ensure(sizeof(int) * (size_t)std::max<long>(n(), 1) * nbs);
-    grid.ensure(sizeof(T) * (size_t)G * ncurves() * nbs);
+    counts.ensure(sizeof(int) * (size_t)std::max<long>(n(), 1) * nbs, s);
+    grid.ensure(sizeof(T) * (size_t)G * ncurves() * nbs, s);
 }
 
 // arguments shared by both modes of the fused bootstrap kernel; computes
@@ -488,14 +581,14 @@ void Plan<T>::bootstrap_ls(const T *y, int nbs, uint32_t seed, T *power, T *peak
             "Lomb-Scargle bootstrap needs a grid of at most 2^15 cells (float) / 2^14 (double) and "
             "m in {6, 8, 10, 12, 13, 16}",
             CUNA_ERROR_UNSUPPORTED);
-    prepare_bootstrap(nbs, true);
+    prepare_bootstrap(nbs, true, s);
     // window spectra workspace: one row of M/2 values per resident workgroup
     // (at most one per kMaxLds of LDS on each CU)
     int dev = 0, ncu = 0;
     CUNA_HIP(hipGetDevice(&dev));
     CUNA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     const int slots = ncu * std::max(1, (int)(kMaxLds / boot_lds_bytes<T>(lgN)));
-    ls_work.ensure(sizeof(cplx<T>) * (size_t)slots * (M / 2));
+    ls_work.ensure(sizeof(cplx<T>) * (size_t)slots * (M / 2), s);
     BootArgs<T> B = fused_args(y, nbs, seed, s);
     B.ls_power = power;
     B.ls_peak = peak;
@@ -517,7 +610,7 @@ void Plan<T>::bootstrap(const T *y, int nbs, uint32_t seed, cplx<T> *out_y, cplx
     require(out_w == nullptr || has_pts2, "window output needs a plan made with CUNA_PLAN_WINDOW2");
     require(out_y != nullptr, "out_y is NULL");
     const int nc = ncurves();
-    prepare_bootstrap(nbs, out_w != nullptr);
+    prepare_bootstrap(nbs, out_w != nullptr, s);
     if (bootstrap_fused_ok(out_w != nullptr)) {
         BootArgs<T> B = fused_args(y, nbs, seed, s);
         B.out_y = out_y;
@@ -561,8 +654,8 @@ template <typename T>
 void Plan<T>::spectrum_to_grid(const cplx<T> *g, int parts, int rot, hipStream_t s) {
     const long N = (long)G / 2;
     const int rows = ncurves() * parts;
-    grid.ensure(sizeof(T) * (size_t)G * rows);
-    work.ensure(sizeof(cplx<T>) * (size_t)N * rows);
+    grid.ensure(sizeof(T) * (size_t)G * rows, s);
+    work.ensure(sizeof(cplx<T>) * (size_t)N * rows, s);
     const double pi = 3.14159265358979323846;
     LoadHermitian<T> ld;
     ld.g = g;
@@ -919,7 +1012,7 @@ struct CompatBatch {
     int idist = 0;
     struct Group {
         // host sources of the group's async uploads, declared first so that
-        // they outlive the device buffers (whose hipFree synchronises)
+        // they outlive the device buffers (whose release synchronises)
         std::vector<int> idx_h;
         std::vector<R> cpar_h, qb_h;
         std::vector<long> ro_h;
@@ -1017,9 +1110,9 @@ static std::unique_ptr<CompatBatch> make_compat_batch(const R *x, const int *n, 
             qb[k] = b * R(0.25);
             ro[k] = (long)cur[k] * B->idist;
         }
-        G->cpar.alloc(sizeof(R) * cp.size());
-        G->qb_row.alloc(sizeof(R) * qb.size());
-        G->row_off.alloc(sizeof(long) * ro.size());
+        G->cpar.alloc(sizeof(R) * cp.size(), s);
+        G->qb_row.alloc(sizeof(R) * qb.size(), s);
+        G->row_off.alloc(sizeof(long) * ro.size(), s);
         CUNA_HIP(hipMemcpyAsync(G->cpar.ptr, cp.data(), sizeof(R) * cp.size(),
                                 hipMemcpyHostToDevice, s));
         CUNA_HIP(hipMemcpyAsync(G->qb_row.ptr, qb.data(), sizeof(R) * qb.size(),
@@ -1260,7 +1353,10 @@ CUNA_API void generate_pinned_filter_properties_batch(const dTyp *x, const int *
 }
 
 CUNA_API void cuna_batch_cache_clear(void) {
-    guarded([&] { batch_drop(nullptr); });
+    guarded([&] {
+        batch_drop(nullptr);
+        BlockPool::clear();
+    });
 }
 
 // ------------------------------------------------------------ plan path --
@@ -1340,24 +1436,29 @@ CUNA_API void free_plan(plan *p) {
     });
 }
 
+// The transform of init_plan + cunfft_adjoint_from_plan + free_plan without the
+// plan struct: its host copies of x, f and f_hat, the E1/E2/E3 arrays and (with
+// CALCULATE_WINDOW_FUNCTION) a window spectrum that this call never returns.
 CUNA_API void cunfft_adjoint(const dTyp *x, const dTyp *f, cTyp *fft, int n, int ng,
                              unsigned int flags) {
+    (void)flags;
     guarded([&] {
         require(fft != nullptr, "fft is NULL");
-        plan *p = (plan *)malloc(sizeof(plan));
-        require(p != nullptr, "host allocation failed", CUNA_ERROR_OUT_OF_MEMORY);
-        memset(p, 0, sizeof *p);
-        init_plan(p, x, f, n, ng, flags & ~DONT_TRANSFER_TO_CPU);
-        int err = g_err;
-        std::string msg = g_msg;
-        if (err == CUNA_SUCCESS) {
-            cunfft_adjoint_from_plan(p);
-            err = g_err;
-            msg = g_msg;
+        require(x != nullptr, "x is NULL");
+        check_compat_sizes(n, ng);
+        DevMem dx, df, dout;
+        dx.alloc(sizeof(R) * n, nullptr);
+        CUNA_HIP(hipMemcpy(dx.ptr, x, sizeof(R) * n, hipMemcpyHostToDevice));
+        if (f) {
+            df.alloc(sizeof(R) * n, nullptr);
+            CUNA_HIP(hipMemcpy(df.ptr, f, sizeof(R) * n, hipMemcpyHostToDevice));
         }
-        if (err == CUNA_SUCCESS) memcpy((void *)fft, p->f_hat, sizeof(Complex) * ng);
-        free_plan(p);
-        if (err != CUNA_SUCCESS) fail(err, msg);
+        dout.alloc(sizeof(cplx<R>) * ng, nullptr);
+        ModeSpec spec;
+        spec.mode = CUNA_MODE_COMPAT;
+        auto p = make_plan_compat<R>(dx.as<R>(), n, ng, nullptr, nullptr, nullptr, spec, nullptr);
+        p->adjoint(f ? df.as<R>() : nullptr, dout.as<cplx<R>>(), nullptr);
+        CUNA_HIP(hipMemcpy((void *)fft, dout.ptr, sizeof(cplx<R>) * ng, hipMemcpyDeviceToHost));
     });
 }
 
@@ -1623,7 +1724,7 @@ CUNA_API int cuna_fft(Complex *data, int n, int batch, int sign, hipStream_t str
             // waits for its stream before the workspace is released
             Bluestein<R> b;
             b.init(n, stream);
-            b.ensure(batch);
+            b.ensure(batch, stream);
             b.run_complex(reinterpret_cast<cplx<R> *>(data), batch, sign, stream);
             CUNA_HIP(hipStreamSynchronize(stream));
             return;

@@ -104,13 +104,13 @@ void Bluestein<T>::init(int ng_, hipStream_t s) {
         b_h[k] = v;
         if (k > 0) b_h[L - k] = v;
     }
-    chirp.alloc(sizeof(cplx<T>) * ng);
-    bhat.alloc(sizeof(cplx<T>) * L);
+    chirp.alloc(sizeof(cplx<T>) * ng, s);
+    bhat.alloc(sizeof(cplx<T>) * L, s);
     CUNA_HIP(hipMemcpyAsync(chirp.ptr, chirp_h.data(), sizeof(cplx<T>) * ng,
                             hipMemcpyHostToDevice, s));
     CUNA_HIP(hipMemcpyAsync(bhat.ptr, b_h.data(), sizeof(cplx<T>) * L, hipMemcpyHostToDevice, s));
     TwiddleCache<T>::get().warm(lgL);
-    ensure(1);
+    ensure(1, s);
     FftShape sh;
     sh.lgN = lgL;
     sh.batch = 1;
@@ -118,9 +118,9 @@ void Bluestein<T>::init(int ng_, hipStream_t s) {
 }
 
 template <typename T>
-void Bluestein<T>::ensure(int batch) {
+void Bluestein<T>::ensure(int batch, hipStream_t s) {
     if (batch <= batch_cap) return;
-    work.alloc(sizeof(cplx<T>) * (size_t)L * 2 * (size_t)batch);
+    work.alloc(sizeof(cplx<T>) * (size_t)L * 2 * (size_t)batch, s);
     batch_cap = batch;
 }
 

@@ -12,18 +12,38 @@
 
 namespace cuna {
 
-// Persistent device allocation (hipMalloc / hipFree).
+// Device blocks kept between plans.  A plan made for one call (a training step,
+// a survey of new curves, the host interface) allocates and frees the same large
+// blocks each time, and hipFree of a large block takes 70 - 260 us, hipMalloc 20 -
+// 60 us.  A freed block of kMinBlock bytes or more is kept for the next
+// allocation of its size class on its device instead.  As hipFree does, a release
+// waits for the device first, so a kept block has no work outstanding on any
+// stream and may go to any other.  At most kMaxKept bytes are kept (the oldest
+// block leaves first); all go back on cuna_batch_cache_clear(), and before an
+// allocation that would otherwise fail.
+struct BlockPool {
+    static constexpr size_t kMinBlock = size_t(64) << 10, kMaxBlock = size_t(256) << 20;
+    static constexpr size_t kMaxKept = size_t(512) << 20;
+    // a block of at least nbytes on the current device (its size in *got).  Like
+    // hipMalloc, refused while `s` is being captured.
+    static void *take(size_t nbytes, size_t *got, int *dev, hipStream_t s);
+    static void give(void *p, size_t bytes, int dev);
+    static void clear();
+};
+
+// Persistent device allocation.
 struct DevMem {
     void *ptr = nullptr;
     size_t bytes = 0;
+    int dev = 0;
     bool owned = true;  // false: a view into another allocation
     DevMem() = default;
     DevMem(const DevMem &) = delete;
     DevMem &operator=(const DevMem &) = delete;
-    void alloc(size_t nbytes) {
+    // s: the stream of the call that allocates (only checked for capture)
+    void alloc(size_t nbytes, hipStream_t s) {
         release();
-        if (nbytes) CUNA_HIP(hipMalloc(&ptr, nbytes));
-        bytes = nbytes;
+        if (nbytes) ptr = BlockPool::take(nbytes, &bytes, &dev, s);
     }
     void view(void *p, size_t nbytes) {
         release();
@@ -31,11 +51,11 @@ struct DevMem {
         bytes = nbytes;
         owned = false;
     }
-    void ensure(size_t nbytes) {
-        if (nbytes > bytes) alloc(nbytes);
+    void ensure(size_t nbytes, hipStream_t s) {
+        if (nbytes > bytes) alloc(nbytes, s);
     }
     void release() {
-        if (ptr && owned) (void)hipFree(ptr);
+        if (ptr && owned) BlockPool::give(ptr, bytes, dev);
         ptr = nullptr;
         bytes = 0;
         owned = true;
@@ -52,7 +72,7 @@ template <typename T>
 struct TiledPoints {
     // host sources of the async uploads (offsets and curve order; the sort's
     // chunk tables), declared first so that they are destroyed after the
-    // device buffers (whose hipFree synchronises)
+    // device buffers (whose release synchronises)
     std::vector<int> plan_h, sort_h;
     int ncurves = 0;
     long n = 0;
@@ -100,7 +120,7 @@ struct Bluestein {
     DevMem work;   // batch_cap x L complex for the data and as much for the FFT passes
     int batch_cap = 0;
     void init(int ng_, hipStream_t s);
-    void ensure(int batch);
+    void ensure(int batch, hipStream_t s);
     // real grids (batch rows of stride gstride, the first ng cells used) ->
     // the compat deconvolution sink, one row per grid
     void run_real(const T *grid, long gstride, int batch, const SinkCompat<T> &sk,
@@ -166,7 +186,7 @@ struct Plan {
     void forward(const cplx<T> *fhat, cplx<T> *f, hipStream_t s);
     // allocate every workspace a later call with these sizes needs (so that
     // the call can be captured into a graph without allocating)
-    void prepare_bootstrap(int nbs, bool window);
+    void prepare_bootstrap(int nbs, bool window, hipStream_t s);
     bool bootstrap_fused_ok(bool window) const;
     int ymax_parts() const;
 

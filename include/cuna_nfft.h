@@ -196,7 +196,8 @@ void cunfft_adjoint_raw_batched_async(const dTyp *x, const dTyp *f_data, Complex
 void generate_pinned_filter_properties_batch(const dTyp *x, const int *n, const int *ng,
                                              const int nlc, filter_properties **h_fprops,
                                              filter_properties **d_fprops, hipStream_t stream);
-/* Frees every cached multi-curve plan. */
+/* Frees every cached multi-curve plan, and the device blocks the library keeps
+ * from destroyed plans (at most 512 MiB). */
 void cuna_batch_cache_clear(void);
 
 /* The FFT stage alone: in-place unnormalised DFT of `batch` sequences of n
