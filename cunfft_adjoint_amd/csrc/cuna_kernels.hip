@@ -59,17 +59,26 @@ constexpr int split_lg1(int lgN) { return lgN / 2; }
 // largest log2 N of the single-workgroup inverse (Hermitian) transform
 constexpr int kC2rSmallLg = 13;
 
+// Radix 8 (8 values per thread, twice the threads of radix 16) up to 2^12: a
+// workgroup is a chain of passes, and more waves shorten each.  Measured radix
+// 16 -> 8 at 2^11: 6.1 -> 4.8 us (one transform, FP32), 22.1 -> 18.1 us (2048),
+// FP64 8.0 -> 6.2 and 44.2 -> 35.0 us.  At 2^13 radix 16 has a pass less and is
+// as fast (9.4 against 9.6 us; 2^14 has 1024 threads only in radix 16).
+constexpr int small_mr(int lg) { return lg >= 5 && lg <= 12 ? 3 : 4; }
+
 template <typename T, int S, int LG, class Loader, class Sink, int MODE>
 static void run_small(const FftShape &sh, const Loader &ld, const Sink &sk, cplx<T> *plain_out,
                       hipStream_t s) {
-    constexpr int NT = fft_threads(LG, 1);
+    constexpr int MR = small_mr(LG), NT = fft_threads(LG, 1, MR);
     auto &tc = TwiddleCache<T>::get();
     const cplx<T> *tw = tc.fine(LG);
     Tw2<T> twG = tc.two_level(LG + 1);
-    size_t lds = (sizeof(cplx<T>) << LG) * (lds_table(LG) ? 2 : 1);
-    auto k = k_fft_small<T, S, LG, NT, Loader, Sink, MODE>;
+    const cplx<T> *tw_lds = lds_table(LG) ? tw : tc.fine(kSplitLg);
+    size_t lds = sizeof(cplx<T>) * (((size_t)1 << LG) + small_table(LG));
+    static_assert(sizeof(cplx<T>) * (((size_t)1 << LG) + small_table(LG)) <= kMaxLds, "FFT LDS");
+    auto k = k_fft_small<T, S, LG, NT, Loader, Sink, MODE, MR>;
     set_lds(k, lds);
-    hipLaunchKernelGGL(k, dim3(sh.batch), dim3(NT), lds, s, ld, sk, plain_out, tw, twG);
+    hipLaunchKernelGGL(k, dim3(sh.batch), dim3(NT), lds, s, ld, sk, plain_out, tw, tw_lds, twG);
     CUNA_LAUNCH_CHECK();
 }
 
