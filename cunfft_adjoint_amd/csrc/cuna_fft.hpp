@@ -20,6 +20,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "cuna_common.hpp"
@@ -137,7 +138,16 @@ constexpr int pass_log2(int lg, int p, int mr = 4) {
 // the stride-16 writes of a radix-16 pass (8- and 16-byte elements, 32 or 64
 // banks) conflict-free; unswizzled, those writes hit 2 of the banks per
 // 64-byte group.
-__device__ __forceinline__ int lds_sw(int a) { return a ^ ((a >> 4) & 31); }
+// The map is linear over XOR, so the address of a sum of terms with disjoint
+// bits is the XOR of their addresses, and a term that is a compile-time constant
+// costs one XOR of its low five bits and an instruction offset.
+__host__ __device__ constexpr int lds_sw(int a) { return a ^ ((a >> 4) & 31); }
+// lds_sw(a + C) from sa = lds_sw(a), where a has no bit in common with C
+template <int C>
+__device__ __forceinline__ int lds_sw_add(int sa) {
+    constexpr int SC = lds_sw(C), low = SC & 31, high = SC & ~31;
+    return (low ? sa ^ low : sa) + high;
+}
 
 // ------------------------------------------------------ twiddle tables --
 // Two-level table for exp(+2 pi i e / Nfull), e < Nfull:
@@ -147,8 +157,8 @@ struct Tw2 {
     const cplx<T> *lo;
     const cplx<T> *hi;
     int lb;  // log2 B
-    __device__ __forceinline__ cplx<T> operator()(long e) const {
-        return lo[e & ((1L << lb) - 1)] * hi[e >> lb];
+    __device__ __forceinline__ cplx<T> operator()(int e) const {
+        return lo[e & ((1 << lb) - 1)] * hi[e >> lb];
     }
     __device__ __forceinline__ cplx<T> operator[](int e) const {
         return lo[e & ((1 << lb) - 1)] * hi[e >> lb];
@@ -224,6 +234,16 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
+template <int N, class F, int... I>
+__device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unroll(F &&f) {
+    unroll_seq<N>(f, std::make_integer_sequence<int, N>{});
+}
+
 // ----------------------------------------------------------- LDS Stockham --
 // W interleaved sequences of length L = 2^LG: element e of sequence w lives at
 // lds[lds_sw(e*W + w)].  Pass 0 reads its inputs through `ld(e, w)`; every pass writes
@@ -260,13 +280,15 @@ __device__ __forceinline__ void fft_pass(cplx<T> *lds, TW tw, const Loader &ld,
             const int g = tid + q * NT;
             if (EXACT || g < NB) {
                 const int w = g % W, j = g / W;
+                if constexpr (P == 0) {
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int e = j + r * Q;
-                    if constexpr (P == 0)
-                        v[q][r] = ld(e, w);
-                    else
-                        v[q][r] = lds[lds_sw(e * W + w)];
+                    for (int r = 0; r < R; ++r) v[q][r] = ld(j + r * Q, w);
+                } else {
+                    // element j + r Q of sequence w: g = j W + w < Q W
+                    const int sg = lds_sw(g);
+                    unroll<R>([&](auto r) __attribute__((always_inline)) {
+                        v[q][r] = lds[lds_sw_add<decltype(r)::value * Q * W>(sg)];
+                    });
                 }
                 // twiddles are global loads: issue them before the barrier
                 // (with several butterflies per thread that would hold all
@@ -290,8 +312,11 @@ __device__ __forceinline__ void fft_pass(cplx<T> *lds, TW tw, const Loader &ld,
                     apply_twiddles<T, S, R, LG - LOGNS - LR, (R <= 4)>(v[q], tw, k);
                 dft<T, R, S>(v[q]);
                 const int base = ((j >> LOGNS) << (LOGNS + LR)) + k;
-#pragma unroll
-                for (int r = 0; r < R; ++r) lds[lds_sw((base + (r << LOGNS)) * W + w)] = v[q][r];
+                // bits [LOGNS, LOGNS + LR) of base are zero
+                const int sb = lds_sw(base * W + w);
+                unroll<R>([&](auto r) __attribute__((always_inline)) {
+                    lds[lds_sw_add<(decltype(r)::value << LOGNS) * W>(sb)] = v[q][r];
+                });
             }
         }
         lds_barrier();
@@ -421,27 +446,37 @@ class TwiddleCache {
     }
 };
 
+// Element i of a row: a row has at most 2^25 (FP32) / 2^24 (FP64) values, so
+// its byte offset fits 32 bits and adds to the row's scalar address in the
+// store instruction.
+template <typename T>
+__device__ __forceinline__ cplx<T> *row_at(cplx<T> *row, int i) {
+    return reinterpret_cast<cplx<T> *>(reinterpret_cast<char *>(row) +
+                                       (unsigned)i * (unsigned)sizeof(cplx<T>));
+}
+
 // ------------------------------------------------------------- sinks --
-// A sink receives one spectral value A[f] of the real grid (f in [0, N]) and
-// writes it, and its conjugate image A[G-f], where the output wants them.
+// A sink receives twice one spectral value A[f] of the real grid (f in [0, N])
+// and writes A[f], and its conjugate image A[G-f], where the output wants them.
 
 // Accurate mode: out[M/2 + k], k = -M/2 .. M/2-1, deconvolved by
 // D(k) = exp(pi^2 beta k^2/G^2)/sqrt(pi beta).
 template <typename T>
 struct SinkAccurate {
     cplx<T> *out;
-    long M;
+    int M;
     long ostride;  // per batch
     T invG, coef, pref;
     // the sink of batch row b and where that row's output starts
     __device__ __forceinline__ const SinkAccurate &for_row(long) const { return *this; }
     __device__ __forceinline__ cplx<T> *row_out(long b) const { return out + b * ostride; }
-    __device__ __forceinline__ void operator()(cplx<T> *o, long f, cplx<T> A) const {
-        if (f <= M / 2) {
+    __device__ __forceinline__ void operator()(cplx<T> *o, int f, cplx<T> A) const {
+        const int half = M / 2;
+        if (f <= half) {
             T kk = (T)f * invG;
-            T D = pref * dexp(coef * kk * kk);
-            if (f < M / 2) o[M / 2 + f] = A * D;
-            if (f > 0) o[M / 2 - f] = conjg(A) * D;
+            T D = (T(0.5) * pref) * dexp(coef * kk * kk);
+            if (f < half) *row_at(o, half + f) = A * D;
+            if (f > 0) *row_at(o, half - f) = conjg(A) * D;
         }
     }
 };
@@ -451,7 +486,7 @@ struct SinkAccurate {
 template <typename T>
 struct SinkCompat {
     cplx<T> *out;
-    long G;
+    int G;
     long ostride;
     T invG, qb, normfac;  // qb = b/4
     // batches of curves with their own b (each nullable): output offset and
@@ -466,25 +501,27 @@ struct SinkCompat {
     __device__ __forceinline__ cplx<T> *row_out(long b) const {
         return out + (row_off ? row_off[b] : b * ostride);
     }
-    __device__ __forceinline__ T fac(long r) const {
+    __device__ __forceinline__ T fac(int r) const {
         T K = (T)r * invG;
         return normfac * dexp(K * K * qb);
     }
-    __device__ __forceinline__ void operator()(cplx<T> *o, long f, cplx<T> A) const {
-        o[f] = A * fac(f);
-        if (f != 0 && 2 * f != G) o[G - f] = conjg(A) * fac(G - f);
+    __device__ __forceinline__ void operator()(cplx<T> *o, int f, cplx<T> A) const {
+        const T h = T(0.5);
+        *row_at(o, f) = A * (h * fac(f));
+        if (f != 0 && 2 * f != G) *row_at(o, G - f) = conjg(A) * (h * fac(G - f));
     }
 };
 
 // A[r] and A[N-r] of the real grid from Z[r], Z[N-r]:
 //   E = (Z[r] + conj Z[N-r])/2, O = (Z[r] - conj Z[N-r])/(2i),
 //   A[r] = E + w_G^r O,  A[N-r] = conj(E - w_G^r O).
+// The halves are left to the sink's factor (exact).
 template <typename T, class Sink>
-__device__ __forceinline__ void emit_pair(const Sink &sk, cplx<T> *o, long r, long N, cplx<T> Zr,
+__device__ __forceinline__ void emit_pair(const Sink &sk, cplx<T> *o, int r, int N, cplx<T> Zr,
                                           cplx<T> Znr, cplx<T> wr) {
     cplx<T> c = conjg(Znr);
-    cplx<T> E = (Zr + c) * T(0.5);
-    cplx<T> D = (Zr - c) * T(0.5);
+    cplx<T> E = Zr + c;
+    cplx<T> D = Zr - c;
     cplx<T> O = cmk(D.y, -D.x);
     cplx<T> wO = wr * O;
     sk(o, r, E + wO);
@@ -500,7 +537,7 @@ struct LoadGrid {
     const cplx<T> *z;
     long stride;  // per batch
     __device__ __forceinline__ void advance(long b) { z += b * stride; }
-    __device__ __forceinline__ cplx<T> at(long n) const { return z[n]; }
+    __device__ __forceinline__ cplx<T> at(int n) const { return z[(unsigned)n]; }
 };
 
 // Backward (C2R of a Hermitian spectrum): Z[q] = E_q + i O_q, 0 <= q < N, with
@@ -530,8 +567,8 @@ struct LoadHermitian {
         }
         g += b * gstride;
     }
-    __device__ __forceinline__ cplx<T> at(long q_) const {
-        const int q = (int)q_, half = M / 2;
+    __device__ __forceinline__ cplx<T> at(int q) const {
+        const int half = M / 2;
         const bool hi = N - q < q;
         const int k = hi ? N - q : q;
         // clamped loads, so that they need no branch; values out of the band
@@ -566,8 +603,8 @@ struct LoadHermitian {
 template <typename T>
 struct Tw2Parts {
     cplx<T> lo, hi;
-    __device__ __forceinline__ void load(const Tw2<T> &t, long e) {
-        lo = t.lo[e & ((1L << t.lb) - 1)];
+    __device__ __forceinline__ void load(const Tw2<T> &t, int e) {
+        lo = t.lo[e & ((1 << t.lb) - 1)];
         hi = t.hi[e >> t.lb];
     }
     __device__ __forceinline__ cplx<T> get() const { return lo * hi; }
@@ -615,7 +652,7 @@ __global__ __launch_bounds__(NT) void k_fft_small(Loader ld, Sink sk, cplx<T> *p
             if (r <= N / 2) {
                 cplx<T> Zr = lds[lds_sw(r)];
                 cplx<T> Zn = lds[lds_sw((N - r) & (N - 1))];
-                emit_pair(skb, o, (long)r, (long)N, Zr, Zn, ot[i].get());
+                emit_pair(skb, o, r, N, Zr, Zn, ot[i].get());
             }
         }
     } else {
@@ -656,11 +693,11 @@ __global__ __launch_bounds__(NT) void k_fft_col(Loader ld, cplx<T> *dst, long ds
             for (int i = 0; i < OPT; ++i) {
                 const int idx = tid + i * NT;
                 if ((W * L2) % NT == 0 || idx < W * L2)
-                    ot[i].load(twN, (long)(n10 + idx % W) * (idx / W));
+                    ot[i].load(twN, (n10 + idx % W) * (idx / W));
             }
         }
     };
-    auto fetch = [&](int e, int w) __attribute__((always_inline)) { return lb.at(n10 + w + (long)L1 * e); };
+    auto fetch = [&](int e, int w) __attribute__((always_inline)) { return lb.at(n10 + w + L1 * e); };
     if constexpr (TAB) {
         auto hook = [&]() __attribute__((always_inline)) {
             tab.store(twl, tid);
@@ -679,15 +716,15 @@ __global__ __launch_bounds__(NT) void k_fft_col(Loader ld, cplx<T> *dst, long ds
                 const int w = idx % W, r2 = idx / W;
                 cplx<T> t = ot[i].get();
                 if constexpr (S < 0) t.y = -t.y;
-                o[n10 + w + (long)L1 * r2] = lds[lds_sw(r2 * W + w)] * t;
+                *row_at(o, n10 + w + L1 * r2) = lds[lds_sw(r2 * W + w)] * t;
             }
         }
     } else {
         for (int idx = tid; idx < W * L2; idx += NT) {
             const int w = idx % W, r2 = idx / W;
-            cplx<T> t = twN((long)(n10 + w) * r2);
+            cplx<T> t = twN((n10 + w) * r2);
             if constexpr (S < 0) t.y = -t.y;
-            o[n10 + w + (long)L1 * r2] = lds[lds_sw(r2 * W + w)] * t;
+            *row_at(o, n10 + w + L1 * r2) = lds[lds_sw(r2 * W + w)] * t;
         }
     }
 }
@@ -711,7 +748,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
     const int2 bs = xcd_block(blockIdx.x, blockIdx.y, nblk, gridDim.y);
     const int i = bs.x;
     const long b = b0 + bs.y;  // launches span at most kMaxGridY batches
-    const long N = (long)L1 * L2;
+    const int N = L1 * L2;
     const cplx<T> *z = src + b * src_stride;
     TableStage<T, (TAB ? L1 : 1), NT> tab;
     if constexpr (TAB) tab.load(tw, tid);
@@ -725,7 +762,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
         for (int k = 0; k < OPT; ++k) {
             const int idx = tid + k * NT;
             if ((H * L1) % NT == 0 || idx < H * L1)
-                ot[k].load(twG, (long)(i * H + idx % H) + (long)L2 * (idx / H));
+                ot[k].load(twG, (i * H + idx % H) + L2 * (idx / H));
         }
     };
     constexpr bool LATE = sizeof(T) == 4;
@@ -736,7 +773,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
         if (s < H) return rho;
         return rho == 0 ? L2 / 2 : L2 - rho;
     };
-    auto fetch = [&](int e, int s) __attribute__((always_inline)) { return z[(long)row_of(s) * L1 + e]; };
+    auto fetch = [&](int e, int s) __attribute__((always_inline)) { return z[(unsigned)(row_of(s) * L1 + e)]; };
     auto late = [&]() __attribute__((always_inline)) {
         if constexpr (LATE) load_ot();
     };
@@ -759,21 +796,21 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
         const int h = idx % H, r1 = idx / H;
         const int rho = i * H + h;
         if (rho != 0) {
-            long r = rho + (long)L2 * r1;
+            const int r = rho + L2 * r1;
             cplx<T> Zr = lds[lds_sw(r1 * W + h)];
             cplx<T> Zn = lds[lds_sw((L1 - 1 - r1) * W + (H + h))];
             emit_pair(skb, o, r, N, Zr, Zn, ot[k].get());
         } else {
             // row 0 (slot h=0): element r1 pairs with (L1 - r1) mod L1, r1 <= L1/2
             if (r1 <= L1 / 2) {
-                long r = (long)L2 * r1;
+                const int r = L2 * r1;
                 cplx<T> Zr = lds[lds_sw(r1 * W + 0)];
                 cplx<T> Zn = lds[lds_sw(((L1 - r1) & (L1 - 1)) * W + 0)];
                 emit_pair(skb, o, r, N, Zr, Zn, ot[k].get());
             }
             // row L2/2 (slot H): element r1 pairs with L1-1-r1, r1 < L1/2
             if (r1 < L1 / 2) {
-                long r = L2 / 2 + (long)L2 * r1;
+                const int r = L2 / 2 + L2 * r1;
                 cplx<T> Zr = lds[lds_sw(r1 * W + H)];
                 cplx<T> Zn = lds[lds_sw((L1 - 1 - r1) * W + H)];
                 emit_pair(skb, o, r, N, Zr, Zn, twG(r));
@@ -800,7 +837,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long s
     const cplx<T> *z = src + b * src_stride;
     TableStage<T, (TAB ? L1 : 1), NT> tab;
     if constexpr (TAB) tab.load(tw, tid);
-    auto fetch = [&](int e, int h) __attribute__((always_inline)) { return z[(long)(i * H + h) * L1 + e]; };
+    auto fetch = [&](int e, int h) __attribute__((always_inline)) { return z[(unsigned)((i * H + h) * L1 + e)]; };
     if constexpr (TAB) {
         auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
         lds_fft<T, S, LG1, H, NT, MR>(lds, (const cplx<T> *)twl, fetch, hook);
@@ -810,7 +847,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long s
     cplx<T> *o = dst + b * dst_stride;
     for (int idx = tid; idx < H * L1; idx += NT) {
         const int h = idx % H, r1 = idx / H;
-        o[(i * H + h) + (long)L2 * r1] = lds[lds_sw(r1 * H + h)];
+        *row_at(o, (i * H + h) + L2 * r1) = lds[lds_sw(r1 * H + h)];
     }
 }
 

@@ -1394,13 +1394,13 @@ struct FixedOf<double> {
     __device__ static I round(double v) { return __double2ll_rn(v); }
 };
 
-// Spectrum value A[r] of the real grid from the pair (Z[r], Z[N-r]) of its
+// Spectrum value 2 A[r] of the real grid from the pair (Z[r], Z[N-r]) of its
 // complex transform (the first of the two values emit_pair produces).
 template <typename T>
 __device__ __forceinline__ cplx<T> real_spectrum_at(cplx<T> Zr, cplx<T> Znr, cplx<T> wr) {
     cplx<T> c = conjg(Znr);
-    cplx<T> E = (Zr + c) * T(0.5);
-    cplx<T> D = (Zr - c) * T(0.5);
+    cplx<T> E = Zr + c;
+    cplx<T> D = Zr - c;
     return E + wr * cmk(D.y, -D.x);
 }
 
@@ -1603,7 +1603,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         const SinkAccurate<T> &sk = A.sink;
         const cplx<T> a = real_spectrum_at(z[lds_sw(f)], z[lds_sw((N - f) & (N - 1))], twG(f));
         const T kk = (T)f * sk.invG;
-        return a * (sk.pref * dexp(sk.coef * kk * kk));
+        return a * ((T(0.5) * sk.pref) * dexp(sk.coef * kk * kk));
     };
 
     for (;;) {
@@ -1628,13 +1628,12 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             SinkAccurate<T> sk = A.sink;
             cplx<T> *o = (tr == 0 ? A.out_y : A.out_w) + ((long)ci * A.nbs + rep) * sk.M;
             for (int r = tid; r <= N / 2; r += NT)
-                emit_pair(sk, o, (long)r, (long)N, z[lds_sw(r)], z[lds_sw((N - r) & (N - 1))],
-                          twG(r));
+                emit_pair(sk, o, r, N, z[lds_sw(r)], z[lds_sw((N - r) & (N - 1))], twG(r));
             __syncthreads();
         } else {
             const int rep = rem;
             const long row = (long)ci * A.nbs + rep;
-            const int half = (int)(A.sink.M / 2);
+            const int half = A.sink.M / 2;
             // moments of the drawn values about the first draw (shifted sums
             // keep the variance accurate when |mean| >> spread)
             double s1 = 0.0, s2 = 0.0;
