@@ -507,19 +507,11 @@ bool Plan<T>::bootstrap_fused_ok(bool window) const {
            (!window || has_pts2);
 }
 
-// partial maxima of |y| per curve: the longest curve's values in at most two
-// rounds of kAbsmaxLoads loads per thread, up to 64 parts
-template <typename T>
-int Plan<T>::ymax_parts() const {
-    const long two_rounds = 2L * kAbsmaxLoads * kAbsmaxThreads;
-    return (int)std::min(64L, std::max(1L, ceil_div(pts.longest, two_rounds)));
-}
-
 template <typename T>
 void Plan<T>::prepare_bootstrap(int nbs, bool window, hipStream_t s) {
     if (bootstrap_fused_ok(window)) {
         counter.ensure(sizeof(int), s);
-        ymax.ensure(sizeof(T) * (size_t)ncurves() * ymax_parts(), s);
+        boot_curves.ensure(sizeof(BootCurve) * (size_t)ncurves(), s);
         cover.ensure(sizeof(int) * 2 * (size_t)ncurves(), s);
         return;
     }
@@ -528,7 +520,8 @@ void Plan<T>::prepare_bootstrap(int nbs, bool window, hipStream_t s) {
 }
 
 // arguments shared by both modes of the fused bootstrap kernel; computes
-// the per-curve cover (once per plan) and max |y| (every call) on stream s
+// the per-curve cover (once per plan) and the queue's entries (every call) on
+// stream s
 template <typename T>
 BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s) {
     const int nc = ncurves();
@@ -541,18 +534,14 @@ BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t 
         }
         cover_ready = true;
     }
-    launch_boot_prepare<T>(y, pts.coff.template as<int>(), nc, ymax_parts(), ymax.as<T>(),
+    launch_boot_prepare<T>(y, pts.coff.template as<int>(), pts.order.template as<int>(), cov,
+                           has_pts2 ? cov + nc : nullptr, nc, boot_curves.as<BootCurve>(),
                            counter.as<int>(), s);
     BootArgs<T> B{};
     B.rec_x = pts.rec_orig.template as<PointRec<T>>();
     B.rec_2x = has_pts2 ? pts2.rec_orig.template as<PointRec<T>>() : nullptr;
     B.y = y;
-    B.ymax = ymax.as<T>();
-    B.ymax_parts = ymax_parts();
-    B.cover_x = cov;
-    B.cover_2x = cov + nc;
-    B.coff = pts.coff.template as<int>();
-    B.order = pts.order.template as<int>();
+    B.curves = boot_curves.as<BootCurve>();
     B.counter = counter.as<int>();
     B.ncurves = nc;
     B.nbs = nbs;

@@ -131,6 +131,13 @@ constexpr int pass_log2(int lg, int p, int mr = 4) {
     return p < n ? mr : rem;
 }
 
+// log2 of the points that passes 0 .. p of a length-2^lg transform combine
+constexpr int cum_log2(int lg, int p, int mr) {
+    int c = 0;
+    for (int q = 0; q <= p; ++q) c += pass_log2(lg, q, mr);
+    return c;
+}
+
 // ------------------------------------------------------------ LDS layout --
 // Element a of the LDS FFT buffer is stored at lds_sw(a): bits 0-3 are XORed
 // with bits 4-7 and bit 4 with bit 8.  The map is a bijection within every
@@ -167,38 +174,46 @@ struct Tw2 {
     __host__ __device__ int n_lo() const { return 1 << lb; }
 };
 
-// Twiddles of a length-2^LG transform too long for a whole table in LDS: the
-// passes whose angles are multiples of 2 pi / 2^LT read the 2^LT-entry table in
-// LDS (the same values), the others the full one in global memory.  Their
-// lanes' indices are consecutive multiples of small numbers there, so a load
-// covers few cache lines; in the earlier passes every lane of a load has a line
-// of its own.  Measured with the earlier passes' twiddles in LDS: 2^13 values
-// 11.8 -> 9.4 us, 256 transforms of 2^14 34.0 -> 29.9 us (FP32).
-template <typename T, int LG, int LT>
-struct TwSplit {
-    const cplx<T> *lds;
-    const cplx<T> *glob;
-    template <int SHIFT>
-    __device__ __forceinline__ cplx<T> get(int kr) const {
-        if constexpr (SHIFT >= LG - LT)
-            return lds[kr << (SHIFT - (LG - LT))];
-        else
-            return glob[kr << SHIFT];
-    }
-};
-template <class TW>
-struct IsTwSplit : std::false_type {};
-template <typename T, int LG, int LT>
-struct IsTwSplit<TwSplit<T, LG, LT>> : std::true_type {};
+// Twiddle rows.  Pass p >= 1 (radix R, Ns = 2^LOGNS points combined before it)
+// multiplies element r of a butterfly by w_{R Ns}^{r k}, k < Ns.  Its table holds
+// R - 1 rows of Ns values, row r - 1 = w_{R Ns}^{r k}: a lane's entry is its own k (an
+// instruction offset picks the row), and lanes with consecutive k read
+// consecutive words, so a lookup costs one LDS read without address arithmetic
+// or bank conflicts.  (One table of w_L^e needs an index product per lookup and
+// strides of r L / (R Ns), which put 4 to 16 lanes on a bank.)  The tables of
+// the passes that combine at most 2^cap points follow each other.
+constexpr int rows_of_pass(int lg, int p, int mr) {
+    return (1 << cum_log2(lg, p, mr)) - (1 << cum_log2(lg, p - 1, mr));
+}
+constexpr int rows_offset(int lg, int p, int mr) {
+    int o = 0;
+    for (int q = 1; q < p; ++q) o += rows_of_pass(lg, q, mr);
+    return o;
+}
+constexpr int rows_count(int lg, int mr, int cap) {
+    int n = 0;
+    for (int q = 1; q < num_passes(lg, mr); ++q)
+        if (cum_log2(lg, q, mr) <= cap) n += rows_of_pass(lg, q, mr);
+    return n > 0 ? n : 1;
+}
 
-// v[r] *= w^(r k 2^SHIFT), r = 1 .. R-1 (conjugated for S = -1).  From the
-// two-level table (two LDS reads per entry) only w^(k 2^SHIFT) is read; the
-// other powers are products of depth <= log2 R: squarings for the powers of
-// two, and w^r = w^h w^(r-h) with h the largest power of two below r.  From
-// a plain table, or with POWERS off (fewer registers: several butterflies
-// per thread), every power is one lookup.
+// The rows of the passes up to 2^CAP points in LDS, and `rest` (w_L^e by index: a
+// table in global memory, or a two-level table) for the later ones.
+template <typename T, int CAP, class Rest>
+struct TwRows {
+    static constexpr int cap = CAP;
+    const cplx<T> *lds;
+    Rest rest;
+};
+
+// v[r] *= w^(r k 2^SHIFT), r = 1 .. R-1 (conjugated for S = -1), by index.  From
+// the two-level table (two LDS reads per entry) with POWERS only w^(k 2^SHIFT)
+// is read; the other powers are products of depth <= log2 R: squarings for the
+// powers of two, and w^r = w^h w^(r-h) with h the largest power of two below r.
+// Otherwise (fewer registers: several butterflies per thread) every power is
+// one lookup.
 template <typename T, int S, int R, int SHIFT, bool POWERS, class TW>
-__device__ __forceinline__ void apply_twiddles(cplx<T> *v, const TW &tw, int k) {
+__device__ __forceinline__ void apply_indexed(cplx<T> *v, const TW &tw, int k) {
     if constexpr (POWERS && std::is_same<TW, Tw2<T>>::value) {
         cplx<T> w[R];
         w[1] = tw[k << SHIFT];
@@ -213,14 +228,27 @@ __device__ __forceinline__ void apply_twiddles(cplx<T> *v, const TW &tw, int k) 
     } else {
 #pragma unroll
         for (int r = 1; r < R; ++r) {
-            cplx<T> t;
-            if constexpr (IsTwSplit<TW>::value)
-                t = tw.template get<SHIFT>(k * r);
-            else
-                t = tw[(k * r) << SHIFT];
+            cplx<T> t = tw[(k * r) << SHIFT];
             if constexpr (S < 0) t.y = -t.y;
             v[r] = v[r] * t;
         }
+    }
+}
+
+// twiddles of pass P of a length-2^LG transform (radices up to 2^MR)
+template <typename T, int S, int LG, int P, int MR, bool POWERS, class TW>
+__device__ __forceinline__ void apply_twiddles(cplx<T> *v, const TW &tw, int k) {
+    constexpr int LR = pass_log2(LG, P, MR), R = 1 << LR, CUM = cum_log2(LG, P, MR);
+    if constexpr (CUM <= TW::cap) {
+        const cplx<T> *row = tw.lds + rows_offset(LG, P, MR) + k;
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+            cplx<T> t = row[(r - 1) << (CUM - LR)];
+            if constexpr (S < 0) t.y = -t.y;
+            v[r] = v[r] * t;
+        }
+    } else {
+        apply_indexed<T, S, R, LG - CUM, POWERS>(v, tw.rest, k);
     }
 }
 
@@ -248,18 +276,17 @@ __device__ __forceinline__ void unroll(F &&f) {
 // W interleaved sequences of length L = 2^LG: element e of sequence w lives at
 // lds[lds_sw(e*W + w)].  Pass 0 reads its inputs through `ld(e, w)`; every pass writes
 // LDS; the routine returns with natural-order results in LDS after a barrier.
-// tw[e] = exp(+2 pi i e / L) (conjugated for S = -1).
+// `tw` is a TwRows (conjugated for S = -1).
 struct NoHook {
     __device__ __forceinline__ void operator()() const {}
 };
 
 // `hook` runs once, after pass 0 has issued its loads and before it writes
 // LDS (used to stage a twiddle table whose loads were issued earlier).
-// `tw` is a table pointer or any object with operator[](int) giving w_L^e.
-template <typename T, int S, int LG, int W, int NT, int P, int LOGNS, class Loader,
-          bool INPLACE = false, class Hook = NoHook, class TW = const cplx<T> *, int MR = 4>
-__device__ __forceinline__ void fft_pass(cplx<T> *lds, TW tw, const Loader &ld,
-                                         const Hook &hook = Hook()) {
+template <typename T, int S, int LG, int W, int NT, int P, int LOGNS, class Loader, bool INPLACE,
+          class Hook, class TW, int MR>
+__device__ __forceinline__ void fft_pass(cplx<T> *lds, const TW &tw, const Loader &ld,
+                                         const Hook &hook) {
     constexpr int NP = num_passes(LG, MR);
     if constexpr (P < NP) {
         constexpr int LR = pass_log2(LG, P, MR);
@@ -294,8 +321,7 @@ __device__ __forceinline__ void fft_pass(cplx<T> *lds, TW tw, const Loader &ld,
                 // (with several butterflies per thread that would hold all
                 // their twiddles in registers at once; they follow it then)
                 if constexpr (P > 0 && BPT == 1)
-                    apply_twiddles<T, S, R, LG - LOGNS - LR, true>(v[q], tw,
-                                                                  j & ((1 << LOGNS) - 1));
+                    apply_twiddles<T, S, LG, P, MR, true>(v[q], tw, j & ((1 << LOGNS) - 1));
             }
         }
         if constexpr (P == 0) hook();
@@ -309,7 +335,7 @@ __device__ __forceinline__ void fft_pass(cplx<T> *lds, TW tw, const Loader &ld,
                 const int w = g % W, j = g / W;
                 const int k = j & ((1 << LOGNS) - 1);
                 if constexpr (P > 0 && BPT > 1)
-                    apply_twiddles<T, S, R, LG - LOGNS - LR, (R <= 4)>(v[q], tw, k);
+                    apply_twiddles<T, S, LG, P, MR, (R <= 4)>(v[q], tw, k);
                 dft<T, R, S>(v[q]);
                 const int base = ((j >> LOGNS) << (LOGNS + LR)) + k;
                 // bits [LOGNS, LOGNS + LR) of base are zero
@@ -327,10 +353,9 @@ __device__ __forceinline__ void fft_pass(cplx<T> *lds, TW tw, const Loader &ld,
 
 // MR: log2 of the largest radix (4: 16 values per butterfly; 3: 8, so that
 // twice the threads share the work)
-template <typename T, int S, int LG, int W, int NT, int MR = 4, class Loader, class Hook = NoHook,
-          class TW = const cplx<T> *>
-__device__ __forceinline__ void lds_fft(cplx<T> *lds, TW tw, const Loader &ld,
-                                        const Hook &hook = Hook()) {
+template <typename T, int S, int LG, int W, int NT, int MR, class Loader, class Hook, class TW>
+__device__ __forceinline__ void lds_fft(cplx<T> *lds, const TW &tw, const Loader &ld,
+                                        const Hook &hook) {
     fft_pass<T, S, LG, W, NT, 0, 0, Loader, false, Hook, TW, MR>(lds, tw, ld, hook);
 }
 
@@ -363,22 +388,22 @@ struct TableStage {
     }
 };
 
-// LDS twiddle tables pay off where a pass's table is small next to its data
-constexpr bool lds_table(int lg) { return lg <= 12; }
-// the LDS table of a longer single-workgroup transform (TwSplit): 2^11 entries,
-// which all passes but the last need at most
-constexpr int kSplitLg = 11;
-// entries of the LDS table of a single-workgroup transform
-constexpr int small_table(int lg) { return lds_table(lg) ? 1 << lg : 1 << kSplitLg; }
-
-// the data is already in `lds` in natural (unswizzled) order; transformed in
-// place, the result is in the swizzled layout
-template <typename T, int S, int LG, int NT, class TW>
-__device__ __forceinline__ void lds_fft_inplace(cplx<T> *lds, TW tw) {
-    auto fetch = [&](int e, int) __attribute__((always_inline)) { return lds[e]; };
-    fft_pass<T, S, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, TW>(lds, tw, fetch);
-}
-
+// Points up to which a single-workgroup transform's passes have their twiddle
+// rows in LDS: all of them up to 2^12; beyond, there is room for the passes up to
+// 2^11 points, and the last reads w_L^e from global memory, where its lanes'
+// indices are consecutive multiples of small numbers (few cache lines a load).
+constexpr int small_cap(int lg) { return lg <= 12 ? lg : 11; }
+// radix of a single-workgroup transform.  Radix 8 (8 values per thread, twice the
+// threads of radix 16) up to 2^12: a workgroup is a chain of passes, and more
+// waves shorten each.  Measured radix 16 -> 8 at 2^11: 6.1 -> 4.8 us (one
+// transform, FP32), 22.1 -> 18.1 us (2048), FP64 8.0 -> 6.2 and 44.2 -> 35.0 us.
+// At 2^13 radix 16 has a pass less and is as fast (9.4 against 9.6 us; 2^14 has
+// 1024 threads only in radix 16).
+constexpr int small_mr(int lg) { return lg >= 5 && lg <= 12 ? 3 : 4; }
+// The two-pass column and row kernels use radix-8 passes (8 values per
+// thread, twice the waves of radix 16): measured at N = 2^20, 0.8 and 1.1 us
+// faster per pass, the more waves per SIMD overlapping LDS work with loads.
+constexpr int kColMr = 3, kRowMr = 3;
 
 // Device twiddle tables, generated in long double on the host once per size
 // and kept for the life of the process (a few KB each).
@@ -400,10 +425,21 @@ class TwiddleCache {
         return t;
     }
 
+    // w_{2^lg}^e for e < count
+    const cplx<T> *head(int lg, long count) { return table(lg, 2, count); }
+    // the twiddle rows of the passes up to 2^cap points (see TwRows)
+    const cplx<T> *rows(int lg, int mr, int cap) {
+        return table(lg, 16 + 64 * mr + cap, rows_count(lg, mr, cap));
+    }
+
     // Every table an FFT of N = 2^lgN complex values (and its real-input
     // epilogue, G = 2N) may use, on the current device.
     void warm(int lgN) {
-        for (int l = 1; l <= std::min(lgN, 14); ++l) fine(l);
+        for (int l = 1; l <= std::min(lgN, 14); ++l) {
+            rows(l, small_mr(l), small_cap(l));
+            if (l <= 12) rows(l, kColMr, l);  // (kRowMr is the same)
+            if (l > 12) fine(l);
+        }
         two_level(lgN);
         two_level(lgN + 1);
     }
@@ -431,12 +467,23 @@ class TwiddleCache {
         require(!flag(), "twiddle table not prepared for this transform size",
                 CUNA_ERROR_INVALID_VALUE);
         std::vector<cplx<T>> h(count);
-        const long double two_pi = 6.283185307179586476925286766559005768L;
-        long N = 1L << lg;
-        for (long e = 0; e < count; ++e) {
-            long double a = two_pi * (long double)e / (long double)N;
-            h[e].x = (T)cosl(a);
-            h[e].y = (T)sinl(a);
+        auto root = [](long e, int l) {  // exp(2 pi i e / 2^l)
+            const long double two_pi = 6.283185307179586476925286766559005768L;
+            const long double a = two_pi * (long double)e / (long double)(1L << l);
+            return cmk((T)cosl(a), (T)sinl(a));
+        };
+        if (kind < 16) {
+            for (long e = 0; e < count; ++e) h[e] = root(e, lg);
+        } else {
+            const int mr = (kind - 16) / 64, cap = (kind - 16) % 64;
+            h[0] = cmk(T(1), T(0));
+            for (int p = 1; p < num_passes(lg, mr) && cum_log2(lg, p, mr) <= cap; ++p) {
+                const int cum = cum_log2(lg, p, mr), lr = pass_log2(lg, p, mr);
+                const long ns = 1L << (cum - lr);
+                cplx<T> *o = h.data() + rows_offset(lg, p, mr);
+                for (long r = 1; r < (1L << lr); ++r)
+                    for (long k = 0; k < ns; ++k) o[(r - 1) * ns + k] = root(r * k, cum);
+            }
         }
         void *d = nullptr;
         CUNA_HIP(hipMalloc(&d, sizeof(cplx<T>) * count));
@@ -532,8 +579,6 @@ __device__ __forceinline__ void emit_pair(const Sink &sk, cplx<T> *o, int r, int
 // Forward: the real grid read as complex z[n] (batch stride N).
 template <typename T>
 struct LoadGrid {
-    // plain loads: the kernel can afford to hold staged twiddles in registers
-    static constexpr bool kStage = true;
     const cplx<T> *z;
     long stride;  // per batch
     __device__ __forceinline__ void advance(long b) { z += b * stride; }
@@ -551,7 +596,6 @@ struct LoadGrid {
 // which takes two values of g, one D(k) and one twiddle.
 template <typename T>
 struct LoadHermitian {
-    static constexpr bool kStage = true;
     const cplx<T> *g;  // M values, natural order k = -M/2..M/2-1
     int parts;         // 2: batch row 2c + part holds the transform of (part ? -i : 1) g_c,
                        // whose grid gives the real and the imaginary part
@@ -593,10 +637,10 @@ struct LoadHermitian {
 
 // ------------------------------------------------------------- kernels --
 // Every kernel issues its twiddle loads together with its data loads: the
-// per-pass table goes to LDS (when small, lds_table) through the pass-0 hook,
+// twiddle rows go to LDS through the pass-0 hook,
 // and the epilogue's twiddles are fetched into registers up front, so the
 // workgroup waits on global memory once instead of once per pass.
-// Launch LDS: (sequences + (lds_table(LG) ? 1 : 0)) * 2^LG complex values.
+// Launch LDS: sequences * 2^LG + rows_count(...) complex values.
 
 // Two-level twiddle w(e) = lo[e mod B] * hi[e / B], split into its two loads
 // (issued early) and the product (formed late).
@@ -616,10 +660,9 @@ template <typename T, int S, int LG, int NT, class Loader, class Sink, int MODE,
 __global__ __launch_bounds__(NT) void k_fft_small(Loader ld, Sink sk, cplx<T> *plain_out,
                                                   const cplx<T> *tw, const cplx<T> *tw_lds,
                                                   Tw2<T> twG) {
-    // tw: the full table; tw_lds: the one staged in LDS (the same one if TAB)
+    // tw_lds: the rows staged in LDS; tw: w_N^e for the passes without (LG > 12)
     constexpr int N = 1 << LG;
-    constexpr bool TAB = lds_table(LG);
-    constexpr int NTAB = small_table(LG);
+    constexpr int CAP = small_cap(LG), NTAB = rows_count(LG, MR, CAP);
     constexpr int OPT = MODE == 0 ? (N / 2) / NT + 1 : 1;  // epilogue pairs per thread
     cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
     cplx<T> *twl = lds + N;
@@ -639,10 +682,7 @@ __global__ __launch_bounds__(NT) void k_fft_small(Loader ld, Sink sk, cplx<T> *p
     }
     auto fetch = [&](int e, int) __attribute__((always_inline)) { return lb.at(e); };
     auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
-    if constexpr (TAB)
-        lds_fft<T, S, LG, 1, NT, MR>(lds, (const cplx<T> *)twl, fetch, hook);
-    else
-        lds_fft<T, S, LG, 1, NT, MR>(lds, TwSplit<T, LG, kSplitLg>{twl, tw}, fetch, hook);
+    lds_fft<T, S, LG, 1, NT, MR>(lds, TwRows<T, CAP, const cplx<T> *>{twl, tw}, fetch, hook);
     if constexpr (MODE == 0) {
         const auto skb = sk.for_row(b);
         cplx<T> *o = sk.row_out(b);
@@ -668,11 +708,11 @@ template <typename T, int S, int LG2, int W, int NT, class Loader, int MR = 4>
 __global__ __launch_bounds__(NT) void k_fft_col(Loader ld, cplx<T> *dst, long dst_stride, int L1,
                                                 const cplx<T> *tw, Tw2<T> twN, long b0) {
     constexpr int L2 = 1 << LG2;
-    constexpr bool TAB = Loader::kStage && lds_table(LG2);
+    constexpr int NTAB = rows_count(LG2, MR, LG2);
     // FP32: the epilogue twiddles are loaded as the first pass's hook, after
     // its data loads (loads return in order, so the pass waits only for its
     // data), and held through the FFT
-    constexpr bool PRE = Loader::kStage && sizeof(T) == 4;
+    constexpr bool PRE = sizeof(T) == 4;
     constexpr int OPT = PRE ? (W * L2 + NT - 1) / NT : 1;
     cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
     cplx<T> *twl = lds + W * L2;
@@ -684,8 +724,8 @@ __global__ __launch_bounds__(NT) void k_fft_col(Loader ld, cplx<T> *dst, long ds
     const int n10 = blk * W;
     Loader lb = ld;
     lb.advance(b);
-    TableStage<T, (TAB ? L2 : 1), NT> tab;
-    if constexpr (TAB) tab.load(tw, tid);
+    TableStage<T, NTAB, NT> tab;
+    tab.load(tw, tid);
     Tw2Parts<T> ot[OPT];
     auto load_ot = [&]() __attribute__((always_inline)) {
         if constexpr (PRE) {
@@ -698,15 +738,11 @@ __global__ __launch_bounds__(NT) void k_fft_col(Loader ld, cplx<T> *dst, long ds
         }
     };
     auto fetch = [&](int e, int w) __attribute__((always_inline)) { return lb.at(n10 + w + L1 * e); };
-    if constexpr (TAB) {
-        auto hook = [&]() __attribute__((always_inline)) {
-            tab.store(twl, tid);
-            load_ot();
-        };
-        lds_fft<T, S, LG2, W, NT, MR>(lds, (const cplx<T> *)twl, fetch, hook);
-    } else {
-        lds_fft<T, S, LG2, W, NT, MR>(lds, tw, fetch, load_ot);
-    }
+    auto hook = [&]() __attribute__((always_inline)) {
+        tab.store(twl, tid);
+        load_ot();
+    };
+    lds_fft<T, S, LG2, W, NT, MR>(lds, TwRows<T, LG2, const cplx<T> *>{twl, tw}, fetch, hook);
     cplx<T> *o = dst + b * dst_stride;
     if constexpr (PRE) {
 #pragma unroll
@@ -739,7 +775,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
                                                      Tw2<T> twG, long b0) {
     constexpr int L1 = 1 << LG1;
     constexpr int W = 2 * H;
-    constexpr bool TAB = lds_table(LG1);
+    constexpr int NTAB = rows_count(LG1, MR, LG1);
     constexpr int OPT = (H * L1 + NT - 1) / NT;
     cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
     cplx<T> *twl = lds + W * L1;
@@ -750,8 +786,8 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
     const long b = b0 + bs.y;  // launches span at most kMaxGridY batches
     const int N = L1 * L2;
     const cplx<T> *z = src + b * src_stride;
-    TableStage<T, (TAB ? L1 : 1), NT> tab;
-    if constexpr (TAB) tab.load(tw, tid);
+    TableStage<T, NTAB, NT> tab;
+    tab.load(tw, tid);
     // epilogue twiddles for r = rho + L2 r1 (row 0 included; its mirror row
     // L2/2 takes its own below): in FP32 loaded as the first pass's hook,
     // after its data loads, so that the pass waits only for its data (loads
@@ -777,15 +813,11 @@ __global__ __launch_bounds__(NT) void k_fft_row_real(const cplx<T> *src, long sr
     auto late = [&]() __attribute__((always_inline)) {
         if constexpr (LATE) load_ot();
     };
-    if constexpr (TAB) {
-        auto hook = [&]() __attribute__((always_inline)) {
-            tab.store(twl, tid);
-            late();
-        };
-        lds_fft<T, 1, LG1, W, NT, MR>(lds, (const cplx<T> *)twl, fetch, hook);
-    } else {
-        lds_fft<T, 1, LG1, W, NT, MR>(lds, tw, fetch, late);
-    }
+    auto hook = [&]() __attribute__((always_inline)) {
+        tab.store(twl, tid);
+        late();
+    };
+    lds_fft<T, 1, LG1, W, NT, MR>(lds, TwRows<T, LG1, const cplx<T> *>{twl, tw}, fetch, hook);
     const auto skb = sk.for_row(b);
     cplx<T> *o = sk.row_out(b);
     // pairs: slot h, element r1 of the primary row with its mirror element
@@ -826,7 +858,7 @@ __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long s
                                                       int L2, cplx<T> *dst, long dst_stride,
                                                       const cplx<T> *tw, long b0) {
     constexpr int L1 = 1 << LG1;
-    constexpr bool TAB = lds_table(LG1);
+    constexpr int NTAB = rows_count(LG1, MR, LG1);
     cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
     cplx<T> *twl = lds + H * L1;
     const int tid = threadIdx.x;
@@ -835,15 +867,11 @@ __global__ __launch_bounds__(NT) void k_fft_row_plain(const cplx<T> *src, long s
     const int i = bs.x;
     const long b = b0 + bs.y;  // launches span at most kMaxGridY batches
     const cplx<T> *z = src + b * src_stride;
-    TableStage<T, (TAB ? L1 : 1), NT> tab;
-    if constexpr (TAB) tab.load(tw, tid);
+    TableStage<T, NTAB, NT> tab;
+    tab.load(tw, tid);
     auto fetch = [&](int e, int h) __attribute__((always_inline)) { return z[(unsigned)((i * H + h) * L1 + e)]; };
-    if constexpr (TAB) {
-        auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
-        lds_fft<T, S, LG1, H, NT, MR>(lds, (const cplx<T> *)twl, fetch, hook);
-    } else {
-        lds_fft<T, S, LG1, H, NT, MR>(lds, tw, fetch);
-    }
+    auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
+    lds_fft<T, S, LG1, H, NT, MR>(lds, TwRows<T, LG1, const cplx<T> *>{twl, tw}, fetch, hook);
     cplx<T> *o = dst + b * dst_stride;
     for (int idx = tid; idx < H * L1; idx += NT) {
         const int h = idx % H, r1 = idx / H;

@@ -45,10 +45,6 @@ static constexpr int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > h
 constexpr int fft_threads(int lg, int w, int mr = 4) {
     return clampi(((1 << lg) * w) >> mr, 64, 1024);
 }
-// The two-pass column and row kernels use radix-8 passes (8 values per
-// thread, twice the waves of radix 16): measured at N = 2^20, 0.8 and 1.1 us
-// faster per pass, the more waves per SIMD overlapping LDS work with loads.
-constexpr int kColMr = 3, kRowMr = 3;
 // sequences per workgroup so that the LDS tile stays at 64 KB
 template <typename T>
 constexpr int seq_per_wg(int lg, int cap) {
@@ -59,23 +55,17 @@ constexpr int split_lg1(int lgN) { return lgN / 2; }
 // largest log2 N of the single-workgroup inverse (Hermitian) transform
 constexpr int kC2rSmallLg = 13;
 
-// Radix 8 (8 values per thread, twice the threads of radix 16) up to 2^12: a
-// workgroup is a chain of passes, and more waves shorten each.  Measured radix
-// 16 -> 8 at 2^11: 6.1 -> 4.8 us (one transform, FP32), 22.1 -> 18.1 us (2048),
-// FP64 8.0 -> 6.2 and 44.2 -> 35.0 us.  At 2^13 radix 16 has a pass less and is
-// as fast (9.4 against 9.6 us; 2^14 has 1024 threads only in radix 16).
-constexpr int small_mr(int lg) { return lg >= 5 && lg <= 12 ? 3 : 4; }
-
 template <typename T, int S, int LG, class Loader, class Sink, int MODE>
 static void run_small(const FftShape &sh, const Loader &ld, const Sink &sk, cplx<T> *plain_out,
                       hipStream_t s) {
     constexpr int MR = small_mr(LG), NT = fft_threads(LG, 1, MR);
     auto &tc = TwiddleCache<T>::get();
-    const cplx<T> *tw = tc.fine(LG);
+    constexpr int CAP = small_cap(LG);
+    const cplx<T> *tw = LG > CAP ? tc.fine(LG) : nullptr;
+    const cplx<T> *tw_lds = tc.rows(LG, MR, CAP);
     Tw2<T> twG = tc.two_level(LG + 1);
-    const cplx<T> *tw_lds = lds_table(LG) ? tw : tc.fine(kSplitLg);
-    size_t lds = sizeof(cplx<T>) * (((size_t)1 << LG) + small_table(LG));
-    static_assert(sizeof(cplx<T>) * (((size_t)1 << LG) + small_table(LG)) <= kMaxLds, "FFT LDS");
+    constexpr size_t lds = sizeof(cplx<T>) * (((size_t)1 << LG) + rows_count(LG, MR, CAP));
+    static_assert(lds <= kMaxLds, "FFT LDS");
     auto k = k_fft_small<T, S, LG, NT, Loader, Sink, MODE, MR>;
     set_lds(k, lds);
     hipLaunchKernelGGL(k, dim3(sh.batch), dim3(NT), lds, s, ld, sk, plain_out, tw, tw_lds, twG);
@@ -87,14 +77,14 @@ static void run_col(const FftShape &sh, const Loader &ld, cplx<T> *dst, int L1, 
     constexpr int NT = fft_threads(LG2, W, kColMr);
     auto &tc = TwiddleCache<T>::get();
     const long N = 1L << sh.lgN;
-    size_t lds = (sizeof(cplx<T>) << LG2) * (W + (lds_table(LG2) ? 1 : 0));
+    const size_t lds = sizeof(cplx<T>) * (((size_t)W << LG2) + rows_count(LG2, kColMr, LG2));
     auto k = k_fft_col<T, S, LG2, W, NT, Loader, kColMr>;
     set_lds(k, lds);
     require(L1 % W == 0, "fft column split");
     for (long b0 = 0; b0 < sh.batch; b0 += kMaxGridY) {
         const int nb = (int)std::min<long>(kMaxGridY, sh.batch - b0);
-        hipLaunchKernelGGL(k, dim3(L1 / W, nb), dim3(NT), lds, s, ld, dst, N, L1, tc.fine(LG2),
-                           tc.two_level(sh.lgN), b0);
+        hipLaunchKernelGGL(k, dim3(L1 / W, nb), dim3(NT), lds, s, ld, dst, N, L1,
+                           tc.rows(LG2, kColMr, LG2), tc.two_level(sh.lgN), b0);
         CUNA_LAUNCH_CHECK();
     }
 }
@@ -105,14 +95,15 @@ static void run_row_real(const FftShape &sh, const cplx<T> *src, int L2, const S
     constexpr int NT = fft_threads(LG1, 2 * H, kRowMr);
     auto &tc = TwiddleCache<T>::get();
     const long N = 1L << sh.lgN;
-    size_t lds = (sizeof(cplx<T>) << LG1) * (2 * H + (lds_table(LG1) ? 1 : 0));
+    const size_t lds =
+        sizeof(cplx<T>) * (((size_t)(2 * H) << LG1) + rows_count(LG1, kRowMr, LG1));
     auto k = k_fft_row_real<T, LG1, H, NT, Sink, kRowMr>;
     set_lds(k, lds);
     require(L2 % (2 * H) == 0, "fft row split");
     for (long b0 = 0; b0 < sh.batch; b0 += kMaxGridY) {
         const int nb = (int)std::min<long>(kMaxGridY, sh.batch - b0);
         hipLaunchKernelGGL(k, dim3(L2 / (2 * H), nb), dim3(NT), lds, s, src, N, L2, sk,
-                           tc.fine(LG1), tc.two_level(sh.lgN + 1), b0);
+                           tc.rows(LG1, kRowMr, LG1), tc.two_level(sh.lgN + 1), b0);
         CUNA_LAUNCH_CHECK();
     }
 }
@@ -123,14 +114,14 @@ static void run_row_plain(const FftShape &sh, const cplx<T> *src, int L2, cplx<T
     constexpr int NT = fft_threads(LG1, H, kRowMr);
     auto &tc = TwiddleCache<T>::get();
     const long N = 1L << sh.lgN;
-    size_t lds = (sizeof(cplx<T>) << LG1) * (H + (lds_table(LG1) ? 1 : 0));
+    const size_t lds = sizeof(cplx<T>) * (((size_t)H << LG1) + rows_count(LG1, kRowMr, LG1));
     auto k = k_fft_row_plain<T, S, LG1, H, NT, kRowMr>;
     set_lds(k, lds);
     require(L2 % H == 0, "fft row split");
     for (long b0 = 0; b0 < sh.batch; b0 += kMaxGridY) {
         const int nb = (int)std::min<long>(kMaxGridY, sh.batch - b0);
-        hipLaunchKernelGGL(k, dim3(L2 / H, nb), dim3(NT), lds, s, src, N, L2, dst, N, tc.fine(LG1),
-                           b0);
+        hipLaunchKernelGGL(k, dim3(L2 / H, nb), dim3(NT), lds, s, src, N, L2, dst, N,
+                           tc.rows(LG1, kRowMr, LG1), b0);
         CUNA_LAUNCH_CHECK();
     }
 }
@@ -608,8 +599,9 @@ template <typename T, int LG, int NTAPS, int MODE>
 static void boot_fused_one(BootArgs<T> A, hipStream_t s) {
     constexpr int NT = fft_threads(LG, 1) < 256 ? 256 : fft_threads(LG, 1);
     auto &tc = TwiddleCache<T>::get();
+    A.twT = tc.rows(LG, kBootMr, boot_cap<T>(LG));
     A.twN = tc.two_level(LG);
-    A.twG = tc.two_level(LG + 1);
+    A.twH = tc.head(LG + 1, NT);
     const size_t lds = boot_lds_bytes<T>(LG);
     static_assert(boot_lds_bytes<T>(LG) <= kMaxLds, "fused bootstrap LDS");
     auto k = k_boot_fused<T, LG, NTAPS, NT, MODE>;
@@ -643,11 +635,11 @@ void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, in
 }
 
 template <typename T>
-void launch_boot_prepare(const T *y, const int *coff, int ncurves, int parts, T *ymax,
-                         int *counter, hipStream_t s) {
-    const int nblk = y ? ncurves * parts : 1;
-    hipLaunchKernelGGL(k_boot_prepare<T>, dim3(std::max(nblk, 1)), dim3(kAbsmaxThreads), 0, s,
-                       ncurves > 0 ? y : nullptr, coff, parts, ymax, counter);
+void launch_boot_prepare(const T *y, const int *coff, const int *order, const int *cover_x,
+                         const int *cover_2x, int ncurves, BootCurve *curves, int *counter,
+                         hipStream_t s) {
+    hipLaunchKernelGGL(k_boot_prepare<T>, dim3(ncurves), dim3(kPrepThreads), 0, s, y, coff, order,
+                       cover_x, cover_2x, curves, counter);
     CUNA_LAUNCH_CHECK();
 }
 
@@ -699,7 +691,7 @@ template bool boot_fused_supported<dTyp>(int, int);
 template void launch_boot_fused<dTyp>(BootArgs<dTyp>, int, int, int, hipStream_t);
 template void launch_curve_cover<dTyp>(const PointRec<dTyp> *, const int *, int, int, int, int *,
                                        hipStream_t);
-template void launch_boot_prepare<dTyp>(const dTyp *, const int *, int, int, dTyp *, int *,
-                                        hipStream_t);
+template void launch_boot_prepare<dTyp>(const dTyp *, const int *, const int *, const int *,
+                                        const int *, int, BootCurve *, int *, hipStream_t);
 
 }  // namespace cuna

@@ -101,10 +101,11 @@ template <typename T>
 void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, int G, int ntaps,
                         int *cover, hipStream_t s);
 template <typename T>
-// zeroes the work-queue head and, with y, fills `parts` partial maxima of |y|
-// per curve (launched before every fused bootstrap)
-void launch_boot_prepare(const T *y, const int *coff, int ncurves, int parts, T *ymax,
-                         int *counter, hipStream_t s);
+// zeroes the work-queue head and fills the queue's curve entries (with max |y|);
+// launched before every fused bootstrap
+void launch_boot_prepare(const T *y, const int *coff, const int *order, const int *cover_x,
+                         const int *cover_2x, int ncurves, BootCurve *curves, int *counter,
+                         hipStream_t s);
 template <typename T>
 // mode 0: spectra of y at x and of the window at 2x; 1: Lomb-Scargle power
 void launch_boot_fused(BootArgs<T> A, int lgN, int ntaps, int mode, hipStream_t s);

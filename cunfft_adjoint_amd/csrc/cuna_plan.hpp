@@ -154,8 +154,8 @@ struct Plan {
     bool has_pts2 = false;
     DevMem grid, work, counts, counter;
     std::unique_ptr<Bluestein<T>> blu;  // compat grids of any other length
-    // fused bootstrap: per-curve max |y| and densest tap window of x and 2x
-    DevMem ymax, cover;
+    // fused bootstrap: queue entries (BootCurve) and densest tap window of x and 2x
+    DevMem boot_curves, cover;
     DevMem ls_work;  // Lomb-Scargle: window spectra of the resident workgroups
     bool cover_ready = false;
     // optional profiling events, recorded on the execution stream before the
@@ -188,7 +188,6 @@ struct Plan {
     // the call can be captured into a graph without allocating)
     void prepare_bootstrap(int nbs, bool window, hipStream_t s);
     bool bootstrap_fused_ok(bool window) const;
-    int ymax_parts() const;
 
     SpreadArgs<T> spread_args(const TiledPoints<T> &P) const;
     GatherArgs<T> gather_args() const;

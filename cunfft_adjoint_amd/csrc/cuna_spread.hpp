@@ -1331,17 +1331,24 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
 // detected from the returned old value and the item is redone at a smaller
 // scale.  The integer grid occupies the same LDS words as the complex
 // buffer of the FFT, whose first pass reads and converts it.
+//
+// What an item needs of its curve, one entry per curve in queue order.
+struct BootCurve {
+    int ci, c0, nc;       // curve, its first point, its points
+    uint32_t fm_m;        // FastMod of max(nc, 1)
+    int fm_s1, fm_s2;
+    int cover_x, cover_2x;  // most points within one tap window
+    double ymax;          // max |y|, NaN values ignored (1 without y)
+};
+constexpr int kBootCurveWords = sizeof(BootCurve) / 4;
+static_assert(sizeof(BootCurve) == 40, "BootCurve is copied word by word");
+
 template <typename T>
 struct BootArgs {
     const PointRec<T> *rec_x;   // (anchor, frac) of x by original index
     const PointRec<T> *rec_2x;  // of 2x (window), nullable
     const T *y;                 // nullable: unit weights
-    const T *ymax;              // per curve ymax_parts partial maxima of |y| (when y is set)
-    int ymax_parts;
-    const int *cover_x;         // per curve: most points within one tap window
-    const int *cover_2x;
-    const int *coff;
-    const int *order;           // curves, longest first
+    const BootCurve *curves;    // longest first
     int *counter;               // work-queue head, zeroed before the launch
     cplx<T> *out_y, *out_w;
     int ncurves, nbs, ntr, total;
@@ -1349,8 +1356,9 @@ struct BootArgs {
     T bi, wscale;
     T e3[kMaxTaps];
     SinkAccurate<T> sink;       // out pointer set per item
+    const cplx<T> *twT;         // twiddle rows up to boot_cap (staged into LDS)
     Tw2<T> twN;                 // w_N^e, e < N (two-level, staged into LDS)
-    Tw2<T> twG;                 // w_G^e, e < G (two-level, staged into LDS)
+    const cplx<T> *twH;         // w_G^e, e < workgroup size
     // Lomb-Scargle mode (each nullable): per replicate, power at k = 0..M/2-1,
     // and its maximum over k >= 1 with the k where it occurs
     T *ls_power;
@@ -1362,16 +1370,41 @@ struct BootArgs {
     int ls_w_slots;
 };
 
-// LDS of the fused kernel: the grid (G reals = N complex) and the four
-// twiddle sub-tables (Tw2 of N and of G).
+// LDS of the fused kernel: the grid (G reals = N complex) between two halos of
+// kBootHalo cells, the twiddle rows of the passes of at most 2^cap points, and the
+// two sub-tables of w_N for the later ones.
+constexpr int kBootHalo = 32, kBootMr = 4;
+// cap: 18 KB of rows at FP32's largest grid, where one workgroup has a CU to
+// itself; a few KB where two share it
+template <typename T>
+__host__ __device__ constexpr int boot_cap(int lg) {
+    return sizeof(T) == 4 && lg == 14 ? 11 : lg < 10 ? lg : 10;
+}
 template <typename T>
 __host__ __device__ constexpr int boot_tw_entries(int lg) {
-    return (1 << ((lg + 1) / 2)) + (1 << (lg - (lg + 1) / 2)) + (1 << ((lg + 2) / 2)) +
-           (1 << (lg + 1 - (lg + 2) / 2));
+    return rows_count(lg, kBootMr, boot_cap<T>(lg)) + (1 << ((lg + 1) / 2)) +
+           (1 << (lg - (lg + 1) / 2));
 }
 template <typename T>
 __host__ __device__ constexpr size_t boot_lds_bytes(int lg) {
-    return sizeof(cplx<T>) * (((size_t)1 << lg) + (size_t)boot_tw_entries<T>(lg));
+    return sizeof(cplx<T>) * (((size_t)1 << lg) + (size_t)boot_tw_entries<T>(lg)) +
+           2 * kBootHalo * sizeof(T);
+}
+
+// cos and sin of 2 pi i / n for the epilogue's constant rotations (compile time
+// from a table of 2 pi / 32 multiples, n <= 32 a power of two)
+template <typename T>
+__device__ __forceinline__ constexpr cplx<T> unit_root_32(int i) {
+    constexpr double c[9] = {1.0,
+                             0.98078528040323044913,
+                             0.92387953251128675613,
+                             0.83146961230254523708,
+                             0.70710678118654752440,
+                             0.55557023301960222474,
+                             0.38268343236508977173,
+                             0.19509032201612826785,
+                             0.0};
+    return i <= 8 ? cplx<T>{(T)c[i], (T)c[8 - i]} : cplx<T>{(T)-c[16 - i], (T)c[i - 8]};
 }
 
 template <typename I>
@@ -1453,27 +1486,44 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     using U = std::make_unsigned_t<I>;
     static_assert(sizeof(I) == sizeof(T), "fixed-point grid aliases the real grid");
     constexpr int N = 1 << LG, G = 2 * N, Q0 = (NTAPS - 1) / 2;
-    constexpr int LBN = (LG + 1) / 2, LBG = (LG + 2) / 2;  // as TwiddleCache::two_level
-    constexpr int NLN = 1 << LBN, NHN = 1 << (LG - LBN), NLG = 1 << LBG, NHG = 1 << (LG + 1 - LBG);
+    constexpr int LBN = (LG + 1) / 2;  // as TwiddleCache::two_level
+    constexpr int NLN = 1 << LBN, NHN = 1 << (LG - LBN);
     constexpr int PB = 4;  // resampled points per thread whose loads are in flight together
     constexpr int kMaxExp = sizeof(T) == 4 ? 100 : 1000;
-    T *grid = reinterpret_cast<T *>(cuna_smem);
-    U *gu = reinterpret_cast<U *>(cuna_smem);
-    cplx<T> *z = reinterpret_cast<cplx<T> *>(cuna_smem);
-    cplx<T> *tl = z + N;  // twiddle sub-tables, staged once per workgroup
+    // the grid's cell 0; kBootHalo cells before it and after cell G - 1 take the
+    // taps that wrap, so that a tap's cell needs no reduction mod G
+    T *grid = reinterpret_cast<T *>(cuna_smem) + kBootHalo;
+    U *gu = reinterpret_cast<U *>(grid);
+    cplx<T> *z = reinterpret_cast<cplx<T> *>(grid);
+    cplx<T> *tl = reinterpret_cast<cplx<T> *>(grid + G + kBootHalo);  // staged once per workgroup
+    constexpr int CAP = boot_cap<T>(LG), NLT = rows_count(LG, kBootMr, CAP);
     const int tid = threadIdx.x;
-    for (int i = tid; i < NLN; i += NT) tl[i] = A.twN.lo[i];
-    for (int i = tid; i < NHN; i += NT) tl[NLN + i] = A.twN.hi[i];
-    for (int i = tid; i < NLG; i += NT) tl[NLN + NHN + i] = A.twG.lo[i];
-    for (int i = tid; i < NHG; i += NT) tl[NLN + NHN + NLG + i] = A.twG.hi[i];
-    Tw2<T> twN, twG;
-    twN.lo = tl;
-    twN.hi = tl + NLN;
-    twN.lb = LBN;
-    twG.lo = tl + NLN + NHN;
-    twG.hi = tl + NLN + NHN + NLG;
-    twG.lb = LBG;
-    __shared__ int item_sh;
+    for (int i = tid; i < NLT; i += NT) tl[i] = A.twT[i];
+    for (int i = tid; i < NLN; i += NT) tl[NLT + i] = A.twN.lo[i];
+    for (int i = tid; i < NHN; i += NT) tl[NLT + NLN + i] = A.twN.hi[i];
+    TwRows<T, CAP, Tw2<T>> tw;
+    tw.lds = tl;
+    tw.rest.lo = tl + NLT;
+    tw.rest.hi = tl + NLT + NLN;
+    tw.rest.lb = LBN;
+    // the epilogue's twiddle w_G^(tid + i NT) = w_G^tid w_(G/NT)^i
+    constexpr int NE = (N / 2 + NT) / NT;  // values of i with tid + i NT <= N/2
+    static_assert(G / NT <= 32 || NE <= 1, "epilogue rotations");
+    const cplx<T> wtid = A.twH[tid];
+    // (thread index and twiddle opaque in each item's epilogue, and its steps
+    // kept apart: the compiler would hoist every step's addresses and rotations
+    // out of the item loop and spill them)
+    auto epilogue = [&](auto &&step) __attribute__((always_inline)) {
+        int t = tid;
+        cplx<T> w0 = wtid;
+        asm volatile("" : "+v"(t), "+v"(w0.x), "+v"(w0.y));
+        unroll<NE>([&](auto i) __attribute__((always_inline)) {
+            constexpr int k = decltype(i)::value;
+            step(t + k * NT, k == 0 ? w0 : w0 * unit_root_32<T>(k * (G / NT > 0 ? 32 * NT / G : 1)));
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    __shared__ int item_sh[kBootCurveWords + 1];
     __shared__ int dmax_sh[NT / 64];
     // draws per block of 32 anchors (at most G/32 = 1024 blocks)
     constexpr int NB = G / 32;
@@ -1485,9 +1535,11 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
 
     // Grid of one transform: the draws of replicate `rep` of the curve at
     // c0 (nc points), positions from P, values y[d] - shift (or 1), |value|
-    // <= vm; spread in fixed point, converted, transformed in place into z.
+    // <= vm; spread in fixed point and transformed in place into z.  Returns the
+    // power of two that the spectrum is to be multiplied by: the integers go
+    // through the FFT as they are.
     auto transform = [&](int c0, int nc, int rep, const FastMod &fm, const PointRec<T> *P,
-                         const T *y, T shift, double vm, int cover) __attribute__((always_inline)) {
+                         const T *y, T shift, double vm, int cover) __attribute__((always_inline)) -> T {
         int sexp = 0;
         if (vm <= 1e300) {  // false for NaN and inf
             // No cell receives more than cnt weights of size <= vm * wscale, so
@@ -1500,10 +1552,12 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             int cnt = 4 * max(cover, 1);
             for (int attempt = 0; attempt < 2; ++attempt) {
                 const double bound = vm * (double)cnt * (double)A.wscale;
-                const int e = bound > 0 ? (int)ceil(log2(bound)) : -kMaxExp;
+                int e = -kMaxExp;  // ceil(log2(bound))
+                if (bound > 0 && frexp(bound, &e) == 0.5) --e;
                 sexp = min(max(FixedOf<T>::headroom_bits - e, -kMaxExp), kMaxExp);
                 const T mul = (T)ldexp((double)A.wscale, sexp);
-                for (int i = tid; i < G; i += NT) gu[i] = U(0);
+                for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
+                    reinterpret_cast<uint4 *>(cuna_smem)[i] = make_uint4(0, 0, 0, 0);
                 for (int i = tid; i < NB; i += NT) hist_sh[i] = 0;
                 __syncthreads();
                 for (int p0 = 0; p0 < nc; p0 += NT * PB) {
@@ -1531,27 +1585,30 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
 #pragma unroll
                     for (int k = 0; k < PB; ++k) {
                         if (p0 + k * NT + tid < nc) {
-                            const int base = pr[k].a - Q0;
+                            U *dst = gu + (pr[k].a - Q0);
                             if constexpr (sizeof(T) == 4) {
                                 // each tap's rounded weight to its atomic as
                                 // it is formed (weights <= 2^headroom_bits)
                                 tap_fixed<T, NTAPS, Fixed32, true>(
-                                    vv[k] * mul, pr[k].e, A.bi, A.e3, T(0), [&](int q, unsigned n) {
-                                        atomicAdd(&gu[(base + q) & (G - 1)], (U)n);
-                                    });
+                                    vv[k] * mul, pr[k].e, A.bi, A.e3, T(0),
+                                    [&](int q, unsigned n) { atomicAdd(dst + q, (U)n); });
                             } else {
                                 T w[NTAPS];
                                 tap_weights<T, NTAPS>(vv[k] * mul, pr[k].e, A.bi, A.e3, w);
 #pragma unroll
                                 for (int q = 0; q < NTAPS; ++q)
-                                    atomicAdd(&gu[(base + q) & (G - 1)],
-                                              (U)FixedOf<T>::round(w[q]));
+                                    atomicAdd(dst + q, (U)FixedOf<T>::round(w[q]));
                             }
                             atomicAdd(&hist_sh[pr[k].a >> 5], 1);
                         }
                     }
                 }
                 __syncthreads();
+                // the taps that wrapped (distinct cells, read after the next barrier)
+                if (tid < kBootHalo) {
+                    gu[G - kBootHalo + tid] += gu[tid - kBootHalo];
+                    gu[tid] += gu[G + tid];
+                }
                 int dmax = 0;
                 for (int b = tid; b < NB; b += NT)
                     dmax = max(dmax, hist_sh[b] + hist_sh[(b + 1) & (NB - 1)]);
@@ -1562,73 +1619,83 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
                 dmax = dmax_sh[0];
 #pragma unroll
                 for (int w = 1; w < NT / 64; ++w) dmax = max(dmax, dmax_sh[w]);
-                // every thread has read dmax_sh before the next attempt or item
-                // writes it (the FFT and the emit below have barriers too)
-                __syncthreads();
                 if (dmax <= cnt) break;  // uniform
                 cnt = dmax;
+                __syncthreads();  // every thread has read dmax_sh
             }
-            const T inv = (T)ldexp(1.0, -sexp);
-            if constexpr (MODE == 0) {
-                // the FFT's first pass reads the fixed-point grid (complex e
-                // = cells 2e, 2e+1) and converts it to reals as it loads
-                auto fetch = [&](int e, int) __attribute__((always_inline)) {
-                    const FixedPair<I> q = reinterpret_cast<const FixedPair<I> *>(gu)[e];
-                    return cmk((T)q.x * inv, (T)q.y * inv);
-                };
-                fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, Tw2<T>>(z, twN,
-                                                                                    fetch);
-            } else {
-                // (Lomb-Scargle keeps the window spectrum in registers; with
-                // the transform outside this branch it needs fewer of them)
-                for (int i = tid; i < G; i += NT) grid[i] = (T)(I)gu[i] * inv;
-            }
-        } else {
-            // a non-finite value: every spectrum value is NaN
-            for (int i = tid; i < G; i += NT) grid[i] = (T)NAN;
-            if constexpr (MODE == 0) __syncthreads();
         }
-        if constexpr (MODE == 1) {
-            __syncthreads();
-            lds_fft_inplace<T, 1, LG, NT>(z, twN);
-        }
+        // the FFT's first pass reads the fixed-point grid (complex e = cells
+        // 2e, 2e+1) and converts it to reals as it loads
+        auto fetch = [&](int e, int) __attribute__((always_inline)) {
+            const FixedPair<I> q = reinterpret_cast<const FixedPair<I> *>(gu)[e];
+            return cmk((T)q.x, (T)q.y);
+        };
+        __syncthreads();
+        fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, decltype(tw), kBootMr>(
+            z, tw, fetch, NoHook());
+        // a non-finite value makes every spectrum value NaN
+        return vm <= 1e300 ? (T)ldexp(1.0, -sexp) : (T)NAN;
     };
-    auto curve_ymax = [&](int ci) {
-        T m = A.ymax[ci * A.ymax_parts];
-        for (int p = 1; p < A.ymax_parts; ++p) m = fmax(m, A.ymax[ci * A.ymax_parts + p]);
-        return (double)m;
-    };
-    // deconvolved spectrum at frequency f (0 <= f < M/2) from z
-    auto spectrum = [&](int f) __attribute__((always_inline)) -> cplx<T> {
+    // deconvolved spectrum, times `scale`, at frequency f (0 <= f < M/2) from z
+    auto spectrum = [&](int f, cplx<T> w, T scale) __attribute__((always_inline)) -> cplx<T> {
         const SinkAccurate<T> &sk = A.sink;
-        const cplx<T> a = real_spectrum_at(z[lds_sw(f)], z[lds_sw((N - f) & (N - 1))], twG(f));
+        const cplx<T> a = real_spectrum_at(z[lds_sw(f)], z[lds_sw((N - f) & (N - 1))], w);
         const T kk = (T)f * sk.invG;
-        return a * ((T(0.5) * sk.pref) * dexp(sk.coef * kk * kk));
+        return a * ((T(0.5) * sk.pref * scale) * dexp(sk.coef * kk * kk));
     };
 
+    // The first wave takes the next item off the queue while the workgroup
+    // works on the current one, and has its curve's entry in LDS by the end: an
+    // item then starts without a chain of global loads.
+    const int per_curve = A.nbs * (MODE == 0 ? A.ntr : 1);
+    const int lane = tid & 63;
+    const bool first_wave = tid < 64;
+    auto take = [&]() __attribute__((always_inline)) -> int {
+        return lane == 0 ? atomicAdd(A.counter, 1) : 0;
+    };
+    auto stage_item = [&](int item) __attribute__((always_inline)) {
+        item = __builtin_amdgcn_readfirstlane(item);
+        int w = -1;
+        if (item < A.total) {
+            const int pos = item / per_curve;
+            if (lane < kBootCurveWords)
+                w = reinterpret_cast<const int *>(A.curves + pos)[lane];
+            else if (lane == kBootCurveWords)
+                w = item - pos * per_curve;
+        }
+        if (lane <= kBootCurveWords) item_sh[lane] = w;  // (rem < 0: no item left)
+    };
+    if (first_wave) stage_item(take());
+    __syncthreads();
     for (;;) {
-        if (tid == 0) item_sh = atomicAdd(A.counter, 1);
-        __syncthreads();
-        // uniform over the workgroup: scalar registers (so are the curve's
-        // offsets and sizes loaded through it)
-        const int item = __builtin_amdgcn_readfirstlane(item_sh);
-        if (item >= A.total) break;  // uniform over the workgroup
-        const int per_curve = A.nbs * (MODE == 0 ? A.ntr : 1);
-        const int ci = A.order[item / per_curve];
-        const int rem = item % per_curve;
-        const int c0 = A.coff[ci];
-        const int nc = A.coff[ci + 1] - c0;
+        // uniform over the workgroup: scalar registers
+        auto word = [&](int k) { return __builtin_amdgcn_readfirstlane(item_sh[k]); };
+        const int rem = word(kBootCurveWords);
+        if (rem < 0) break;  // uniform over the workgroup
+        const int ci = word(0), c0 = word(1), nc = word(2);
         FastMod fm;
-        fm.init((uint32_t)max(nc, 1));
+        fm.d = (uint32_t)max(nc, 1);
+        fm.m = (uint32_t)word(3);
+        fm.s1 = word(4);
+        fm.s2 = word(5);
+        const int cover_x = word(6), cover_2x = word(7);
+        const double ymax = __longlong_as_double(((long long)word(9) << 32) | (unsigned)word(8));
+        int next = 0;
+        if (first_wave) next = take();
         if constexpr (MODE == 0) {
             const int rep = rem / A.ntr, tr = rem % A.ntr;
             const bool usey = tr == 0 && A.y;
-            transform(c0, nc, rep, fm, tr == 0 ? A.rec_x : A.rec_2x, usey ? A.y : nullptr, T(0),
-                      usey ? curve_ymax(ci) : 1.0, tr == 0 ? A.cover_x[ci] : A.cover_2x[ci]);
+            const T scale = transform(c0, nc, rep, fm, tr == 0 ? A.rec_x : A.rec_2x,
+                                      usey ? A.y : nullptr, T(0), usey ? ymax : 1.0,
+                                      tr == 0 ? cover_x : cover_2x);
+            if (first_wave) stage_item(next);
             SinkAccurate<T> sk = A.sink;
+            sk.pref *= scale;
             cplx<T> *o = (tr == 0 ? A.out_y : A.out_w) + ((long)ci * A.nbs + rep) * sk.M;
-            for (int r = tid; r <= N / 2; r += NT)
-                emit_pair(sk, o, r, N, z[lds_sw(r)], z[lds_sw((N - r) & (N - 1))], twG(r));
+            epilogue([&](int r, cplx<T> w) __attribute__((always_inline)) {
+                if (r <= N / 2)
+                    emit_pair(sk, o, r, N, z[lds_sw(r)], z[lds_sw((N - r) & (N - 1))], w);
+            });
             __syncthreads();
         } else {
             const int rep = rem;
@@ -1682,23 +1749,28 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             const T ybar = (T)((double)shift + mean_off);
             const T yy = (T)fmax(0.0, s2 - s1 * mean_off);
             // window W(2w), parked in this workgroup's workspace row
-            transform(c0, nc, rep, fm, A.rec_2x, nullptr, T(0), 1.0, A.cover_2x[ci]);
+            const T wscale = transform(c0, nc, rep, fm, A.rec_2x, nullptr, T(0), 1.0, cover_2x);
             cplx<T> *wrow = A.ls_w + (long)blockIdx.x * half;
-            for (int f = tid; f < half; f += NT) wrow[f] = spectrum(f);
+            epilogue([&](int f, cplx<T> w) __attribute__((always_inline)) {
+                if (f < half) wrow[f] = spectrum(f, w, wscale);
+            });
             __syncthreads();
             // F(w) of the mean-subtracted values, then the power
-            const double vm = curve_ymax(ci) + fabs((double)ybar);
-            transform(c0, nc, rep, fm, A.rec_x, A.y, ybar, vm, A.cover_x[ci]);
+            const double vm = ymax + fabs((double)ybar);
+            const T yscale = transform(c0, nc, rep, fm, A.rec_x, A.y, ybar, vm, cover_x);
+            if (first_wave) stage_item(next);
             T best = T(-1);
             int kbest = 0;
-            for (int f = tid; f < half; f += NT) {
-                const T pw = ls_power(spectrum(f), wrow[f], (T)nc, yy);
-                if (A.ls_power) A.ls_power[row * half + f] = pw;
-                if (f >= 1 && pw > best) {
-                    best = pw;
-                    kbest = f;
+            epilogue([&](int f, cplx<T> w) __attribute__((always_inline)) {
+                if (f < half) {
+                    const T pw = ls_power(spectrum(f, w, yscale), wrow[f], (T)nc, yy);
+                    if (A.ls_power) A.ls_power[row * half + f] = pw;
+                    if (f >= 1 && pw > best) {
+                        best = pw;
+                        kbest = f;
+                    }
                 }
-            }
+            });
             if (A.ls_peak || A.ls_kpeak) {
                 // block arg-max (ties: smallest k)
 #pragma unroll
@@ -1731,37 +1803,54 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     }
 }
 
-// Work-queue head := 0, and per-curve max |y| (NaN values ignored) in `parts`
-// partial maxima out[c * parts + p], part p taking every parts-th block of the
-// curve's values.  Latency-bound: a thread keeps 8 loads in flight, and the
-// host picks the parts so that it needs few rounds of them.  One workgroup of
-// 256 threads per curve with one load in flight took 80 us for 128 curves of up
-// to 50,000 values, and resetting the queue was a launch of its own (4.7 us).
-constexpr int kAbsmaxThreads = 256, kAbsmaxLoads = 8;
+// Queue head := 0, and one BootCurve per workgroup (position in the queue order)
+// with the curve's max |y|.  Latency-bound: a thread keeps 8 loads in flight.
+// One workgroup of 256 threads per curve with one load in flight took 80 us for
+// 128 curves of up to 50,000 values, and resetting the queue was a launch of its
+// own (4.7 us).
+constexpr int kPrepThreads = 1024, kPrepLoads = 8;
 template <typename T>
-__global__ __launch_bounds__(kAbsmaxThreads) void k_boot_prepare(const T *y, const int *coff,
-                                                                 int parts, T *out, int *counter) {
+__global__ __launch_bounds__(kPrepThreads) void k_boot_prepare(const T *y, const int *coff,
+                                                               const int *order,
+                                                               const int *cover_x,
+                                                               const int *cover_2x,
+                                                               BootCurve *curves, int *counter) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0;
-    if (!y) return;
-    const int c = blockIdx.x / parts, p = blockIdx.x % parts;
-    const int b = coff[c], e = coff[c + 1];
+    const int ci = order[blockIdx.x];
+    const int b = coff[ci], e = coff[ci + 1];
     T m = T(0);
-    const long step = (long)parts * kAbsmaxThreads;
-    for (long i = b + (long)p * kAbsmaxThreads + threadIdx.x; i < e; i += kAbsmaxLoads * step) {
-        T v[kAbsmaxLoads];
+    if (y) {
+        for (long i = b + (long)threadIdx.x; i < e; i += kPrepLoads * kPrepThreads) {
+            T v[kPrepLoads];
 #pragma unroll
-        for (int k = 0; k < kAbsmaxLoads; ++k) v[k] = y[i + k * step < e ? i + k * step : i];
+            for (int k = 0; k < kPrepLoads; ++k)
+                v[k] = y[i + k * kPrepThreads < e ? i + k * kPrepThreads : i];
 #pragma unroll
-        for (int k = 0; k < kAbsmaxLoads; ++k) m = fmax(m, fabs(v[k]));
+            for (int k = 0; k < kPrepLoads; ++k) m = fmax(m, fabs(v[k]));
+        }
+    } else {
+        m = T(1);
     }
-    __shared__ T red[kAbsmaxThreads / 64];
+    __shared__ T red[kPrepThreads / 64];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < kAbsmaxThreads / 64; ++w) m = fmax(m, red[w]);
-        out[blockIdx.x] = m;
+        for (int w = 1; w < kPrepThreads / 64; ++w) m = fmax(m, red[w]);
+        FastMod fm;
+        fm.init((uint32_t)max(e - b, 1));
+        BootCurve c;
+        c.ci = ci;
+        c.c0 = b;
+        c.nc = e - b;
+        c.fm_m = fm.m;
+        c.fm_s1 = fm.s1;
+        c.fm_s2 = fm.s2;
+        c.cover_x = cover_x[ci];
+        c.cover_2x = cover_2x ? cover_2x[ci] : 0;
+        c.ymax = (double)m;
+        curves[blockIdx.x] = c;
     }
 }
 
