@@ -401,7 +401,7 @@ void Plan<T>::prepare_fft(hipStream_t s) {
     }
     require(spec.mode == CUNA_MODE_COMPAT, "accurate-mode grids are powers of two");
     blu = std::make_unique<Bluestein<T>>();
-    blu->init(G, s);
+    blu->init(G, true, s);
     blu->ensure(std::max(ncurves(), 1), s);
 }
 
@@ -1712,7 +1712,7 @@ CUNA_API int cuna_fft(Complex *data, int n, int batch, int sign, hipStream_t str
             // reference creates its cuFFT plan on every call); the call
             // waits for its stream before the workspace is released
             Bluestein<R> b;
-            b.init(n, stream);
+            b.init(n, false, stream);
             b.ensure(batch, stream);
             b.run_complex(reinterpret_cast<cplx<R> *>(data), batch, sign, stream);
             CUNA_HIP(hipStreamSynchronize(stream));

@@ -3,170 +3,421 @@
 //
 // The reference's cuFFT stage takes any ng (cufftPlan1d / cufftPlanMany,
 // src/cuna_kernel.cu:82,169,208,261; its test program uses ng = R*N,
-// test.cpp:114).  Here a real grid of ng cells is transformed through
-//   A[r] = c_r * sum_g (z_g c_g) conj(c_{r-g}),  c_k = exp(+i pi k^2/ng),
-// with the convolution done circularly at L = 2^lgL >= 2 ng - 1.  The chirp
-// is tabulated on the host in long double from k^2 mod 2 ng (exact integer),
-// so its phase carries no error that grows with k.
+// test.cpp:114).  A length-n transform is
+//   A[r] = c_r * sum_g (z_g c_g) conj(c_{r-g}),  c_k = exp(+i pi k^2/n),
+// with the convolution done circularly at L = 2^lgL >= 2 n - 1.  A real grid of
+// even ng is read as n = ng/2 complex values, and its spectrum recovered from
+// Z[r], Z[n-r] as in the power-of-two path; an odd one is transformed as n = ng
+// complex values.  The chirp is tabulated on the host in long double from
+// k^2 mod 2 n (exact integer), so its phase carries no error that grows with k.
+//
+// The chirp products, the two FFTs and the product with the convolution kernel's
+// transform are fused: one launch when L fits a workgroup's LDS, else three (the
+// first column pass reads and premultiplies the grid; a row pass transforms each
+// row forward, multiplies and transforms it back in LDS; the last column pass
+// applies the chirp and writes the output), plus the even grid's pairing.  Bound
+// by the passes' loads and stores, as the power-of-two FFT.  Measured at ng =
+// 300,000, FP32: 63 us in seven launches over L = 2^20 -> 27 us
+// in four over 2^19 (rocprofv3 sums).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 
+#include "cuna_dispatch.hpp"
 #include "cuna_plan.hpp"
 
 namespace cuna {
 
-// a[b][i] = c_i * z[b][i] for i < ng, 0 for ng <= i < L (z real, or complex
-// and optionally conjugated)
-template <typename T, class In>
-__global__ void k_chirp_premul(const In *z, long zstride, int ng, const cplx<T> *chirp, long L,
-                               int batch, int conj_in, cplx<T> *a) {
-    for (int b = blockIdx.y; b < batch; b += gridDim.y) {
-        for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < L;
-             i += (long)gridDim.x * blockDim.x) {
-            cplx<T> v = cmk(T(0), T(0));
-            if (i < ng) {
-                if constexpr (std::is_same<In, T>::value) {
-                    v = chirp[i] * z[b * zstride + i];
-                } else {
-                    cplx<T> w = z[b * zstride + i];
-                    if (conj_in) w.y = -w.y;
-                    v = chirp[i] * w;
-                }
-            }
-            a[(long)b * L + i] = v;
+// z_g c_g, zero from n on: the input of the first transform (row stride `stride`
+// in elements of the source)
+template <typename T>
+struct LoadChirp {
+    const cplx<T> *zc;  // complex values (a real grid's pairs), or
+    const T *zr;        // a real grid of odd length
+    const cplx<T> *chirp;
+    long stride;
+    int n;
+    int conj_in;
+    __device__ __forceinline__ void advance(long b) {
+        if (zr)
+            zr += b * stride;
+        else
+            zc += b * stride;
+    }
+    __device__ __forceinline__ cplx<T> at(int g) const {
+        if (g >= n) return cmk(T(0), T(0));
+        const cplx<T> c = chirp[(unsigned)g];
+        if (zr) return c * zr[(unsigned)g];
+        cplx<T> w = zc[(unsigned)g];
+        if (conj_in) w.y = -w.y;
+        return c * w;
+    }
+};
+
+// what becomes of y_r, r < n: the transform is c_r y_r
+enum ChirpOut {
+    CHIRP_STORE = 0,   // kept in place (row stride L) for the pairing launch
+    CHIRP_COMPAT = 1,  // through the compat deconvolution (odd real grids)
+    CHIRP_PLAIN = 2    // data[b][r], conjugated on request
+};
+template <typename T>
+struct ChirpSink {
+    const cplx<T> *chirp;
+    int n, mode, conj_out;
+    cplx<T> *data;  // CHIRP_STORE / CHIRP_PLAIN
+    long stride;
+    SinkCompat<T> sk;  // CHIRP_COMPAT
+    // the sink of batch row b (its data pointer advanced)
+    __device__ __forceinline__ ChirpSink for_row(long b) const {
+        ChirpSink r = *this;
+        if (mode == CHIRP_COMPAT) {
+            r.sk = sk.for_row(b);
+            r.data = sk.row_out(b);
+        } else {
+            r.data = data + b * stride;
+        }
+        return r;
+    }
+    __device__ __forceinline__ void operator()(int r, cplx<T> y) const {
+        if (r >= n) return;
+        cplx<T> v = chirp[(unsigned)r] * y;
+        if (mode == CHIRP_COMPAT) v = v * sk.fac(r);
+        if (mode == CHIRP_PLAIN && conj_out) v.y = -v.y;
+        *row_at(data, r) = v;
+    }
+};
+
+// Row pass of the convolution: H consecutive rows r2 of the L1-contiguous data
+// per workgroup.  Length-L1 transform (sign -1), product with bt (the kernel's
+// transform over L, row-major: bt[r2 L1 + r1] = bhat[r2 + L2 r1] / L), length-L1
+// transform (sign +1) and the twiddle w_L^(r2 n1), in place.
+template <typename T, int LG1, int H, int NT, int MR>
+__global__ __launch_bounds__(NT) void k_chirp_row(cplx<T> *a, long stride, int L2,
+                                                  const cplx<T> *bt, const cplx<T> *tw,
+                                                  Tw2<T> twL, long b0) {
+    constexpr int L1 = 1 << LG1, NTAB = rows_count(LG1, MR, LG1);
+    constexpr int NV = (H * L1 + NT - 1) / NT;
+    static_assert(NV <= (1 << MR), "one butterfly per thread");
+    cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
+    cplx<T> *twl = lds + H * L1;
+    const int tid = threadIdx.x;
+    const int2 bs = xcd_block(blockIdx.x, blockIdx.y, L2 / H, gridDim.y);
+    const int i = bs.x;
+    cplx<T> *z = a + (b0 + bs.y) * stride;
+    TableStage<T, NTAB, NT> tab;
+    tab.load(tw, tid);
+    // the kernel's values in the order in which the second transform's first
+    // pass takes them, and the epilogue's twiddles: loaded behind the data
+    cplx<T> bv[1 << MR];
+    Tw2Parts<T> ot[NV];
+    auto row_index = [&](int e, int h) __attribute__((always_inline)) {
+        return (unsigned)((i * H + h) * L1 + e);
+    };
+    auto fetch = [&](int e, int h) __attribute__((always_inline)) { return z[row_index(e, h)]; };
+    auto hook = [&]() __attribute__((always_inline)) {
+        tab.store(twl, tid);
+        constexpr int Q = L1 >> pass_log2(LG1, 0, MR);
+#pragma unroll
+        for (int r = 0; r < (1 << pass_log2(LG1, 0, MR)); ++r)
+            if ((H * Q) % NT == 0 || tid < H * Q) bv[r] = bt[row_index(tid / H + r * Q, tid % H)];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const int idx = tid + k * NT;
+            if ((H * L1) % NT == 0 || idx < H * L1)
+                ot[k].load(twL, (i * H + idx % H) * (idx / H));
+        }
+    };
+    const TwRows<T, LG1, const cplx<T> *> rows{twl, tw};
+    lds_fft<T, -1, LG1, H, NT, MR>(lds, rows, fetch, hook);
+    int nv = 0;
+    auto product = [&](int e, int h) __attribute__((always_inline)) {
+        return lds[lds_sw(e * H + h)] * bv[nv++];
+    };
+    fft_pass<T, 1, LG1, H, NT, 0, 0, decltype(product), true, NoHook, decltype(rows), MR>(
+        lds, rows, product, NoHook());
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int idx = tid + k * NT;
+        if ((H * L1) % NT == 0 || idx < H * L1) {
+            const int h = idx % H, n1 = idx / H;
+            z[row_index(n1, h)] = lds[lds_sw(n1 * H + h)] * ot[k].get();
         }
     }
 }
 
-// a[b][k] *= bhat[k] * scale
-template <typename T>
-__global__ void k_chirp_mul(cplx<T> *a, const cplx<T> *bhat, long L, int batch, T scale) {
-    for (int b = blockIdx.y; b < batch; b += gridDim.y) {
-        for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < L;
-             k += (long)gridDim.x * blockDim.x) {
-            a[(long)b * L + k] = a[(long)b * L + k] * bhat[k] * scale;
-        }
+// Last column pass: W columns n1 per workgroup, length-L2 transform over r2 (sign
+// +1); element n2 of column n1 is y_r, r = n1 + L1 n2.
+template <typename T, int LG2, int W, int NT, int MR>
+__global__ __launch_bounds__(NT) void k_chirp_col(const cplx<T> *a, long stride, int L1,
+                                                  ChirpSink<T> sink, const cplx<T> *tw, long b0) {
+    constexpr int L2 = 1 << LG2, NTAB = rows_count(LG2, MR, LG2);
+    cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
+    cplx<T> *twl = lds + W * L2;
+    const int tid = threadIdx.x;
+    const int2 bs = xcd_block(blockIdx.x, blockIdx.y, L1 / W, gridDim.y);
+    const int n10 = bs.x * W;
+    const long b = b0 + bs.y;
+    const cplx<T> *z = a + b * stride;
+    TableStage<T, NTAB, NT> tab;
+    tab.load(tw, tid);
+    auto fetch = [&](int e, int w) __attribute__((always_inline)) {
+        return z[(unsigned)(n10 + w + L1 * e)];
+    };
+    auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
+    lds_fft<T, 1, LG2, W, NT, MR>(lds, TwRows<T, LG2, const cplx<T> *>{twl, tw}, fetch, hook);
+    const ChirpSink<T> sk = sink.for_row(b);
+    for (int idx = tid; idx < W * L2; idx += NT) {
+        const int w = idx % W, n2 = idx / W;
+        sk(n10 + w + L1 * n2, lds[lds_sw(n2 * W + w)]);
     }
 }
 
-// compat sink: out row b, r < ng: c_r conv[b][r] * normfac exp((r/ng)^2 b/4)
+// The spectrum of an even real grid from Z[r] = conv row b, r < n = ng/2
+// (A[r] and A[n-r] from the pair Z[r], Z[n-r]; wr = exp(2 pi i r/ng)).
 template <typename T>
-__global__ void k_chirp_post_compat(const cplx<T> *conv, long L, int ng, const cplx<T> *chirp,
-                                    int batch, SinkCompat<T> sk) {
+__global__ __launch_bounds__(256) void k_chirp_pairs(const cplx<T> *Z, long L, int n,
+                                                     const cplx<T> *wng, int batch,
+                                                     SinkCompat<T> sk) {
     for (int b = blockIdx.y; b < batch; b += gridDim.y) {
         const SinkCompat<T> skb = sk.for_row(b);
         cplx<T> *o = sk.row_out(b);
-        for (long r = (long)blockIdx.x * blockDim.x + threadIdx.x; r < ng;
-             r += (long)gridDim.x * blockDim.x)
-            o[r] = chirp[r] * conv[(long)b * L + r] * skb.fac(r);
+        const cplx<T> *z = Z + b * L;
+        for (int r = blockIdx.x * blockDim.x + threadIdx.x; r <= n / 2; r += gridDim.x * blockDim.x)
+            emit_pair(skb, o, r, n, z[r], z[r == 0 ? 0 : n - r], wng[r]);
     }
 }
 
-// plain output, in place: data[b][r] = c_r conv[b][r] (conjugated on request)
-template <typename T>
-__global__ void k_chirp_post_plain(const cplx<T> *conv, long L, int ng, const cplx<T> *chirp,
-                                   int batch, int conj_out, cplx<T> *data) {
-    for (int b = blockIdx.y; b < batch; b += gridDim.y) {
-        for (long r = (long)blockIdx.x * blockDim.x + threadIdx.x; r < ng;
-             r += (long)gridDim.x * blockDim.x) {
-            cplx<T> v = chirp[r] * conv[(long)b * L + r];
-            if (conj_out) v.y = -v.y;
-            data[(long)b * ng + r] = v;
+// The whole transform of one batch row in LDS (L = 2^LG).  bt[k] = bhat[k] / L;
+// wng: the pairing twiddles of an even real grid, else null.
+template <typename T, int LG, int NT, int MR>
+__global__ __launch_bounds__(NT) void k_chirp_small(LoadChirp<T> ld, ChirpSink<T> sink,
+                                                    const cplx<T> *bt, const cplx<T> *wng,
+                                                    const cplx<T> *tw, const cplx<T> *tw_rows) {
+    constexpr int L = 1 << LG, CAP = small_cap(LG), NTAB = rows_count(LG, MR, CAP);
+    cplx<T> *lds = reinterpret_cast<cplx<T> *>(cuna_smem);
+    cplx<T> *twl = lds + L;
+    const int tid = threadIdx.x;
+    const long b = blockIdx.x;
+    LoadChirp<T> lb = ld;
+    lb.advance(b);
+    TableStage<T, NTAB, NT> tab;
+    tab.load(tw_rows, tid);
+    auto fetch = [&](int e, int) __attribute__((always_inline)) { return lb.at(e); };
+    auto hook = [&]() __attribute__((always_inline)) { tab.store(twl, tid); };
+    const TwRows<T, CAP, const cplx<T> *> rows{twl, tw};
+    lds_fft<T, -1, LG, 1, NT, MR>(lds, rows, fetch, hook);
+    auto product = [&](int e, int) __attribute__((always_inline)) {
+        return lds[lds_sw(e)] * bt[(unsigned)e];
+    };
+    fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(product), true, NoHook, decltype(rows), MR>(
+        lds, rows, product, NoHook());
+    const ChirpSink<T> sk = sink.for_row(b);
+    const int n = sk.n;
+    if (wng) {
+        for (int r = tid; r <= n / 2; r += NT) {
+            const int rn = r == 0 ? 0 : n - r;
+            emit_pair(sk.sk, sk.data, r, n, sk.chirp[r] * lds[lds_sw(r)],
+                      sk.chirp[rn] * lds[lds_sw(rn)], wng[r]);
         }
+    } else {
+        for (int r = tid; r < n; r += NT) sk(r, lds[lds_sw(r)]);
     }
 }
 
-static dim3 elem_grid(long n, int batch) {
-    const long bx = std::min<long>(ceil_div(std::max(n, 1L), 256), 4096);
-    return dim3((unsigned)bx, (unsigned)std::min(std::max(batch, 1), 65535));
+// b_k = b_{L-k} = conj(c_k), k < n, zero between
+template <typename T>
+__global__ void k_chirp_kernel(const cplx<T> *chirp, int n, long L, cplx<T> *out) {
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= L) return;
+    const long m = k < n ? k : L - k;
+    out[k] = m < n ? conjg(chirp[m]) : cmk(T(0), T(0));
+}
+// bt[r2 L1 + r1] = bhat[r2 + L2 r1] * scale
+template <typename T>
+__global__ void k_chirp_rows(const cplx<T> *bhat, int L1, int L2, T scale, cplx<T> *bt) {
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= (long)L1 * L2) return;
+    const long r2 = k / L1, r1 = k % L1;
+    bt[k] = bhat[r2 + (long)L2 * r1] * scale;
 }
 
 template <typename T>
-void Bluestein<T>::init(int ng_, hipStream_t s) {
-    require(ng_ >= 1, "transform length must be positive");
-    ng = ng_;
-    lgL = std::max(1, ilog2(2L * ng - 1));
+void Bluestein<T>::init(int length, bool real, hipStream_t s) {
+    require(length >= 1, "transform length must be positive");
+    ng = length;
+    pairs = real && length % 2 == 0;
+    n = pairs ? length / 2 : length;
+    lgL = std::max(1, ilog2(2L * n - 1));
     L = 1L << lgL;
     require(lgL <= max_fft_lg<T>(), "transform length too large", CUNA_ERROR_UNSUPPORTED);
     const long double pi = 3.141592653589793238462643383279502884L;
-    chirp_h.resize(ng);
-    for (long k = 0; k < ng; ++k) {
-        const unsigned long long q = ((unsigned long long)k * (unsigned long long)k) %
-                                     (2ull * (unsigned long long)ng);
-        const long double a = pi * (long double)q / (long double)ng;
-        chirp_h[k] = cmk((T)cosl(a), (T)sinl(a));
+    const int nw = pairs ? n / 2 + 1 : 0;
+    tab_h.resize((size_t)n + nw);
+    for (long k = 0; k < n; ++k) {
+        const unsigned long long q =
+            ((unsigned long long)k * (unsigned long long)k) % (2ull * (unsigned long long)n);
+        const long double a = pi * (long double)q / (long double)n;
+        tab_h[k] = cmk((T)cosl(a), (T)sinl(a));
     }
-    b_h.assign(L, cmk(T(0), T(0)));
-    for (long k = 0; k < ng; ++k) {
-        const cplx<T> v = conjg(chirp_h[k]);
-        b_h[k] = v;
-        if (k > 0) b_h[L - k] = v;
+    for (long r = 0; r < nw; ++r) {
+        const long double a = 2 * pi * (long double)r / (long double)ng;
+        tab_h[n + r] = cmk((T)cosl(a), (T)sinl(a));
     }
-    chirp.alloc(sizeof(cplx<T>) * ng, s);
-    bhat.alloc(sizeof(cplx<T>) * L, s);
-    CUNA_HIP(hipMemcpyAsync(chirp.ptr, chirp_h.data(), sizeof(cplx<T>) * ng,
+    tab.alloc(sizeof(cplx<T>) * tab_h.size(), s);
+    bt.alloc(sizeof(cplx<T>) * L, s);
+    CUNA_HIP(hipMemcpyAsync(tab.ptr, tab_h.data(), sizeof(cplx<T>) * tab_h.size(),
                             hipMemcpyHostToDevice, s));
-    CUNA_HIP(hipMemcpyAsync(bhat.ptr, b_h.data(), sizeof(cplx<T>) * L, hipMemcpyHostToDevice, s));
     TwiddleCache<T>::get().warm(lgL);
     ensure(1, s);
+    // the kernel's transform, scaled, in the order in which the passes take it
+    // (bt is the FFT's workspace before it receives the result)
+    cplx<T> *const w = work.as<cplx<T>>();
+    hipLaunchKernelGGL(k_chirp_kernel<T>, dim3(ceil_div(L, 256)), dim3(256), 0, s, chirp(), n, L,
+                       w);
+    CUNA_LAUNCH_CHECK();
     FftShape sh;
     sh.lgN = lgL;
     sh.batch = 1;
-    fft_complex<T>(sh, bhat.as<cplx<T>>(), work.as<cplx<T>>() + L, -1, s);
+    fft_complex<T>(sh, w, bt.as<cplx<T>>(), -1, s);
+    const int lg1 = lgL <= max_small_lg<T>() ? 0 : split_lg1(lgL);
+    hipLaunchKernelGGL(k_chirp_rows<T>, dim3(ceil_div(L, 256)), dim3(256), 0, s, w, 1 << lg1,
+                       1 << (lgL - lg1), T(1) / (T)L, bt.as<cplx<T>>());
+    CUNA_LAUNCH_CHECK();
 }
 
 template <typename T>
 void Bluestein<T>::ensure(int batch, hipStream_t s) {
     if (batch <= batch_cap) return;
-    work.alloc(sizeof(cplx<T>) * (size_t)L * 2 * (size_t)batch, s);
+    work.alloc(sizeof(cplx<T>) * (size_t)L * (size_t)batch, s);
     batch_cap = batch;
+}
+
+template <typename T>
+void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch,
+                       hipStream_t s) {
+    require(batch <= batch_cap, "Bluestein workspace too small for this batch");
+    auto &tc = TwiddleCache<T>::get();
+    const cplx<T> *const wng = pairs ? chirp() + n : nullptr;
+    if (lgL <= max_small_lg<T>()) {
+        dispatch_lg<1, max_small_lg<T>()>(lgL, [&](auto c) {
+            constexpr int LG = decltype(c)::value, MR = small_mr(LG), CAP = small_cap(LG);
+            constexpr int NT = fft_threads(LG, 1, MR);
+            constexpr size_t lds =
+                sizeof(cplx<T>) * (((size_t)1 << LG) + rows_count(LG, MR, CAP));
+            auto k = k_chirp_small<T, LG, NT, MR>;
+            set_lds(k, lds);
+            hipLaunchKernelGGL(k, dim3(batch), dim3(NT), lds, s, ld, sink, bt.as<cplx<T>>(), wng,
+                               LG > CAP ? tc.fine(LG) : nullptr, tc.rows(LG, MR, CAP));
+            CUNA_LAUNCH_CHECK();
+        });
+        return;
+    }
+    const int lg1 = split_lg1(lgL), lg2 = lgL - lg1, L1 = 1 << lg1, L2 = 1 << lg2;
+    const int W = pick_seq<T>(lg2, L1, batch, 1, "CUNA_FFT_W", 0, num_cus());
+    const int H = pick_seq<T>(lg1, L2, batch, 1, "CUNA_FFT_H", 0, num_cus());
+    cplx<T> *const a = work.as<cplx<T>>();
+    auto batches = [&](auto &&launch) {
+        for (long b0 = 0; b0 < batch; b0 += kMaxGridY) {
+            launch(b0, (int)std::min<long>(kMaxGridY, batch - b0));
+            CUNA_LAUNCH_CHECK();
+        }
+    };
+    dispatch_lg<7, 12>(lg2, [&](auto c) {
+        constexpr int LG2 = decltype(c)::value;
+        dispatch_w<T, LG2>(W, [&](auto w) {
+            constexpr int WW = decltype(w)::value, NT = fft_threads(LG2, WW, kColMr);
+            constexpr size_t lds =
+                sizeof(cplx<T>) * (((size_t)WW << LG2) + rows_count(LG2, kColMr, LG2));
+            auto k = k_fft_col<T, -1, LG2, WW, NT, LoadChirp<T>, kColMr>;
+            set_lds(k, lds);
+            batches([&](long b0, int nb) {
+                hipLaunchKernelGGL(k, dim3(L1 / WW, nb), dim3(NT), lds, s, ld, a, L, L1,
+                                   tc.rows(LG2, kColMr, LG2), tc.two_level(lgL), b0);
+            });
+        });
+    });
+    dispatch_lg<7, 12>(lg1, [&](auto c) {
+        constexpr int LG1 = decltype(c)::value;
+        dispatch_w<T, LG1>(H, [&](auto h) {
+            constexpr int HH = decltype(h)::value, NT = fft_threads(LG1, HH, kRowMr);
+            constexpr size_t lds =
+                sizeof(cplx<T>) * (((size_t)HH << LG1) + rows_count(LG1, kRowMr, LG1));
+            auto k = k_chirp_row<T, LG1, HH, NT, kRowMr>;
+            set_lds(k, lds);
+            batches([&](long b0, int nb) {
+                hipLaunchKernelGGL(k, dim3(L2 / HH, nb), dim3(NT), lds, s, a, L, L2,
+                                   bt.as<cplx<T>>(), tc.rows(LG1, kRowMr, LG1), tc.two_level(lgL),
+                                   b0);
+            });
+        });
+    });
+    ChirpSink<T> out = sink;
+    if (pairs) {
+        out.mode = CHIRP_STORE;
+        out.data = a;
+        out.stride = L;
+    }
+    dispatch_lg<7, 12>(lg2, [&](auto c) {
+        constexpr int LG2 = decltype(c)::value;
+        dispatch_w<T, LG2>(W, [&](auto w) {
+            constexpr int WW = decltype(w)::value, NT = fft_threads(LG2, WW, kColMr);
+            constexpr size_t lds =
+                sizeof(cplx<T>) * (((size_t)WW << LG2) + rows_count(LG2, kColMr, LG2));
+            auto k = k_chirp_col<T, LG2, WW, NT, kColMr>;
+            set_lds(k, lds);
+            batches([&](long b0, int nb) {
+                hipLaunchKernelGGL(k, dim3(L1 / WW, nb), dim3(NT), lds, s, a, L, L1, out,
+                                   tc.rows(LG2, kColMr, LG2), b0);
+            });
+        });
+    });
+    if (pairs) {
+        const long bx = std::min<long>(ceil_div(n / 2 + 1, 256), 4096);
+        hipLaunchKernelGGL(k_chirp_pairs<T>, dim3(bx, std::min(batch, kMaxGridY)), dim3(256), 0, s,
+                           a, L, n, wng, batch, sink.sk);
+        CUNA_LAUNCH_CHECK();
+    }
 }
 
 template <typename T>
 void Bluestein<T>::run_real(const T *grid, long gstride, int batch, const SinkCompat<T> &sk,
                             hipStream_t s) {
-    require(batch <= batch_cap, "Bluestein workspace too small for this batch");
-    cplx<T> *a = work.as<cplx<T>>();
-    cplx<T> *tmp = a + (size_t)L * batch;
-    hipLaunchKernelGGL((k_chirp_premul<T, T>), elem_grid(L, batch), dim3(256), 0, s, grid,
-                       gstride, ng, chirp.as<cplx<T>>(), L, batch, 0, a);
-    CUNA_LAUNCH_CHECK();
-    FftShape sh;
-    sh.lgN = lgL;
-    sh.batch = batch;
-    fft_complex<T>(sh, a, tmp, -1, s);
-    hipLaunchKernelGGL(k_chirp_mul<T>, elem_grid(L, batch), dim3(256), 0, s, a,
-                       bhat.as<cplx<T>>(), L, batch, T(1) / (T)L);
-    CUNA_LAUNCH_CHECK();
-    fft_complex<T>(sh, a, tmp, 1, s);
-    hipLaunchKernelGGL(k_chirp_post_compat<T>, elem_grid(ng, batch), dim3(256), 0, s, a, L, ng,
-                       chirp.as<cplx<T>>(), batch, sk);
-    CUNA_LAUNCH_CHECK();
+    LoadChirp<T> ld{};
+    ld.chirp = chirp();
+    ld.n = n;
+    if (pairs) {
+        ld.zc = reinterpret_cast<const cplx<T> *>(grid);
+        ld.stride = gstride / 2;
+    } else {
+        ld.zr = grid;
+        ld.stride = gstride;
+    }
+    ChirpSink<T> sink{};
+    sink.chirp = chirp();
+    sink.n = n;
+    sink.mode = CHIRP_COMPAT;
+    sink.sk = sk;
+    run(ld, sink, batch, s);
 }
 
 template <typename T>
 void Bluestein<T>::run_complex(cplx<T> *data, int batch, int sign, hipStream_t s) {
-    require(batch <= batch_cap, "Bluestein workspace too small for this batch");
     // sign -1 as the conjugate of the sign +1 transform of the conjugate
-    const int cj = sign < 0 ? 1 : 0;
-    cplx<T> *a = work.as<cplx<T>>();
-    cplx<T> *tmp = a + (size_t)L * batch;
-    hipLaunchKernelGGL((k_chirp_premul<T, cplx<T>>), elem_grid(L, batch), dim3(256), 0, s, data,
-                       (long)ng, ng, chirp.as<cplx<T>>(), L, batch, cj, a);
-    CUNA_LAUNCH_CHECK();
-    FftShape sh;
-    sh.lgN = lgL;
-    sh.batch = batch;
-    fft_complex<T>(sh, a, tmp, -1, s);
-    hipLaunchKernelGGL(k_chirp_mul<T>, elem_grid(L, batch), dim3(256), 0, s, a,
-                       bhat.as<cplx<T>>(), L, batch, T(1) / (T)L);
-    CUNA_LAUNCH_CHECK();
-    fft_complex<T>(sh, a, tmp, 1, s);
-    hipLaunchKernelGGL(k_chirp_post_plain<T>, elem_grid(ng, batch), dim3(256), 0, s, a, L, ng,
-                       chirp.as<cplx<T>>(), batch, cj, data);
-    CUNA_LAUNCH_CHECK();
+    LoadChirp<T> ld{};
+    ld.zc = data;
+    ld.stride = ng;
+    ld.chirp = chirp();
+    ld.n = n;
+    ld.conj_in = sign < 0 ? 1 : 0;
+    ChirpSink<T> sink{};
+    sink.chirp = chirp();
+    sink.n = n;
+    sink.mode = CHIRP_PLAIN;
+    sink.conj_out = ld.conj_in;
+    sink.data = data;
+    sink.stride = ng;
+    run(ld, sink, batch, s);
 }
 
 template struct Bluestein<dTyp>;

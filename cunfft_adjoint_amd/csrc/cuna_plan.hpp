@@ -103,23 +103,30 @@ struct ModeSpec {
 // Bluestein (chirp-z) transform of length ng, for grids whose length is not
 // a power of two >= 4 (the reference hands any ng to cuFFT,
 // src/cuna_kernel.cu:82,169,208,261):
-//   A[r] = sum_g z_g e^{+2 pi i g r/ng} = c_r sum_g (z_g c_g) conj(c_{r-g}),
-//   c_k = exp(+i pi k^2/ng),
-// a circular convolution of length L = 2^lgL >= 2 ng - 1 done with the
+//   A[r] = sum_g z_g e^{+2 pi i g r/n} = c_r sum_g (z_g c_g) conj(c_{r-g}),
+//   c_k = exp(+i pi k^2/n),
+// a circular convolution of length L = 2^lgL >= 2 n - 1 done with the
 // power-of-two FFT: conv = FFT_+(FFT_-(z c) * FFT_-(b)) / L, with
-// b_k = b_{L-k} = conj(c_k) for 0 <= k < ng and zero between.
+// b_k = b_{L-k} = conj(c_k) for 0 <= k < n and zero between.
+template <typename T>
+struct LoadChirp;
+template <typename T>
+struct ChirpSink;
+
 template <typename T>
 struct Bluestein {
-    // host sources of the (async) uploads, declared first so that they are
-    // destroyed after the device buffers (whose hipFree synchronises)
-    std::vector<cplx<T>> chirp_h, b_h;
-    int ng = 0, lgL = 0;
+    // host source of the (async) upload, declared first so that it is destroyed
+    // after the device buffers (whose release synchronises)
+    std::vector<cplx<T>> tab_h;
+    int ng = 0, n = 0, lgL = 0;  // n: complex values transformed
+    bool pairs = false;          // an even real grid: n = ng/2 pairs of cells
     long L = 0;
-    DevMem chirp;  // c_k, k < ng
-    DevMem bhat;   // FFT_-(b), L values
-    DevMem work;   // batch_cap x L complex for the data and as much for the FFT passes
+    DevMem tab;   // c_k, k < n, then (pairs) exp(2 pi i r/ng), r <= n/2
+    DevMem bt;    // FFT_-(b) / L, in the order of the passes
+    DevMem work;  // batch_cap x L complex
     int batch_cap = 0;
-    void init(int ng_, hipStream_t s);
+    // real: run_real will be called (else run_complex)
+    void init(int length, bool real, hipStream_t s);
     void ensure(int batch, hipStream_t s);
     // real grids (batch rows of stride gstride, the first ng cells used) ->
     // the compat deconvolution sink, one row per grid
@@ -127,6 +134,10 @@ struct Bluestein {
                   hipStream_t s);
     // in place on batch x ng complex values: data[r] = sum_g data[g] e^{sign 2 pi i g r/ng}
     void run_complex(cplx<T> *data, int batch, int sign, hipStream_t s);
+
+  private:
+    const cplx<T> *chirp() const { return tab.template as<cplx<T>>(); }
+    void run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch, hipStream_t s);
 };
 
 // true when a real grid of G cells takes the power-of-two FFT (else Bluestein)
