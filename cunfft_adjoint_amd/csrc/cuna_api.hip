@@ -290,11 +290,8 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
 template <typename T>
 void TiledPoints<T>::sort_points(hipStream_t s) {
     const std::vector<int> &offsets = coff_h;
-    const int K1 = 1 << tlog;
-    // chunk table: chunks of at most CH points, never crossing a curve.  One
-    // wave ranks a chunk against per-chunk counts of every key: 512 points
-    // for the 256-key passes, up to 2048 for larger tiles (first digit)
-    const int CH = std::max(512, std::min(2048, 2 * K1));
+    // chunk table: chunks of at most CH points, never crossing a curve
+    const int CH = kSortChunk;
     std::vector<int4> chunks;
     std::vector<int> base(ncurves), nch(ncurves);
     int total_chunks = 0;
@@ -309,14 +306,13 @@ void TiledPoints<T>::sort_points(hipStream_t s) {
         }
         total_chunks += k;
     }
-    const long hist_len = (long)std::max(K1, 256) * std::max(total_chunks, 1);
+    const long hist_len = (1L << kSortBits) * std::max(total_chunks, 1);
     const long n1 = std::max<long>(n, 1);
     // the sort's stream-ordered temporaries, in one allocation
     Carve tc;
     const size_t o_chunks = tc.add(sizeof(int4) * std::max<size_t>(chunks.size(), 1));
     const size_t o_base = tc.add(sizeof(int) * ncurves);
     const size_t o_nch = tc.add(sizeof(int) * ncurves);
-    const size_t o_keys = tc.add(sizeof(int) * n1);
     const size_t o_recA = tc.add(sizeof(PointRec<T>) * n1);
     const size_t o_permA = tc.add(sizeof(int) * n1);
     const size_t o_hist = tc.add(sizeof(int) * hist_len);
@@ -325,13 +321,12 @@ void TiledPoints<T>::sort_points(hipStream_t s) {
     tmp.alloc(tc.total, s);
     char *tb = tmp.as<char>();
     // chunk table, chunk bases and counts, laid out as in the temporaries
-    sort_h.assign((o_keys - o_chunks) / sizeof(int), 0);
+    sort_h.assign((o_recA - o_chunks) / sizeof(int), 0);
     if (!chunks.empty()) std::memcpy(sort_h.data(), chunks.data(), sizeof(int4) * chunks.size());
     std::memcpy(sort_h.data() + o_base / sizeof(int), base.data(), sizeof(int) * ncurves);
     std::memcpy(sort_h.data() + o_nch / sizeof(int), nch.data(), sizeof(int) * ncurves);
     CUNA_HIP(hipMemcpyAsync(tb, sort_h.data(), sizeof(int) * sort_h.size(), hipMemcpyHostToDevice,
                             s));
-    int *const keys = reinterpret_cast<int *>(tb + o_keys);
     PointRec<T> *const recA = reinterpret_cast<PointRec<T> *>(tb + o_recA);
     int *const permA = reinterpret_cast<int *>(tb + o_permA);
     SortWork W;
@@ -344,22 +339,16 @@ void TiledPoints<T>::sort_points(hipStream_t s) {
     W.total_chunks = total_chunks;
     W.hist = reinterpret_cast<int *>(tb + o_hist);
     W.bsum = reinterpret_cast<int *>(tb + o_bsum);
-    // an LSD sort by anchor: the cell within the tile, then the tile index in
-    // digits of at most 8 bits; the passes alternate between rec/perm and
-    // recA/permA, ending in rec/perm
-    launch_digit_keys<T>(rec_orig.as<PointRec<T>>(), n, 0, K1 - 1, keys, s);
-    const int tbits = ilog2(ntiles);
-    const int npass = 1 + (tbits + 7) / 8;
+    // an LSD sort by anchor, in digits of at most kSortBits bits; the passes
+    // alternate between rec/perm and recA/permA, ending in rec/perm
+    const int abits = std::max(1, ilog2(G)), npass = (int)ceil_div(abits, kSortBits);
     PointRec<T> *const rbuf[2] = {rec.as<PointRec<T>>(), recA};
     int *const pbuf[2] = {perm.as<int>(), permA};
-    auto dst = [&](int p) { return (npass - 1 - p) & 1; };
-    launch_sort_pass<T>(W, K1, keys, rec_orig.as<PointRec<T>>(), nullptr, rbuf[dst(0)],
-                        pbuf[dst(0)], s);
-    for (int p = 1; p < npass; ++p) {
-        const int shift = 8 * (p - 1), bits = std::min(8, tbits - shift);
-        launch_digit_keys<T>(rbuf[dst(p - 1)], n, tlog + shift, (1 << bits) - 1, keys, s);
-        launch_sort_pass<T>(W, 1 << bits, keys, rbuf[dst(p - 1)], pbuf[dst(p - 1)],
-                            rbuf[dst(p)], pbuf[dst(p)], s);
+    for (int p = 0, shift = 0; p < npass; ++p) {
+        const int bits = (int)ceil_div(abits - shift, npass - p), dst = (npass - 1 - p) & 1;
+        launch_sort_pass<T>(W, shift, bits, p == 0 ? rec_orig.as<PointRec<T>>() : rbuf[1 - dst],
+                            p == 0 ? nullptr : pbuf[1 - dst], rbuf[dst], pbuf[dst], s);
+        shift += bits;
     }
     launch_buckets<T>(coff.as<int>(), ncurves, Kc, rec.as<PointRec<T>>(), tlog, olo,
                       olo + ntaps - 1, G, bucket.as<int>(), s);

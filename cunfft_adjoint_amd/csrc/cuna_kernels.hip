@@ -214,49 +214,28 @@ void launch_point_setup(const SetupArgs<T> &A, hipStream_t s) {
 }
 
 template <typename T>
-void launch_digit_keys(const PointRec<T> *rec, long n, int shift, int mask, int *key,
-                       hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_digit_keys<T>, dim3(ceil_div(n, 256)), dim3(256), 0, s, rec, n, shift,
-                       mask, key);
-    CUNA_LAUNCH_CHECK();
-}
-
-static SortArgs sort_args(const SortWork &W, int K, const int *keys) {
+void launch_sort_pass(const SortWork &W, int shift, int bits, const PointRec<T> *rec_in,
+                      const int *perm_in, PointRec<T> *rec_out, int *perm_out, hipStream_t s) {
+    if (W.nchunks == 0) return;
+    require(bits >= 1 && bits <= kSortBits, "sort digit too wide");
     SortArgs S;
     S.chunks = W.chunks;
     S.chunk_base = W.chunk_base;
     S.nch = W.nch;
     S.nchunks = W.nchunks;
-    S.K = K;
-    S.kbits = ilog2(K);
-    S.keys = keys;
+    S.K = 1 << bits;
+    S.shift = shift;
     S.hist = W.hist;
-    return S;
-}
-
-template <typename T>
-void launch_sort_pass(const SortWork &W, int K, const int *keys, const PointRec<T> *rec_in,
-                      const int *perm_in, PointRec<T> *rec_out, int *perm_out, hipStream_t s) {
-    if (W.nchunks == 0) return;
-    const SortArgs S = sort_args(W, K, keys);
-    // waves per block limited by the per-wave LDS counters
-    size_t per_wave = sizeof(int) * (size_t)K;
-    require(per_wave <= kMaxLds, "too many sort keys", CUNA_ERROR_UNSUPPORTED);
-    int wpb = (int)std::max<size_t>(1, std::min<size_t>(4, (64 * 1024) / per_wave));
-    size_t lds = per_wave * wpb;
-    int nblk = (int)ceil_div(W.nchunks, wpb);
-    set_lds(k_hist, lds);
-    set_lds(k_scatter<T>, lds);
-    hipLaunchKernelGGL(k_hist, dim3(nblk), dim3(64 * wpb), lds, s, S);
+    constexpr int wpb = 4;  // waves per block
+    const size_t lds = sizeof(int) * (size_t)wpb * S.K;
+    const int nblk = (int)ceil_div(W.nchunks, wpb);
+    hipLaunchKernelGGL(k_hist<T>, dim3(nblk), dim3(64 * wpb), lds, s, S, rec_in);
     CUNA_LAUNCH_CHECK();
     // exclusive scan of the key-major count matrix
-    const long n = (long)K * W.total_chunks;
+    const long n = (long)S.K * W.total_chunks;
     const long nb = ceil_div(std::max(n, 1L), kScanTile);
     size_t slds = sizeof(int) * kScanNT;
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kScanNT), slds, s, W.hist, n, W.bsum);
-    CUNA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanNT), slds, s, W.bsum, nb);
     CUNA_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kScanNT), slds, s, W.hist, n, W.bsum, W.hist);
     CUNA_LAUNCH_CHECK();
@@ -543,9 +522,8 @@ template void fft_c2r_inverse<dTyp>(const FftShape &, const LoadHermitian<dTyp> 
                                     dTyp *, hipStream_t);
 template void fft_complex<dTyp>(const FftShape &, cplx<dTyp> *, cplx<dTyp> *, int, hipStream_t);
 template void launch_point_setup<dTyp>(const SetupArgs<dTyp> &, hipStream_t);
-template void launch_sort_pass<dTyp>(const SortWork &, int, const int *, const PointRec<dTyp> *,
+template void launch_sort_pass<dTyp>(const SortWork &, int, int, const PointRec<dTyp> *,
                                      const int *, PointRec<dTyp> *, int *, hipStream_t);
-template void launch_digit_keys<dTyp>(const PointRec<dTyp> *, long, int, int, int *, hipStream_t);
 template void launch_buckets<dTyp>(const int *, int, int, const PointRec<dTyp> *, int, int, int, int,
                                    int *, hipStream_t);
 template void launch_spread<dTyp>(const SpreadArgs<dTyp> &, int, int, int, hipStream_t, hipEvent_t,

@@ -53,19 +53,15 @@ struct SortWork {
     const int *nch;
     const int *coff;
     int nchunks, ncurves, total_chunks;
-    int *hist;  // >= K * total_chunks entries for the largest K used
+    int *hist;  // 2^kSortBits * total_chunks entries
     int *bsum;
 };
 template <typename T>
 void launch_point_setup(const SetupArgs<T> &A, hipStream_t s);
-// one stable counting-sort pass over keys in [0, K)
+// one stable counting-sort pass over the anchors' bits [shift, shift + bits)
 template <typename T>
-void launch_sort_pass(const SortWork &W, int K, const int *keys, const PointRec<T> *rec_in,
+void launch_sort_pass(const SortWork &W, int shift, int bits, const PointRec<T> *rec_in,
                       const int *perm_in, PointRec<T> *rec_out, int *perm_out, hipStream_t s);
-// key = (anchor >> shift) & mask, the digits of the tile index
-template <typename T>
-void launch_digit_keys(const PointRec<T> *rec, long n, int shift, int mask, int *key,
-                       hipStream_t s);
 // first sorted index of every (curve, 3 * tile + edge class) key, from points
 // sorted by anchor
 template <typename T>

@@ -164,24 +164,36 @@ __device__ __forceinline__ int tile_key(int a, int tlog, int olo, int ohi, int G
     return 3 * tile + cls;
 }
 
-// sort digits after the first: bits [shift, shift + log2(mask + 1)) of the
-// tile index a >> tlog
-template <typename T>
-__global__ void k_digit_keys(const PointRec<T> *rec, long n, int shift, int mask, int *key) {
-    const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n) key[s] = (rec[s].a >> shift) & mask;
+// The lanes of the wave with the same digit (of at most NBITS bits) as this one,
+// among those in `act`: rank below the lane and count (NBITS ballots, about four
+// instructions each).
+template <int NBITS>
+__device__ __forceinline__ void match_digit(unsigned d, unsigned long long act, int &rank,
+                                            int &count) {
+    unsigned lo = (unsigned)act, hi = (unsigned)(act >> 32);
+#pragma unroll
+    for (int b = 0; b < NBITS; ++b) {  // (bits past the digit's are 0)
+        const int t = __builtin_amdgcn_sbfe((int)d, b, 1);  // 0 or ~0
+        const unsigned long long m = __ballot(t < 0);
+        lo &= ~((unsigned)m ^ (unsigned)t);
+        hi &= ~((unsigned)(m >> 32) ^ (unsigned)t);
+    }
+    rank = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+    count = __popc(lo) + __popc(hi);
 }
 
-// A stable counting sort pass over K keys.  Points are cut into chunks that
-// never cross a curve; the per-chunk counts form a key-major matrix
-// hist[curve base + key * nch + chunk], whose exclusive scan gives every
-// chunk's first position for every key.  One wave handles one chunk.
+// A stable counting sort pass over the digit (anchor >> shift) & (K - 1).  Points
+// are cut into chunks of at most kSortChunk that never cross a curve; the
+// per-chunk counts form a key-major matrix hist[curve base + key * nch + chunk],
+// whose exclusive scan gives every chunk's first position for every key.  One
+// wave handles one chunk, all of whose loads it issues first: with a step's loads
+// issued when its turn came, the scatter of 1e6 points took 24 us, now 15 us.
+constexpr int kSortChunk = 512, kSortBits = 8, kSortSteps = kSortChunk / 64;
 struct SortArgs {
     const int4 *chunks;     // {curve, start, len, column}
     const int *chunk_base;  // chunks before each curve
     const int *nch;         // chunks per curve
-    int nchunks, K, kbits;
-    const int *keys;
+    int nchunks, K, shift;
     int *hist;
 };
 
@@ -189,21 +201,25 @@ __device__ __forceinline__ long hist_index(const SortArgs &S, int4 cd, int k) {
     return (long)S.K * S.chunk_base[cd.x] + (long)k * S.nch[cd.x] + cd.w;
 }
 
-static __global__ void k_hist(SortArgs S) {
+template <typename T>
+__global__ void k_hist(SortArgs S, const PointRec<T> *rec) {
     int *cnt_all = reinterpret_cast<int *>(cuna_smem);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int ch = blockIdx.x * (blockDim.x >> 6) + wave;
     int *cnt = cnt_all + wave * S.K;
     for (int k = lane; k < S.K; k += 64) cnt[k] = 0;
-    __syncthreads();
-    int4 cd = make_int4(0, 0, 0, 0);
-    if (ch < S.nchunks) {
-        cd = S.chunks[ch];
-        for (int q = lane; q < cd.z; q += 64) atomicAdd(&cnt[S.keys[(long)cd.y + q]], 1);
-    }
-    __syncthreads();
-    if (ch < S.nchunks)
-        for (int k = lane; k < S.K; k += 64) S.hist[hist_index(S, cd, k)] = cnt[k];
+    if (ch >= S.nchunks) return;  // (no workgroup barriers)
+    const int4 cd = S.chunks[ch];
+    int a[kSortSteps];  // (clamped loads: all issue together)
+#pragma unroll
+    for (int r = 0; r < kSortSteps; ++r)
+        a[r] = rec[(long)cd.y + min(r * 64 + lane, cd.z - 1)].a;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int r = 0; r < kSortSteps; ++r)
+        if (r * 64 + lane < cd.z) atomicAdd(&cnt[(a[r] >> S.shift) & (S.K - 1)], 1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int k = lane; k < S.K; k += 64) S.hist[hist_index(S, cd, k)] = cnt[k];
 }
 
 // scatter with ranks that keep the input order among equal keys
@@ -214,37 +230,34 @@ __global__ void k_scatter(SortArgs S, const PointRec<T> *rec_in, const int *perm
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int ch = blockIdx.x * (blockDim.x >> 6) + wave;
     int *cur = cur_all + wave * S.K;
-    int4 cd = make_int4(0, 0, 0, 0);
-    if (ch < S.nchunks) {
-        cd = S.chunks[ch];
-        for (int k = lane; k < S.K; k += 64) cur[k] = S.hist[hist_index(S, cd, k)];
+    if (ch >= S.nchunks) return;  // (no workgroup barriers)
+    const int4 cd = S.chunks[ch];
+    PointRec<T> pr[kSortSteps];
+    int pm[kSortSteps];
+#pragma unroll
+    for (int r = 0; r < kSortSteps; ++r) {
+        const long i = (long)cd.y + min(r * 64 + lane, cd.z - 1);
+        pr[r] = rec_in[i];
+        pm[r] = perm_in ? perm_in[i] : (int)i;
     }
-    __syncthreads();
-    if (ch < S.nchunks) {
-        const unsigned long long lt = (1ull << lane) - 1ull;
-        for (int r0 = 0; r0 < cd.z; r0 += 64) {
-            const int q = r0 + lane;
-            const bool act = q < cd.z;
-            const long i = (long)cd.y + q;
-            const int key = act ? S.keys[i] : 0;
-            unsigned long long peers = __ballot(act);
-            for (int bit = 0; bit < S.kbits; ++bit) {
-                const int bv = (key >> bit) & 1;
-                unsigned long long m = __ballot(bv);
-                peers &= bv ? m : ~m;
-            }
-            const int rank = __popcll(peers & lt);
-            const int gcount = __popcll(peers);
-            int pos = 0;
-            if (act) pos = cur[key] + rank;
-            __builtin_amdgcn_wave_barrier();
-            if (act) {
-                rec_out[pos] = rec_in[i];
-                perm_out[pos] = perm_in ? perm_in[i] : (int)i;
-                if (rank == gcount - 1) cur[key] = pos + 1;
-            }
-            __builtin_amdgcn_wave_barrier();
+    for (int k = lane; k < S.K; k += 64) cur[k] = S.hist[hist_index(S, cd, k)];
+#pragma unroll
+    for (int r = 0; r < kSortSteps; ++r) {
+        const int na = cd.z - r * 64;
+        if (na <= 0) break;  // uniform
+        const unsigned d = (unsigned)(pr[r].a >> S.shift) & (unsigned)(S.K - 1);
+        int rank, count;
+        match_digit<kSortBits>(d, na >= 64 ? ~0ull : (1ull << na) - 1ull, rank, count);
+        const int pos = cur[d] + rank;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < na) {
+            rec_out[pos] = pr[r];
+            perm_out[pos] = pm[r];
+            if (rank == count - 1) cur[d] = pos + 1;
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -323,20 +336,13 @@ __global__ __launch_bounds__(NT) void k_plan_curve(const PointRec<T> *rec_orig, 
             const unsigned long long act = na == 64 ? ~0ull : (1ull << na) - 1ull;
             const int q = min(q0 + lane, w1 - 1);
             const unsigned d = (sv[q] >> shift) & mask;
-            unsigned plo = (unsigned)act, phi = (unsigned)(act >> 32);
-#pragma unroll
-            for (int b = 0; b < kPlanDigitBits; ++b) {  // (bits past the digit's are 0)
-                const int t = __builtin_amdgcn_sbfe((int)d, b, 1);  // 0 or ~0
-                const unsigned long long m = __ballot(t < 0);
-                plo &= ~((unsigned)m ^ (unsigned)t);
-                phi &= ~((unsigned)(m >> 32) ^ (unsigned)t);
-            }
             // (a lane past the end counts all its peers as lower: it never writes)
-            const int r = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0));
+            int r, peers;
+            match_digit<kPlanDigitBits>(d, act, r, peers);
             const int cur = cw[d];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
-            if (r == __popc(plo) + __popc(phi) - 1) cw[d] = (unsigned short)(cur + r + 1);
+            if (r == peers - 1) cw[d] = (unsigned short)(cur + r + 1);
             if (lane < na) rk[q] = (unsigned short)(cur + r);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -461,20 +467,6 @@ static __global__ __launch_bounds__(kScanNT) void k_scan_reduce(const int *in, l
     if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-static __global__ __launch_bounds__(kScanNT) void k_scan_sums(int *bsum, long nb) {
-    int *sh = reinterpret_cast<int *>(cuna_smem);
-    int carry = 0;
-    for (long c0 = 0; c0 < nb; c0 += kScanNT) {
-        long i = c0 + threadIdx.x;
-        int v = i < nb ? bsum[i] : 0;
-        int total;
-        int ex = block_exclusive_scan(v, sh, total);
-        if (i < nb) bsum[i] = ex + carry;
-        carry += total;
-        __syncthreads();
-    }
-}
-
 static __global__ __launch_bounds__(kScanNT) void k_scan_apply(const int *in, long n, const int *bsum,
                                                         int *out) {
     int *sh = reinterpret_cast<int *>(cuna_smem);
@@ -486,8 +478,11 @@ static __global__ __launch_bounds__(kScanNT) void k_scan_apply(const int *in, lo
         v[q] = base + q < n ? in[base + q] : 0;
         s += v[q];
     }
-    int total;
-    int ex = block_exclusive_scan(s, sh, total) + bsum[blockIdx.x];
+    // the earlier blocks' sums
+    int before = 0, total;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kScanNT) before += bsum[b];
+    block_exclusive_scan(before, sh, before);
+    int ex = block_exclusive_scan(s, sh, total) + before;
 #pragma unroll
     for (int q = 0; q < kScanIPT; ++q) {
         if (base + q < n) out[base + q] = ex;
