@@ -31,10 +31,6 @@ extern __shared__ __attribute__((aligned(16))) unsigned char cuna_smem[];
 
 // ---------------------------------------------------------- butterflies --
 // In-register DFTs of radix 2/4/8/16, v[n] -> v[k] = sum_n v[n] w_R^{S n k}.
-template <typename T>
-__device__ __forceinline__ cplx<T> rot(cplx<T> z, T c, T s) {  // z * (c + i s)
-    return cmk(z.x * c - z.y * s, z.x * s + z.y * c);
-}
 template <typename T, int S>
 __device__ __forceinline__ cplx<T> mul_si(cplx<T> z) {  // z * (S i)
     return S > 0 ? cmk(-z.y, z.x) : cmk(z.y, -z.x);
@@ -56,30 +52,39 @@ __device__ __forceinline__ void dft4(cplx<T> &a0, cplx<T> &a1, cplx<T> &a2, cplx
     a3 = t1 - t3;
 }
 
+// a + f b and a - f b
+template <typename T>
+__device__ __forceinline__ void pm(cplx<T> a, T f, cplx<T> b, cplx<T> &plus, cplx<T> &minus) {
+    plus = cmk(a.x + f * b.x, a.y + f * b.y);
+    minus = cmk(a.x - f * b.x, a.y - f * b.y);
+}
+
+// The odd half's rotations by c + i s are factored as c (1 + i t): (1 + i t) o
+// takes two multiply-adds and the sums with the even half four, 6 operations in
+// place of 8 (and two roundings less).
 template <typename T, int S>
 __device__ __forceinline__ void dft8(cplx<T> *v) {
-    const T h = T(0.70710678118654752440);
+    const T h = T(0.70710678118654752440), sg = T(S);
     cplx<T> e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
     cplx<T> o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
     dft4<T, S>(e0, e1, e2, e3);
     dft4<T, S>(o0, o1, o2, o3);
-    o1 = rot(o1, h, S * h);
+    o1 = cmk(o1.x - sg * o1.y, o1.y + sg * o1.x);     // (1 + i S) o1
     o2 = mul_si<T, S>(o2);
-    o3 = rot(o3, -h, S * h);
+    o3 = cmk(-o3.x - sg * o3.y, sg * o3.x - o3.y);    // (-1 + i S) o3
     v[0] = e0 + o0;
     v[4] = e0 - o0;
-    v[1] = e1 + o1;
-    v[5] = e1 - o1;
+    pm(e1, h, o1, v[1], v[5]);
     v[2] = e2 + o2;
     v[6] = e2 - o2;
-    v[3] = e3 + o3;
-    v[7] = e3 - o3;
+    pm(e3, h, o3, v[3], v[7]);
 }
 
 template <typename T, int S>
 __device__ __forceinline__ void dft16(cplx<T> *v) {
-    const T c1 = T(0.92387953251128675613), s1 = T(0.38268343236508977173);
-    const T h = T(0.70710678118654752440);
+    // cos(pi/8), tan(pi/8), 1/sqrt 2
+    const T c1 = T(0.92387953251128675613), t = T(0.41421356237309504880);
+    const T h = T(0.70710678118654752440), sg = T(S), st = T(S) * t;
     cplx<T> e[8], o[8];
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
@@ -88,18 +93,17 @@ __device__ __forceinline__ void dft16(cplx<T> *v) {
     }
     dft8<T, S>(e);
     dft8<T, S>(o);
-    o[1] = rot(o[1], c1, S * s1);
-    o[2] = rot(o[2], h, S * h);
-    o[3] = rot(o[3], s1, S * c1);
+    v[0] = e[0] + o[0];
+    v[8] = e[0] - o[0];
+    pm(e[1], c1, cmk(o[1].x - st * o[1].y, o[1].y + st * o[1].x), v[1], v[9]);
+    pm(e[2], h, cmk(o[2].x - sg * o[2].y, o[2].y + sg * o[2].x), v[2], v[10]);
+    pm(e[3], c1, cmk(t * o[3].x - sg * o[3].y, t * o[3].y + sg * o[3].x), v[3], v[11]);
     o[4] = mul_si<T, S>(o[4]);
-    o[5] = rot(o[5], -s1, S * c1);
-    o[6] = rot(o[6], -h, S * h);
-    o[7] = rot(o[7], -c1, S * s1);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        v[k] = e[k] + o[k];
-        v[k + 8] = e[k] - o[k];
-    }
+    v[4] = e[4] + o[4];
+    v[12] = e[4] - o[4];
+    pm(e[5], c1, cmk(-t * o[5].x - sg * o[5].y, sg * o[5].x - t * o[5].y), v[5], v[13]);
+    pm(e[6], h, cmk(-o[6].x - sg * o[6].y, sg * o[6].x - o[6].y), v[6], v[14]);
+    pm(e[7], c1, cmk(-o[7].x - st * o[7].y, st * o[7].x - o[7].y), v[7], v[15]);
 }
 
 template <typename T, int R, int S>

@@ -1533,8 +1533,12 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     // <= vm; spread in fixed point and transformed in place into z.  Returns the
     // power of two that the spectrum is to be multiplied by: the integers go
     // through the FFT as they are.
-    auto transform = [&](int c0, int nc, int rep, const FastMod &fm, const PointRec<T> *P,
-                         const T *y, T shift, double vm, int cover) __attribute__((always_inline)) -> T {
+    // With `moments`, y (whose values are not spread: unit weights) only adds the
+    // drawn values' shifted sums s1, s2 to the workgroup's red_sh.
+    auto transform = [&](auto moments, int c0, int nc, int rep, const FastMod &fm,
+                         const PointRec<T> *P, const T *y, T shift, double vm,
+                         int cover) __attribute__((always_inline)) -> T {
+        constexpr bool MOM = decltype(moments)::value;
         int sexp = 0;
         if (vm <= 1e300) {  // false for NaN and inf
             // No cell receives more than cnt weights of size <= vm * wscale, so
@@ -1554,6 +1558,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
                 for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
                     reinterpret_cast<uint4 *>(cuna_smem)[i] = make_uint4(0, 0, 0, 0);
                 for (int i = tid; i < NB; i += NT) hist_sh[i] = 0;
+                double s1 = 0.0, s2 = 0.0;
                 __syncthreads();
                 for (int p0 = 0; p0 < nc; p0 += NT * PB) {
                     PointRec<T> pr[PB];
@@ -1570,7 +1575,19 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
                     }
 #pragma unroll
                     for (int k = 0; k < PB; ++k) pr[k] = P[dk[k]];
-                    if (y) {
+                    if constexpr (MOM) {
+#pragma unroll
+                        for (int k = 0; k < PB; ++k) vv[k] = y[dk[k]];
+#pragma unroll
+                        for (int k = 0; k < PB; ++k) {
+                            if (p0 + k * NT + tid < nc) {
+                                const double d = (double)vv[k] - (double)shift;
+                                s1 += d;
+                                s2 += d * d;
+                            }
+                            vv[k] = T(1);
+                        }
+                    } else if (y) {
 #pragma unroll
                         for (int k = 0; k < PB; ++k) vv[k] = y[dk[k]] - shift;
                     } else {
@@ -1610,6 +1627,17 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) dmax = max(dmax, __shfl_xor(dmax, o));
                 if ((tid & 63) == 0) dmax_sh[tid >> 6] = dmax;
+                if constexpr (MOM) {
+#pragma unroll
+                    for (int o = 32; o > 0; o >>= 1) {
+                        s1 += __shfl_xor(s1, o);
+                        s2 += __shfl_xor(s2, o);
+                    }
+                    if ((tid & 63) == 0) {
+                        red_sh[2 * (tid >> 6)] = s1;
+                        red_sh[2 * (tid >> 6) + 1] = s2;
+                    }
+                }
                 __syncthreads();
                 dmax = dmax_sh[0];
 #pragma unroll
@@ -1680,9 +1708,9 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         if constexpr (MODE == 0) {
             const int rep = rem / A.ntr, tr = rem % A.ntr;
             const bool usey = tr == 0 && A.y;
-            const T scale = transform(c0, nc, rep, fm, tr == 0 ? A.rec_x : A.rec_2x,
-                                      usey ? A.y : nullptr, T(0), usey ? ymax : 1.0,
-                                      tr == 0 ? cover_x : cover_2x);
+            const T scale = transform(std::false_type{}, c0, nc, rep, fm,
+                                      tr == 0 ? A.rec_x : A.rec_2x, usey ? A.y : nullptr, T(0),
+                                      usey ? ymax : 1.0, tr == 0 ? cover_x : cover_2x);
             if (first_wave) stage_item(next);
             SinkAccurate<T> sk = A.sink;
             sk.pref *= scale;
@@ -1696,43 +1724,15 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             const int rep = rem;
             const long row = (long)ci * A.nbs + rep;
             const int half = A.sink.M / 2;
-            // moments of the drawn values about the first draw (shifted sums
-            // keep the variance accurate when |mean| >> spread)
+            // window W(2w), parked in this workgroup's workspace row; its draws
+            // also give the moments of the drawn values about the first one
+            // (shifted sums keep the variance accurate when |mean| >> spread)
+            const T shift =
+                nc > 0 ? A.y[c0 + (int)fm(xorshift32(wang_hash(A.seed + (uint32_t)rep * (uint32_t)nc)))]
+                       : T(0);
+            const T wscale = transform(std::true_type{}, c0, nc, rep, fm, A.rec_2x, A.y, shift, 1.0,
+                                       cover_2x);
             double s1 = 0.0, s2 = 0.0;
-            T shift = T(0);
-            if (nc > 0) {
-                shift = A.y[c0 + (int)fm(xorshift32(wang_hash(A.seed + (uint32_t)rep * (uint32_t)nc)))];
-                for (int p0 = 0; p0 < nc; p0 += NT * PB) {
-                    T vv[PB];
-#pragma unroll
-                    for (int k = 0; k < PB; ++k) {
-                        int p = p0 + k * NT + tid;
-                        p = p < nc ? p : 0;
-                        const uint32_t t = (uint32_t)rep * (uint32_t)nc + (uint32_t)p;
-                        vv[k] = A.y[c0 + (int)fm(xorshift32(wang_hash(A.seed + t)))];
-                    }
-#pragma unroll
-                    for (int k = 0; k < PB; ++k) {
-                        if (p0 + k * NT + tid < nc) {
-                            const double d = (double)vv[k] - (double)shift;
-                            s1 += d;
-                            s2 += d * d;
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                s1 += __shfl_xor(s1, o);
-                s2 += __shfl_xor(s2, o);
-            }
-            if ((tid & 63) == 0) {
-                red_sh[2 * (tid >> 6)] = s1;
-                red_sh[2 * (tid >> 6) + 1] = s2;
-            }
-            __syncthreads();
-            s1 = 0.0;
-            s2 = 0.0;
             for (int w = 0; w < NT / 64; ++w) {
                 s1 += red_sh[2 * w];
                 s2 += red_sh[2 * w + 1];
@@ -1743,8 +1743,6 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             const double mean_off = s1 / nd;
             const T ybar = (T)((double)shift + mean_off);
             const T yy = (T)fmax(0.0, s2 - s1 * mean_off);
-            // window W(2w), parked in this workgroup's workspace row
-            const T wscale = transform(c0, nc, rep, fm, A.rec_2x, nullptr, T(0), 1.0, cover_2x);
             cplx<T> *wrow = A.ls_w + (long)blockIdx.x * half;
             epilogue([&](int f, cplx<T> w) __attribute__((always_inline)) {
                 if (f < half) wrow[f] = spectrum(f, w, wscale);
@@ -1752,7 +1750,8 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             __syncthreads();
             // F(w) of the mean-subtracted values, then the power
             const double vm = ymax + fabs((double)ybar);
-            const T yscale = transform(c0, nc, rep, fm, A.rec_x, A.y, ybar, vm, cover_x);
+            const T yscale = transform(std::false_type{}, c0, nc, rep, fm, A.rec_x, A.y, ybar, vm,
+                                       cover_x);
             if (first_wave) stage_item(next);
             T best = T(-1);
             int kbest = 0;
