@@ -496,11 +496,26 @@ bool Plan<T>::bootstrap_fused_ok(bool window) const {
            (!window || has_pts2);
 }
 
+// workgroups of the fused kernels that can be resident (at most one per
+// boot_lds_bytes of each CU's LDS): rows of their workspaces
+template <typename T>
+int Plan<T>::boot_slots() const {
+    int dev = 0, ncu = 0;
+    CUNA_HIP(hipGetDevice(&dev));
+    CUNA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    return std::max(ncu, 1) * std::max(1, (int)(kMaxLds / boot_lds_bytes<T>(lgN)));
+}
+template <typename T>
+int Plan<T>::boot_list_cap() const {
+    return std::max(4, std::min(pts.longest, boot_list_max<T>(lgN)));
+}
+
 template <typename T>
 void Plan<T>::prepare_bootstrap(int nbs, bool window, hipStream_t s) {
     if (bootstrap_fused_ok(window)) {
         counter.ensure(sizeof(int), s);
         boot_curves.ensure(sizeof(BootCurve) * (size_t)ncurves(), s);
+        boot_list.ensure(sizeof(unsigned) * (size_t)boot_slots() * boot_list_cap(), s);
         cover.ensure(sizeof(int) * 2 * (size_t)ncurves(), s);
         return;
     }
@@ -531,6 +546,9 @@ BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t 
     B.rec_2x = has_pts2 ? pts2.rec_orig.template as<PointRec<T>>() : nullptr;
     B.y = y;
     B.curves = boot_curves.as<BootCurve>();
+    B.slots = boot_slots();
+    B.list = boot_list.as<unsigned>();
+    B.list_cap = boot_list_cap();
     B.counter = counter.as<int>();
     B.ncurves = nc;
     B.nbs = nbs;
@@ -561,18 +579,12 @@ void Plan<T>::bootstrap_ls(const T *y, int nbs, uint32_t seed, T *power, T *peak
             CUNA_ERROR_UNSUPPORTED);
     prepare_bootstrap(nbs, true, s);
     // window spectra workspace: one row of M/2 values per resident workgroup
-    // (at most one per kMaxLds of LDS on each CU)
-    int dev = 0, ncu = 0;
-    CUNA_HIP(hipGetDevice(&dev));
-    CUNA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    const int slots = ncu * std::max(1, (int)(kMaxLds / boot_lds_bytes<T>(lgN)));
-    ls_work.ensure(sizeof(cplx<T>) * (size_t)slots * (M / 2), s);
+    ls_work.ensure(sizeof(cplx<T>) * (size_t)boot_slots() * (M / 2), s);
     BootArgs<T> B = fused_args(y, nbs, seed, s);
     B.ls_power = power;
     B.ls_peak = peak;
     B.ls_kpeak = kpeak;
     B.ls_w = ls_work.as<cplx<T>>();
-    B.ls_w_slots = slots;
     B.ntr = 1;
     const long total = (long)ncurves() * nbs;
     require(total < (1L << 31), "too many bootstrap items");
@@ -594,8 +606,8 @@ void Plan<T>::bootstrap(const T *y, int nbs, uint32_t seed, cplx<T> *out_y, cplx
         B.out_y = out_y;
         B.out_w = out_w;
         B.ntr = out_w ? 2 : 1;
-        const long total = (long)nc * nbs * B.ntr;
-        require(total < (1L << 31), "too many bootstrap items");
+        const long total = (long)nc * nbs;
+        require(total * B.ntr < (1L << 31), "too many bootstrap items");
         B.total = (int)total;
         launch_boot_fused<T>(B, lgN, ntaps, 0, s);
         return;

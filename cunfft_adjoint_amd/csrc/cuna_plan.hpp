@@ -167,6 +167,7 @@ struct Plan {
     std::unique_ptr<Bluestein<T>> blu;  // compat grids of any other length
     // fused bootstrap: queue entries (BootCurve) and densest tap window of x and 2x
     DevMem boot_curves, cover;
+    DevMem boot_list;  // draws of the resident workgroups
     DevMem ls_work;  // Lomb-Scargle: window spectra of the resident workgroups
     bool cover_ready = false;
     // optional profiling events, recorded on the execution stream before the
@@ -199,6 +200,8 @@ struct Plan {
     // the call can be captured into a graph without allocating)
     void prepare_bootstrap(int nbs, bool window, hipStream_t s);
     bool bootstrap_fused_ok(bool window) const;
+    int boot_slots() const;
+    int boot_list_cap() const;
 
     SpreadArgs<T> spread_args(const TiledPoints<T> &P) const;
     GatherArgs<T> gather_args() const;

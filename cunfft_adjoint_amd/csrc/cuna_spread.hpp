@@ -1312,8 +1312,8 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
 }
 
 // ------------------------------------------- fused batched bootstrap --
-// One persistent workgroup per CU drains a queue of (curve, replicate,
-// transform) items.  An item draws the replicate's points
+// One persistent workgroup per CU drains a queue of (curve, replicate) items.
+// An item draws the replicate's points
 // d = c0 + xorshift(wang(seed + rep*n_c + p)) % n_c, p < n_c, spreads them
 // into a grid of G = 2N cells held entirely in LDS, transforms it in place
 // (real input as N complex) and writes the deconvolved spectrum:
@@ -1347,6 +1347,9 @@ struct BootArgs {
     int *counter;               // work-queue head, zeroed before the launch
     cplx<T> *out_y, *out_w;
     int ncurves, nbs, ntr, total;
+    int split;                  // MODE 0: a replicate's transforms are items of their own
+    unsigned *list;             // one row of list_cap words per workgroup
+    int list_cap;
     uint32_t seed;
     T bi, wscale;
     T e3[kMaxTaps];
@@ -1359,10 +1362,10 @@ struct BootArgs {
     T *ls_power;
     T *ls_peak;
     int *ls_kpeak;
-    // ... and a workspace of ls_w_slots rows of M/2 values: a workgroup keeps
-    // its current window spectrum in row blockIdx.x
+    // ... and a workspace of a row of M/2 values per workgroup, which keeps its
+    // current window spectrum in row blockIdx.x
     cplx<T> *ls_w;
-    int ls_w_slots;
+    int slots;  // rows of list and ls_w
 };
 
 // LDS of the fused kernel: the grid (G reals = N complex) between two halos of
@@ -1384,6 +1387,14 @@ template <typename T>
 __host__ __device__ constexpr size_t boot_lds_bytes(int lg) {
     return sizeof(cplx<T>) * (((size_t)1 << lg) + (size_t)boot_tw_entries<T>(lg)) +
            2 * kBootHalo * sizeof(T);
+}
+
+// the longest curve whose draws are merged: 16-bit counters in the grid's space,
+// 16-bit point indices
+template <typename T>
+__host__ __device__ constexpr int boot_list_max(int lg) {
+    const long fit = (2L << lg) * (long)sizeof(T) / 2;
+    return fit < 65535 ? (int)fit : 65535;
 }
 
 // cos and sin of 2 pi i / n for the epilogue's constant rotations (compile time
@@ -1469,7 +1480,8 @@ __device__ __forceinline__ double uniform_f64(double v) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// MODE 0: items (curve, replicate, transform) -> deconvolved spectra.
+// MODE 0: items (curve, replicate) -> the deconvolved spectra of its transforms
+// (or one of them, with A.split: few items would leave CUs idle).
 // MODE 1: items (curve, replicate) -> Lomb-Scargle power of the replicate:
 // the window transform (unit weights at 2x) goes to the workgroup's row of
 // the workspace (each thread writes, and later reads back, its own
@@ -1519,6 +1531,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         });
     };
     __shared__ int item_sh[kBootCurveWords + 1];
+    __shared__ int nlist_sh;
     __shared__ int dmax_sh[NT / 64];
     // draws per block of 32 anchors (at most G/32 = 1024 blocks)
     constexpr int NB = G / 32;
@@ -1528,17 +1541,86 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     __shared__ T peak_sh[NT / 64];
     __shared__ int kpk_sh[NT / 64];
 
-    // Grid of one transform: the draws of replicate `rep` of the curve at
-    // c0 (nc points), positions from P, values y[d] - shift (or 1), |value|
-    // <= vm; spread in fixed point and transformed in place into z.  Returns the
-    // power of two that the spectrum is to be multiplied by: the integers go
-    // through the FFT as they are.
-    // With `moments`, y (whose values are not spread: unit weights) only adds the
-    // drawn values' shifted sums s1, s2 to the workgroup's red_sh.
-    auto transform = [&](auto moments, int c0, int nc, int rep, const FastMod &fm,
-                         const PointRec<T> *P, const T *y, T shift, double vm,
-                         int cover) __attribute__((always_inline)) -> T {
+    // The draws of replicate `rep` of the curve at c0 (nc points).  Up to
+    // A.list_cap points, equal draws are merged: their multiplicities are counted
+    // in 16-bit LDS counters (in the grid's space), and the distinct points, about
+    // 63 % of nc, go to this workgroup's list with their counts, in any order (the
+    // grid's integer sums do not depend on it).  The spread, bound by its LDS
+    // atomics, then adds each point once with the weight count * y.  A longer curve
+    // is drawn point by point in the spread.  With `moments`, red_sh receives the
+    // sums over the draws of (y - shift) and its square.  Returns the length of the
+    // list (nc without one).
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned *const list = A.list + (long)blockIdx.x * A.list_cap;
+    auto draw = [&](int nc, int rep, const FastMod &fm, int p) __attribute__((always_inline)) {
+        const uint32_t t = (uint32_t)rep * (uint32_t)nc + (uint32_t)p;
+        return fm(xorshift32(wang_hash(A.seed + t)));
+    };
+    auto prepare_draws = [&](auto moments, int c0, int nc, int rep, const FastMod &fm,
+                             T shift) __attribute__((always_inline)) -> int {
         constexpr bool MOM = decltype(moments)::value;
+        double s1 = 0.0, s2 = 0.0;
+        auto moment = [&](double mult, T yv) __attribute__((always_inline)) {
+            const double d = (double)yv - (double)shift;
+            s1 += mult * d;
+            s2 += mult * d * d;
+        };
+        const bool merged = nc <= A.list_cap;  // uniform
+        if (merged) {
+            unsigned *cw = reinterpret_cast<unsigned *>(gu);
+            const int nw = (nc + 1) / 2;
+            for (int i = tid; i < (nw + 3) / 4; i += NT)
+                reinterpret_cast<uint4 *>(cw)[i] = make_uint4(0, 0, 0, 0);
+            if (tid == 0) nlist_sh = 0;
+            __syncthreads();
+            for (int p = tid; p < nc; p += NT) {
+                const unsigned d = draw(nc, rep, fm, p);
+                atomicAdd(&cw[d >> 1], 1u << (16 * (d & 1)));
+            }
+            __syncthreads();
+            for (int i0 = wave_id * 64; i0 < nw; i0 += NT) {  // uniform
+                const int i = i0 + (tid & 63);
+                const unsigned w = i < nw ? cw[i] : 0u, lo = w & 0xffffu, hi = w >> 16;
+                if constexpr (MOM) {
+                    if (lo) moment((double)lo, A.y[c0 + 2 * i]);
+                    if (hi) moment((double)hi, A.y[c0 + 2 * i + 1]);
+                }
+                const unsigned long long b0 = __ballot(lo != 0), b1 = __ballot(hi != 0);
+                int at = 0;
+                if ((tid & 63) == 0) at = atomicAdd(&nlist_sh, __popcll(b0) + __popcll(b1));
+                at = __builtin_amdgcn_readfirstlane(at);
+                at += __builtin_amdgcn_mbcnt_hi((unsigned)(b0 >> 32),
+                                                __builtin_amdgcn_mbcnt_lo((unsigned)b0, 0));
+                at += __builtin_amdgcn_mbcnt_hi((unsigned)(b1 >> 32),
+                                                __builtin_amdgcn_mbcnt_lo((unsigned)b1, 0));
+                if (lo) list[at] = (unsigned)(2 * i) | lo << 16;
+                if (hi) list[at + (lo ? 1 : 0)] = (unsigned)(2 * i + 1) | hi << 16;
+            }
+        } else if constexpr (MOM) {
+            for (int p = tid; p < nc; p += NT) moment(1.0, A.y[c0 + (int)draw(nc, rep, fm, p)]);
+        }
+        if constexpr (MOM) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                s1 += __shfl_xor(s1, o);
+                s2 += __shfl_xor(s2, o);
+            }
+            if ((tid & 63) == 0) {
+                red_sh[2 * (tid >> 6)] = s1;
+                red_sh[2 * (tid >> 6) + 1] = s2;
+            }
+        }
+        __syncthreads();
+        return merged ? __builtin_amdgcn_readfirstlane(nlist_sh) : nc;
+    };
+
+    // Grid of one transform: the nl entries of prepare_draws, positions from P,
+    // values y[d] - shift (or 1), |value| <= vm; spread in fixed point and
+    // transformed in place into z.  Returns the power of two that the spectrum is
+    // to be multiplied by: the integers go through the FFT as they are.
+    auto transform = [&](int c0, int nc, int nl, int rep, const FastMod &fm, const PointRec<T> *P,
+                         const T *y, T shift, double vm, int cover) __attribute__((always_inline)) -> T {
+        const bool merged = nc <= A.list_cap;  // uniform
         int sexp = 0;
         if (vm <= 1e300) {  // false for NaN and inf
             // No cell receives more than cnt weights of size <= vm * wscale, so
@@ -1555,48 +1637,48 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
                 if (bound > 0 && frexp(bound, &e) == 0.5) --e;
                 sexp = min(max(FixedOf<T>::headroom_bits - e, -kMaxExp), kMaxExp);
                 const T mul = (T)ldexp((double)A.wscale, sexp);
+                // thread t takes the spl consecutive entries from t spl on: the list
+                // follows the points, often in order of position, and neighbouring
+                // lanes on neighbouring points would put one atomic's lanes on the
+                // same cells, which serialises them.  PB at a time, loaded ahead of
+                // their use (slots past the end take entry 0 and are skipped below)
+                const int spl = (nl + NT - 1) / NT;  // uniform
+                unsigned wn[PB];
+                auto entries = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int k = 0; k < PB; ++k) {
+                        int p = tid * spl + k0 + k;
+                        p = k0 + k < spl && p < nl ? p : 0;
+                        wn[k] = merged ? list[p] : draw(nc, rep, fm, p);
+                    }
+                };
+                if (nl > 0) entries(0);
                 for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
                     reinterpret_cast<uint4 *>(cuna_smem)[i] = make_uint4(0, 0, 0, 0);
                 for (int i = tid; i < NB; i += NT) hist_sh[i] = 0;
-                double s1 = 0.0, s2 = 0.0;
                 __syncthreads();
-                for (int p0 = 0; p0 < nc; p0 += NT * PB) {
+                for (int k0 = 0; k0 < spl; k0 += PB) {
                     PointRec<T> pr[PB];
                     T vv[PB];
-                    // branch-free: out-of-range slots draw for p = 0 (and are
-                    // skipped below), so all loads issue together
-                    int dk[PB];
+                    int dk[PB], mk[PB];  // point and multiplicity
 #pragma unroll
                     for (int k = 0; k < PB; ++k) {
-                        int p = p0 + k * NT + tid;
-                        p = p < nc ? p : 0;
-                        const uint32_t t = (uint32_t)rep * (uint32_t)nc + (uint32_t)p;
-                        dk[k] = c0 + (int)fm(xorshift32(wang_hash(A.seed + t)));
+                        dk[k] = c0 + (int)(merged ? wn[k] & 0xffffu : wn[k]);
+                        mk[k] = merged ? (int)(wn[k] >> 16) : 1;
                     }
 #pragma unroll
                     for (int k = 0; k < PB; ++k) pr[k] = P[dk[k]];
-                    if constexpr (MOM) {
+                    if (y) {
 #pragma unroll
-                        for (int k = 0; k < PB; ++k) vv[k] = y[dk[k]];
-#pragma unroll
-                        for (int k = 0; k < PB; ++k) {
-                            if (p0 + k * NT + tid < nc) {
-                                const double d = (double)vv[k] - (double)shift;
-                                s1 += d;
-                                s2 += d * d;
-                            }
-                            vv[k] = T(1);
-                        }
-                    } else if (y) {
-#pragma unroll
-                        for (int k = 0; k < PB; ++k) vv[k] = y[dk[k]] - shift;
+                        for (int k = 0; k < PB; ++k) vv[k] = (T)mk[k] * (y[dk[k]] - shift);
                     } else {
 #pragma unroll
-                        for (int k = 0; k < PB; ++k) vv[k] = T(1);
+                        for (int k = 0; k < PB; ++k) vv[k] = (T)mk[k];
                     }
+                    if (k0 + PB < spl) entries(k0 + PB);
 #pragma unroll
                     for (int k = 0; k < PB; ++k) {
-                        if (p0 + k * NT + tid < nc) {
+                        if (k0 + k < spl && tid * spl + k0 + k < nl) {
                             U *dst = gu + (pr[k].a - Q0);
                             if constexpr (sizeof(T) == 4) {
                                 // each tap's rounded weight to its atomic as
@@ -1611,7 +1693,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
                                 for (int q = 0; q < NTAPS; ++q)
                                     atomicAdd(dst + q, (U)FixedOf<T>::round(w[q]));
                             }
-                            atomicAdd(&hist_sh[pr[k].a >> 5], 1);
+                            atomicAdd(&hist_sh[pr[k].a >> 5], mk[k]);
                         }
                     }
                 }
@@ -1627,17 +1709,6 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
 #pragma unroll
                 for (int o = 32; o > 0; o >>= 1) dmax = max(dmax, __shfl_xor(dmax, o));
                 if ((tid & 63) == 0) dmax_sh[tid >> 6] = dmax;
-                if constexpr (MOM) {
-#pragma unroll
-                    for (int o = 32; o > 0; o >>= 1) {
-                        s1 += __shfl_xor(s1, o);
-                        s2 += __shfl_xor(s2, o);
-                    }
-                    if ((tid & 63) == 0) {
-                        red_sh[2 * (tid >> 6)] = s1;
-                        red_sh[2 * (tid >> 6) + 1] = s2;
-                    }
-                }
                 __syncthreads();
                 dmax = dmax_sh[0];
 #pragma unroll
@@ -1670,7 +1741,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     // The first wave takes the next item off the queue while the workgroup
     // works on the current one, and has its curve's entry in LDS by the end: an
     // item then starts without a chain of global loads.
-    const int per_curve = A.nbs * (MODE == 0 ? A.ntr : 1);
+    const int per_curve = A.nbs * (A.split ? A.ntr : 1);
     const int lane = tid & 63;
     const bool first_wave = tid < 64;
     auto take = [&]() __attribute__((always_inline)) -> int {
@@ -1706,32 +1777,32 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         int next = 0;
         if (first_wave) next = take();
         if constexpr (MODE == 0) {
-            const int rep = rem / A.ntr, tr = rem % A.ntr;
-            const bool usey = tr == 0 && A.y;
-            const T scale = transform(std::false_type{}, c0, nc, rep, fm,
-                                      tr == 0 ? A.rec_x : A.rec_2x, usey ? A.y : nullptr, T(0),
-                                      usey ? ymax : 1.0, tr == 0 ? cover_x : cover_2x);
-            if (first_wave) stage_item(next);
-            SinkAccurate<T> sk = A.sink;
-            sk.pref *= scale;
-            cplx<T> *o = (tr == 0 ? A.out_y : A.out_w) + ((long)ci * A.nbs + rep) * sk.M;
-            epilogue([&](int r, cplx<T> w) __attribute__((always_inline)) {
-                if (r <= N / 2)
-                    emit_pair(sk, o, r, N, z[lds_sw(r)], z[lds_sw((N - r) & (N - 1))], w);
-            });
-            __syncthreads();
+            const int rep = A.split ? rem / A.ntr : rem;
+            const int tr0 = A.split ? rem % A.ntr : 0, tr1 = A.split ? tr0 + 1 : A.ntr;
+            const int nl = prepare_draws(std::false_type{}, c0, nc, rep, fm, T(0));
+            for (int tr = tr0; tr < tr1; ++tr) {
+                const bool usey = tr == 0 && A.y;
+                const T scale = transform(c0, nc, nl, rep, fm, tr == 0 ? A.rec_x : A.rec_2x,
+                                          usey ? A.y : nullptr, T(0), usey ? ymax : 1.0,
+                                          tr == 0 ? cover_x : cover_2x);
+                if (first_wave && tr == tr1 - 1) stage_item(next);
+                SinkAccurate<T> sk = A.sink;
+                sk.pref *= scale;
+                cplx<T> *o = (tr == 0 ? A.out_y : A.out_w) + ((long)ci * A.nbs + rep) * sk.M;
+                epilogue([&](int r, cplx<T> w) __attribute__((always_inline)) {
+                    if (r <= N / 2)
+                        emit_pair(sk, o, r, N, z[lds_sw(r)], z[lds_sw((N - r) & (N - 1))], w);
+                });
+                __syncthreads();
+            }
         } else {
             const int rep = rem;
             const long row = (long)ci * A.nbs + rep;
             const int half = A.sink.M / 2;
-            // window W(2w), parked in this workgroup's workspace row; its draws
-            // also give the moments of the drawn values about the first one
-            // (shifted sums keep the variance accurate when |mean| >> spread)
-            const T shift =
-                nc > 0 ? A.y[c0 + (int)fm(xorshift32(wang_hash(A.seed + (uint32_t)rep * (uint32_t)nc)))]
-                       : T(0);
-            const T wscale = transform(std::true_type{}, c0, nc, rep, fm, A.rec_2x, A.y, shift, 1.0,
-                                       cover_2x);
+            // moments of the drawn values about the first draw (shifted sums
+            // keep the variance accurate when |mean| >> spread)
+            const T shift = nc > 0 ? A.y[c0 + (int)draw(nc, rep, fm, 0)] : T(0);
+            const int nl = prepare_draws(std::true_type{}, c0, nc, rep, fm, shift);
             double s1 = 0.0, s2 = 0.0;
             for (int w = 0; w < NT / 64; ++w) {
                 s1 += red_sh[2 * w];
@@ -1743,6 +1814,9 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             const double mean_off = s1 / nd;
             const T ybar = (T)((double)shift + mean_off);
             const T yy = (T)fmax(0.0, s2 - s1 * mean_off);
+            // window W(2w), parked in this workgroup's workspace row
+            const T wscale =
+                transform(c0, nc, nl, rep, fm, A.rec_2x, nullptr, T(0), 1.0, cover_2x);
             cplx<T> *wrow = A.ls_w + (long)blockIdx.x * half;
             epilogue([&](int f, cplx<T> w) __attribute__((always_inline)) {
                 if (f < half) wrow[f] = spectrum(f, w, wscale);
@@ -1750,8 +1824,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             __syncthreads();
             // F(w) of the mean-subtracted values, then the power
             const double vm = ymax + fabs((double)ybar);
-            const T yscale = transform(std::false_type{}, c0, nc, rep, fm, A.rec_x, A.y, ybar, vm,
-                                       cover_x);
+            const T yscale = transform(c0, nc, nl, rep, fm, A.rec_x, A.y, ybar, vm, cover_x);
             if (first_wave) stage_item(next);
             T best = T(-1);
             int kbest = 0;
