@@ -11,6 +11,7 @@
 #include <unordered_map>
 
 #include "cuna.h"
+#include "cuna_dispatch.hpp"
 #include "cuna_filter.h"
 #include "cuna_nfft.h"
 #include "cuna_plan.hpp"
@@ -197,7 +198,7 @@ struct Carve {
 
 template <typename T>
 void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int G_, int tlog_,
-                           int ntaps_, bool periodic_, bool keep_eps, hipStream_t s) {
+                           int ntaps_, bool periodic_, bool keep_eps, bool lazy, hipStream_t s) {
     ncurves = (int)offsets.size() - 1;
     coff_h = offsets;
     n = offsets.back();
@@ -229,42 +230,54 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     std::stable_sort(ord.begin(), ord.end(), [&](int u, int v) {
         return offsets[u + 1] - offsets[u] > offsets[v + 1] - offsets[v];
     });
-    // the plan's device memory in one allocation, filled by one upload:
-    // allocation and copy calls are most of a plan build's host time
+    // device memory in few allocations, filled by one upload: allocation and copy
+    // calls are most of a plan build's host time
     const long n1 = std::max<long>(n, 1);
-    const size_t ncov = (size_t)std::max(ncurves, 1) * std::max(ntiles, 1);
     Carve pc;
     const size_t o_up = pc.add(sizeof(int) * (2 * (size_t)ncurves + 1));  // coff, order
-    const size_t o_rec = pc.add(sizeof(PointRec<T>) * n1);
-    const size_t o_perm = pc.add(sizeof(int) * n1);
     const size_t o_orig = pc.add(sizeof(PointRec<T>) * n1);
-    const size_t o_bk = pc.add(sizeof(int) * (size_t)ncurves * (Kc + 1));
     const size_t o_eps = keep_eps ? pc.add(sizeof(T) * n1) : 0;
-    const size_t o_desc = pc.add(sizeof(TileDesc) * ncov);
     arena.alloc(pc.total, s);
     char *pb = arena.as<char>();
     coff.view(pb + o_up, sizeof(int) * (ncurves + 1));
     order.view(pb + o_up + sizeof(int) * (ncurves + 1), sizeof(int) * ncurves);
-    rec.view(pb + o_rec, sizeof(PointRec<T>) * n1);
-    perm.view(pb + o_perm, sizeof(int) * n1);
     rec_orig.view(pb + o_orig, sizeof(PointRec<T>) * n1);
-    bucket.view(pb + o_bk, sizeof(int) * (size_t)ncurves * (Kc + 1));
     if (keep_eps) {
         eps_orig.view(pb + o_eps, sizeof(T) * n1);
         A.eps_orig = eps_orig.as<T>();
     } else {
         eps_orig.release();
     }
-    tile_desc.view(pb + o_desc, sizeof(TileDesc) * ncov);
     plan_h.assign(offsets.begin(), offsets.end());
     plan_h.insert(plan_h.end(), ord.begin(), ord.end());
     CUNA_HIP(hipMemcpyAsync(pb + o_up, plan_h.data(), sizeof(int) * plan_h.size(),
                             hipMemcpyHostToDevice, s));
+    // phase reduction / compat decisions
     A.n = n;
     A.G = G;
     A.rec = rec_orig.as<PointRec<T>>();
-    // phase reduction / compat decisions, then the sort by anchor
     launch_point_setup<T>(A, s);
+    tiled = false;
+    if (!lazy) tiles(s);
+}
+
+template <typename T>
+void TiledPoints<T>::tiles(hipStream_t s) {
+    if (tiled) return;
+    const long n1 = std::max<long>(n, 1);
+    const size_t ncov = (size_t)std::max(ncurves, 1) * std::max(ntiles, 1);
+    Carve pc;
+    const size_t o_rec = pc.add(sizeof(PointRec<T>) * n1);
+    const size_t o_perm = pc.add(sizeof(int) * n1);
+    const size_t o_bk = pc.add(sizeof(int) * (size_t)ncurves * (Kc + 1));
+    const size_t o_desc = pc.add(sizeof(TileDesc) * ncov);
+    tile_arena.alloc(pc.total, s);
+    char *pb = tile_arena.as<char>();
+    rec.view(pb + o_rec, sizeof(PointRec<T>) * n1);
+    perm.view(pb + o_perm, sizeof(int) * n1);
+    bucket.view(pb + o_bk, sizeof(int) * (size_t)ncurves * (Kc + 1));
+    tile_desc.view(pb + o_desc, sizeof(TileDesc) * ncov);
+    // the sort by anchor
     if (!launch_plan_curves<T>(rec_orig.as<PointRec<T>>(), coff.as<int>(), ncurves, longest, tlog,
                                G, Kc, olo, olo + ntaps - 1, rec.as<PointRec<T>>(), perm.as<int>(),
                                bucket.as<int>(), s))
@@ -284,6 +297,7 @@ void TiledPoints<T>::build(SetupArgs<T> A, const std::vector<int> &offsets, int 
     C.periodic = periodic ? 1 : 0;
     C.wrap1 = (periodic && ntiles == 1) ? 1 : 0;
     launch_tile_order<T>(C, ncurves, tile_desc.as<TileDesc>(), s);
+    tiled = true;
 }
 
 // Sort and buckets of curves of any length, in several launches.
@@ -402,15 +416,7 @@ void Plan<T>::run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s, hipEv
     sh.w = spec.fft_w;
     sh.h = spec.fft_h;
     if (spec.mode == CUNA_MODE_ACCURATE) {
-        SinkAccurate<T> sk;
-        sk.out = out;
-        sk.M = M;
-        sk.ostride = M;
-        sk.invG = T(1) / (T)G;
-        const double pi = 3.14159265358979323846;
-        sk.coef = (T)(pi * pi * (double)beta);
-        sk.pref = (T)(1.0 / std::sqrt(pi * (double)beta));
-        fft_real_forward<T>(sh, grid_ptr, sk, s, mid);
+        fft_real_forward<T>(sh, grid_ptr, accurate_sink(out), s, mid);
     } else {
         SinkCompat<T> sk;
         sk.out = out;
@@ -431,8 +437,50 @@ void Plan<T>::run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s, hipEv
 template <typename T>
 void Plan<T>::adjoint(const T *y, cplx<T> *out, hipStream_t s) {
     require(out != nullptr, "output pointer is NULL");
+    if (fused_adjoint) {
+        adjoint_fused(y, 1, out, s);
+        return;
+    }
+    pts.tiles(s);
     grid.ensure(sizeof(T) * (size_t)G * ncurves(), s);
     adjoint_into(y, out, grid.as<T>(), s);
+}
+
+// rows c * nrhs + r of out: curve c with value vector r
+template <typename T>
+void Plan<T>::adjoint_fused(const T *y, int nrhs, cplx<T> *out, hipStream_t s) {
+    AdjointArgs<T> A{};
+    A.total = ncurves() * nrhs;
+    if (sizeof(T) == 4)  // dense curves' first round
+        grid.ensure(sizeof(int) * (size_t)G * std::min(A.total, fused_slots<T>(lgN)), s);
+    A.cover = covers(s);
+    A.rec = pts.rec_orig.template as<PointRec<T>>();
+    A.y = y;
+    A.y_stride = n();
+    A.coff = pts.coff.template as<int>();
+    A.order = pts.order.template as<int>();
+    A.nrhs = nrhs;
+    A.hi = grid.as<int>();
+    A.bi = T(1) / beta;
+    A.wscale = wscale;
+    for (int q = 0; q < kMaxTaps; ++q) A.e3[q] = e3[q];
+    A.sink = accurate_sink(out);
+    launch_adjoint_fused<T>(A, lgN, ntaps, s, prof[0], prof[1]);
+    if (prof[2]) CUNA_HIP(hipEventRecord(prof[2], s));
+    if (prof[3]) CUNA_HIP(hipEventRecord(prof[3], s));
+}
+
+template <typename T>
+SinkAccurate<T> Plan<T>::accurate_sink(cplx<T> *out) const {
+    const double pi = 3.14159265358979323846;
+    SinkAccurate<T> sk;
+    sk.out = out;
+    sk.M = M;
+    sk.ostride = M;
+    sk.invG = T(1) / (T)G;
+    sk.coef = (T)(pi * pi * (double)beta);
+    sk.pref = (T)(1.0 / std::sqrt(pi * (double)beta));
+    return sk;
 }
 
 template <typename T>
@@ -460,6 +508,11 @@ void Plan<T>::adjoint_many(const T *y, int nrhs, cplx<T> *out, hipStream_t s) {
     require(nrhs >= 1, "nrhs must be positive");
     const int nc = ncurves();
     require((long)nc * nrhs <= INT_MAX, "ncurves * nrhs too large", CUNA_ERROR_UNSUPPORTED);
+    if (fused_adjoint) {
+        adjoint_fused(y, nrhs, out, s);
+        return;
+    }
+    pts.tiles(s);
     grid.ensure(sizeof(T) * (size_t)G * nc * nrhs, s);
     SpreadArgs<T> A = spread_args(pts);
     A.y = y;
@@ -496,15 +549,6 @@ bool Plan<T>::bootstrap_fused_ok(bool window) const {
            (!window || has_pts2);
 }
 
-// workgroups of the fused kernels that can be resident (at most one per
-// boot_lds_bytes of each CU's LDS): rows of their workspaces
-template <typename T>
-int Plan<T>::boot_slots() const {
-    int dev = 0, ncu = 0;
-    CUNA_HIP(hipGetDevice(&dev));
-    CUNA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    return std::max(ncu, 1) * std::max(1, (int)(kMaxLds / boot_lds_bytes<T>(lgN)));
-}
 template <typename T>
 int Plan<T>::boot_list_cap() const {
     return std::max(4, std::min(pts.longest, boot_list_max<T>(lgN)));
@@ -515,20 +559,17 @@ void Plan<T>::prepare_bootstrap(int nbs, bool window, hipStream_t s) {
     if (bootstrap_fused_ok(window)) {
         counter.ensure(sizeof(int), s);
         boot_curves.ensure(sizeof(BootCurve) * (size_t)ncurves(), s);
-        boot_list.ensure(sizeof(unsigned) * (size_t)boot_slots() * boot_list_cap(), s);
-        cover.ensure(sizeof(int) * 2 * (size_t)ncurves(), s);
+        boot_list.ensure(sizeof(unsigned) * (size_t)fused_slots<T>(lgN) * boot_list_cap(), s);
         return;
     }
     counts.ensure(sizeof(int) * (size_t)std::max<long>(n(), 1) * nbs, s);
     grid.ensure(sizeof(T) * (size_t)G * ncurves() * nbs, s);
 }
 
-// arguments shared by both modes of the fused bootstrap kernel; computes
-// the per-curve cover (once per plan) and the queue's entries (every call) on
-// stream s
 template <typename T>
-BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s) {
+const int *Plan<T>::covers(hipStream_t s) {
     const int nc = ncurves();
+    cover.ensure(sizeof(int) * 2 * (size_t)nc, s);
     int *cov = cover.as<int>();
     if (!cover_ready) {
         for (int w = 0; w < (has_pts2 ? 2 : 1); ++w) {
@@ -538,6 +579,16 @@ BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t 
         }
         cover_ready = true;
     }
+    return cov;
+}
+
+// arguments shared by both modes of the fused bootstrap kernel; computes
+// the per-curve cover (once per plan) and the queue's entries (every call) on
+// stream s
+template <typename T>
+BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s) {
+    const int nc = ncurves();
+    const int *cov = covers(s);
     launch_boot_prepare<T>(y, pts.coff.template as<int>(), pts.order.template as<int>(), cov,
                            has_pts2 ? cov + nc : nullptr, nc, boot_curves.as<BootCurve>(),
                            counter.as<int>(), s);
@@ -546,7 +597,7 @@ BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t 
     B.rec_2x = has_pts2 ? pts2.rec_orig.template as<PointRec<T>>() : nullptr;
     B.y = y;
     B.curves = boot_curves.as<BootCurve>();
-    B.slots = boot_slots();
+    B.slots = fused_slots<T>(lgN);
     B.list = boot_list.as<unsigned>();
     B.list_cap = boot_list_cap();
     B.counter = counter.as<int>();
@@ -556,12 +607,7 @@ BootArgs<T> Plan<T>::fused_args(const T *y, int nbs, uint32_t seed, hipStream_t 
     B.bi = T(1) / beta;
     B.wscale = wscale;
     for (int q = 0; q < kMaxTaps; ++q) B.e3[q] = e3[q];
-    const double pi = 3.14159265358979323846;
-    B.sink.M = M;
-    B.sink.ostride = M;
-    B.sink.invG = T(1) / (T)G;
-    B.sink.coef = (T)(pi * pi * (double)beta);
-    B.sink.pref = (T)(1.0 / std::sqrt(pi * (double)beta));
+    B.sink = accurate_sink(nullptr);
     return B;
 }
 
@@ -579,7 +625,7 @@ void Plan<T>::bootstrap_ls(const T *y, int nbs, uint32_t seed, T *power, T *peak
             CUNA_ERROR_UNSUPPORTED);
     prepare_bootstrap(nbs, true, s);
     // window spectra workspace: one row of M/2 values per resident workgroup
-    ls_work.ensure(sizeof(cplx<T>) * (size_t)boot_slots() * (M / 2), s);
+    ls_work.ensure(sizeof(cplx<T>) * (size_t)fused_slots<T>(lgN) * (M / 2), s);
     BootArgs<T> B = fused_args(y, nbs, seed, s);
     B.ls_power = power;
     B.ls_peak = peak;
@@ -625,7 +671,8 @@ void Plan<T>::bootstrap(const T *y, int nbs, uint32_t seed, cplx<T> *out_y, cplx
     for (int pass = 0; pass < 2; ++pass) {
         cplx<T> *out = pass == 0 ? out_y : out_w;
         if (!out) continue;
-        const TiledPoints<T> &P = pass == 0 ? pts : pts2;
+        TiledPoints<T> &P = pass == 0 ? pts : pts2;
+        P.tiles(s);
         SpreadArgs<T> A = spread_args(P);
         A.y = pass == 0 ? y : nullptr;
         A.grid = grid.as<T>();
@@ -692,6 +739,7 @@ void Plan<T>::backward(const T *y, const cplx<T> *g, T *dy, T *dx, hipStream_t s
     require(spec.mode == CUNA_MODE_ACCURATE, "backward needs an accurate-mode plan");
     require(g != nullptr, "gradient pointer is NULL");
     if (!dy && !dx) return;
+    pts.tiles(s);
     spectrum_to_grid(g, 1, 0, s);
     GatherArgs<T> A = gather_args();
     A.y = y;
@@ -713,6 +761,7 @@ void Plan<T>::forward(const cplx<T> *fhat, cplx<T> *f, hipStream_t s) {
     require(spec.mode == CUNA_MODE_ACCURATE, "forward needs an accurate-mode plan");
     require(fhat != nullptr && f != nullptr, "NULL pointer");
     const int nc = ncurves();
+    pts.tiles(s);
     constexpr size_t kBothPartsBytes = size_t(4) << 30;
     const size_t both = 4 * sizeof(T) * (size_t)G * nc;  // two grids and two FFT buffers
     if (both <= kBothPartsBytes) {
@@ -747,6 +796,28 @@ static int default_tlog(long n, long ncurves, long G) {
     const int most = sizeof(T) == 4 ? 10 : 9;
     while (tl < most && n <= 80 * ncurves * (G >> tl) && ncurves * (G >> (tl + 1)) >= 8192) ++tl;
     return tl;
+}
+
+// Whether a small grid's adjoint goes through the fused kernel.  Its time is that
+// of its longest curve in one workgroup (1 - 2 ns per point in FP32, 3 - 4 in
+// FP64) and it saves the tile path a launch and each cell's way through memory, so
+// a curve may be the longer the more cells the batch has; and where the batch
+// fills the chip anyway, its points cost more than the tile path's and its cells
+// less.  Measured, fused against tiles of 256 cells, plan kept, us, with the points
+// per curve: FP32, one curve, M = 2^11 1000 8.2 / 9.0, 2500 11.4 / 9.2; 64 curves,
+// M = 2^13 2500 14.9 / 15.1, 4700 17.6 / 15.7; 256 curves, M = 2^14 4700 34 / 52;
+// 600 curves, M = 2^9 1000 9.4 / 13.1, 2500 20.6 / 17.8.  FP64, one curve, M = 2^11
+// 300 10.4 / 10.9, 1000 12.6 / 11.5; 128 curves, M = 2^13 2500 27.7 / 30.4, 4700
+// 37 / 33; 400 curves, M = 2^13 2500 54 / 63, 4700 74 / 70.
+template <typename T>
+static bool fused_adjoint_wins(const std::vector<int> &offsets, int G) {
+    const long nc = (long)offsets.size() - 1, cells = nc * G, n = offsets.back();
+    long longest = 0;
+    for (long c = 0; c < nc; ++c) longest = std::max<long>(longest, offsets[c + 1] - offsets[c]);
+    if (sizeof(T) == 4)
+        return longest <= 1000 + cells * fused_threads(ilog2(G) - 1) / 430000 &&
+               n <= cells / 4 + 500000;
+    return longest <= 250 + cells / 1024 && n <= cells / 5 + 400000;
 }
 
 template <typename T>
@@ -787,14 +858,20 @@ std::unique_ptr<Plan<T>> make_plan_accurate(const T *x, const double *t, double 
     A.mode = t ? SETUP_ACC_T : SETUP_ACC_X;
     int tl = spec.tile_log2 > 0 ? spec.tile_log2
                                 : default_tlog<T>(n, (long)offsets.size() - 1, P->G);
-    P->pts.build(A, offsets, P->G, tl, P->ntaps, true, false, s);
+    const bool fused = boot_fused_supported<T>(P->lgN, P->ntaps) &&
+                       !(spec.flags & (CUNA_PLAN_UNFUSED | CUNA_PLAN_GATHER));
+    // explicit tile and FFT shapes ask for the tile path
+    P->fused_adjoint = fused && spec.tile_log2 == 0 && spec.fft_w == 0 && spec.fft_h == 0 &&
+                       fused_adjoint_wins<T>(offsets, P->G);
+    const bool lazy = P->fused_adjoint || (fused && (spec.flags & CUNA_PLAN_WINDOW2));
+    P->pts.build(A, offsets, P->G, tl, P->ntaps, true, false, lazy, s);
     if (spec.flags & CUNA_PLAN_WINDOW2) {
         // the points 2x: times with 2 df (FP64), or x doubled (exact in
         // binary floating point)
         SetupArgs<T> B = A;
         if (t) {
             B.df = 2.0 * df;
-            P->pts2.build(B, offsets, P->G, tl, P->ntaps, true, false, s);
+            P->pts2.build(B, offsets, P->G, tl, P->ntaps, true, false, fused, s);
         } else {
             DevBuf x2;
             x2.alloc(sizeof(T) * std::max<long>(n, 1), s);
@@ -804,10 +881,11 @@ std::unique_ptr<Plan<T>> make_plan_accurate(const T *x, const double *t, double 
                 CUNA_LAUNCH_CHECK();
             }
             B.x = x2.as<T>();
-            P->pts2.build(B, offsets, P->G, tl, P->ntaps, true, false, s);
+            P->pts2.build(B, offsets, P->G, tl, P->ntaps, true, false, fused, s);
         }
         P->has_pts2 = true;
     }
+    if (P->fused_adjoint) P->covers(s);
     P->prepare_fft(s);
     return P;
 }
@@ -878,7 +956,7 @@ std::unique_ptr<Plan<T>> make_plan_compat(const T *x, int n, int ng, T *E1, T *E
     A.E3 = E3;
     int tl = spec.tile_log2 > 0 ? spec.tile_log2 : default_tlog<T>(n, 1, ng);
     std::vector<int> off = {0, n};
-    P->pts.build(A, off, ng, tl, P->ntaps, false, true, s);
+    P->pts.build(A, off, ng, tl, P->ntaps, false, true, false, s);
     P->prepare_fft(s);
     return P;
 }
@@ -1090,7 +1168,7 @@ static std::unique_ptr<CompatBatch> make_compat_batch(const R *x, const int *n, 
         A.b = P->b_c;
         A.e1s = P->wscale;
         P->pts.build(A, goff, g, default_tlog<R>(gn, nc, g), P->ntaps, false,
-                     false, s);
+                     false, false, s);
         P->prepare_fft(s);
         hipLaunchKernelGGL(k_compose, dim3(ceil_div(std::max(gn, 1L), 256)), dim3(256), 0, s,
                            P->pts.perm.as<int>(), d_idx.as<int>(), gn);

@@ -47,6 +47,11 @@ static constexpr int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > h
 constexpr int fft_threads(int lg, int w, int mr = 4) {
     return clampi(((1 << lg) * w) >> mr, 64, 1024);
 }
+
+// threads of the fused kernels: as the FFT takes them, at least 256 for the spread
+constexpr int fused_threads(int lg) {
+    return fft_threads(lg, 1, small_mr(lg)) < 256 ? 256 : fft_threads(lg, 1, small_mr(lg));
+}
 // two-pass split N = L1 * L2, L2 >= L1
 constexpr int split_lg1(int lgN) { return lgN / 2; }
 // largest log2 N of the single-workgroup inverse (Hermitian) transform

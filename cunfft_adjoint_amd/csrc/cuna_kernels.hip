@@ -441,11 +441,64 @@ bool boot_fused_supported(int lgN, int ntaps) {
                                                     ntaps == 24 || ntaps == 26 || ntaps == 32);
 }
 
+// workgroups that a fused kernel is launched with at most: as many as a CU's LDS
+// holds, on every CU (rows of their workspaces)
+template <typename T>
+int fused_slots(int lgN) {
+    return num_cus() * std::max(1, (int)(kMaxLds / boot_lds_bytes<T>(lgN)));
+}
+
+template <typename T, int LG, int NTAPS>
+static void adjoint_fused_one(AdjointArgs<T> A, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
+    constexpr int NT = fused_threads(LG);
+    auto &tc = TwiddleCache<T>::get();
+    constexpr int CAP = adjoint_cap<T>(LG);
+    A.twT = tc.rows(LG, small_mr(LG), CAP);
+    A.fine = sizeof(T) == 4 && LG > CAP ? tc.fine(LG) : nullptr;
+    A.twN = tc.two_level(LG);
+    A.twH = tc.head(LG + 1, NT);
+    constexpr size_t lds = adjoint_lds_bytes<T>(LG);
+    static_assert(lds <= kMaxLds - 256, "fused adjoint LDS");
+    auto k = k_adjoint_fused<T, LG, NTAPS, NT>;
+    set_lds(k, lds);
+    const int nblk = std::max(1, std::min(A.total, fused_slots<T>(LG)));
+    if (ev0 || ev1)
+        hipExtLaunchKernelGGL(k, dim3(nblk), dim3(NT), (uint32_t)lds, s, ev0, ev1, 0, A);
+    else
+        hipLaunchKernelGGL(k, dim3(nblk), dim3(NT), lds, s, A);
+    CUNA_LAUNCH_CHECK();
+}
+
+// f(integral_constant) of a filter width that the fused kernels have
+template <class F>
+static void dispatch_fused_taps(int ntaps, F &&f) {
+    switch (ntaps) {
+        case 12: f(std::integral_constant<int, 12>{}); break;
+        case 16: f(std::integral_constant<int, 16>{}); break;
+        case 20: f(std::integral_constant<int, 20>{}); break;
+        case 24: f(std::integral_constant<int, 24>{}); break;
+        case 26: f(std::integral_constant<int, 26>{}); break;
+        default: f(std::integral_constant<int, 32>{}); break;
+    }
+}
+
+template <typename T>
+void launch_adjoint_fused(const AdjointArgs<T> &A, int lgN, int ntaps, hipStream_t s,
+                          hipEvent_t ev0, hipEvent_t ev1) {
+    require(boot_fused_supported<T>(lgN, ntaps), "no fused adjoint kernel for this size",
+            CUNA_ERROR_UNSUPPORTED);
+    dispatch_lg<6, max_small_lg<T>()>(lgN, [&](auto c) {
+        dispatch_fused_taps(ntaps, [&](auto t) {
+            adjoint_fused_one<T, decltype(c)::value, decltype(t)::value>(A, s, ev0, ev1);
+        });
+    });
+}
+
 template <typename T, int LG, int NTAPS, int MODE>
 static void boot_fused_one(BootArgs<T> A, hipStream_t s) {
-    constexpr int NT = fft_threads(LG, 1) < 256 ? 256 : fft_threads(LG, 1);
+    constexpr int NT = fused_threads(LG);
     auto &tc = TwiddleCache<T>::get();
-    A.twT = tc.rows(LG, kBootMr, boot_cap<T>(LG));
+    A.twT = tc.rows(LG, small_mr(LG), boot_cap<T>(LG));
     A.twN = tc.two_level(LG);
     A.twH = tc.head(LG + 1, NT);
     const size_t lds = boot_lds_bytes<T>(LG);
@@ -478,7 +531,7 @@ void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, in
                         int *cover, hipStream_t s) {
     require(is_pow2(G) && G <= (1 << 15), "cover histogram needs a power-of-two grid <= 2^15");
     if (ncurves <= 0) return;
-    const size_t lds = sizeof(int) * (size_t)G;
+    const size_t lds = 16 * (((size_t)cover_slot(G) + 3) / 4);
     set_lds(k_curve_cover<T>, lds);
     hipLaunchKernelGGL(k_curve_cover<T>, dim3(ncurves), dim3(1024), lds, s, rec, coff, G, ntaps,
                        cover);
@@ -501,15 +554,9 @@ void launch_boot_fused(BootArgs<T> A, int lgN, int ntaps, int mode, hipStream_t 
     dispatch_lg<6, max_small_lg<T>()>(lgN, [&](auto c) {
         constexpr int LG = decltype(c)::value;
         auto go = [&](auto m) {
-            constexpr int MODE = decltype(m)::value;
-            switch (ntaps) {
-                case 12: boot_fused_one<T, LG, 12, MODE>(A, s); break;
-                case 16: boot_fused_one<T, LG, 16, MODE>(A, s); break;
-                case 20: boot_fused_one<T, LG, 20, MODE>(A, s); break;
-                case 24: boot_fused_one<T, LG, 24, MODE>(A, s); break;
-                case 26: boot_fused_one<T, LG, 26, MODE>(A, s); break;
-                default: boot_fused_one<T, LG, 32, MODE>(A, s); break;
-            }
+            dispatch_fused_taps(ntaps, [&](auto t) {
+                boot_fused_one<T, LG, decltype(t)::value, decltype(m)::value>(A, s);
+            });
         };
         if (mode == 0)
             go(std::integral_constant<int, 0>{});
@@ -538,6 +585,9 @@ template void launch_tile_order<dTyp>(const SpreadArgs<dTyp> &, int, TileDesc *,
 template bool launch_plan_curves<dTyp>(const PointRec<dTyp> *, const int *, int, int, int, int, int,
                                        int, int, PointRec<dTyp> *, int *, int *, hipStream_t);
 template bool boot_fused_supported<dTyp>(int, int);
+template int fused_slots<dTyp>(int);
+template void launch_adjoint_fused<dTyp>(const AdjointArgs<dTyp> &, int, int, hipStream_t,
+                                         hipEvent_t, hipEvent_t);
 template void launch_boot_fused<dTyp>(BootArgs<dTyp>, int, int, int, hipStream_t);
 template void launch_curve_cover<dTyp>(const PointRec<dTyp> *, const int *, int, int, int, int *,
                                        hipStream_t);

@@ -92,6 +92,14 @@ bool launch_plan_curves(const PointRec<T> *rec_orig, const int *coff, int ncurve
 // fused kernel
 template <typename T>
 bool boot_fused_supported(int lgN, int ntaps);
+// workgroups a fused kernel is launched with at most
+template <typename T>
+int fused_slots(int lgN);
+// adjoint of small grids, one workgroup per (curve, value vector) item; A.hi holds
+// min(A.total, fused_slots) x G integers (FP32)
+template <typename T>
+void launch_adjoint_fused(const AdjointArgs<T> &A, int lgN, int ntaps, hipStream_t s,
+                          hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // per-curve densest tap window (G <= 2^15)
 template <typename T>
 void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, int G, int ntaps,

@@ -80,15 +80,23 @@ struct TiledPoints {
     int longest = 0;  // points of the longest curve
     int G = 0, tlog = 0, ntiles = 0, Kc = 0, olo = 0, ntaps = 0;
     bool periodic = true;
-    DevMem arena;  // one allocation; the buffers below are views into it
-    DevMem coff, rec, perm, bucket, eps_orig;
+    // two allocations; the buffers below are views into them
+    DevMem arena, tile_arena;
+    DevMem coff, eps_orig;
     DevMem rec_orig;  // (anchor, e) by original index
     DevMem order;     // curves by decreasing length (work-queue order)
+    // the points sorted by tile, for the paths that work by tiles (see tiles())
+    bool tiled = false;
+    DevMem rec, perm, bucket;
     DevMem tile_desc;   // per curve: the scatter's work order (TileDesc per tile)
 
-    // src: setup arguments with x/t/mode/compat fields filled
+    // src: setup arguments with x/t/mode/compat fields filled.  lazy: the points
+    // are sorted when a call first needs them (the fused kernels of small grids
+    // take them in their original order)
     void build(SetupArgs<T> A, const std::vector<int> &offsets, int G_, int tlog_, int ntaps_,
-               bool periodic_, bool keep_eps, hipStream_t s);
+               bool periodic_, bool keep_eps, bool lazy, hipStream_t s);
+    // sorted points, buckets and work order, made on the first call
+    void tiles(hipStream_t s);
 
   private:
     void sort_points(hipStream_t s);
@@ -200,11 +208,15 @@ struct Plan {
     // the call can be captured into a graph without allocating)
     void prepare_bootstrap(int nbs, bool window, hipStream_t s);
     bool bootstrap_fused_ok(bool window) const;
-    int boot_slots() const;
     int boot_list_cap() const;
 
+    bool fused_adjoint = false;  // adjoint() and adjoint_many() by launch_adjoint_fused
+    void adjoint_fused(const T *y, int nrhs, cplx<T> *out, hipStream_t s);
+    // per-curve cover of x (and 2x) for the fused kernels, once per plan
+    const int *covers(hipStream_t s);
     SpreadArgs<T> spread_args(const TiledPoints<T> &P) const;
     GatherArgs<T> gather_args() const;
+    SinkAccurate<T> accurate_sink(cplx<T> *out) const;
     void spectrum_to_grid(const cplx<T> *g, int parts, int rot, hipStream_t s);
     BootArgs<T> fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s);
     void run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s,

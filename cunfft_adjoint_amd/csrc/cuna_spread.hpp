@@ -1371,7 +1371,7 @@ struct BootArgs {
 // LDS of the fused kernel: the grid (G reals = N complex) between two halos of
 // kBootHalo cells, the twiddle rows of the passes of at most 2^cap points, and the
 // two sub-tables of w_N for the later ones.
-constexpr int kBootHalo = 32, kBootMr = 4;
+constexpr int kBootHalo = 32;
 // cap: 18 KB of rows at FP32's largest grid, where one workgroup has a CU to
 // itself; a few KB where two share it
 template <typename T>
@@ -1380,7 +1380,7 @@ __host__ __device__ constexpr int boot_cap(int lg) {
 }
 template <typename T>
 __host__ __device__ constexpr int boot_tw_entries(int lg) {
-    return rows_count(lg, kBootMr, boot_cap<T>(lg)) + (1 << ((lg + 1) / 2)) +
+    return rows_count(lg, small_mr(lg), boot_cap<T>(lg)) + (1 << ((lg + 1) / 2)) +
            (1 << (lg - (lg + 1) / 2));
 }
 template <typename T>
@@ -1503,7 +1503,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     U *gu = reinterpret_cast<U *>(grid);
     cplx<T> *z = reinterpret_cast<cplx<T> *>(grid);
     cplx<T> *tl = reinterpret_cast<cplx<T> *>(grid + G + kBootHalo);  // staged once per workgroup
-    constexpr int CAP = boot_cap<T>(LG), NLT = rows_count(LG, kBootMr, CAP);
+    constexpr int MR = small_mr(LG), CAP = boot_cap<T>(LG), NLT = rows_count(LG, MR, CAP);
     const int tid = threadIdx.x;
     for (int i = tid; i < NLT; i += NT) tl[i] = A.twT[i];
     for (int i = tid; i < NLN; i += NT) tl[NLT + i] = A.twN.lo[i];
@@ -1725,7 +1725,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             return cmk((T)q.x, (T)q.y);
         };
         __syncthreads();
-        fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, decltype(tw), kBootMr>(
+        fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, decltype(tw), MR>(
             z, tw, fetch, NoHook());
         // a non-finite value makes every spectrum value NaN
         return vm <= 1e300 ? (T)ldexp(1.0, -sexp) : (T)NAN;
@@ -1921,31 +1921,289 @@ __global__ __launch_bounds__(kPrepThreads) void k_boot_prepare(const T *y, const
     }
 }
 
-// per-curve densest window: the most points whose anchors fall in one
-// cyclic run of NTAPS cells of the G-cell grid.  One workgroup per curve,
-// anchor histogram in LDS (G ints).
+// Per-curve densest window: the most points whose anchors fall in one cyclic run
+// of ntaps cells of the G-cell grid.  One workgroup per curve, anchor histogram in
+// LDS, where each thread slides the window over its share of the cells (a word of
+// padding per 32 cells keeps the threads' walks on different banks).  What is left
+// is the histogram's loads.  256 curves of 100 - 20,000 points on 2^15 cells
+// take 10.9 us (22.6 with the windows as differences of a wave's prefix sums,
+// whose chain of lane exchanges bounds it).
+__host__ __device__ constexpr int cover_slot(int i) { return i + (i >> 5); }
+
 template <typename T>
-__global__ void k_curve_cover(const PointRec<T> *rec, const int *coff, int G, int ntaps,
-                              int *cover) {
+__global__ __launch_bounds__(1024) void k_curve_cover(const PointRec<T> *rec, const int *coff,
+                                                      int G, int ntaps, int *cover) {
     int *h = reinterpret_cast<int *>(cuna_smem);
-    const int c = blockIdx.x;
-    for (int i = threadIdx.x; i < G; i += blockDim.x) h[i] = 0;
-    __syncthreads();
-    for (int i = coff[c] + threadIdx.x; i < coff[c + 1]; i += blockDim.x)
-        atomicAdd(&h[rec[i].a & (G - 1)], 1);
-    __syncthreads();
-    int best = 0;
-    for (int g = threadIdx.x; g < G; g += blockDim.x) {
-        int sum = 0;
-        for (int k = 0; k < ntaps; ++k) sum += h[(g + k) & (G - 1)];
-        best = max(best, sum);
-    }
     __shared__ int red;
-    if (threadIdx.x == 0) red = 0;
+    const int c = blockIdx.x, b = coff[c], e = coff[c + 1];
+    const int tid = threadIdx.x, NT = blockDim.x;
+    for (int i = tid; i < (cover_slot(G) + 3) / 4; i += NT)
+        reinterpret_cast<int4 *>(h)[i] = make_int4(0, 0, 0, 0);
+    if (tid == 0) red = 0;
     __syncthreads();
-    atomicMax(&red, best);
+    constexpr int U = 8;  // loads in flight
+    for (int i = b + tid; i < e; i += U * NT) {
+        int a[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) a[k] = rec[min(i + k * NT, e - 1)].a;
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (i + k * NT < e) atomicAdd(&h[cover_slot(a[k] & (G - 1))], 1);
+    }
     __syncthreads();
-    if (threadIdx.x == 0) cover[c] = red;
+    const int share = (G + NT - 1) / NT, g0 = tid * share, g1 = min(g0 + share, G);
+    int best = 0, win = 0;  // win: cells g - ntaps .. g - 1
+    if (g0 < G)
+        for (int g = g0 - ntaps; g < g0; ++g) win += h[cover_slot(g & (G - 1))];
+#pragma unroll 4
+    for (int g = g0; g < g1; ++g) {
+        win += h[cover_slot(g)] - h[cover_slot((g - ntaps) & (G - 1))];
+        best = max(best, win);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) best = max(best, __shfl_xor(best, o));
+    if ((tid & 63) == 0) atomicMax(&red, best);
+    __syncthreads();
+    if (tid == 0) cover[c] = red;
+}
+
+// --------------------------------------------- fused adjoint of small grids --
+// The whole adjoint of one (curve, value vector) item in one workgroup, for grids
+// that fit its LDS: the points in their original order, spread in fixed point into
+// the halo grid of the fused bootstrap, transformed in place, and the deconvolved
+// spectrum written.  The tile path's sort, spread launch and passes of the grid
+// through memory fall away; the bound is the LDS atomics and vector instructions
+// of the workgroup's points (1.15 ns each at 2^15 cells in FP32), so the host takes
+// this path only for curves that are not long next to the whole batch.  256 curves
+// of 100 - 20,000 points, M = 2^14, new plan each time: 100 us, 143 with the sort,
+// tiles and FFT; one curve of 1000 points, M = 2^11, plan kept: 8.3 us, 8.9.
+//
+// Scale: with `cover` the curve's densest window of NTAPS anchors and vm its
+// largest |value|, no cell sum exceeds cover * vm * wscale, kept within 2^30
+// (FP32) / 2^61 (FP64).  In FP32 a curve denser than kDenseCover takes a second
+// round over its points that accumulates what rounding each weight dropped, scaled
+// by up to 2^kDenseBits, so that a dense cell costs no precision; the first round's
+// integers wait in the workspace row of the workgroup.
+constexpr int kDenseCover = 64, kDenseBits = 14;
+
+// What tap_fixed (FP32, table) rounded off each weight: it repeats its operations,
+// so n_q is the same integer, and the rest up e3 - n_q is exact up to one rounding.
+template <int NTAPS, class Emit>
+__device__ __forceinline__ void tap_rest(float v, float e, float bi, const float *e3,
+                                         Emit &&emit) {
+    constexpr int Q0 = (NTAPS - 1) / 2;
+    const float E1 = dexp(-e * e * bi);
+    const float E2 = dexp(2.0f * e * bi);
+    const float E2i = dexp(-2.0f * e * bi);
+    const float h = copysignf(0.5f, v);
+    float up = v * E1;
+#pragma unroll
+    for (int q = Q0; q < NTAPS; ++q) {
+        emit(q, fmaf(up, e3[q], -(float)(int)fmaf(up, e3[q], h)));
+        up *= E2;
+    }
+    float dn = v * E1 * E2i;
+#pragma unroll
+    for (int q = Q0 - 1; q >= 0; --q) {
+        emit(q, fmaf(dn, e3[q], -(float)(int)fmaf(dn, e3[q], h)));
+        dn *= E2i;
+    }
+}
+
+// Twiddles: FP32 as the single-workgroup FFT takes them, rows in LDS and the last
+// pass of 2^13 and 2^14 points from the full table in global memory (two-level
+// products there raised the error of a survey's spectra from 2.3e-7 to 3.4e-7);
+// FP64, whose rows of 2^13 do not fit beside the grid and whose filter's error is
+// far above, as the fused bootstrap.
+template <typename T>
+__host__ __device__ constexpr int adjoint_cap(int lg) {
+    return sizeof(T) == 4 ? small_cap(lg) : boot_cap<T>(lg);
+}
+template <typename T>
+__host__ __device__ constexpr size_t adjoint_lds_bytes(int lg) {
+    const size_t two_level =
+        sizeof(T) == 4 ? 0 : ((size_t)1 << ((lg + 1) / 2)) + ((size_t)1 << (lg - (lg + 1) / 2));
+    return sizeof(cplx<T>) * (((size_t)1 << lg) +
+                              rows_count(lg, small_mr(lg), adjoint_cap<T>(lg)) + two_level) +
+           2 * kBootHalo * sizeof(T);
+}
+
+template <typename T>
+struct AdjointArgs {
+    const PointRec<T> *rec;  // (anchor, e) by original index
+    const T *y;              // nullable: unit weights
+    long y_stride;           // per value vector
+    const int *coff, *order, *cover;
+    int nrhs, total;         // total = curves * nrhs
+    int *hi;                 // dense curves: G integers per workgroup
+    T bi, wscale;
+    T e3[kMaxTaps];
+    SinkAccurate<T> sink;
+    const cplx<T> *twT;   // twiddle rows up to adjoint_cap
+    const cplx<T> *fine;  // FP32: w_N^e
+    Tw2<T> twN;           // FP64: the same by two levels
+    const cplx<T> *twH;   // w_G^e, e < workgroup size
+};
+
+template <typename T, int LG, int NTAPS, int NT>
+__global__ __launch_bounds__(NT) void k_adjoint_fused(AdjointArgs<T> A) {
+    using I = typename FixedOf<T>::I;
+    using U = std::make_unsigned_t<I>;
+    constexpr int N = 1 << LG, G = 2 * N, Q0 = (NTAPS - 1) / 2, PB = 4;
+    constexpr int LBN = (LG + 1) / 2, NLN = 1 << LBN, NHN = 1 << (LG - LBN);
+    constexpr int MR = small_mr(LG), CAP = adjoint_cap<T>(LG), NLT = rows_count(LG, MR, CAP);
+    using Rest = std::conditional_t<sizeof(T) == 4, const cplx<T> *, Tw2<T>>;
+    constexpr int kMaxExp = sizeof(T) == 4 ? 100 : 1000;
+    constexpr T kBig = sizeof(T) == 4 ? T(3.0e38f) : T(1.0e300);
+    T *grid = reinterpret_cast<T *>(cuna_smem) + kBootHalo;
+    U *gu = reinterpret_cast<U *>(grid);
+    cplx<T> *z = reinterpret_cast<cplx<T> *>(grid);
+    cplx<T> *tl = reinterpret_cast<cplx<T> *>(grid + G + kBootHalo);
+    __shared__ T vmax_sh[NT / 64];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < NLT; i += NT) tl[i] = A.twT[i];
+    TwRows<T, CAP, Rest> tw;
+    tw.lds = tl;
+    if constexpr (sizeof(T) == 4) {
+        tw.rest = A.fine;
+    } else {
+        for (int i = tid; i < NLN; i += NT) tl[NLT + i] = A.twN.lo[i];
+        for (int i = tid; i < NHN; i += NT) tl[NLT + NLN + i] = A.twN.hi[i];
+        tw.rest.lo = tl + NLT;
+        tw.rest.hi = tl + NLT + NLN;
+        tw.rest.lb = LBN;
+    }
+    constexpr int NE = (N / 2 + NT) / NT;
+    const cplx<T> wtid = A.twH[tid];
+    int *const hi = A.hi + (long)blockIdx.x * G;
+
+    for (int item = blockIdx.x; item < A.total; item += gridDim.x) {
+        const int ci = A.order[item / A.nrhs], r = item % A.nrhs;
+        const int c0 = A.coff[ci], nc = A.coff[ci + 1] - c0, cover = max(A.cover[ci], 1);
+        const PointRec<T> *P = A.rec + c0;
+        const T *y = A.y ? A.y + r * A.y_stride + c0 : nullptr;
+        // largest |value|; a non-finite value or position (NaN x gives NaN e)
+        // makes it infinite and the spectrum NaN
+        T vm = y ? T(0) : T(1);
+        for (int p0 = tid; p0 < nc; p0 += PB * NT) {
+            T v[PB], e[PB];
+#pragma unroll
+            for (int k = 0; k < PB; ++k) {
+                const int p = min(p0 + k * NT, nc - 1);
+                v[k] = y ? fabs(y[p]) : T(1);
+                e[k] = fabs(P[p].e);
+            }
+#pragma unroll
+            for (int k = 0; k < PB; ++k)
+                vm = fmax(vm, v[k] <= kBig && e[k] <= kBig ? v[k] : T(INFINITY));
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) vm = fmax(vm, __shfl_xor(vm, o));
+        if ((tid & 63) == 0) vmax_sh[tid >> 6] = vm;
+        for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
+            reinterpret_cast<uint4 *>(cuna_smem)[i] = make_uint4(0, 0, 0, 0);
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) vm = fmax(vm, vmax_sh[w]);
+        const bool finite = vm <= kBig;  // uniform
+        int sexp = 0;
+        const double bound = (double)vm * (double)cover * (double)A.wscale;
+        int eb = -kMaxExp;  // ceil(log2(bound))
+        if (bound > 0 && finite && frexp(bound, &eb) == 0.5) --eb;
+        sexp = min(max(FixedOf<T>::headroom_bits - eb, -kMaxExp), kMaxExp);
+        const T mul = (T)ldexp((double)A.wscale, sexp);
+        // dense curves: rests of at most 1/2, `cover` of them in a cell, within 2^30
+        const int lowbits = min(kDenseBits, 31 - (32 - __clz(cover - 1)));
+        const float lowmul = ldexpf(1.0f, lowbits);
+        // one round over the points: each tap's integer, or (LOW) the scaled rest
+        // of its rounding, to its cell.  Thread t takes spl consecutive points:
+        // neighbours in neighbouring lanes would meet on one cell (see k_boot_fused)
+        const int spl = (nc + NT - 1) / NT;
+        auto round = [&](auto low) __attribute__((always_inline)) {
+            constexpr bool LOW = decltype(low)::value;
+            for (int k0 = 0; k0 < spl; k0 += PB) {
+                PointRec<T> pr[PB];
+                T vv[PB];
+#pragma unroll
+                for (int k = 0; k < PB; ++k) {
+                    const int p = tid * spl + k0 + k, q = k0 + k < spl && p < nc ? p : 0;
+                    pr[k] = P[q];
+                    vv[k] = y ? y[q] : T(1);
+                }
+#pragma unroll
+                for (int k = 0; k < PB; ++k) {
+                    if (k0 + k < spl && tid * spl + k0 + k < nc) {
+                        U *dst = gu + (pr[k].a - Q0);
+                        if constexpr (LOW) {
+                            tap_rest<NTAPS>(vv[k] * mul, pr[k].e, A.bi, A.e3,
+                                            [&](int q, float rest) {
+                                                atomicAdd(dst + q, (U)__float2int_rn(rest * lowmul));
+                                            });
+                        } else if constexpr (sizeof(T) == 4) {
+                            tap_fixed<T, NTAPS, Fixed32, true>(
+                                vv[k] * mul, pr[k].e, A.bi, A.e3, T(0),
+                                [&](int q, unsigned n) { atomicAdd(dst + q, (U)n); });
+                        } else {
+                            T w[NTAPS];
+                            tap_weights<T, NTAPS>(vv[k] * mul, pr[k].e, A.bi, A.e3, w);
+#pragma unroll
+                            for (int q = 0; q < NTAPS; ++q)
+                                atomicAdd(dst + q, (U)FixedOf<T>::round(w[q]));
+                        }
+                    }
+                }
+            }
+        };
+        auto fold = [&]() __attribute__((always_inline)) {
+            __syncthreads();
+            if (tid < kBootHalo) {
+                gu[G - kBootHalo + tid] += gu[tid - kBootHalo];
+                gu[tid] += gu[G + tid];
+            }
+            __syncthreads();
+        };
+        if (finite) round(std::false_type{});
+        fold();
+        bool dense = false;
+        if constexpr (sizeof(T) == 4) {
+            dense = finite && cover > kDenseCover;  // uniform
+            if (dense) {
+                for (int i = tid; i < G; i += NT) hi[i] = (int)gu[i];
+                __syncthreads();
+                for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
+                    reinterpret_cast<uint4 *>(cuna_smem)[i] = make_uint4(0, 0, 0, 0);
+                __syncthreads();
+                round(std::true_type{});
+                fold();
+                // both parts as reals, in the integers' unit
+                for (int i = tid; i < G; i += NT)
+                    grid[i] = (T)hi[i] + (T)(int)gu[i] * (T)(1.0f / lowmul);
+                __syncthreads();
+            }
+        }
+        auto fetch = [&](int e, int) __attribute__((always_inline)) {
+            const FixedPair<I> q = reinterpret_cast<const FixedPair<I> *>(gu)[e];
+            return dense ? z[e] : cmk((T)q.x, (T)q.y);
+        };
+        fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, decltype(tw), MR>(
+            z, tw, fetch, NoHook());
+        SinkAccurate<T> sk = A.sink;
+        sk.pref *= finite ? (T)ldexp(1.0, -sexp) : (T)NAN;
+        cplx<T> *o = sk.row_out((long)ci * A.nrhs + r);
+        int t = tid;
+        cplx<T> w0 = wtid;
+        asm volatile("" : "+v"(t), "+v"(w0.x), "+v"(w0.y));
+        unroll<NE>([&](auto i) __attribute__((always_inline)) {
+            constexpr int k = decltype(i)::value;
+            const int f = t + k * NT;
+            const cplx<T> w =
+                k == 0 ? w0 : w0 * unit_root_32<T>(k * (G / NT > 0 ? 32 * NT / G : 1));
+            if (f <= N / 2)
+                emit_pair(sk, o, f, N, z[lds_sw(f)], z[lds_sw((N - f) & (N - 1))], w);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        __syncthreads();
+    }
 }
 
 // ----------------------------------------------------------- gather --
