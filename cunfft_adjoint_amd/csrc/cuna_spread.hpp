@@ -1619,7 +1619,9 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
     // transformed in place into z.  Returns the power of two that the spectrum is
     // to be multiplied by: the integers go through the FFT as they are.
     auto transform = [&](int c0, int nc, int nl, int rep, const FastMod &fm, const PointRec<T> *P,
-                         const T *y, T shift, double vm, int cover) __attribute__((always_inline)) -> T {
+                         const T *y, T shift, double vm, int cover,
+                         auto &&ahead) __attribute__((always_inline)) -> T {
+        ahead();
         const bool merged = nc <= A.list_cap;  // uniform
         int sexp = 0;
         if (vm <= 1e300) {  // false for NaN and inf
@@ -1738,14 +1740,21 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         return a * ((T(0.5) * sk.pref * scale) * dexp(sk.coef * kk * kk));
     };
 
-    // The first wave takes the next item off the queue while the workgroup
-    // works on the current one, and has its curve's entry in LDS by the end: an
-    // item then starts without a chain of global loads.
+    // The first item is the workgroup's index.  The first wave takes each further
+    // one off the queue while the workgroup works on the current one, and has its
+    // curve's entry in LDS by the end: an item then starts without a chain of global
+    // loads.  With many items per workgroup it does so first thing, otherwise before
+    // the current item's last transform, so that none waits behind a long one while
+    // other workgroups run dry.  Measured, early / late: 128 curves x 25 replicates,
+    // M = 2^14, 12 items each, 544 / 566 us; 64 x 25 periodograms, M = 2^13, 3 items
+    // each, 158 / 148 us.  (All off the queue and early, the first workgroups had a
+    // second item before the last ones had any: 8 curves x 24 replicates, M = 2^13,
+    // FP64 periodograms 88 us, now 52.)
     const int per_curve = A.nbs * (A.split ? A.ntr : 1);
     const int lane = tid & 63;
     const bool first_wave = tid < 64;
     auto take = [&]() __attribute__((always_inline)) -> int {
-        return lane == 0 ? atomicAdd(A.counter, 1) : 0;
+        return lane == 0 ? (int)gridDim.x + atomicAdd(A.counter, 1) : 0;
     };
     auto stage_item = [&](int item) __attribute__((always_inline)) {
         item = __builtin_amdgcn_readfirstlane(item);
@@ -1759,7 +1768,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         }
         if (lane <= kBootCurveWords) item_sh[lane] = w;  // (rem < 0: no item left)
     };
-    if (first_wave) stage_item(take());
+    if (first_wave) stage_item(blockIdx.x);
     __syncthreads();
     for (;;) {
         // uniform over the workgroup: scalar registers
@@ -1775,7 +1784,11 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
         const int cover_x = word(6), cover_2x = word(7);
         const double ymax = __longlong_as_double(((long long)word(9) << 32) | (unsigned)word(8));
         int next = 0;
-        if (first_wave) next = take();
+        const bool early = A.total >= 8 * (int)gridDim.x;
+        if (first_wave && early) next = take();
+        auto take_next = [&]() __attribute__((always_inline)) {
+            if (first_wave && !early) next = take();
+        };
         if constexpr (MODE == 0) {
             const int rep = A.split ? rem / A.ntr : rem;
             const int tr0 = A.split ? rem % A.ntr : 0, tr1 = A.split ? tr0 + 1 : A.ntr;
@@ -1784,7 +1797,9 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
                 const bool usey = tr == 0 && A.y;
                 const T scale = transform(c0, nc, nl, rep, fm, tr == 0 ? A.rec_x : A.rec_2x,
                                           usey ? A.y : nullptr, T(0), usey ? ymax : 1.0,
-                                          tr == 0 ? cover_x : cover_2x);
+                                          tr == 0 ? cover_x : cover_2x, [&] {
+                                              if (tr == tr1 - 1) take_next();
+                                          });
                 if (first_wave && tr == tr1 - 1) stage_item(next);
                 SinkAccurate<T> sk = A.sink;
                 sk.pref *= scale;
@@ -1816,7 +1831,7 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             const T yy = (T)fmax(0.0, s2 - s1 * mean_off);
             // window W(2w), parked in this workgroup's workspace row
             const T wscale =
-                transform(c0, nc, nl, rep, fm, A.rec_2x, nullptr, T(0), 1.0, cover_2x);
+                transform(c0, nc, nl, rep, fm, A.rec_2x, nullptr, T(0), 1.0, cover_2x, [] {});
             cplx<T> *wrow = A.ls_w + (long)blockIdx.x * half;
             epilogue([&](int f, cplx<T> w) __attribute__((always_inline)) {
                 if (f < half) wrow[f] = spectrum(f, w, wscale);
@@ -1824,7 +1839,8 @@ __global__ __launch_bounds__(NT) void k_boot_fused(BootArgs<T> A) {
             __syncthreads();
             // F(w) of the mean-subtracted values, then the power
             const double vm = ymax + fabs((double)ybar);
-            const T yscale = transform(c0, nc, nl, rep, fm, A.rec_x, A.y, ybar, vm, cover_x);
+            const T yscale =
+                transform(c0, nc, nl, rep, fm, A.rec_x, A.y, ybar, vm, cover_x, take_next);
             if (first_wave) stage_item(next);
             T best = T(-1);
             int kbest = 0;
