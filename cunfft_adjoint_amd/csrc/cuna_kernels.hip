@@ -370,20 +370,28 @@ template <typename T>
 bool launch_plan_curves(const PointRec<T> *rec_orig, const int *coff, int ncurves, int longest,
                         int tlog, int G, int Kc, int olo, int ohi, PointRec<T> *rec, int *perm,
                         int *bucket, hipStream_t s) {
-    const int abits = std::max(1, ilog2(G)), ibits = std::max(1, ilog2(std::max(longest, 1)));
-    if (longest > kPlanCurveMax || abits + ibits > 32) return false;
+    const int ibits = std::max(1, ilog2(std::max(longest, 1)));
+    if (longest > kPlanCurveMax || std::max(1, ilog2(G)) + ibits > 32) return false;
     if (ncurves <= 0) return true;
     // 256 threads where they hold a curve in 8 points each, so that several
     // curves share a CU
     const int NT = longest <= 2048 ? 256 : 1024;
+    // as many workgroups per curve as keep to one per CU (their LDS takes all of
+    // it) and have a point per thread on average; one curve of 20,011 points takes
+    // 53 us with one workgroup, 26 with 16
+    int parts = 1;
+    while (NT == 1024 && parts < 16 && 2L * parts * ncurves <= num_cus() &&
+           longest >= 2 * parts * NT && G >= 128 * parts)
+        parts *= 2;
+    const int abits = std::max(1, ilog2(ceil_div(G, parts)));  // of an anchor in its part
     const int cap = (std::max(longest, 1) + 7) & ~7;
     const int npass = (int)ceil_div(abits, kPlanDigitBits), bits = (int)ceil_div(abits, npass);
     const size_t lds = (sizeof(unsigned) + sizeof(short)) * (size_t)cap +
                        sizeof(short) * ((size_t)(NT / 64) << bits);
     auto go = [&](auto k) {
         set_lds(k, lds);
-        hipLaunchKernelGGL(k, dim3(ncurves), dim3(NT), lds, s, rec_orig, coff, cap, abits, ibits,
-                           tlog, G, Kc, olo, ohi, rec, perm, bucket);
+        hipLaunchKernelGGL(k, dim3(ncurves, parts), dim3(NT), lds, s, rec_orig, coff, cap, abits,
+                           ibits, tlog, G, Kc, olo, ohi, rec, perm, bucket);
         CUNA_LAUNCH_CHECK();
     };
     if (NT == 256)

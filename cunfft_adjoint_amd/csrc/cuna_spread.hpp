@@ -283,20 +283,24 @@ __global__ void k_buckets(const int *coff, int ncurves, int Kc, const PointRec<T
 }
 
 // ---------------------------------------- sort of short curves: one launch --
-// The sort by anchor and the buckets of one curve in one workgroup, for curves
-// of at most kPlanCurveMax points whose (anchor, index) pairs fit 32 bits.  A
-// point is the word anchor << ibits | index, held in LDS; an LSD radix sort over
-// the anchor's bits (digits of at most 9) permutes the words: stable, so the
-// order is that of the multi-launch sort.  Wave w ranks the consecutive words
-// [w seg, (w + 1) seg), 64 per step: a word's rank is the count of equal digits
-// in the wave's earlier steps (16-bit counters per wave) plus the lower lanes
-// with the same digit (nine ballots); the scan of the
-// counters turns it into a place, and every thread moves its IPT words through
-// registers.  Bound by instruction issue in the ranking steps (one workgroup
-// per CU, four waves per SIMD).  It stands in for the sort's launches (digits,
-// histogram, three scan steps and scatter per digit, and the buckets): at 64
-// curves of 20,000 points and 2^17 cells 18 launches and 172 us -> 1 launch and
-// 52 us; at one curve of 20,011 points and 2^16 cells (FP64) 77 -> 55 us.
+// The sort by anchor and the buckets of a curve, for curves of at most
+// kPlanCurveMax points whose (anchor, index) pairs fit 32 bits, by gridDim.y
+// workgroups that share the curve's anchor range: each takes the points of its
+// part of the range, in order of index, sorts them alone and writes them behind
+// the points of the parts below, which it has counted on the way.  A point is the
+// word anchor << ibits | index, held in LDS (room for all of the curve, so that
+// clustered points change only the time); an LSD radix sort over the anchor's bits
+// (digits of at most 9) permutes the words: stable, so the order is that of the
+// multi-launch sort.  Wave w ranks the consecutive words [w seg, (w + 1) seg), 64
+// per step: a word's rank is the count of equal digits in the wave's earlier steps
+// (16-bit counters per wave) plus the lower lanes with the same digit (nine
+// ballots); the scan of the counters turns it into a place, and every thread moves
+// its IPT words through registers.  Bound by instruction issue in the ranking
+// steps, hence the split where curves are fewer than CUs.  It stands in for the
+// sort's launches (histogram, two scan steps and scatter per digit, and the
+// buckets).  Measured: 64 curves of 20,000 points and 2^17 cells 34 us with 4 parts
+// (50 with one); one curve of 20,011 points and 2^16 cells, FP64, 26 us with 16 (53
+// with one).
 constexpr int kPlanCurveMax = 23 * 1024, kPlanDigitBits = 9;
 
 template <typename T, int NT, int IPT>
@@ -308,22 +312,65 @@ __global__ __launch_bounds__(NT) void k_plan_curve(const PointRec<T> *rec_orig, 
     unsigned *sv = reinterpret_cast<unsigned *>(cuna_smem);              // cap words
     unsigned short *rk = reinterpret_cast<unsigned short *>(sv + cap);   // cap ranks
     unsigned short *cnt = rk + cap;                                      // [wave][digit]
-    __shared__ int wsum[NW];
-    const int c = blockIdx.x, c0 = coff[c], n = coff[c + 1] - c0;
+    __shared__ int wsum[NW], wbelow[NW];
+    const int c = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // this workgroup's anchors [alo, ahi); the outer parts are open
+    const int part = blockIdx.y, parts = gridDim.y;
+    const int alo = part > 0 ? (int)((long)part * G / parts) : INT_MIN;
+    const int ahi = part + 1 < parts ? (int)((long)(part + 1) * G / parts) : INT_MAX;
+    const int abase = part > 0 ? alo : 0;  // the words' anchors count from here
+    const int c0 = coff[c];
+    int n = coff[c + 1] - c0;
+    int below = 0;  // points of the parts below
+    {
+        const int len = (n + NT - 1) / NT * 64, q0 = min(wave * len, n), q1 = min(q0 + len, n);
+        int a[IPT], mine = 0;
+#pragma unroll
+        for (int s = 0; s < IPT; ++s)  // (clamped loads: all issue together)
+            a[s] = s * 64 < len ? rec_orig[c0 + max(min(q0 + s * 64 + lane, q1 - 1), 0)].a : 0;
+#pragma unroll
+        for (int s = 0; s < IPT; ++s) {
+            if (s * 64 < len) {
+                const bool in = q0 + s * 64 + lane < q1;
+                below += __popcll(__ballot(in && a[s] < alo));
+                mine += __popcll(__ballot(in && a[s] >= alo && a[s] < ahi));
+            }
+        }
+        if (lane == 0) {
+            wsum[wave] = mine;
+            wbelow[wave] = below;
+        }
+        __syncthreads();
+        int at = 0;
+        mine = below = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            if (w < wave) at += wsum[w];
+            mine += wsum[w];
+            below += wbelow[w];
+        }
+#pragma unroll
+        for (int s = 0; s < IPT; ++s) {
+            if (s * 64 < len) {
+                const int q = q0 + s * 64 + lane;
+                const bool in = q < q1 && a[s] >= alo && a[s] < ahi;
+                const unsigned long long m = __ballot(in);
+                if (in)
+                    sv[at + __builtin_amdgcn_mbcnt_hi(
+                                (unsigned)(m >> 32),
+                                __builtin_amdgcn_mbcnt_lo((unsigned)m, 0))] =
+                        (unsigned)(a[s] - abase) << ibits | (unsigned)q;
+                at += __popcll(m);
+            }
+        }
+        n = __builtin_amdgcn_readfirstlane(mine);
+        below = __builtin_amdgcn_readfirstlane(below);
+        __syncthreads();
+    }
     const int seg = (n + NT - 1) / NT * 64;  // words per wave
     const int w0 = min(wave * seg, n), w1 = min(w0 + seg, n);
-    for (int p0 = tid; p0 < n; p0 += UN * NT) {
-        int a[UN];  // (clamped loads: all issue together)
-#pragma unroll
-        for (int k = 0; k < UN; ++k) a[k] = rec_orig[c0 + min(p0 + k * NT, n - 1)].a;
-#pragma unroll
-        for (int k = 0; k < UN; ++k) {
-            const int p = p0 + k * NT;
-            if (p < n) sv[p] = (unsigned)a[k] << ibits | (unsigned)p;
-        }
-    }
     int shift = ibits, left = abits;
     for (int pass = (abits + kPlanDigitBits - 1) / kPlanDigitBits; pass > 0; --pass) {
         const int bits = (left + pass - 1) / pass, K = 1 << bits;
@@ -338,7 +385,10 @@ __global__ __launch_bounds__(NT) void k_plan_curve(const PointRec<T> *rec_orig, 
             const unsigned d = (sv[q] >> shift) & mask;
             // (a lane past the end counts all its peers as lower: it never writes)
             int r, peers;
-            match_digit<kPlanDigitBits>(d, act, r, peers);
+            if (bits <= 6)  // uniform
+                match_digit<6>(d, act, r, peers);
+            else
+                match_digit<kPlanDigitBits>(d, act, r, peers);
             const int cur = cw[d];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -388,9 +438,13 @@ __global__ __launch_bounds__(NT) void k_plan_curve(const PointRec<T> *rec_orig, 
         unsigned short to[IPT];
 #pragma unroll
         for (int s = 0; s < IPT; ++s) {
-            const int q = max(min(w0 + s * 64 + lane, w1 - 1), 0);
-            v[s] = sv[q];
-            to[s] = (unsigned short)(rk[q] + cw[(v[s] >> shift) & mask]);
+            v[s] = 0;
+            to[s] = 0;
+            if (s * 64 < seg) {  // uniform
+                const int q = max(min(w0 + s * 64 + lane, w1 - 1), 0);
+                v[s] = sv[q];
+                to[s] = (unsigned short)(rk[q] + cw[(v[s] >> shift) & mask]);
+            }
             if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // fewer registers
         }
         __syncthreads();
@@ -415,24 +469,27 @@ __global__ __launch_bounds__(NT) void k_plan_curve(const PointRec<T> *rec_orig, 
             const int j = j0 + k * NT;
             if (j < n) {
                 PointRec<T> pr;
-                pr.a = (int)(w[k] >> ibits);
+                pr.a = abase + (int)(w[k] >> ibits);
                 pr.e = e[k];
-                rec[c0 + j] = pr;
-                perm[c0 + j] = c0 + (int)(w[k] & imask);
+                rec[c0 + below + j] = pr;
+                perm[c0 + below + j] = c0 + (int)(w[k] & imask);
             }
         }
     }
-    // bucket[k]: first sorted point with tile_key >= k, as in k_buckets
-    for (int k = tid; k <= Kc; k += NT) {
+    // bucket[k]: first sorted point with tile_key >= k, as in k_buckets; the keys
+    // whose first anchor lies in this part
+    const int k0 = part > 0 ? tile_key(alo - 1, tlog, olo, ohi, G) + 1 : 0;
+    const int k1 = part + 1 < parts ? tile_key(ahi - 1, tlog, olo, ohi, G) : Kc;
+    for (int k = k0 + tid; k <= k1; k += NT) {
         int lo = k < Kc ? 0 : n, hi = n;
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
-            if (tile_key((int)(sv[mid] >> ibits), tlog, olo, ohi, G) < k)
+            if (tile_key(abase + (int)(sv[mid] >> ibits), tlog, olo, ohi, G) < k)
                 lo = mid + 1;
             else
                 hi = mid;
         }
-        bucket[(long)c * (Kc + 1) + k] = c0 + lo;
+        bucket[(long)c * (Kc + 1) + k] = c0 + below + lo;
     }
 }
 
