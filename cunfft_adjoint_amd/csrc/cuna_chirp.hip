@@ -12,13 +12,13 @@
 // k^2 mod 2 n (exact integer), so its phase carries no error that grows with k.
 //
 // The chirp products, the two FFTs and the product with the convolution kernel's
-// transform are fused: one launch when L fits a workgroup's LDS, else three (the
-// first column pass reads and premultiplies the grid; a row pass transforms each
-// row forward, multiplies and transforms it back in LDS; the last column pass
-// applies the chirp and writes the output), plus the even grid's pairing.  Bound
-// by the passes' loads and stores, as the power-of-two FFT.  Measured at ng =
-// 300,000, FP32: 63 us in seven launches over L = 2^20 -> 27 us
-// in four over 2^19 (rocprofv3 sums).
+// transform are fused: one launch when L fits a workgroup's LDS (and, at its
+// largest, the rows are many), else three (the first column pass reads and
+// premultiplies the grid; a row pass transforms each row forward, multiplies and
+// transforms it back in LDS; the last column pass applies the chirp and writes the
+// output), plus the even grid's pairing.  Bound by the passes' loads and stores, as
+// the power-of-two FFT.  Measured at ng = 300,000, FP32: 63 us in seven launches
+// over L = 2^20 -> 27 us in four over 2^19 (rocprofv3 sums).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -284,6 +284,28 @@ void Bluestein<T>::init(int length, bool real, hipStream_t s) {
     hipLaunchKernelGGL(k_chirp_rows<T>, dim3(ceil_div(L, 256)), dim3(256), 0, s, w, 1 << lg1,
                        1 << (lgL - lg1), T(1) / (T)L, bt.as<cplx<T>>());
     CUNA_LAUNCH_CHECK();
+    if (both_forms()) {
+        bt_rows.alloc(sizeof(cplx<T>) * L, s);
+        const int l1 = split_lg1(lgL);
+        hipLaunchKernelGGL(k_chirp_rows<T>, dim3(ceil_div(L, 256)), dim3(256), 0, s, w, 1 << l1,
+                           1 << (lgL - l1), T(1) / (T)L, bt_rows.as<cplx<T>>());
+        CUNA_LAUNCH_CHECK();
+    }
+}
+
+// The largest length that one workgroup holds.  Its two FFTs take one CU 20 us, so
+// few rows go through the three passes, which spread them over the chip.  Measured,
+// with the spread, one workgroup per row / three passes: FP32, L = 2^14, 2 rows
+// 34.5 / 22.6 us, 64 rows 38.1 / 32.8, 100 rows 41.8 / 42.5; FP64, L = 2^13, 2 rows
+// 26.7 / 19.2 us, 32 rows 26.8 / 22.5, 64 rows 27.6 / 28.6.  (FP32 at 2^13: 20.5 /
+// 21.9 us at 2 rows, 21.0 / 23.3 at 48.)
+template <typename T>
+bool Bluestein<T>::both_forms() const {
+    return lgL == max_small_lg<T>();
+}
+template <typename T>
+static constexpr int chirp_pass_rows() {
+    return sizeof(T) == 4 ? 64 : 32;
 }
 
 template <typename T>
@@ -299,7 +321,7 @@ void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int bat
     require(batch <= batch_cap, "Bluestein workspace too small for this batch");
     auto &tc = TwiddleCache<T>::get();
     const cplx<T> *const wng = pairs ? chirp() + n : nullptr;
-    if (lgL <= max_small_lg<T>()) {
+    if (lgL <= max_small_lg<T>() && !(both_forms() && batch <= chirp_pass_rows<T>())) {
         dispatch_lg<1, max_small_lg<T>()>(lgL, [&](auto c) {
             constexpr int LG = decltype(c)::value, MR = small_mr(LG), CAP = small_cap(LG);
             constexpr int NT = fft_threads(LG, 1, MR);
@@ -317,6 +339,7 @@ void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int bat
     const int W = pick_seq<T>(lg2, L1, batch, 1, "CUNA_FFT_W", 0, num_cus());
     const int H = pick_seq<T>(lg1, L2, batch, 1, "CUNA_FFT_H", 0, num_cus());
     cplx<T> *const a = work.as<cplx<T>>();
+    const cplx<T> *const b = (both_forms() ? bt_rows : bt).template as<cplx<T>>();
     auto batches = [&](auto &&launch) {
         for (long b0 = 0; b0 < batch; b0 += kMaxGridY) {
             launch(b0, (int)std::min<long>(kMaxGridY, batch - b0));
@@ -337,7 +360,7 @@ void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int bat
             });
         });
     });
-    dispatch_lg<7, 12>(lg1, [&](auto c) {
+    dispatch_lg<6, 12>(lg1, [&](auto c) {
         constexpr int LG1 = decltype(c)::value;
         dispatch_w<T, LG1>(H, [&](auto h) {
             constexpr int HH = decltype(h)::value, NT = fft_threads(LG1, HH, kRowMr);
@@ -347,8 +370,7 @@ void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int bat
             set_lds(k, lds);
             batches([&](long b0, int nb) {
                 hipLaunchKernelGGL(k, dim3(L2 / HH, nb), dim3(NT), lds, s, a, L, L2,
-                                   bt.as<cplx<T>>(), tc.rows(LG1, kRowMr, LG1), tc.two_level(lgL),
-                                   b0);
+                                   b, tc.rows(LG1, kRowMr, LG1), tc.two_level(lgL), b0);
             });
         });
     });

@@ -131,6 +131,7 @@ struct Bluestein {
     long L = 0;
     DevMem tab;   // c_k, k < n, then (pairs) exp(2 pi i r/ng), r <= n/2
     DevMem bt;    // FFT_-(b) / L, in the order of the passes
+    DevMem bt_rows;  // both_forms(): bt in the order of the three passes
     DevMem work;  // batch_cap x L complex
     int batch_cap = 0;
     // real: run_real will be called (else run_complex)
@@ -145,6 +146,7 @@ struct Bluestein {
 
   private:
     const cplx<T> *chirp() const { return tab.template as<cplx<T>>(); }
+    bool both_forms() const;
     void run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch, hipStream_t s);
 };
 

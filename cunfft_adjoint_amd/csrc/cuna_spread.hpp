@@ -1379,10 +1379,10 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
 // LDS float atomics are slow on this hardware, so the grid accumulates in
 // fixed point with integer atomics (int32 in the FP32 library, int64 in FP64),
 // which are also order-independent.  The power-of-two scale comes from the
-// curve's max |y| and its densest tap window; an addition that overflows is
-// detected from the returned old value and the item is redone at a smaller
-// scale.  The integer grid occupies the same LDS words as the complex
-// buffer of the FFT, whose first pass reads and converts it.
+// curve's max |y| and its densest tap window; the draws' own density is counted on
+// the way, and an item denser than the scale allows is redone.  The integer grid
+// occupies the same LDS words as the complex buffer of the FFT, whose first pass
+// reads and converts it.
 //
 // What an item needs of its curve, one entry per curve in queue order.
 struct BootCurve {
