@@ -81,6 +81,17 @@ static void run_row_plain(const FftShape &sh, const cplx<T> *src, int L2, cplx<T
     }
 }
 
+// Rows up to which the largest transform that one workgroup holds goes through two
+// passes all the same: one workgroup per row leaves the chip idle and takes the
+// whole transform's LDS passes in a row.  Measured, spread and transform, one
+// workgroup per row / two passes: FP32, 2^14, 1 row 21.6 / 15.9 us, 64 rows 29.5 /
+// 25.0, 100 rows 35.0 / 32.6, 160 rows 41.1 / 42.4; FP64, 2^13, 1 row 20.1 / 16.0
+// us, 32 rows 28.9 / 27.4, 48 rows 32.9 / 33.0.
+template <typename T>
+static bool few_rows(const FftShape &sh) {
+    return sh.lgN == max_small_lg<T>() && sh.batch <= (sizeof(T) == 4 ? 100 : 32);
+}
+
 template <typename T, class Sink>
 static void real_forward_impl(const FftShape &sh, T *grid, const Sink &sk, hipStream_t s,
                               hipEvent_t mid) {
@@ -89,7 +100,7 @@ static void real_forward_impl(const FftShape &sh, T *grid, const Sink &sk, hipSt
     LoadGrid<T> ld;
     ld.z = reinterpret_cast<const cplx<T> *>(grid);
     ld.stride = 1L << sh.lgN;
-    if (sh.lgN <= max_small_lg<T>()) {
+    if (sh.lgN <= max_small_lg<T>() && !few_rows<T>(sh)) {
         dispatch_lg<1, max_small_lg<T>()>(sh.lgN, [&](auto c) {
             run_small<T, 1, decltype(c)::value, LoadGrid<T>, Sink, 0>(sh, ld, sk, nullptr, s);
         });
@@ -106,7 +117,7 @@ static void real_forward_impl(const FftShape &sh, T *grid, const Sink &sk, hipSt
         });
     });
     if (mid) CUNA_HIP(hipEventRecord(mid, s));
-    dispatch_lg<7, 12>(lg1, [&](auto c) {
+    dispatch_lg<6, 12>(lg1, [&](auto c) {
         constexpr int LG1 = decltype(c)::value;
         dispatch_h<T, LG1>(H, [&](auto h) {
             run_row_real<T, LG1, decltype(h)::value, Sink>(sh, z, 1 << lg2, sk, s);
@@ -134,8 +145,8 @@ void fft_c2r_inverse(const FftShape &sh, const LoadHermitian<T> &ld, cplx<T> *wo
     SinkAccurate<T> dummy{};
     // the Hermitian loader is register-heavy: a 1024-thread workgroup (N =
     // 2^14) would spill, so N >= 2^14 takes the two-pass path in both
-    // libraries, whose first split then has L1 >= 2^7
-    if (sh.lgN <= kC2rSmallLg) {
+    // libraries; FP64 at 2^13 does so for few rows, as the forward transform
+    if (sh.lgN <= kC2rSmallLg && !few_rows<T>(sh)) {
         dispatch_lg<1, kC2rSmallLg>(sh.lgN, [&](auto c) {
             run_small<T, -1, decltype(c)::value, LoadHermitian<T>, SinkAccurate<T>, 1>(
                 sh, ld, dummy, z, s);
@@ -151,7 +162,7 @@ void fft_c2r_inverse(const FftShape &sh, const LoadHermitian<T> &ld, cplx<T> *wo
             run_col<T, -1, LG2, decltype(w)::value, LoadHermitian<T>>(sh, ld, work, 1 << lg1, s);
         });
     });
-    dispatch_lg<7, 12>(lg1, [&](auto c) {
+    dispatch_lg<6, 12>(lg1, [&](auto c) {
         constexpr int LG1 = decltype(c)::value;
         dispatch_w<T, LG1>(H, [&](auto h) {
             run_row_plain<T, -1, LG1, decltype(h)::value>(sh, work, 1 << lg2, z, s);
