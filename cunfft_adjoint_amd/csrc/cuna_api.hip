@@ -125,9 +125,7 @@ void *BlockPool::take(size_t nbytes, size_t *got, int *dev, hipStream_t s) {
         std::lock_guard<std::mutex> lk(K.mu);
         for (auto it = K.blocks.begin(); it != K.blocks.end(); ++it) {
             if (it->bytes != n || it->dev != *dev) continue;
-            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-            CUNA_HIP(hipStreamIsCapturing(s, &st));
-            require(st == hipStreamCaptureStatusNone,
+            require(!capturing(s),
                     "device memory cannot be allocated while the stream is captured "
                     "(run the call once before capturing it)",
                     CUNA_ERROR_HIP);

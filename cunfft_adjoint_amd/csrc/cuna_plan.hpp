@@ -31,12 +31,29 @@ struct BlockPool {
     static void clear();
 };
 
+// true while `s` is being captured into a graph (the null stream never is)
+inline bool capturing(hipStream_t s) {
+    if (!s) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    CUNA_HIP(hipStreamIsCapturing(s, &st));
+    return st != hipStreamCaptureStatusNone;
+}
+
 // Persistent device allocation.
 struct DevMem {
     void *ptr = nullptr;
     size_t bytes = 0;
     int dev = 0;
     bool owned = true;  // false: a view into another allocation
+    // a captured call used this memory: its graph holds the address, so a block
+    // that ensure() outgrows stays this object's own until release()
+    bool in_graph = false;
+    struct Outgrown {
+        void *p;
+        size_t bytes;
+        int dev;
+    };
+    std::vector<Outgrown> outgrown;
     DevMem() = default;
     DevMem(const DevMem &) = delete;
     DevMem &operator=(const DevMem &) = delete;
@@ -51,11 +68,33 @@ struct DevMem {
         bytes = nbytes;
         owned = false;
     }
+    // at least nbytes, for a call on s (its contents are not kept).  A captured
+    // call that is refused memory leaves what there was.
     void ensure(size_t nbytes, hipStream_t s) {
-        if (nbytes > bytes) alloc(nbytes, s);
+        const bool now = capturing(s);
+        if (nbytes > bytes) {
+            if (!now && !in_graph) {
+                alloc(nbytes, s);
+            } else {
+                size_t got = 0;
+                int d = 0;
+                void *p = BlockPool::take(nbytes, &got, &d, s);
+                if (ptr) outgrown.push_back(Outgrown{ptr, bytes, dev});
+                ptr = p;
+                bytes = got;
+                dev = d;
+                in_graph = false;
+            }
+        }
+        in_graph = in_graph || now;
     }
+    // a call on s reads or writes this memory as it is
+    void use(hipStream_t s) { in_graph = in_graph || capturing(s); }
     void release() {
         if (ptr && owned) BlockPool::give(ptr, bytes, dev);
+        for (const Outgrown &o : outgrown) BlockPool::give(o.p, o.bytes, o.dev);
+        outgrown.clear();
+        in_graph = false;
         ptr = nullptr;
         bytes = 0;
         owned = true;
