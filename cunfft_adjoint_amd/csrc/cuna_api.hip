@@ -883,7 +883,10 @@ std::unique_ptr<Plan<T>> make_plan_accurate(const T *x, const double *t, double 
         }
         P->has_pts2 = true;
     }
-    if (P->fused_adjoint) P->covers(s);
+    if (P->fused_adjoint) {
+        P->covers(s);
+        warm_adjoint_fused<T>(P->lgN);
+    }
     P->prepare_fft(s);
     return P;
 }

@@ -467,15 +467,28 @@ int fused_slots(int lgN) {
     return num_cus() * std::max(1, (int)(kMaxLds / boot_lds_bytes<T>(lgN)));
 }
 
-template <typename T, int LG, int NTAPS>
-static void adjoint_fused_one(AdjointArgs<T> A, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
-    constexpr int NT = fused_threads(LG);
+template <typename T, int LG>
+static void adjoint_fused_tables(AdjointArgs<T> &A) {
     auto &tc = TwiddleCache<T>::get();
     constexpr int CAP = adjoint_cap<T>(LG);
     A.twT = tc.rows(LG, small_mr(LG), CAP);
     A.fine = sizeof(T) == 4 && LG > CAP ? tc.fine(LG) : nullptr;
     A.twN = tc.two_level(LG);
-    A.twH = tc.head(LG + 1, NT);
+    A.twH = tc.head(LG + 1, fused_threads(LG));
+}
+
+template <typename T>
+void warm_adjoint_fused(int lgN) {
+    dispatch_lg<6, max_small_lg<T>()>(lgN, [&](auto c) {
+        AdjointArgs<T> A{};
+        adjoint_fused_tables<T, decltype(c)::value>(A);
+    });
+}
+
+template <typename T, int LG, int NTAPS>
+static void adjoint_fused_one(AdjointArgs<T> A, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
+    constexpr int NT = fused_threads(LG);
+    adjoint_fused_tables<T, LG>(A);
     constexpr size_t lds = adjoint_lds_bytes<T>(LG);
     static_assert(lds <= kMaxLds - 256, "fused adjoint LDS");
     auto k = k_adjoint_fused<T, LG, NTAPS, NT>;
@@ -605,6 +618,7 @@ template bool launch_plan_curves<dTyp>(const PointRec<dTyp> *, const int *, int,
                                        int, int, PointRec<dTyp> *, int *, int *, hipStream_t);
 template bool boot_fused_supported<dTyp>(int, int);
 template int fused_slots<dTyp>(int);
+template void warm_adjoint_fused<dTyp>(int);
 template void launch_adjoint_fused<dTyp>(const AdjointArgs<dTyp> &, int, int, hipStream_t,
                                          hipEvent_t, hipEvent_t);
 template void launch_boot_fused<dTyp>(BootArgs<dTyp>, int, int, int, hipStream_t);

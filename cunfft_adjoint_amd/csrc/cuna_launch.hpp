@@ -100,6 +100,10 @@ int fused_slots(int lgN);
 template <typename T>
 void launch_adjoint_fused(const AdjointArgs<T> &A, int lgN, int ntaps, hipStream_t s,
                           hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// the twiddle tables of its launches (made at plan creation, so that a captured
+// call makes none)
+template <typename T>
+void warm_adjoint_fused(int lgN);
 // per-curve densest tap window (G <= 2^15)
 template <typename T>
 void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, int G, int ntaps,

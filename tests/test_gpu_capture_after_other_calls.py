@@ -1,0 +1,50 @@
+"""Calls that can be captured once another call of the plan has run, because all
+they need is there by then."""
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+FUSED = """
+import numpy as np, torch
+import cunfft_adjoint_amd as cu
+dt, cdt, prec = {dt}
+rng = np.random.default_rng(2)
+n, M = 200, {M}
+x = torch.from_numpy(rng.uniform(-0.5, 0.5, n).astype(dt)).cuda()
+y = torch.from_numpy(rng.standard_normal(n).astype(dt)).cuda()
+plan = cu.NFFTPlan(x, M)
+s = torch.cuda.Stream()
+out = torch.empty((1, M), dtype=cdt, device="cuda")
+plan.backward(y, torch.ones((1, M), dtype=cdt, device="cuda"))
+torch.cuda.synchronize()
+g = cu.capture(lambda: plan.adjoint(y, out=out, stream=s), s, prec)
+for _ in range(3):
+    out.zero_()
+    torch.cuda.synchronize()
+    g.launch(s)
+    s.synchronize()
+    got = out.cpu().numpy()
+    assert np.array_equal(got, plan.adjoint(y).cpu().numpy())
+print("done")
+"""
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+@pytest.mark.parametrize("dt", ["np.float32, torch.complex64, 'f'", "np.float64, torch.complex128, 'd'"])
+@pytest.mark.parametrize("M", [1 << 8, 1 << 12])
+def test_fused_adjoint_after_a_backward(dt, M):
+    """In a process of its own: twiddle tables are kept per process."""
+    r = subprocess.run([sys.executable, "-c", FUSED.format(dt=dt, M=M)], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and "done" in r.stdout, r.stdout + r.stderr
