@@ -310,15 +310,14 @@ static constexpr int chirp_pass_rows() {
 
 template <typename T>
 void Bluestein<T>::ensure(int batch, hipStream_t s) {
-    if (batch <= batch_cap) return;
     work.ensure(sizeof(cplx<T>) * (size_t)L * (size_t)batch, s);
-    batch_cap = batch;
 }
 
 template <typename T>
 void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch,
                        hipStream_t s) {
-    require(batch <= batch_cap, "Bluestein workspace too small for this batch");
+    require(sizeof(cplx<T>) * (size_t)L * (size_t)batch <= work.bytes,
+            "Bluestein workspace too small for this batch");
     work.use(s);
     auto &tc = TwiddleCache<T>::get();
     const cplx<T> *const wng = pairs ? chirp() + n : nullptr;

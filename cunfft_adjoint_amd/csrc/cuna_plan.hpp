@@ -74,7 +74,8 @@ struct DevMem {
         const bool now = capturing(s);
         if (nbytes > bytes) {
             if (!now && !in_graph) {
-                alloc(nbytes, s);
+                drop();
+                ptr = BlockPool::take(nbytes, &bytes, &dev, s);
             } else {
                 size_t got = 0;
                 int d = 0;
@@ -90,14 +91,18 @@ struct DevMem {
     }
     // a call on s reads or writes this memory as it is
     void use(hipStream_t s) { in_graph = in_graph || capturing(s); }
-    void release() {
+    // gives up the current memory, not what graphs hold of earlier memory
+    void drop() {
         if (ptr && owned) BlockPool::give(ptr, bytes, dev);
-        for (const Outgrown &o : outgrown) BlockPool::give(o.p, o.bytes, o.dev);
-        outgrown.clear();
-        in_graph = false;
         ptr = nullptr;
         bytes = 0;
         owned = true;
+    }
+    void release() {
+        drop();
+        for (const Outgrown &o : outgrown) BlockPool::give(o.p, o.bytes, o.dev);
+        outgrown.clear();
+        in_graph = false;
     }
     ~DevMem() { release(); }
     template <typename U>
@@ -171,8 +176,7 @@ struct Bluestein {
     DevMem tab;   // c_k, k < n, then (pairs) exp(2 pi i r/ng), r <= n/2
     DevMem bt;    // FFT_-(b) / L, in the order of the passes
     DevMem bt_rows;  // both_forms(): bt in the order of the three passes
-    DevMem work;  // batch_cap x L complex
-    int batch_cap = 0;
+    DevMem work;  // batch x L complex, batch as large as ensure() asked for
     // real: run_real will be called (else run_complex)
     void init(int length, bool real, hipStream_t s);
     void ensure(int batch, hipStream_t s);

@@ -46,7 +46,7 @@ def replays_equal(g, s, out, want):
         assert np.array_equal(out.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("later", ["forward", "adjoint_many"])
+@pytest.mark.parametrize("later", ["forward", "adjoint_many", "both"])
 def test_adjoint_graph_after_larger_calls(later):
     M = 1 << 16
     cu.batch_cache_clear("f")
@@ -59,9 +59,9 @@ def test_adjoint_graph_after_larger_calls(later):
     s.synchronize()
     want = out.cpu().numpy().copy()
     g = cu.capture(lambda: plan.adjoint(y, out=out, stream=s), s)
-    if later == "forward":
+    if later != "adjoint_many":
         plan.forward(spectrum(M))
-    else:
+    if later != "forward":
         plan.adjoint_many(torch.stack([y, 2 * y, 3 * y]).contiguous())
     torch.cuda.synchronize()
     p2, y2, want2 = other_plan()
