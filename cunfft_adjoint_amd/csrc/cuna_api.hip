@@ -751,18 +751,38 @@ void Plan<T>::backward(const T *y, const cplx<T> *g, T *dy, T *dx, hipStream_t s
 // by linearity the imaginary part is the same with -i fhat.  Both grids of a
 // curve go through one batched inverse FFT and one gather, which forms each
 // point's weights once.  Measured at M = 2^18, 300,007 clustered points, FP32:
-// 20.5 us, against 52.3 us with one FFT and one gather per part.  Beyond
-// kBothPartsBytes of workspace the parts follow each other instead (half the
-// memory; a transform that large fills the chip by itself).
+// 20.5 us, against 52.3 us with one FFT and one gather per part.  The parts follow
+// each other instead where there is no room for both: beyond kBothPartsBytes of
+// workspace (a transform that large fills the chip by itself), when the device has
+// not that much left, and in a captured call whose plan has only run calls of one
+// grid per curve so far (a capture allocates nothing).
+template <typename T>
+bool Plan<T>::room_for_both_parts(hipStream_t s) {
+    constexpr size_t kBothPartsBytes = size_t(4) << 30;
+    const size_t grids = 2 * sizeof(T) * (size_t)G * ncurves();  // the FFT's buffers are as large
+    if (2 * grids > kBothPartsBytes) return false;
+    if (grids <= grid.bytes && grids <= work.bytes) return true;
+    if (capturing(s)) return false;
+    try {
+        grid.ensure(grids, s);
+        work.ensure(grids, s);
+        return true;
+    } catch (const Error &e) {
+        if (e.code != CUNA_ERROR_OUT_OF_MEMORY) throw;
+        (void)hipGetLastError();
+        if (!grid.in_graph) grid.drop();
+        if (!work.in_graph) work.drop();
+        return false;
+    }
+}
+
 template <typename T>
 void Plan<T>::forward(const cplx<T> *fhat, cplx<T> *f, hipStream_t s) {
     require(spec.mode == CUNA_MODE_ACCURATE, "forward needs an accurate-mode plan");
     require(fhat != nullptr && f != nullptr, "NULL pointer");
     const int nc = ncurves();
     pts.tiles(s);
-    constexpr size_t kBothPartsBytes = size_t(4) << 30;
-    const size_t both = 4 * sizeof(T) * (size_t)G * nc;  // two grids and two FFT buffers
-    if (both <= kBothPartsBytes) {
+    if (room_for_both_parts(s)) {
         spectrum_to_grid(fhat, 2, 0, s);
         GatherArgs<T> A = gather_args();
         A.dy = reinterpret_cast<T *>(f);

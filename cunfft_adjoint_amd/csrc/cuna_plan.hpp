@@ -263,6 +263,7 @@ struct Plan {
     GatherArgs<T> gather_args() const;
     SinkAccurate<T> accurate_sink(cplx<T> *out) const;
     void spectrum_to_grid(const cplx<T> *g, int parts, int rot, hipStream_t s);
+    bool room_for_both_parts(hipStream_t s);
     BootArgs<T> fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s);
     void run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s,
                  hipEvent_t mid = nullptr) const;
