@@ -369,10 +369,14 @@ void launch_tile_order(const SpreadArgs<T> &A, int ncurves, TileDesc *desc, hipS
     const size_t lds = sizeof(int) * kDescWaves * (((size_t)1 << A.tlog) + 2 * (size_t)A.ntaps + 1);
     require(lds <= kMaxLds, "spread tile too large", CUNA_ERROR_UNSUPPORTED);
     set_lds(k_tile_desc<T>, lds);
-    const long npos = (long)ncurves * A.ntiles;
-    hipLaunchKernelGGL(k_tile_desc<T>, dim3(ceil_div(npos, kDescWaves)), dim3(64 * kDescWaves), lds,
-                       s, A, npos, desc);
-    CUNA_LAUNCH_CHECK();
+    // a launch holds fewer than 2^32 threads
+    const long npos = (long)ncurves * A.ntiles, most = 1L << 25;
+    for (long p0 = 0; p0 < npos; p0 += most) {
+        const long p1 = std::min(npos, p0 + most);
+        hipLaunchKernelGGL(k_tile_desc<T>, dim3(ceil_div(p1 - p0, kDescWaves)),
+                           dim3(64 * kDescWaves), lds, s, A, p0, p1, desc);
+        CUNA_LAUNCH_CHECK();
+    }
 }
 
 // sort and buckets of short curves in one launch; false when a curve is too

@@ -992,12 +992,12 @@ static __global__ __launch_bounds__(kOrderThreads) void k_tile_order(const int *
 constexpr int kDescWaves = 4;
 
 template <typename T>
-__global__ __launch_bounds__(64 * kDescWaves) void k_tile_desc(SpreadArgs<T> A, long npos,
-                                                               TileDesc *desc) {
+__global__ __launch_bounds__(64 * kDescWaves) void k_tile_desc(SpreadArgs<T> A, long pos0,
+                                                               long npos, TileDesc *desc) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int TT = 1 << A.tlog, nt = A.ntaps, Q0 = (nt - 1) / 2, NH = TT + 2 * nt;
     int *h = reinterpret_cast<int *>(cuna_smem) + wave * (NH + 1);  // cells -nt .. TT+nt-1
-    const long pos = (long)blockIdx.x * kDescWaves + wave;
+    const long pos = pos0 + (long)blockIdx.x * kDescWaves + wave;  // pos0 <= pos < npos
     if (pos >= npos) return;  // no workgroup barriers below
     const int c = (int)(pos / A.ntiles);
     const int tile = desc[pos].tile;
