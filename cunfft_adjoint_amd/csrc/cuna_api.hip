@@ -621,6 +621,10 @@ void Plan<T>::bootstrap_ls(const T *y, int nbs, uint32_t seed, T *power, T *peak
             "Lomb-Scargle bootstrap needs a grid of at most 2^15 cells (float) / 2^14 (double) and "
             "m in {6, 8, 10, 12, 13, 16}",
             CUNA_ERROR_UNSUPPORTED);
+    // there is only the fused kernel, and such a plan has no workspaces for it
+    require(bootstrap_fused_ok(true),
+            "Lomb-Scargle bootstrap needs a plan made without CUNA_PLAN_UNFUSED",
+            CUNA_ERROR_UNSUPPORTED);
     prepare_bootstrap(nbs, true, s);
     // window spectra workspace: one row of M/2 values per resident workgroup
     ls_work.ensure(sizeof(cplx<T>) * (size_t)fused_slots<T>(lgN) * (M / 2), s);

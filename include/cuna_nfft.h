@@ -105,8 +105,8 @@ int cuna_nfft_adjoint_many(cuna_nfft_plan plan, const dTyp *y, int nrhs, Complex
 int cuna_nfft_bootstrap(cuna_nfft_plan plan, const dTyp *y, int nbs, unsigned int seed,
                         Complex *out_y, Complex *out_w, hipStream_t stream);
 
-/* accurate mode, CUNA_PLAN_WINDOW2 plan: Lomb-Scargle periodograms of the
- * same replicates (Press & Rybicki 1989; data centred on the replicate mean,
+/* accurate mode, CUNA_PLAN_WINDOW2 plan without CUNA_PLAN_UNFUSED:
+ * Lomb-Scargle periodograms of the same replicates (Press & Rybicki 1989; data centred on the replicate mean,
  * "standard" normalisation, 0 <= P <= 1), computed in the fused bootstrap
  * kernel without writing the spectra.  Frequency k*df (times plans; k/1 for
  * x plans), k = 0 .. M/2-1:
