@@ -119,8 +119,10 @@ size_t size_class(size_t n) {
 
 void *BlockPool::take(size_t nbytes, size_t *got, int *dev, hipStream_t s) {
     CUNA_HIP(hipGetDevice(dev));
-    const size_t n = nbytes >= kMinBlock ? size_class(nbytes) : nbytes;
-    if (nbytes >= kMinBlock) {
+    // blocks that are never kept are allocated as they are
+    const bool keep = nbytes >= kMinBlock && size_class(nbytes) <= kMaxBlock;
+    const size_t n = keep ? size_class(nbytes) : nbytes;
+    if (keep) {
         Kept &K = kept();
         std::lock_guard<std::mutex> lk(K.mu);
         for (auto it = K.blocks.begin(); it != K.blocks.end(); ++it) {
