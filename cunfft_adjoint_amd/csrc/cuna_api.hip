@@ -150,9 +150,18 @@ void *BlockPool::take(size_t nbytes, size_t *got, int *dev, hipStream_t s) {
     return p;
 }
 
+namespace {
+// A release has no caller to report an error to (a thread that destroys a plan while
+// it captures a stream gets one here), and the runtime would hand it to the next
+// launch check.
+void free_block(void *p) {
+    if (hipFree(p) != hipSuccess) (void)hipGetLastError();
+}
+}  // namespace
+
 void BlockPool::give(void *p, size_t bytes, int dev) {
     if (bytes < kMinBlock || bytes > kMaxBlock) {
-        (void)hipFree(p);
+        free_block(p);
         return;
     }
     int cur = dev;
@@ -161,7 +170,8 @@ void BlockPool::give(void *p, size_t bytes, int dev) {
     const hipError_t e = hipDeviceSynchronize();
     if (cur != dev) (void)hipSetDevice(cur);
     if (e != hipSuccess) {
-        (void)hipFree(p);
+        (void)hipGetLastError();
+        free_block(p);
         return;
     }
     Kept &K = kept();
@@ -169,7 +179,7 @@ void BlockPool::give(void *p, size_t bytes, int dev) {
     K.blocks.push_back(Block{p, bytes, dev});
     K.bytes += bytes;
     while (K.bytes > kMaxKept) {
-        (void)hipFree(K.blocks.front().p);
+        free_block(K.blocks.front().p);
         K.bytes -= K.blocks.front().bytes;
         K.blocks.pop_front();
     }
@@ -178,7 +188,7 @@ void BlockPool::give(void *p, size_t bytes, int dev) {
 void BlockPool::clear() {
     Kept &K = kept();
     std::lock_guard<std::mutex> lk(K.mu);
-    for (const Block &b : K.blocks) (void)hipFree(b.p);
+    for (const Block &b : K.blocks) free_block(b.p);
     K.blocks.clear();
     K.bytes = 0;
 }
@@ -775,7 +785,6 @@ bool Plan<T>::room_for_both_parts(hipStream_t s) {
         return true;
     } catch (const Error &e) {
         if (e.code != CUNA_ERROR_OUT_OF_MEMORY) throw;
-        (void)hipGetLastError();
         if (!grid.in_graph) grid.drop();
         if (!work.in_graph) work.drop();
         return false;

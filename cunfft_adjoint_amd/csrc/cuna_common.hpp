@@ -32,6 +32,7 @@ struct Error {
 
 inline void hip_check(hipError_t e, const char *what, const char *file, int line) {
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not again by the next launch check
         char buf[512];
         snprintf(buf, sizeof buf, "%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
         fail(e == hipErrorOutOfMemory ? CUNA_ERROR_OUT_OF_MEMORY : CUNA_ERROR_HIP, buf);
