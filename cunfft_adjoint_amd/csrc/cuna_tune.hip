@@ -3,8 +3,8 @@
 // For a point set and an accuracy target it picks the oversampling sigma and
 // filter half-width m (the smallest m per sigma whose Gaussian-gridding error
 // bound meets the target), then measures on the device the spread tile size
-// and the FFT workgroup shapes, and keeps the fastest combination.  Results
-// are cached in a text file keyed by device, precision, n (rounded to a power
+// and the FFT workgroup shapes, and for small grids the one-launch adjoint, and
+// keeps the fastest combination.  Results are cached in a text file keyed by device, precision, n (rounded to a power
 // of two), M and the target.
 #include <hip/hip_runtime.h>
 
@@ -120,6 +120,23 @@ struct Timer {
         std::sort(t.begin(), t.end());
         return t[t.size() / 2];
     }
+    // median time of one of kCalls calls in a row (launches count as they do for a
+    // caller, which the events around one call's kernels do not see)
+    float calls(Plan<R> &P, const R *y, cplx<R> *out, hipStream_t s) {
+        constexpr int kCalls = 32;
+        std::vector<float> t;
+        for (int r = 0; r < 6; ++r) {
+            CUNA_HIP(hipEventRecord(ev[0], s));
+            for (int i = 0; i < kCalls; ++i) P.adjoint(y, out, s);
+            CUNA_HIP(hipEventRecord(ev[3], s));
+            CUNA_HIP(hipStreamSynchronize(s));
+            float ms = 0;
+            CUNA_HIP(hipEventElapsedTime(&ms, ev[0], ev[3]));
+            if (r > 0) t.push_back(ms / kCalls);  // the first run allocates
+        }
+        std::sort(t.begin(), t.end());
+        return t[t.size() / 2];
+    }
 };
 
 }  // namespace
@@ -197,7 +214,21 @@ CUNA_API int cuna_nfft_autotune(const dTyp *x, int n, int M, double tol, const c
                         }
                     }
             }
-            const double total = (double)best_spread + best_fft;
+            double total = (double)best_spread + best_fft;
+            // a small grid's adjoint may do better in one launch, which a plan with
+            // the library's own tile and FFT shapes takes by its rule
+            spec.tile_log2 = 0;
+            auto D = make_plan_accurate<R>(x, nullptr, 0.0, {0, n}, M, spec, stream);
+            if (D->fused_adjoint) {
+                keep->spec.fft_w = bw;
+                keep->spec.fft_h = bh;
+                const float two = tm.calls(*keep, y.as<R>(), out.as<cplx<R>>(), stream);
+                const float one = tm.calls(*D, y.as<R>(), out.as<cplx<R>>(), stream);
+                if (one < two) {
+                    total *= one / two;
+                    best_t = bw = bh = 0;
+                }
+            }
             if (total < best_ms) {
                 best_ms = total;
                 best.sigma = sigma;

@@ -149,10 +149,11 @@ int cuna_nfft_plan_destroy(cuna_nfft_plan plan);
  * sigma in {2, 4} it takes the smallest m whose Gaussian-gridding error bound
  * exp(-pi m (1 - 1/(2 sigma - 1))) plus the arithmetic's rounding floor meets
  * tol (relative L2 error vs the direct NDFT), then times the spread tile
- * (2^8..2^11 cells) and FFT workgroup shapes on the device and keeps the
- * fastest.  Results are cached (appended) in a text file keyed by GPU,
- * precision, n rounded to a power of two, M and tol: cache_path NULL uses
- * $CUNA_TUNE_CACHE or ~/.cache/cuna_tune.txt, "" disables the cache. */
+ * (2^8..2^11 cells) and FFT workgroup shapes, and on small grids the library's
+ * one-launch adjoint (tile_log2 = 0), on the device and keeps the fastest.
+ * Results are cached (appended) in a text file keyed by GPU, precision, n
+ * rounded to a power of two, M and tol: cache_path NULL uses $CUNA_TUNE_CACHE
+ * or ~/.cache/cuna_tune.txt, "" disables the cache. */
 int cuna_nfft_autotune(const dTyp *x, int n, int M, double tol, const char *cache_path,
                        cuna_nfft_params *params, hipStream_t stream);
 
