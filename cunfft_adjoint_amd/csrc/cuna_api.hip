@@ -419,10 +419,12 @@ void Plan<T>::prepare_fft(hipStream_t s) {
 }
 
 template <typename T>
-void Plan<T>::run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s, hipEvent_t mid) const {
+void Plan<T>::run_fft(T *grid_ptr, cplx<T> *out, int batch, int rows, hipStream_t s,
+                      hipEvent_t mid) const {
     FftShape sh;
     sh.lgN = lgN;
     sh.batch = batch;
+    sh.rows = rows;
     sh.w = spec.fft_w;
     sh.h = spec.fft_h;
     if (spec.mode == CUNA_MODE_ACCURATE) {
@@ -438,7 +440,7 @@ void Plan<T>::run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s, hipEv
         sk.row_off = row_off_c;
         sk.qb_row = qb_row_c;
         if (blu)
-            blu->run_real(grid_ptr, G, batch, sk, s);
+            blu->run_real(grid_ptr, G, batch, rows, sk, s);
         else
             fft_real_forward<T>(sh, grid_ptr, sk, s, mid);
     }
@@ -503,7 +505,8 @@ void Plan<T>::adjoint_into(const T *y, cplx<T> *out, T *grid_ptr, hipStream_t s)
     A.grid_stride = G;
     // prof[0] and prof[1] take the spread kernel's own start and stop times
     launch_spread<T>(A, ntaps, VAL_PLAIN, nc, s, prof[0], prof[1]);
-    run_fft(grid_ptr, out, nc, s, prof[2]);
+    // a curve of a compat batch has the bits of its own call
+    run_fft(grid_ptr, out, nc, spec.mode == CUNA_MODE_COMPAT ? 1 : nc, s, prof[2]);
     if (prof[3]) CUNA_HIP(hipEventRecord(prof[3], s));
 }
 
@@ -531,7 +534,7 @@ void Plan<T>::adjoint_many(const T *y, int nrhs, cplx<T> *out, hipStream_t s) {
     A.grid = grid.as<T>();
     A.grid_stride = G;
     launch_spread<T>(A, ntaps, VAL_PLAIN, nc * nrhs, s, prof[0], prof[1]);
-    run_fft(grid.as<T>(), out, nc * nrhs, s, prof[2]);
+    run_fft(grid.as<T>(), out, nc * nrhs, nc, s, prof[2]);
     if (prof[3]) CUNA_HIP(hipEventRecord(prof[3], s));
 }
 
@@ -550,7 +553,7 @@ void Plan<T>::bootstrap_compat(const T *y, cplx<T> *out, int nbs, uint32_t seed,
     A.seed = seed;
     A.eps_orig = pts.eps_orig.template as<T>();
     launch_spread<T>(A, ntaps, VAL_COMPAT_BOOT, nbs, s);
-    run_fft(grid.as<T>(), out, nbs, s);
+    run_fft(grid.as<T>(), out, nbs, nbs, s);
 }
 
 template <typename T>
@@ -695,7 +698,7 @@ void Plan<T>::bootstrap(const T *y, int nbs, uint32_t seed, cplx<T> *out_y, cplx
         A.counts = counts.as<int>();
         A.counts_stride = n_;
         launch_spread<T>(A, ntaps, VAL_COUNTS, nc * nbs, s);
-        run_fft(grid.as<T>(), out, nc * nbs, s);
+        run_fft(grid.as<T>(), out, nc * nbs, nc * nbs, s);
     }
 }
 

@@ -294,18 +294,25 @@ void Bluestein<T>::init(int length, bool real, hipStream_t s) {
 }
 
 // The largest length that one workgroup holds.  Its two FFTs take one CU 20 us, so
-// few rows go through the three passes, which spread them over the chip.  Measured,
-// with the spread, one workgroup per row / three passes: FP32, L = 2^14, 2 rows
-// 34.5 / 22.6 us, 64 rows 38.1 / 32.8, 100 rows 41.8 / 42.5; FP64, L = 2^13, 2 rows
-// 26.7 / 19.2 us, 32 rows 26.8 / 22.5, 64 rows 27.6 / 28.6.  (FP32 at 2^13: 20.5 /
-// 21.9 us at 2 rows, 21.0 / 23.3 at 48.)
+// few rows go through the three passes, which spread them over the chip.  `rows`
+// decides, not the batch, and the passes have one shape (kBothW, both_h), because a
+// curve's bits do not depend on the batch that it is in.  Measured with the spread,
+// one workgroup per row / three passes: FP32, ng = 5001, 1 row 32.6 / 16.8 us, 64
+// rows 33.9 / 27.9, 100 rows 35.7 / 36.9, 256 rows 46 / 69; FP64, ng = 2501, 1 row
+// 25.5 / 18.9, 16 rows 25.5 / 19.3, 64 rows 26.6 / 26.6, 256 rows 31 / 55.  (FP32 at
+// 2^13: 20.5 / 21.9 us at 2 rows.)  Eight sequences per workgroup 18.5 and 56 us.
 template <typename T>
 bool Bluestein<T>::both_forms() const {
     return lgL == max_small_lg<T>();
 }
 template <typename T>
-static constexpr int chirp_pass_rows() {
-    return sizeof(T) == 4 ? 64 : 32;
+static constexpr int cus_per_pass_row() {  // rows up to num_cus() over this are few
+    return sizeof(T) == 4 ? 4 : 8;
+}
+constexpr int kBothW = 2;
+template <typename T>
+constexpr int both_h() {
+    return sizeof(T) == 4 ? 2 : 4;
 }
 
 template <typename T>
@@ -314,14 +321,15 @@ void Bluestein<T>::ensure(int batch, hipStream_t s) {
 }
 
 template <typename T>
-void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch,
+void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch, int rows,
                        hipStream_t s) {
     require(sizeof(cplx<T>) * (size_t)L * (size_t)batch <= work.bytes,
             "Bluestein workspace too small for this batch");
     work.use(s);
     auto &tc = TwiddleCache<T>::get();
     const cplx<T> *const wng = pairs ? chirp() + n : nullptr;
-    if (lgL <= max_small_lg<T>() && !(both_forms() && batch <= chirp_pass_rows<T>())) {
+    const bool both = both_forms();
+    if (lgL <= max_small_lg<T>() && !(both && rows <= num_cus() / cus_per_pass_row<T>())) {
         dispatch_lg<1, max_small_lg<T>()>(lgL, [&](auto c) {
             constexpr int LG = decltype(c)::value, MR = small_mr(LG), CAP = small_cap(LG);
             constexpr int NT = fft_threads(LG, 1, MR);
@@ -336,10 +344,10 @@ void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int bat
         return;
     }
     const int lg1 = split_lg1(lgL), lg2 = lgL - lg1, L1 = 1 << lg1, L2 = 1 << lg2;
-    const int W = pick_seq<T>(lg2, L1, batch, 1, "CUNA_FFT_W", 0, num_cus());
-    const int H = pick_seq<T>(lg1, L2, batch, 1, "CUNA_FFT_H", 0, num_cus());
+    const int W = pick_seq<T>(lg2, L1, batch, 1, "CUNA_FFT_W", both ? kBothW : 0, num_cus());
+    const int H = pick_seq<T>(lg1, L2, batch, 1, "CUNA_FFT_H", both ? both_h<T>() : 0, num_cus());
     cplx<T> *const a = work.as<cplx<T>>();
-    const cplx<T> *const b = (both_forms() ? bt_rows : bt).template as<cplx<T>>();
+    const cplx<T> *const b = (both ? bt_rows : bt).template as<cplx<T>>();
     auto batches = [&](auto &&launch) {
         for (long b0 = 0; b0 < batch; b0 += kMaxGridY) {
             launch(b0, (int)std::min<long>(kMaxGridY, batch - b0));
@@ -403,8 +411,8 @@ void Bluestein<T>::run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int bat
 }
 
 template <typename T>
-void Bluestein<T>::run_real(const T *grid, long gstride, int batch, const SinkCompat<T> &sk,
-                            hipStream_t s) {
+void Bluestein<T>::run_real(const T *grid, long gstride, int batch, int rows,
+                            const SinkCompat<T> &sk, hipStream_t s) {
     LoadChirp<T> ld{};
     ld.chirp = chirp();
     ld.n = n;
@@ -420,7 +428,7 @@ void Bluestein<T>::run_real(const T *grid, long gstride, int batch, const SinkCo
     sink.n = n;
     sink.mode = CHIRP_COMPAT;
     sink.sk = sk;
-    run(ld, sink, batch, s);
+    run(ld, sink, batch, rows, s);
 }
 
 template <typename T>
@@ -439,7 +447,7 @@ void Bluestein<T>::run_complex(cplx<T> *data, int batch, int sign, hipStream_t s
     sink.conj_out = ld.conj_in;
     sink.data = data;
     sink.stride = ng;
-    run(ld, sink, batch, s);
+    run(ld, sink, batch, batch, s);
 }
 
 template struct Bluestein<dTyp>;

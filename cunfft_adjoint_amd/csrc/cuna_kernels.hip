@@ -81,15 +81,22 @@ static void run_row_plain(const FftShape &sh, const cplx<T> *src, int L2, cplx<T
     }
 }
 
-// Rows up to which the largest transform that one workgroup holds goes through two
-// passes all the same: one workgroup per row leaves the chip idle and takes the
-// whole transform's LDS passes in a row.  Measured, spread and transform, one
-// workgroup per row / two passes: FP32, 2^14, 1 row 21.6 / 15.9 us, 64 rows 29.5 /
-// 25.0, 100 rows 35.0 / 32.6, 160 rows 41.1 / 42.4; FP64, 2^13, 1 row 20.1 / 16.0
-// us, 32 rows 28.9 / 27.4, 48 rows 32.9 / 33.0.
+// Whether the largest transform that one workgroup holds goes through two passes
+// all the same: for few rows, which leave the chip idle at one workgroup per row and
+// take the whole transform's LDS passes in a row.  sh.rows decides, not the batch,
+// and the passes have one shape (kFewW, kFewH), because calls that are promised to
+// agree bit for bit differ in their batches.  Measured with the spread, values of one
+// plan, one workgroup per row / two passes: FP32, 2^14, 20,000 points: 1 row 22.4 /
+// 12.3 us, 64 rows 31.4 / 27.5, 100 rows 38.0 / 37.4, 128 rows 42.7 / 43.9, 256 rows
+// 62 / 75; FP64, 2^13, 8000 points: 1 row 19.8 / 14.8, 32 rows 23.2 / 19.6, 64 rows
+// 28.4 / 27.1, 100 rows 34.4 / 36.8.  Other shapes: 12.2 us at one row and 95 at 256
+// with one sequence per workgroup, 14.3 and 70 with eight and four.
+constexpr int kFewW = 8, kFewH = 1;
 template <typename T>
 static bool few_rows(const FftShape &sh) {
-    return sh.lgN == max_small_lg<T>() && sh.batch <= (sizeof(T) == 4 ? 100 : 32);
+    const int rows = sh.rows > 0 ? sh.rows : sh.batch;
+    return sh.lgN == max_small_lg<T>() &&
+           rows <= (sizeof(T) == 4 ? num_cus() * 3 / 8 : num_cus() * 3 / 16);
 }
 
 template <typename T, class Sink>
@@ -100,7 +107,8 @@ static void real_forward_impl(const FftShape &sh, T *grid, const Sink &sk, hipSt
     LoadGrid<T> ld;
     ld.z = reinterpret_cast<const cplx<T> *>(grid);
     ld.stride = 1L << sh.lgN;
-    if (sh.lgN <= max_small_lg<T>() && !few_rows<T>(sh)) {
+    const bool few = few_rows<T>(sh);
+    if (sh.lgN <= max_small_lg<T>() && !few) {
         dispatch_lg<1, max_small_lg<T>()>(sh.lgN, [&](auto c) {
             run_small<T, 1, decltype(c)::value, LoadGrid<T>, Sink, 0>(sh, ld, sk, nullptr, s);
         });
@@ -108,8 +116,10 @@ static void real_forward_impl(const FftShape &sh, T *grid, const Sink &sk, hipSt
     }
     const int lg1 = split_lg1(sh.lgN), lg2 = sh.lgN - lg1;
     cplx<T> *z = reinterpret_cast<cplx<T> *>(grid);
-    const int W = pick_seq<T>(lg2, 1L << lg1, sh.batch, 1, "CUNA_FFT_W", sh.w, num_cus());
-    const int H = std::min(4, pick_seq<T>(lg1, 1L << lg2, sh.batch, 2, "CUNA_FFT_H", sh.h));
+    const int W = pick_seq<T>(lg2, 1L << lg1, sh.batch, 1, "CUNA_FFT_W",
+                              few && !sh.w ? kFewW : sh.w, num_cus());
+    const int H = std::min(4, pick_seq<T>(lg1, 1L << lg2, sh.batch, 2, "CUNA_FFT_H",
+                                          few && !sh.h ? kFewH : sh.h));
     dispatch_lg<7, 12>(lg2, [&](auto c) {
         constexpr int LG2 = decltype(c)::value;
         dispatch_w<T, LG2>(W, [&](auto w) {
@@ -145,8 +155,10 @@ void fft_c2r_inverse(const FftShape &sh, const LoadHermitian<T> &ld, cplx<T> *wo
     SinkAccurate<T> dummy{};
     // the Hermitian loader is register-heavy: a 1024-thread workgroup (N =
     // 2^14) would spill, so N >= 2^14 takes the two-pass path in both
-    // libraries; FP64 at 2^13 does so for few rows, as the forward transform
-    if (sh.lgN <= kC2rSmallLg && !few_rows<T>(sh)) {
+    // libraries; FP64 at 2^13 does so for few rows, as the forward transform (18.4 ->
+    // 15.4 us with the gather, one curve)
+    const bool few = sh.lgN == max_small_lg<T>() && sh.batch <= num_cus() / 8;
+    if (sh.lgN <= kC2rSmallLg && !few) {
         dispatch_lg<1, kC2rSmallLg>(sh.lgN, [&](auto c) {
             run_small<T, -1, decltype(c)::value, LoadHermitian<T>, SinkAccurate<T>, 1>(
                 sh, ld, dummy, z, s);

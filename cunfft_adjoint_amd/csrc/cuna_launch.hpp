@@ -14,6 +14,9 @@ struct FftShape {
     int batch = 1;
     int w = 0;  // columns per workgroup in pass 1 (0: heuristic)
     int h = 0;  // rows (real: row pairs) per workgroup in pass 2 (0: heuristic)
+    // rows by which a form with other roundings is chosen (0: batch): the same for
+    // calls that have to agree bit for bit
+    int rows = 0;
 };
 
 template <typename T>

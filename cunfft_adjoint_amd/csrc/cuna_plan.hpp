@@ -181,8 +181,8 @@ struct Bluestein {
     void init(int length, bool real, hipStream_t s);
     void ensure(int batch, hipStream_t s);
     // real grids (batch rows of stride gstride, the first ng cells used) ->
-    // the compat deconvolution sink, one row per grid
-    void run_real(const T *grid, long gstride, int batch, const SinkCompat<T> &sk,
+    // the compat deconvolution sink, one row per grid (rows: see FftShape)
+    void run_real(const T *grid, long gstride, int batch, int rows, const SinkCompat<T> &sk,
                   hipStream_t s);
     // in place on batch x ng complex values: data[r] = sum_g data[g] e^{sign 2 pi i g r/ng}
     void run_complex(cplx<T> *data, int batch, int sign, hipStream_t s);
@@ -190,7 +190,8 @@ struct Bluestein {
   private:
     const cplx<T> *chirp() const { return tab.template as<cplx<T>>(); }
     bool both_forms() const;
-    void run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch, hipStream_t s);
+    void run(const LoadChirp<T> &ld, const ChirpSink<T> &sink, int batch, int rows,
+             hipStream_t s);
 };
 
 // true when a real grid of G cells takes the power-of-two FFT (else Bluestein)
@@ -265,7 +266,8 @@ struct Plan {
     void spectrum_to_grid(const cplx<T> *g, int parts, int rot, hipStream_t s);
     bool room_for_both_parts(hipStream_t s);
     BootArgs<T> fused_args(const T *y, int nbs, uint32_t seed, hipStream_t s);
-    void run_fft(T *grid_ptr, cplx<T> *out, int batch, hipStream_t s,
+    // rows: see FftShape
+    void run_fft(T *grid_ptr, cplx<T> *out, int batch, int rows, hipStream_t s,
                  hipEvent_t mid = nullptr) const;
     // twiddle tables (and the Bluestein set-up for other lengths) for this
     // plan's transform; run once at plan creation

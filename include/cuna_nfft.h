@@ -91,7 +91,9 @@ int cuna_nfft_adjoint(cuna_nfft_plan plan, const dTyp *y, Complex *out, hipStrea
 /* accurate mode: nrhs value vectors of one plan in one spread launch and one
  * batched FFT.  y: nrhs x n (row r holds the values of right-hand side r, in
  * the plan's point order); out: ncurves x nrhs x M complex, row c*nrhs + r
- * equal to cuna_nfft_adjoint of row r for curve c.
+ * equal to cuna_nfft_adjoint of row r for curve c: bit for bit on grids of up to
+ * 2^15 cells (libcunaf) / 2^14 (libcunad), within rounding on larger ones, whose
+ * FFT takes its shape from the number of transforms.
  * No counterpart in the reference (its batching is over bootstrap replicates,
  * src/cuna_kernel.cu:236-289). */
 int cuna_nfft_adjoint_many(cuna_nfft_plan plan, const dTyp *y, int nrhs, Complex *out,
@@ -174,9 +176,11 @@ int cuna_graph_destroy(cuna_graph graph);
  * src/gaussian_filter.cu:67-99 generate_pinned_filter_properties_batch).
  * Curve i has n[i] points of the concatenated x (and f_data; NULL = unit
  * weights) and ng[i] grid cells (any ng[i] >= 1, n[i] < 2 ng[i]); its
- * ng[i] outputs (exactly those of cunfft_adjoint_raw_async on that curve)
- * go to the start of slab i of f_hat, slab stride idist = max ng, f_hat
- * holding nlc * idist values; the rest of each slab is left as it was.
+ * ng[i] outputs (those of cunfft_adjoint_raw_async on that curve: bit for bit
+ * for powers of two up to 2^15 (libcunaf) / 2^14 (libcunad) and other ng up to
+ * 2^13 / 2^12, within rounding for larger ng) go to the start of slab i of
+ * f_hat, slab stride idist = max ng, f_hat holding nlc * idist values; the rest
+ * of each slab is left as it was.
  * n, ng and gpu_fprops are HOST arrays; gpu_fprops[i] is curve i's device
  * filter_properties from generate_*filter_properties*.  When all of them
  * are such registered structs, the multi-curve plan (curves of equal ng

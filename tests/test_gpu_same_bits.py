@@ -42,3 +42,23 @@ def compat_batch_equals_single_calls(prec, ng, curves, n):
 @pytest.mark.parametrize("prec", ["f", "d"])
 def test_compat_batch_of_sparse_curves(prec):
     compat_batch_equals_single_calls(prec, 1 << 13, 520, 100)
+
+
+@pytest.mark.parametrize("prec,ng", [("f", 1 << 15), ("f", 3001), ("f", 4097), ("f", 5001), ("f", 8191),
+                                     ("d", 1 << 14), ("d", 2049), ("d", 2501), ("d", 4095)])
+@pytest.mark.parametrize("curves", [2, 70, 130])
+def test_compat_batch(prec, ng, curves):
+    compat_batch_equals_single_calls(prec, ng, curves, 900)
+
+
+@pytest.mark.parametrize("prec,M", [("f", 1 << 13), ("f", 1 << 14), ("d", 1 << 12), ("d", 1 << 13)])
+@pytest.mark.parametrize("curves,nrhs", [(1, 2), (1, 60), (1, 130), (40, 3), (60, 2), (110, 2)])
+def test_adjoint_many(prec, M, curves, nrhs):
+    rng = np.random.default_rng(M + nrhs)
+    n = 1500 * curves
+    x = torch.from_numpy(rng.uniform(-0.5, 0.5, n)).to(RT[prec]).cuda()
+    y = torch.from_numpy(rng.standard_normal((nrhs, n))).to(RT[prec]).cuda()
+    plan = cu.NFFTPlan(x, M, offsets=np.arange(curves + 1, dtype=np.int32) * 1500, tile_log2=8)
+    many = plan.adjoint_many(y).reshape(curves, nrhs, M)
+    for r in (0, nrhs - 1):
+        assert torch.equal(many[:, r], plan.adjoint(y[r]))
