@@ -1169,16 +1169,20 @@ __device__ __forceinline__ void tap_fixed(T v, T e, T bi, const T *e3, T c1, Emi
 // Each wave of the tile's workgroup accumulates its own share of the points
 // into its own LDS cells, in fixed point with integer atomics (32-bit cells
 // in FP32, 64-bit in FP64), with its own power-of-two scale:
-//   min(cnt, cover) * vmax * wscale * 2^s <= 2^headroom,
-// cnt = the wave's points this round (<= 64 * kSpreadSlots), vmax their
-// largest |value| (compat filters: largest kept weight / wscale), cover = the
-// tile's most points in one window of ntaps anchors.  No cell can overflow,
+//   min(cover * vmax, vsum) * wscale * 2^s <= 2^headroom,
+// vmax and vsum = the largest and the sum of the |values| of the wave's points this
+// round (at most 64 * kSpreadSlots; compat filters: of the largest kept weights /
+// wscale; FP64 takes their number times vmax for vsum), cover = the tile's most
+// points in one window of ntaps anchors.  No cell can overflow,
 // whatever the density, so no wider fallback and no plan-time read-back is
 // needed; a wave's scale needs no workgroup barrier; and the waves never
 // contend for one address.  After the last round the waves' cells are
 // converted and summed in a fixed wave order, so the grid is bitwise
-// reproducible.  Resolution: 2^-headroom * min(cnt, cover) of the round's
-// largest weight (FP32: 2^-24 for cover <= 64, 2^-22 at worst).  A wave with
+// reproducible.  Resolution: 2^-headroom * min(cover, vsum / vmax) of the round's
+// largest weight (FP32: 2^-24 for cover <= 64, 2^-22 at worst, and 2^-29 next to one
+// value that dominates, whose rounding the other points of its tile share: with
+// cover alone, spectra in tiles of 1024 cells were up to 1.26 times as far off as in
+// tiles of 256, log-normal values, now 1.02 times).  A wave with
 // several rounds folds each into its own float (double) cells.
 constexpr int kSpreadSlots = 4;  // point slots per lane in a round
 
@@ -1272,7 +1276,7 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
             am[k] = pr.a - rk[k];
             ev[k] = pr.e;
         }
-        T vmax = T(0);
+        T vmax = T(0), vsum = T(0);
 #pragma unroll
         for (int k = 0; k < PPT; ++k) {
             T v, e = ev[k];
@@ -1293,11 +1297,17 @@ __global__ __launch_bounds__(64 * WPT) void k_spread_wv(SpreadArgs<T> A) {
             // tile's output NaN
             if (!(av <= kBig) || (ok && !(fabs(e) <= kBig))) av = T(INFINITY);
             vmax = fmax(vmax, av);
+            vsum += av;
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) vmax = fmax(vmax, __shfl_xor(vmax, o));
+        for (int o = 32; o > 0; o >>= 1) {
+            vmax = fmax(vmax, __shfl_xor(vmax, o));
+            if constexpr (sizeof(T) == 4) vsum += __shfl_xor(vsum, o);
+        }
         if (!(vmax <= kBig)) finite = false;
-        const T bound = (T)min(wcnt, cover) * vmax * wscale;
+        // (FP64: the bound on single weights decides)
+        const T bound =
+            (sizeof(T) == 4 ? fmin((T)cover * vmax, vsum) : (T)min(wcnt, cover) * vmax) * wscale;
         int eb = -64;
         if (bound > T(0) && finite) (void)frexp(bound, &eb);
         sexp = min(FX::headroom - eb, kMaxExp - ew);
