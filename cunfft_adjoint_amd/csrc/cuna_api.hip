@@ -463,7 +463,7 @@ template <typename T>
 void Plan<T>::adjoint_fused(const T *y, int nrhs, cplx<T> *out, hipStream_t s) {
     AdjointArgs<T> A{};
     A.total = ncurves() * nrhs;
-    if (sizeof(T) == 4)  // dense curves' first round
+    if (sizeof(T) == 4)  // the first of two rounds
         grid.ensure(sizeof(int) * (size_t)G * std::min(A.total, fused_slots<T>(lgN)), s);
     A.cover = covers(s);
     A.rec = pts.rec_orig.template as<PointRec<T>>();

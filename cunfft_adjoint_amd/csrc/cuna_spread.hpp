@@ -2063,11 +2063,22 @@ __global__ __launch_bounds__(1024) void k_curve_cover(const PointRec<T> *rec, co
 //
 // Scale: with `cover` the curve's densest window of NTAPS anchors and vm its
 // largest |value|, no cell sum exceeds cover * vm * wscale, kept within 2^30
-// (FP32) / 2^61 (FP64).  In FP32 a curve denser than kDenseCover takes a second
-// round over its points that accumulates what rounding each weight dropped, scaled
-// by up to 2^kDenseBits, so that a dense cell costs no precision; the first round's
-// integers wait in the workspace row of the workgroup.
-constexpr int kDenseCover = 64, kDenseBits = 14;
+// (FP32) / 2^61 (FP64).  All of the curve shares it, and with one unit of the scale
+// at u the grid's rounding is 0.94 u / mean |value| of the spectrum's norm (m = 8).
+// In FP32 a curve whose mean |value| has fewer than kMeanUnits of them, so that this
+// would pass 0.75e-7 (the FFT's own is 2e-7), is looked at closer: the sums of the
+// |values| per 16 anchors bound a cell's sum by that of the blocks which its window
+// touches, a few times less than cover * vm.  If that is not enough, where one value
+// dominates or the points are dense, a second round over the points accumulates what
+// rounding each weight dropped, scaled by up to 2^kRestBits, and the first round's
+// integers wait in the workspace row of the workgroup.  Errors with cover * vm alone /
+// this / tiles, whose scales are each tile's: 4700 points, M = 2^14, one value 30 times
+// the others 5.0e-7 / 2.2e-7 / 2.1e-7, log-normal values 6.9e-7 / 2.2e-7 / 2.3e-7;
+// 20,000 points, one value 1000 times the others 41e-7 / 1.9e-7 / 1.9e-7.  It costs 256
+// ordinary curves of 100 - 20,000 points 3.6 us of 54 for the sums; where the longest
+// takes the second round they take 82.
+constexpr float kMeanUnits = 0.75f * 16777216.0f;
+constexpr int kRestBits = 14;
 
 // What tap_fixed (FP32, table) rounded off each weight: it repeats its operations,
 // so n_q is the same integer, and the rest up e3 - n_q is exact up to one rounding.
@@ -2118,7 +2129,7 @@ struct AdjointArgs {
     long y_stride;           // per value vector
     const int *coff, *order, *cover;
     int nrhs, total;         // total = curves * nrhs
-    int *hi;                 // dense curves: G integers per workgroup
+    int *hi;                 // FP32, two rounds: G integers per workgroup
     T bi, wscale;
     T e3[kMaxTaps];
     SinkAccurate<T> sink;
@@ -2142,7 +2153,8 @@ __global__ __launch_bounds__(NT) void k_adjoint_fused(AdjointArgs<T> A) {
     U *gu = reinterpret_cast<U *>(grid);
     cplx<T> *z = reinterpret_cast<cplx<T> *>(grid);
     cplx<T> *tl = reinterpret_cast<cplx<T> *>(grid + G + kBootHalo);
-    __shared__ T vmax_sh[NT / 64];
+    __shared__ T vmax_sh[NT / 64], vsum_sh[NT / 64];
+    __shared__ unsigned block_sh[NT / 64];
     const int tid = threadIdx.x;
     for (int i = tid; i < NLT; i += NT) tl[i] = A.twT[i];
     TwRows<T, CAP, Rest> tw;
@@ -2165,38 +2177,97 @@ __global__ __launch_bounds__(NT) void k_adjoint_fused(AdjointArgs<T> A) {
         const int c0 = A.coff[ci], nc = A.coff[ci + 1] - c0, cover = max(A.cover[ci], 1);
         const PointRec<T> *P = A.rec + c0;
         const T *y = A.y ? A.y + r * A.y_stride + c0 : nullptr;
+        // f(|value|, record, counts) for every point, the last one also for the
+        // slots past the end
+        auto scan = [&](auto &&f) __attribute__((always_inline)) {
+            for (int p0 = tid; p0 < nc; p0 += PB * NT) {
+                T v[PB];
+                PointRec<T> pr[PB];
+#pragma unroll
+                for (int k = 0; k < PB; ++k) {
+                    const int p = min(p0 + k * NT, nc - 1);
+                    v[k] = y ? fabs(y[p]) : T(1);
+                    pr[k] = P[p];
+                }
+#pragma unroll
+                for (int k = 0; k < PB; ++k) f(v[k], pr[k], p0 + k * NT < nc);
+            }
+        };
         // largest |value|; a non-finite value or position (NaN x gives NaN e)
         // makes it infinite and the spectrum NaN
-        T vm = y ? T(0) : T(1);
-        for (int p0 = tid; p0 < nc; p0 += PB * NT) {
-            T v[PB], e[PB];
+        T vm = y ? T(0) : T(1), vs = T(0);  // largest, and (FP32) sum of the |values|
+        scan([&](T v, const PointRec<T> &pr, bool in) __attribute__((always_inline)) {
+            vm = fmax(vm, v <= kBig && fabs(pr.e) <= kBig ? v : T(INFINITY));
+            vs += in ? v : T(0);
+        });
 #pragma unroll
-            for (int k = 0; k < PB; ++k) {
-                const int p = min(p0 + k * NT, nc - 1);
-                v[k] = y ? fabs(y[p]) : T(1);
-                e[k] = fabs(P[p].e);
-            }
-#pragma unroll
-            for (int k = 0; k < PB; ++k)
-                vm = fmax(vm, v[k] <= kBig && e[k] <= kBig ? v[k] : T(INFINITY));
+        for (int o = 32; o > 0; o >>= 1) {
+            vm = fmax(vm, __shfl_xor(vm, o));
+            if constexpr (sizeof(T) == 4) vs += __shfl_xor(vs, o);
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) vm = fmax(vm, __shfl_xor(vm, o));
-        if ((tid & 63) == 0) vmax_sh[tid >> 6] = vm;
+        if ((tid & 63) == 0) {
+            vmax_sh[tid >> 6] = vm;
+            vsum_sh[tid >> 6] = vs;
+        }
         for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
             reinterpret_cast<uint4 *>(cuna_smem)[i] = make_uint4(0, 0, 0, 0);
         __syncthreads();
 #pragma unroll
         for (int w = 0; w < NT / 64; ++w) vm = fmax(vm, vmax_sh[w]);
         const bool finite = vm <= kBig;  // uniform
-        int sexp = 0;
-        const double bound = (double)vm * (double)cover * (double)A.wscale;
-        int eb = -kMaxExp;  // ceil(log2(bound))
-        if (bound > 0 && finite && frexp(bound, &eb) == 0.5) --eb;
-        sexp = min(max(FixedOf<T>::headroom_bits - eb, -kMaxExp), kMaxExp);
+        // the scale's exponent for cell sums within `bound`
+        auto exponent = [&](double bound) __attribute__((always_inline)) -> int {
+            int eb = -kMaxExp;  // ceil(log2(bound))
+            if (bound > 0 && finite && frexp(bound, &eb) == 0.5) --eb;
+            return min(max(FixedOf<T>::headroom_bits - eb, -kMaxExp), kMaxExp);
+        };
+        int sexp = exponent((double)vm * (double)cover * (double)A.wscale);
+        bool second = false;  // a second round (uniform)
+        if constexpr (sizeof(T) == 4) {
+            float mean = 0.0f;
+#pragma unroll
+            for (int w = 0; w < NT / 64; ++w) mean += vsum_sh[w];
+            mean *= A.wscale / (float)max(nc, 1);
+            if (finite && mean > 0.0f && ldexpf(mean, sexp) < kMeanUnits) {
+                // block sums in the grid's first cells (cleared above, cleared again
+                // below), in units of 2^(ev - q), rounded up: within 2^31 in all.
+                // Lanes count in four copies: points in order of position meet on one
+                // block.
+                constexpr int NBK = G >> 4, NW = (NTAPS + 14) / 16 + 1;
+                static_assert(NW <= NBK, "blocks that a window touches");
+                uint4 *const blocks = reinterpret_cast<uint4 *>(gu);
+                int ev = 0;
+                (void)frexpf(vm, &ev);
+                const int q = 30 - (32 - __clz(nc)), copy = tid & 3;
+                scan([&](float v, const PointRec<T> &pr, bool in) __attribute__((always_inline)) {
+                    if (in) atomicAdd(&gu[(pr.a >> 4) * 4 + copy], (U)ceilf(ldexpf(v, q - ev)));
+                });
+                __syncthreads();
+                unsigned most = 0;
+                for (int b = tid; b < NBK; b += NT) {
+                    unsigned sum = 0;
+#pragma unroll
+                    for (int i = 0; i < NW; ++i) {
+                        const uint4 u = blocks[(b + i) & (NBK - 1)];
+                        sum += u.x + u.y + u.z + u.w;
+                    }
+                    most = max(most, sum);
+                }
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) most = max(most, (unsigned)__shfl_xor((int)most, o));
+                if ((tid & 63) == 0) block_sh[tid >> 6] = most;
+                __syncthreads();
+                for (int b = tid; b < NBK; b += NT) blocks[b] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int w = 0; w < NT / 64; ++w) most = max(most, block_sh[w]);
+                sexp = max(sexp, exponent(ldexp((double)most * (double)A.wscale, ev - q)));
+                second = ldexpf(mean, sexp) < kMeanUnits;
+                __syncthreads();
+            }
+        }
         const T mul = (T)ldexp((double)A.wscale, sexp);
-        // dense curves: rests of at most 1/2, `cover` of them in a cell, within 2^30
-        const int lowbits = min(kDenseBits, 31 - (32 - __clz(cover - 1)));
+        // the second round: rests of at most 1/2, `cover` of them in a cell, within 2^30
+        const int lowbits = min(kRestBits, 31 - (32 - __clz(cover - 1)));
         const float lowmul = ldexpf(1.0f, lowbits);
         // one round over the points: each tap's integer, or (LOW) the scaled rest
         // of its rounding, to its cell.  Thread t takes spl consecutive points:
@@ -2247,10 +2318,8 @@ __global__ __launch_bounds__(NT) void k_adjoint_fused(AdjointArgs<T> A) {
         };
         if (finite) round(std::false_type{});
         fold();
-        bool dense = false;
         if constexpr (sizeof(T) == 4) {
-            dense = finite && cover > kDenseCover;  // uniform
-            if (dense) {
+            if (second) {
                 for (int i = tid; i < G; i += NT) hi[i] = (int)gu[i];
                 __syncthreads();
                 for (int i = tid; i < (int)((G + 2 * kBootHalo) * sizeof(T) / 16); i += NT)
@@ -2266,7 +2335,7 @@ __global__ __launch_bounds__(NT) void k_adjoint_fused(AdjointArgs<T> A) {
         }
         auto fetch = [&](int e, int) __attribute__((always_inline)) {
             const FixedPair<I> q = reinterpret_cast<const FixedPair<I> *>(gu)[e];
-            return dense ? z[e] : cmk((T)q.x, (T)q.y);
+            return second ? z[e] : cmk((T)q.x, (T)q.y);
         };
         fft_pass<T, 1, LG, 1, NT, 0, 0, decltype(fetch), true, NoHook, decltype(tw), MR>(
             z, tw, fetch, NoHook());

@@ -69,3 +69,28 @@ def test_large_spread_tiles(pts, kind):
     assert large.info().tile_log2 > 8
     e = [error(p.adjoint(y)[:rows], ref) for p in (large, small)]
     assert e[0] <= 1.1 * e[1], e
+
+
+@pytest.mark.parametrize("n,M,curves,pts", [
+    (1000, 1 << 11, 1, "uniform"), (1000, 1 << 11, 1, "clustered"), (200, 1 << 9, 4, "uniform"),
+    (4700, 1 << 14, 256, "uniform"), (4700, 1 << 14, 256, "clustered"),
+    (12_000, 1 << 14, 256, "uniform"), (12_000, 1 << 14, 256, "clustered")])
+@pytest.mark.parametrize("kind", ["even", "lognormal", "30", "100", "1000", "1e6"])
+def test_fused_adjoint(n, M, curves, pts, kind):
+    """One workgroup's FFT rounds near 2.1e-7 (2.6e-7 for dense clumps), and the rule
+    keeps the grid's rounding below 0.75e-7: together 2.7e-7, times a margin of 1.2.
+    One curve of the kind asked for, the rest short, so that the batch is fused."""
+    x, y = batch(pts, kind, n, 1, 1)
+    if curves > 1:
+        rng = np.random.default_rng(12)
+        fill = 100 * (curves - 1)
+        x = torch.cat([x, torch.from_numpy(rng.uniform(-0.5, 0.5, fill).astype(np.float32)).cuda()])
+        y = torch.cat([y, torch.from_numpy(rng.standard_normal(fill).astype(np.float32)).cuda()])
+    offs = np.concatenate([[0, n], n + 100 * np.arange(1, curves)]).astype(np.int32)
+    ref = reference(x, y, n, 1, M)
+    fused, tiles = (cu.NFFTPlan(x, M, offsets=offs, unfused=u) for u in (False, True))
+    got = fused.adjoint(y)
+    assert error(got[:1], ref) <= 3.2e-7
+    assert error(tiles.adjoint(y)[:1], ref) <= 3.2e-7  # and so have the tiles
+    # the same bits each time, whatever the order in which the rounds' atomics land
+    assert torch.equal(got, fused.adjoint(y))
