@@ -111,14 +111,14 @@ void warm_adjoint_fused(int lgN);
 template <typename T>
 void launch_curve_cover(const PointRec<T> *rec, const int *coff, int ncurves, int G, int ntaps,
                         int *cover, hipStream_t s);
-template <typename T>
 // zeroes the work-queue head and fills the queue's curve entries (with max |y|);
 // launched before every fused bootstrap
+template <typename T>
 void launch_boot_prepare(const T *y, const int *coff, const int *order, const int *cover_x,
                          const int *cover_2x, int ncurves, BootCurve *curves, int *counter,
                          hipStream_t s);
-template <typename T>
 // mode 0: spectra of y at x and of the window at 2x; 1: Lomb-Scargle power
+template <typename T>
 void launch_boot_fused(BootArgs<T> A, int lgN, int ntaps, int mode, hipStream_t s);
 
 // bytes of dynamic LDS a launch may use on gfx950

@@ -3,9 +3,9 @@
 //
 // Replaces fast_gridding / fast_gridding_bootstrap (src/gridding.cu:36-117),
 // which scatter every tap of every point with a global atomicAdd.  Here the
-// points of one x are binned once per plan by a stable two-pass counting sort
-// into buckets key = 3*tile + class (class 0: taps reach the previous tile,
-// 2: the next tile, 1: interior), ordered by anchor within a bucket.  One
+// points of one x are sorted once per plan by anchor (a stable radix sort, in one
+// launch for short curves), which orders them by the buckets key = 3*tile + class
+// (class 0: taps reach the previous tile, 2: the next tile, 1: interior).  One
 // workgroup owns one tile: it takes the points of its own bucket plus the
 // boundary classes of its two neighbours and accumulates the taps that land
 // in its tile in LDS, then writes the tile once with coalesced stores.  No

@@ -35,8 +35,9 @@ typedef struct cuna_nfft_plan_s *cuna_nfft_plan;
 
 /* plan flags */
 #define CUNA_PLAN_WINDOW2 0x1 /* also bin the points 2x (window transform at 2f) */
-#define CUNA_PLAN_UNFUSED 0x2 /* bootstrap through spread + batched FFT kernels instead of
-                                 the fused single-launch kernel (grids <= 2^15 cells) */
+#define CUNA_PLAN_UNFUSED 0x2 /* bootstrap and adjoint through spread + batched FFT kernels
+                                 instead of the fused single-launch kernels (grids <= 2^15
+                                 cells; the adjoint's for short curves) */
 #define CUNA_PLAN_GATHER 0x4  /* spread in gather form (each cell sums the points that
                                  reach it) instead of the default scatter with fixed-point
                                  integer LDS atomics; both are deterministic */
@@ -45,7 +46,9 @@ typedef struct {
     int mode;      /* CUNA_MODE_ACCURATE (default) or CUNA_MODE_COMPAT */
     int sigma;     /* accurate: oversampling, G = sigma*M, power of two >= 2 (default 2) */
     int m;         /* accurate: filter half-width, 2m taps, 2..16 (default 8 / 13) */
-    int tile_log2; /* spread tile of 2^tile_log2 cells; 0 = library default */
+    int tile_log2; /* spread tile of 2^tile_log2 cells; 0 = library default.  A size
+                      given here, or an FFT shape below, asks for the spread and the
+                      FFT as launches of their own, also where the default is one */
     int flags;     /* CUNA_PLAN_* */
     int fft_w;     /* FFT pass 1: columns per workgroup (1,2,4,8; 0 = library choice) */
     int fft_h;     /* FFT pass 2: rows (row pairs) per workgroup (1,2,4; 0 = library choice) */
@@ -143,6 +146,8 @@ int cuna_nfft_plan_info(cuna_nfft_plan plan, cuna_nfft_info *info);
  * events[1] the start and stop times of its spread kernel (taken by that
  * kernel's dispatch), events[2] between the two FFT passes (large grids
  * only) and events[3] after the last kernel, all on the execution stream.
+ * Where the adjoint is one launch, events[0] and events[1] are that launch's
+ * and events[2] follows it.
  * nevents = 0 clears them. */
 int cuna_nfft_set_profile_events(cuna_nfft_plan plan, hipEvent_t *events, int nevents);
 int cuna_nfft_plan_destroy(cuna_nfft_plan plan);
@@ -163,7 +168,8 @@ int cuna_nfft_autotune(const dTyp *x, int n, int M, double tol, const char *cach
  * cuna_stream_capture_end on `stream` (a created stream, not the null
  * stream) is recorded instead of run; cuna_graph_launch replays the sequence.
  * Run each captured call once beforehand so that its workspaces exist: a
- * capture allocates nothing.  The captured kernels use no memset nodes. */
+ * capture allocates nothing.  A plan keeps the memory that its captured calls
+ * use until it is destroyed, also where later calls need more.  The captured kernels use no memset nodes. */
 typedef struct cuna_graph_s *cuna_graph;
 int cuna_stream_capture_begin(hipStream_t stream);
 int cuna_stream_capture_end(hipStream_t stream, cuna_graph *graph);
