@@ -62,3 +62,20 @@ def test_adjoint_many(prec, M, curves, nrhs):
     many = plan.adjoint_many(y).reshape(curves, nrhs, M)
     for r in (0, nrhs - 1):
         assert torch.equal(many[:, r], plan.adjoint(y[r]))
+
+
+@pytest.mark.parametrize("prec,ng,rows", [("f", 1 << 15, 97), ("f", 1 << 15, 96), ("d", 1 << 14, 49),
+                                          ("d", 1 << 14, 48)])
+def test_compat_bootstrap_within_rounding(prec, ng, rows):
+    """Replicates choose the form by their number: the same ones in a call on the other
+    side of the line (3/8 and 3/16 of the CUs) within rounding, 1e-6 and 1e-14."""
+    rng = np.random.default_rng(rows)
+    n = 700
+    x = torch.from_numpy(rng.uniform(-0.5, 0.5, n)).to(RT[prec]).cuda()
+    y = torch.from_numpy(rng.standard_normal(n)).to(RT[prec]).cuda()
+    fp = cu.generate_filter_properties(x, n, ng)
+    many, few = (torch.empty((r, ng), dtype=CT[prec], device="cuda") for r in (rows, 5))
+    cu.cunfft_adjoint_raw_async_bootstrap(x, y, many, n, ng, rows, fp, seed=9)
+    cu.cunfft_adjoint_raw_async_bootstrap(x, y, few, n, ng, 5, fp, seed=9)
+    assert torch.linalg.norm(many[:5] - few) <= (1e-6 if prec == "f" else 1e-14) * torch.linalg.norm(few)
+    fp.free()
